@@ -127,9 +127,9 @@ static_assert((unsigned long long)kMaxK * 512ull < kOobOffset && kMaxK % 8 == 0,
 // Elements of a side-job array: its byte size must stay below the out-of-range offset the kernels use.
 constexpr long long kMaxSideElems = (long long)(kOobOffset / 16) * 8;
 
-// Validates a gemmrc problem.  *generic is set when it is well formed but outside what the tiled kernels take
-// (rows of A / B that are not multiples of 16 bytes, i.e. K % 8 != 0; operands not 16-byte or output not
-// 8-byte aligned; K beyond the descriptor range): such problems run on the plain kernel of aux_kernels.hip.
+// Validates a gemmrc problem.  *generic is set when it is well formed but outside what the tiled kernels take (K
+// shorter than one 16-byte chunk, or beyond the descriptor range): such problems run on the plain kernel of
+// aux_kernels.hip.
 int check_problem(const void* A, const void* B, const void* C, int M, int N, int K, int dtype, bool* generic) {
   *generic = false;
   if (M < 0 || N < 0 || K < 0) return fail(BEAM_ERR_INVALID, "negative dimension (M=%d N=%d K=%d)", M, N, K);
@@ -140,8 +140,14 @@ int check_problem(const void* A, const void* B, const void* C, int M, int N, int
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 1) return fail(BEAM_ERR_INVALID, "A, B and C must be aligned to their 16-bit elements");
   if ((size_t)M * (size_t)N >= ((size_t)1 << 40)) return fail(BEAM_ERR_UNSUPPORTED, "M*N too large");
   if ((M + 63) / 64 > 65535) return fail(BEAM_ERR_UNSUPPORTED, "M=%d too large", M);
-  *generic = K > kMaxK || K % 8 != 0 || ((((uintptr_t)A | (uintptr_t)B) & 15) != 0) || (((uintptr_t)C & 7) != 0);
+  *generic = K > kMaxK || (K > 0 && K < 8);
   return BEAM_OK;
+}
+
+// Rows of A or B that do not start on 16 bytes, or C not on 8: what the kernels take at a lower rate (gemm_kernel.h:
+// load_short_tile), and what may call split-K without a workspace.
+bool rows_unaligned(const void* A, const void* B, const void* C, int K) {
+  return K % 8 != 0 || (((uintptr_t)A | (uintptr_t)B) & 15) != 0 || ((uintptr_t)C & 7) != 0;
 }
 
 // Slices for `tiles` output tiles when the caller leaves the choice to the library: as many as make
@@ -504,8 +510,8 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     BEAM_HIP(launch_zero_u16(C, (size_t)M * N, st));
     return BEAM_OK;
   }
-  // rows of B ([K][N]) that are not multiples of 16 bytes, or more than a descriptor spans: the plain kernel
-  if (generic || N % 8 != 0 || N > (1 << 24)) {
+  // rows of B ([K][N]) shorter than a chunk of 16 bytes, or more than a descriptor spans: the plain kernel
+  if (generic || N < 8 || N > (N % 8 != 0 ? 1 << 23 : 1 << 24)) {
     BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, true, false, st));
     return BEAM_OK;
   }
@@ -673,7 +679,7 @@ int beam_splitk_effective(int M, int N, int K, const beam_tile_cfg* cfg, int spl
   beam_tile_cfg c;
   const KernelSet* ks;
   if (M <= 0 || N <= 0 || K < 0) return 1;
-  if (K % 8 != 0 || K > kMaxK) return 1;  // the plain kernel: no slices
+  if ((K > 0 && K < 8) || K > kMaxK) return 1;  // the plain kernel: no slices
   if (resolve_cfg(cfg, M, N, K, &c, &ks, split_k > 0 ? split_k : 0)) return -1;
   return effective_split(M, N, K, c, split_k);
 }
@@ -714,14 +720,16 @@ int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int 
     BEAM_HIP(launch_zero_u16(C, (size_t)M * N, st));
     return BEAM_OK;
   }
-  if (generic) {  // one pass of the plain kernel, no slices (beam_splitk_effective says 1 for K % 8 != 0)
+  if (generic) {  // one pass of the plain kernel, no slices (beam_splitk_effective says 1)
     BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, false, false, st));
     return BEAM_OK;
   }
   beam_tile_cfg c;
   const KernelSet* ks;
   if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, split_k > 0 ? split_k : 0))) return rc;
-  const int s = effective_split(M, N, K, c, split_k);
+  int s = effective_split(M, N, K, c, split_k);
+  // Operands whose rows are not 16-byte aligned may be given without room for slices (they need none: one pass).
+  if (rows_unaligned(A, B, C, K) && (!ws || ws_bytes < splitk_partial_bytes(M, N, s))) s = 1;
   if (split_k <= 0 && g_verbose.load(std::memory_order_relaxed)) log_split_choice_once(M, N, K, dtype, c, s);
   if (s == 1) {  // nothing to reduce: the plain kernel writes C directly
     GemmParams p = base_params(A, B, M, N, K, c);
@@ -797,7 +805,7 @@ int beam_gemmrc_splitk_noalloc(const void* A, const void* B, void* C, int M, int
   if (rc) return rc;
   bool generic = false;
   if ((rc = check_problem(A, B, C, M, N, K, dtype, &generic))) return rc;
-  if (M > 0 && N > 0 && K > 0 && !generic) {  // (the plain kernel, one pass, needs no workspace)
+  if (M > 0 && N > 0 && K > 0 && !generic && !rows_unaligned(A, B, C, K)) {  // (those run without slices if need be)
     const int s = beam_splitk_effective(M, N, K, cfg, split_k);
     if (s < 0) return BEAM_ERR_UNSUPPORTED;  // the message is already set
     const size_t need = s > 1 ? splitk_partial_bytes(M, N, s) : 0;
@@ -919,8 +927,9 @@ static int ln_resolve_cfg(const beam_tile_cfg* cfg, int M, int N, int K, int mod
 
 // What a GEMM+LayerNorm call does and the workspace it needs: one function, so that the entry point and the
 // workspace queries cannot disagree.
-//   plain     the problem is outside what the tiled kernels take (K % 8, K beyond a descriptor, operands aligned to
-//             an element only): plain GEMM into fp32 X, then a row-wise LayerNorm
+//   plain     the problem is outside what the tiled kernels take (K below 8 or beyond a descriptor, gamma or beta not
+//             8-byte aligned): plain GEMM into fp32 X, then a row-wise LayerNorm.  (Also for the one combination
+//             that has always been computed and never refused: BEAM_LN_FUSED where it does not apply, K % 8 != 0.)
 //   capturing the stream is being captured: AUTO then means two passes (a replayed graph may share the device with
 //             other work, which the fused kernel's residency argument does not cover); an explicit FUSED is honoured
 //   wide_io   Y, gamma and beta are 16-byte aligned (the 4-wavefront kernel's vector accesses)
@@ -943,6 +952,11 @@ static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool
   int rc = ln_resolve_cfg(cfg, M, N, K, mode, &out->c, &out->ks);
   if (rc) return rc;
   beam_tile_cfg& c = out->c;
+  if (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N) && K % 8 != 0) {
+    out->kind = LnPlan::kPlain;
+    out->need = ln_generic_need(M, N);
+    return BEAM_OK;
+  }
   if (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N))
     return fail(BEAM_ERR_UNSUPPORTED, "fused LayerNorm: needs a device of %d CUs and at most 64 column tiles (N=%d, block_n=%d, %d CUs)",
                 kNumXcd * 32, N, c.block_n, g_dev.cus);
@@ -967,7 +981,7 @@ static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool
 // beam_gemmrc_ln_checked), which also covers the plain path.
 size_t beam_gemmrc_ln_workspace_bytes_for(int M, int N, int K, const beam_tile_cfg* cfg, int mode) {
   if (M <= 0 || N <= 0 || K < 0) return 0;
-  if (K % 8 != 0 || K > kMaxK) return ln_generic_need(M, N);
+  if ((K > 0 && K < 8) || K > kMaxK) return ln_generic_need(M, N);
   (void)beam_init();  // AUTO depends on the device
   LnPlan eager, captured;
   if (ln_plan(M, N, K, cfg, mode, false, false, true, &eager)) return 0;
@@ -1005,7 +1019,7 @@ size_t beam_gemmrc_ln_workspace_bytes(int M, int N, const beam_tile_cfg* cfg) {
 
 size_t beam_dbg_ln_plan_bytes(int M, int N, int K, const beam_tile_cfg* cfg, int mode, int plain, int capturing, int wide_io) {
   LnPlan plan;
-  if (M <= 0 || N <= 0 || K < 0 || ln_plan(M, N, K, cfg, mode, plain != 0 || K % 8 != 0 || K > kMaxK, capturing != 0, wide_io != 0, &plan)) return 0;
+  if (M <= 0 || N <= 0 || K < 0 || ln_plan(M, N, K, cfg, mode, plain != 0 || (K > 0 && K < 8) || K > kMaxK, capturing != 0, wide_io != 0, &plan)) return 0;
   return plan.need;
 }
 

@@ -49,6 +49,7 @@
 namespace beam {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_at_4 __attribute__((ext_vector_type(4), aligned(4)));  // at any float's address
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -497,8 +498,15 @@ struct GemmTile {
     int klen = K - kb;
     if (klen > p.k_slice) klen = p.k_slice;
     if (klen < 0) klen = 0;
-    const int kt_full = klen / kBK;
-    const int k_tail = klen - kt_full * kBK;         // multiple of 8 (host guarantees K % 8 == 0)
+    // [K][N] with rows of B that are not whole 16-byte chunks: the last K tile is treated as a short one even if it
+    // is whole, because the last row's last chunk must not be fetched as it stands (see load_short_tile).
+    const bool n_odd = B_KMAJOR && (N & 7) != 0;
+    int kt_full = klen / kBK;
+    int k_tail = klen - kt_full * kBK;
+    if (n_odd && k_tail == 0 && kt_full > 0) {
+      k_tail = kBK;
+      --kt_full;
+    }
     const int n_tiles = kt_full + (k_tail ? 1 : 0);  // the short tile, if any, is tile 0
 
     // Buffer descriptors cover exactly the rows of this tile that exist and the K range of
@@ -566,7 +574,9 @@ struct GemmTile {
         const int koff = tile_koff(t);
         int rows = klen - koff;
         if (rows > kBK) rows = kBK;
-        const unsigned bytes = (t < n_tiles && rows > 0) ? ((unsigned)(rows - 1) * N + rows_b) * 2u : 0u;
+        // (n_odd: another row of at least 8 elements follows every tile fetched here, so its last row may be read to a
+        // whole chunk; the range check works on whole dwords and would cut an odd last column off)
+        const unsigned bytes = (t < n_tiles && rows > 0) ? ((unsigned)(rows - 1) * N + rows_b + (n_odd ? 7 : 0)) * 2u : 0u;
         const __amdgpu_buffer_rsrc_t r = make_rsrc(b_base + (size_t)koff * N, bytes);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16,
                                                  (int)voff_b[i], 0, 0, 0);
@@ -576,36 +586,80 @@ struct GemmTile {
                                                  (int)voff_b[i], tile_koff(t) * 2, 0, 0);
       }
     };
-    // The short tile goes through registers so that chunks at or past `kvalid` are zero-filled.
-    // (A K-major B needs none of this: its rows past the end of K are out of range by themselves.)
+    // The short tile goes through registers: chunks at or past `kvalid` are zero-filled, and a chunk that K ends
+    // inside (K % 8 != 0) is fetched as the 16 bytes that end where its row ends, then shifted down -- one in-bounds
+    // load per chunk whatever K is, never a byte past a row (the host guarantees K >= 8).  Nothing here or in the
+    // LDS-direct loads needs more alignment than the element's: the memory path takes a 16-byte access at any byte
+    // address.  What that costs is rate: rows that do not start on a 128-byte line fill LDS at 57 (odd K) to 68 GB/s
+    // per CU (K % 8 == 0) against 122 for rows of whole lines (a fill loop with nothing else in it).  3001 x 5001 x 2001
+    // bf16: 58 us, against 1594 on the plain kernel that such rows ran on before; 3000 x 5000 x 2000 53.5 against 54.3
+    // for the one trip to memory.
+    // (A K-major B with whole chunks needs none of this: its rows past the end of K are out of range by themselves.
+    // With N % 8 != 0 the chunk that the very last row of B ends inside is fetched the same way.)
     const bool loader = LDW == NW || wave < LDW;
-    auto fill_short_tile = [&](int kvalid) __attribute__((always_inline)) {
-      if (!loader) return;
-      const int koff = tile_koff(0);
-      i32x4 ra[LA], rb[LB];
+    struct ShortTile {
+      i32x4 a[LA], b[LB];
+    };
+    // v >> bits for a uniform 0 < bits < 128
+    auto shift_down = [](i32x4 v, int bits) __attribute__((always_inline)) -> i32x4 {
+      typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+      const u64x2 w = __builtin_bit_cast(u64x2, v);
+      u64x2 o;
+      o[0] = bits >= 64 ? w[1] >> (bits - 64) : (w[0] >> bits) | (w[1] << (64 - bits));
+      o[1] = bits >= 64 ? 0ull : w[1] >> bits;
+      return __builtin_bit_cast(i32x4, o);
+    };
+    auto load_short_tile = [&](ShortTile& st, int kvalid) __attribute__((always_inline)) {
+      const int koff = kb + tile_koff(0);  // first K element of the tile, from the row's start
+      const int kend = koff + kvalid;      // the row's end in this slice
+      const int r = kvalid & 7;            // elements of the chunk that K ends inside
+      // rows of A or B ([N][K]) from their own start, so that the shifted chunk's offset is never negative
+      auto load_rows = [&](const void* base, int rows, auto n_tag, i32x4* regs) __attribute__((always_inline)) {
+        constexpr int L = decltype(n_tag)::value;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, ((unsigned)(rows - 1) * (unsigned)K + (unsigned)kend) * 2u);
 #pragma unroll
-      for (int i = 0; i < LA; ++i) {
-        const int q = i * NTL + tid;
-        const int chunk = (q & 7) ^ swizzle_of_row(q >> 3);
-        const unsigned off = (chunk * 8 < kvalid) ? voff_a[i] + (unsigned)koff * 2u : kOobOffset;
-        ra[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)off, 0, 0);
-      }
-      if (!B_KMAJOR) {
+        for (int i = 0; i < L; ++i) {
+          const int q = i * NTL + tid;
+          const int c8 = ((q & 7) ^ swizzle_of_row(q >> 3)) * 8;
+          const int at = c8 + 8 <= kvalid ? koff + c8 : kend - 8;
+          const unsigned off = c8 < kvalid ? ((unsigned)(q >> 3) * (unsigned)K + (unsigned)at) * 2u : kOobOffset;
+          regs[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
+        }
+        if (r != 0) {  // (uniform)
+#pragma unroll
+          for (int i = 0; i < L; ++i) {
+            const int q = i * NTL + tid;
+            const int c8 = ((q & 7) ^ swizzle_of_row(q >> 3)) * 8;
+            if (c8 + 8 > kvalid) regs[i] = shift_down(regs[i], 128 - 16 * r);
+          }
+        }
+      };
+      load_rows((const T*)p.A + (size_t)row0 * K, rows_a, std::integral_constant<int, LA>{}, st.a);
+      if constexpr (!B_KMAJOR) {
+        load_rows((const T*)p.B + (size_t)col0 * K, rows_b, std::integral_constant<int, LB>{}, st.b);
+      } else if (n_odd) {
+        constexpr int CPR = BN / 8;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc((const T*)p.B + (size_t)koff * N, (unsigned)kvalid * (unsigned)N * 2u);
+        const int nr = N & 7;
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
           const int q = i * NTL + tid;
-          const int chunk = (q & 7) ^ swizzle_of_row(q >> 3);
-          const unsigned off = (chunk * 8 < kvalid) ? voff_b[i] + (unsigned)koff * 2u : kOobOffset;
-          rb[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, (int)off, 0, 0);
+          const int k = q / CPR, n = col0 + ((q % CPR) ^ kmajor_swizzle(k, BN)) * 8;
+          const bool cut = k == kvalid - 1 && n + 8 > N;  // the matrix ends inside this chunk, or in front of it
+          const unsigned off = k < kvalid && !(cut && n >= N) ? ((unsigned)k * (unsigned)N + (unsigned)(cut ? N - 8 : n)) * 2u : kOobOffset;
+          st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
+          if (cut) st.b[i] = shift_down(st.b[i], 128 - 16 * nr);
         }
       }
+    };
+    auto store_short_tile = [&](const ShortTile& st) __attribute__((always_inline)) {
       char* sa = smem + tid * 16;
       char* sb = smem + B_REGION + tid * 16;
 #pragma unroll
-      for (int i = 0; i < LA; ++i) *(i32x4*)(sa + i * (NTL * 16)) = ra[i];
-      if (!B_KMAJOR) {
+      for (int i = 0; i < LA; ++i) *(i32x4*)(sa + i * (NTL * 16)) = st.a[i];
+      if (!B_KMAJOR || n_odd) {
 #pragma unroll
-        for (int i = 0; i < LB; ++i) *(i32x4*)(sb + i * (NTL * 16)) = rb[i];
+        for (int i = 0; i < LB; ++i) *(i32x4*)(sb + i * (NTL * 16)) = st.b[i];
       }
     };
 
@@ -859,20 +913,34 @@ struct GemmTile {
     };
 
     // Prologue: A tiles 0 .. AST-2 and B tiles 0 .. BST-2, oldest first (tile 0 is what the first
-    // wait of the loop is about).  A short tile 0 goes through registers instead.
+    // wait of the loop is about).  A short tile 0 goes through registers instead; it is written to LDS when the
+    // other tiles are on their way, so that one trip to memory covers all of them.
     auto issue_prologue = [&]() __attribute__((always_inline)) {
-      if (k_tail) fill_short_tile(k_tail);
+      const bool short_b = !B_KMAJOR || n_odd;  // the short tile's B goes through registers as well
+      auto fills = [&](auto short_tag) __attribute__((always_inline)) {
+        constexpr bool SHORT = decltype(short_tag)::value;
 #pragma unroll
-      for (int s = 0; s < (loader ? AST - 1 : 0); ++s) {
-        if (!(s == 0 && k_tail)) {
+        for (int s = 0; s < (loader ? AST - 1 : 0); ++s) {
+          if (!(s == 0 && SHORT)) {
 #pragma unroll
-          for (int i = 0; i < LA; ++i) load_a(i, s);
+            for (int i = 0; i < LA; ++i) load_a(i, s);
+          }
+          if (s < BST - 1 && !(s == 0 && SHORT && short_b)) {
+#pragma unroll
+            for (int i = 0; i < LB; ++i) load_b(i, s);
+          }
         }
-        if (s < BST - 1 && (B_KMAJOR || !(s == 0 && k_tail))) {
-#pragma unroll
-          for (int i = 0; i < LB; ++i) load_b(i, s);
+      };
+      if constexpr (!LOOP) {  // (no short tile there: the host sees to it; its registers would not fit beside the accumulators)
+        if (k_tail && loader) {
+          ShortTile st;
+          load_short_tile(st, k_tail);
+          fills(std::true_type{});
+          store_short_tile(st);
+          return;
         }
       }
+      fills(std::false_type{});
     };
     using W16 = std::integral_constant<int, 16>;
     using W8 = std::integral_constant<int, 8>;
@@ -1066,7 +1134,6 @@ struct GemmTile {
       constexpr int RPI = 64 / LPR;     // rows per store instruction
       auto chunk_xor = [](int r) { return RB == 64 ? (r >> 1) & 3 : r & 7; };
       char* stage = smem + RESERVED + wave * (FMH * 16 * RB);
-      const bool wide_ok = (N % 8) == 0 && ((size_t)C & 15) == 0;
       const int srow = lane / LPR, schunk = lane % LPR;
       const int wr = lane & 15, wg = lane >> 4;  // writer: row of the block, column group
       const int w_off = wr * RB + (((wg & 1) ^ (wr >> 3)) << 3);
@@ -1088,11 +1155,8 @@ struct GemmTile {
           const int m = row0 + wm * TM + hf * FMH * 16 + r;
           if (m < M) {
             T* dst = C + (size_t)m * N + n_st;
-            if (wide_ok && n_st + 7 < N) {
+            if (n_st + 7 < N) {  // (at any element's address)
               store_through_16(dst, __builtin_bit_cast(i32x4, v));
-            } else if (vec_ok && n_st + 7 < N) {  // C only 8-byte aligned, or N % 8 == 4
-              *(vec4*)dst = vec4{v[0], v[1], v[2], v[3]};
-              *(vec4*)(dst + 4) = vec4{v[4], v[5], v[6], v[7]};
             } else {
 #pragma unroll
               for (int e = 0; e < 8; ++e)
@@ -1347,8 +1411,8 @@ struct GemmTile {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
           const int n = n_base + j * 16;
-          if (vec_ok && n + 3 < N) {
-            *(f32x4*)(wrow + n) = acc[i][j];
+          if (n + 3 < N) {
+            *(f32x4_at_4*)(wrow + n) = acc[i][j];
           } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)

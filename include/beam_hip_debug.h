@@ -59,8 +59,8 @@ int beam_dbg_lds_offset(int row, int chunk);
 /* Byte offset of element (k, n), n a multiple of 4, inside a K-major LDS stage of block_n columns
  * (B stored [K][N], beam_matmul_nn). */
 int beam_dbg_kmajor_lds_offset(int k, int n, int block_n);
-/* Workspace bytes beam_gemmrc_ln_ex(M, N, K, cfg, mode) insists on, by the path the call takes: `plain` (operands
- * aligned to an element only; K % 8 != 0 implies it), `capturing` (the stream is being captured), `wide_io` (Y, gamma
+/* Workspace bytes beam_gemmrc_ln_ex(M, N, K, cfg, mode) insists on, by the path the call takes: `plain` (gamma or
+ * beta off an 8-byte boundary; 0 < K < 8 implies it), `capturing` (the stream is being captured), `wide_io` (Y, gamma
  * and beta 16-byte aligned).  The entry point computes its requirement with the same function; the workspace queries
  * are tested against it.  0 on error. */
 size_t beam_dbg_ln_plan_bytes(int M, int N, int K, const beam_tile_cfg* cfg, int mode, int plain, int capturing, int wide_io);

@@ -1,0 +1,116 @@
+"""Rows that do not start on 16 bytes: K not a multiple of 8, [K][N] with N not a multiple of 8, operands and outputs
+at any element's address, on the tiled kernels.  Every operand lies inside a larger buffer of NaNs: an element read
+from beside a row, or beyond a matrix, that reached an output would show.  Every output lies inside a larger buffer
+too, which must stay as it was around it."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from test_gpu_edges import close_enough
+from test_gpu_gemm import F16, BF16, all_configs, assert_close
+from test_gpu_ln import check_ln, make_ln_inputs
+
+pytestmark = pytest.mark.gpu
+
+PAD = 16
+NAN = 0xFFFF
+
+
+class Embedded:
+    """`bits` on the device, `off` elements past a 16-byte boundary, NaNs (or a guard pattern) in front and behind."""
+
+    def __init__(self, beamc, shape, dtype, off, bits=None):
+        self.beamc, self.shape, self.n, self.off = beamc, shape, int(np.prod(shape)), off
+        host = np.full(self.n + 2 * PAD, NAN, np.uint16)
+        if bits is not None:
+            host[off:off + self.n] = bits.ravel()
+        self.buf = beamc.DeviceArray.from_numpy(host, dtype)
+        self.ptr = self.buf.ptr + 2 * off
+
+    def result(self):
+        out = self.buf.to_numpy()
+        assert (out[:self.off] == NAN).all() and (out[self.off + self.n:] == NAN).all(), "written outside the output"
+        return out[self.off:self.off + self.n].reshape(self.shape)
+
+
+def run(beamc, call, a, b, shape, dtype, offs):
+    da, db, c = Embedded(beamc, a.shape, dtype, offs[0], a), Embedded(beamc, b.shape, dtype, offs[1], b), Embedded(beamc, shape, dtype, offs[2])
+    beamc._check(call(da.ptr, db.ptr, c.ptr))
+    out = c.result()
+    for x in (da, db, c):
+        x.buf.free()
+    return out
+
+
+# K around one chunk of 8, one K tile of 64 and several of them; M and N around the smallest tile
+@pytest.mark.parametrize("K", [8, 9, 15, 57, 63, 65, 71, 127, 129, 1001])
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_any_k(gpu, beamc, oracle, K, dtype):
+    L = beamc.lib
+    for M, N, offs in ((65, 63, (0, 0, 0)), (1, 9, (1, 3, 5)), (130, 257, (7, 2, 1))):
+        a, b = beamc.host_uniform((M, K), dtype, 71, 0), beamc.host_uniform((N, K), dtype, 71, 1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offs)
+        close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"gemmrc {(M, N, K)} at {offs}")
+        # slices whose last one ends in a short tile, with and without room for them
+        for slices, room in ((3, True), (3, False)):
+            ws = beamc.DeviceArray((max(L.beam_splitk_workspace_bytes(M, N, 3), 256),), itemsize=1)
+            out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, dtype, None, slices, ws.ptr if room else None,
+                                                                     ws.nbytes if room else 0, None), a, b, (M, N), dtype,
+                      offs if K % 8 or room else (1, 0, 0))
+            ws.free()
+            close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"split-K {(M, N, K)} room {room}")
+
+
+# N around one chunk, around the tiles' widths, and a last K tile that is whole (64, 128) or short
+@pytest.mark.parametrize("N", [8, 9, 63, 65, 127, 129, 255, 257, 1001])
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_any_n_kmajor(gpu, beamc, oracle, N, dtype):
+    L = beamc.lib
+    for M, K, offs in ((65, 64, (0, 0, 0)), (3, 9, (1, 1, 1)), (130, 128, (0, 5, 3)), (129, 331, (0, 0, 0))):
+        a, b = beamc.host_uniform((M, K), dtype, 72, 0), beamc.host_uniform((K, N), dtype, 72, 1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offs)
+        close_enough(oracle, out, oracle.matmul_nn(a, b, dtype), K, dtype, f"matmul {(M, N, K)} at {offs}")
+
+
+def test_every_tile(gpu, beamc, oracle):
+    """Every compiled tile and LDS depth, both layouts: several tiles each way, a short K tile behind several whole ones."""
+    M, N, K = 515, 773, 459
+    L = beamc.lib
+    a, b, bt = beamc.host_uniform((M, K), F16, 73, 0), beamc.host_uniform((N, K), F16, 73, 1), beamc.host_uniform((K, N), F16, 73, 1)
+    ref, ref_nn = oracle.gemmrc(a, b, F16), oracle.matmul_nn(a, bt, F16)
+    for cfg in all_configs(beamc):
+        c = cfg.to_c()
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, F16, ctypes.byref(c), None), a, b, (M, N), F16, (0, 3, 1))
+        assert_close(oracle, out, ref, K, F16, f"gemmrc {cfg.name}")
+        out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, ctypes.byref(c), None), a, bt, (M, N), F16, (0, 3, 1))
+        assert_close(oracle, out, ref_nn, K, F16, f"matmul {cfg.name}")
+
+
+# the persistent kernels: more tiles than CUs, K a multiple of 64, operands off a 16-byte boundary
+@pytest.mark.parametrize("wave_n", [64, 128])
+def test_walking_kernels_at_any_address(gpu, beamc, oracle, wave_n):
+    M, N, K = 4200, 4200, 192
+    L = beamc.lib
+    a, b = beamc.host_uniform((M, K), F16, 74, 0), beamc.host_uniform((N, K), F16, 74, 1)
+    c = beamc.TileConfig(256, 256, 128, wave_n).to_c()
+    out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, F16, ctypes.byref(c), None), a, b, (M, N), F16, (1, 3, 0))
+    assert_close(oracle, out, oracle.gemmrc(a, b, F16), K, F16, f"256x256, wavefronts 128x{wave_n}")
+
+
+@pytest.mark.parametrize("shape", [(65, 63, 9), (130, 257, 71), (33, 1001, 331), (300, 515, 129)])
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_layer_norm(gpu, beamc, oracle, shape, dtype):
+    M, N, K = shape
+    L = beamc.lib
+    a, b, g, bt = make_ln_inputs(beamc, M, N, K, dtype, 75)
+    ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, dtype)
+    dg, dbt = beamc.DeviceArray.from_numpy(g, dtype), beamc.DeviceArray.from_numpy(bt, dtype)
+    for mode in (beamc.LN_AUTO, beamc.LN_TWOPASS):
+        ws = beamc.DeviceArray((L.beam_gemmrc_ln_workspace_bytes_for(M, N, K, None, mode),), itemsize=1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_ln_ex(pa, pb, dg.ptr, dbt.ptr, 1e-5, pc, M, N, K, dtype, None, mode, ws.ptr,
+                                                                ws.nbytes, None), a, b, (M, N), dtype, (1, 0, 3))
+        check_ln(oracle, out, ref, dtype, f"LayerNorm {shape} mode {mode}")
+        ws.free()
+    dg.free()
+    dbt.free()
