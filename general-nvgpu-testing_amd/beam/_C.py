@@ -12,6 +12,7 @@ code of the library becomes a BeamError.
 from __future__ import annotations
 
 import ctypes
+import math
 import os
 import sys
 from dataclasses import dataclass
@@ -145,6 +146,27 @@ def _load() -> ctypes.CDLL:
 _TORCH_FIRST = False
 lib = _load()
 
+# What the operators need of torch, looked up once.  torch.cuda.current_stream() builds a Stream object after a walk
+# through the device index' conversions (2.8 us on the machine measured, three times per call before: 10.6 of a call's
+# 14.6 us); the raw handle of the current device's current stream is what a launch takes, and costs 0.1 us: a call of
+# gemmrc returns after 5.9 us, 4.3 of them in the library's launch.
+if _TORCH_FIRST:
+    import torch as _torch
+    _Tensor = _torch.Tensor
+    _TORCH_DTYPES = {_torch.float16: F16, _torch.bfloat16: BF16}
+    _raw_stream = getattr(_torch._C, "_cuda_getCurrentRawStream", None)
+    _raw_device = getattr(_torch._C, "_cuda_getDevice", None)
+else:
+    _torch = _Tensor = _raw_stream = _raw_device = None
+    _TORCH_DTYPES = {}
+
+
+def _torch_stream() -> int:
+    """Handle of torch's current stream on its current device."""
+    if _raw_stream is not None and _raw_device is not None:
+        return _raw_stream(_raw_device())
+    return _torch.cuda.current_stream().cuda_stream
+
 
 def _check(status: int) -> None:
     if status != 0:
@@ -252,49 +274,50 @@ class DeviceArray:
 
 
 def _is_torch(x) -> bool:
-    return type(x).__module__.split(".")[0] == "torch"
+    return (_Tensor is not None and isinstance(x, _Tensor)) or type(x).__module__.split(".")[0] == "torch"
 
 
 def _describe(x):
-    """(pointer, shape, dtype code, stream handle) of a torch tensor or DeviceArray."""
-    if isinstance(x, DeviceArray):
-        return x.ptr, x.shape, x.dtype, None
-    if _is_torch(x):
-        if not _TORCH_FIRST:
-            raise BeamError(1, "torch tensors need `import torch` before `import beam` (one HIP runtime per "
-                               "process); use beam.DeviceArray otherwise")
-        import torch
+    """(pointer, shape, dtype code) of a torch tensor or DeviceArray."""
+    if _Tensor is not None and isinstance(x, _Tensor):
+        d = _TORCH_DTYPES.get(x.dtype)
+        if d is not None and x.is_cuda and x.is_contiguous():
+            return x.data_ptr(), x.shape, d
         if not x.is_cuda:
             raise BeamError(1, "tensor is not on the GPU")
         if not x.is_contiguous():
             raise BeamError(1, "tensor is not contiguous")
-        if x.dtype == torch.float16:
-            d = F16
-        elif x.dtype == torch.bfloat16:
-            d = BF16
-        else:
-            raise BeamError(2, f"unsupported tensor type {x.dtype}")
-        return x.data_ptr(), tuple(x.shape), d, torch.cuda.current_stream().cuda_stream
+        raise BeamError(2, f"unsupported tensor type {x.dtype}")
+    if isinstance(x, DeviceArray):
+        return x.ptr, x.shape, x.dtype
+    if _is_torch(x):
+        raise BeamError(1, "torch tensors need `import torch` before `import beam` (one HIP runtime per "
+                           "process); use beam.DeviceArray otherwise")
     raise TypeError(f"expected a torch CUDA tensor or beam.DeviceArray, got {type(x)!r}")
+
+
+def _stream_of(x):
+    """What a launch on x goes to: torch's current stream for a tensor, the default stream for a DeviceArray."""
+    return _torch_stream() if _Tensor is not None and isinstance(x, _Tensor) else None
 
 
 def _problem(a, b, c):
     """Shape conventions of cuda/cutlass_kernels/main.cc:25-35: M=a.size(0), N=b.size(0),
     K=a.size(1); a.size(1)==b.size(1), c is [M, N]; all three of one 16-bit dtype."""
-    pa, sa, da, st = _describe(a)
-    pb, sb, db, _ = _describe(b)
-    pc, sc, dc, _ = _describe(c)
+    pa, sa, da = _describe(a)
+    pb, sb, db = _describe(b)
+    pc, sc, dc = _describe(c)
     if len(sa) != 2 or len(sb) != 2 or len(sc) != 2:
         raise BeamError(1, "a, b, c must be 2-D")
     M, K = sa
-    N = sb[0]
-    if sb[1] != K:
-        raise BeamError(1, f"a.size(1)={K} != b.size(1)={sb[1]}")
+    N, kb = sb
+    if kb != K:
+        raise BeamError(1, f"a.size(1)={K} != b.size(1)={kb}")
     if sc != (M, N):
-        raise BeamError(1, f"c has shape {sc}, expected {(M, N)}")
+        raise BeamError(1, f"c has shape {tuple(sc)}, expected {(M, N)}")
     if not (da == db == dc):
         raise BeamError(2, "a, b, c must share one dtype (fp16 or bf16)")
-    return pa, pb, pc, M, N, K, da, st
+    return pa, pb, pc, M, N, K, da, _stream_of(a)
 
 
 def _cfg_from_shapes(shape_threadblock, shape_warp, pipeline=0, group_m=0) -> _TileCfg:
@@ -412,8 +435,8 @@ def gemmrc_ln(a, b, c, gamma, beta, eps: float = 1e-5, config: Optional[TileConf
     an explicit LN_FUSED raises BeamError.  check=False launches and returns at once, like the other operators: the
     rows concerned are NaN if that ever happens, and gemmrc_ln_timed_out() tells."""
     pa, pb, pc, M, N, K, d, st = _problem(a, b, c)
-    pg, sg, dg, _ = _describe(gamma)
-    pbt, sbt, dbt, _ = _describe(beta)
+    pg, sg, dg = _describe(gamma)
+    pbt, sbt, dbt = _describe(beta)
     if tuple(sg) != (N,) or tuple(sbt) != (N,) or dg != d or dbt != d:
         raise BeamError(1, "gamma and beta must be [N] of the same dtype as a, b, c")
     cfg = config.to_c() if config is not None else None
@@ -448,8 +471,8 @@ def gemmrc_ln_timed_out() -> bool:
 def matmul(a, b, c=None, config: Optional[TileConfig] = None):
     """c = a @ b with a [M, K] and b [K, N], both row-major; returns c (allocated like the inputs when
     not given).  Reference: matmul(a, b) of python/beam/triton_kernels/gemm.py:78-99."""
-    pa, sa, da, st = _describe(a)
-    pb, sb, db, _ = _describe(b)
+    pa, sa, da = _describe(a)
+    pb, sb, db = _describe(b)
     if len(sa) != 2 or len(sb) != 2 or sa[1] != sb[0]:
         raise BeamError(1, "Incompatible dimensions")
     if da != db:
@@ -458,27 +481,26 @@ def matmul(a, b, c=None, config: Optional[TileConfig] = None):
     N = sb[1]
     if c is None:
         if _is_torch(a):
-            import torch
-            c = torch.empty((M, N), device=a.device, dtype=a.dtype)
+            c = _torch.empty((M, N), device=a.device, dtype=a.dtype)
         else:
             c = DeviceArray((M, N), da)
-    pc, sc, dc, _ = _describe(c)
+    pc, sc, dc = _describe(c)
     if tuple(sc) != (M, N) or dc != da:
         raise BeamError(1, f"c must be {(M, N)} of the inputs' dtype")
     cfg = config.to_c() if config is not None else None
-    _check(lib.beam_matmul_nn(pa, pb, pc, M, N, K, da, ctypes.byref(cfg) if cfg else None, st))
+    _check(lib.beam_matmul_nn(pa, pb, pc, M, N, K, da, ctypes.byref(cfg) if cfg else None, _stream_of(a)))
     return c
 
 
 def _flat_pair(x, y, d=None):
-    px, sx, dx, st = _describe(x)
-    py, sy, dy, _ = _describe(y)
-    nx, ny = int(np.prod(sx, dtype=np.int64)), int(np.prod(sy, dtype=np.int64))
+    px, sx, dx = _describe(x)
+    py, sy, dy = _describe(y)
+    nx, ny = math.prod(sx), math.prod(sy)
     if nx != ny:
         raise BeamError(1, f"elementwise input has {nx} elements, output {ny}")
     if dx != dy or (d is not None and dx != d):
         raise BeamError(2, "elementwise input and output must share the GEMM's dtype")
-    return px, py, nx, dx, st
+    return px, py, nx, dx, _stream_of(x)
 
 
 def silu(x, y) -> None:
@@ -537,8 +559,9 @@ def bench(op: int, a, b, c, config: Optional[TileConfig] = None, split_k: int = 
           eps: float = 1e-5, warmup: int = 5, iters: int = 20, x=None, y=None, ln_mode: int = 0) -> float:
     """Average milliseconds per call (HIP events around `iters` back-to-back launches)."""
     if op == OP_MATMUL_NN:  # b is [K, N]
-        pa, (M, K), d, st = _describe(a)
-        pb, (kb, N), _, _ = _describe(b)
+        pa, (M, K), d = _describe(a)
+        pb, (kb, N), _ = _describe(b)
+        st = _stream_of(a)
         pc = _describe(c)[0]
         if kb != K or tuple(_describe(c)[1]) != (M, N):
             raise BeamError(1, "Incompatible dimensions")

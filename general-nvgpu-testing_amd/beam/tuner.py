@@ -85,7 +85,7 @@ class Operator:
         if self.native is not None:
             return _C.bench(self.native["op"], a, b, c, config=self.native.get("config"),
                             split_k=self.native.get("split_k", 0), warmup=warmup, iters=rep)
-        stream = _C._describe(a)[3]
+        stream = _C._stream_of(a)
         return _C.do_bench(lambda: self.func(a=a, b=b, c=c), warmup=warmup, rep=rep, stream=stream)
 
     def get_performance(self, a, b, c, warmup: int = 5, rep: int = 20, min_ms: float = 0.0) -> float:
