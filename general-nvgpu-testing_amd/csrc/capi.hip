@@ -54,6 +54,12 @@ struct Device {
 };
 Device g_dev;
 std::mutex g_dev_mu;
+// A word of pinned host memory that every fused GEMM+LayerNorm launch in which a workgroup gave up sets to its own tag
+// (made once, by beam_init; the process keeps it).  A checked call that finds it as it was before its launch knows that
+// nobody gave up, without copying the workspace header back: that blocking copy of 16 bytes cost more than a small
+// call's kernel (64 x 64 x 64: 24 us of a checked call beyond its launch with the copy, 11 without).  Tags never repeat, so any time-out between the two looks changes the word, whichever thread's or stream's
+// launch it was; the header then says whose.
+unsigned* g_ln_host_timeout = nullptr;
 // Polls before a waiting thread gives up: of statistics slots in the fused LayerNorm (3-4 us each once the pauses
 // between tries have grown: about 60 ms), of a tile's flags in the one-launch split-K (about 1 us each).  What a
 // workgroup legitimately waits for is resident with it and at most a tile's K loop behind, so the bound is there
@@ -303,6 +309,13 @@ int beam_init(void) {
     return fail(BEAM_ERR_DEVICE, "device 0 is %s; this library holds gfx950 code only", prop.gcnArchName);
   }
   g_dev.status = BEAM_OK;
+  void* word = nullptr;
+  if (hipHostMalloc(&word, 64, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+    *(unsigned*)word = 0;
+    g_ln_host_timeout = (unsigned*)word;
+  } else {
+    (void)hipGetLastError();  // without it every checked call reads the header
+  }
   void* ignored;
   return scratch_on_current_device(&ignored);  // the no-allocation entry point's memory, looked up at set-up
 }
@@ -1086,6 +1099,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     p.stats = sets;
     p.next_stats = (float*)((char*)sets + set_bytes);
     p.timeout_flag = (int*)ws;
+    p.host_timeout = g_ln_host_timeout;
     p.gamma = gamma;
     p.beta = beta;
     p.eps = eps;
@@ -1163,7 +1177,11 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (st != nullptr) (void)hipStreamIsCapturing(st, &capturing);
   // (captured: AUTO is two passes, which wait for nothing; a stream being captured cannot be waited for anyway)
-  int rc = beam_gemmrc_ln_ex(A, B, gamma, beta, eps, Y, M, N, K, dtype, cfg, BEAM_LN_AUTO, ws, ws_bytes, stream);
+  int rc = beam_init();
+  if (rc && M > 0 && N > 0) return rc;
+  const volatile unsigned* word = g_ln_host_timeout;
+  const unsigned before = word ? *word : 0u;
+  rc = beam_gemmrc_ln_ex(A, B, gamma, beta, eps, Y, M, N, K, dtype, cfg, BEAM_LN_AUTO, ws, ws_bytes, stream);
   if (rc || capturing != hipStreamCaptureStatusNone || M == 0 || N == 0) return rc;
   bool generic;
   (void)check_problem(A, B, Y, M, N, K, dtype, &generic);
@@ -1171,6 +1189,10 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   if (ln_plan(M, N, K, cfg, BEAM_LN_AUTO, ln_is_generic(generic, gamma, beta), false,
               (((uintptr_t)Y | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0, &plan) || plan.kind != LnPlan::kFused)
     return BEAM_OK;  // nothing in the call waits for anything
+  if (word) {
+    BEAM_HIP(hipStreamSynchronize(st));
+    if (*word == before) return BEAM_OK;
+  }
   int timed_out = 0;
   if ((rc = beam_gemmrc_ln_timed_out(ws, stream, &timed_out))) return rc;
   if (!timed_out) return BEAM_OK;

@@ -109,6 +109,9 @@ struct GemmParams {
   float* next_stats;    // kEpiLnFused: 8-byte words [tiles_m][tiles_n][BM] = (M2, ~tag)
   // kEpiLnFused: the workspace header (tile_map.h: kLnHdr*); never has to be initialised
   int* timeout_flag;
+  // kEpiLnFused: a word in host memory that a launch in which a workgroup gave up waiting sets to its tag (may be null).
+  // The host takes an unchanged word for "nobody gave up" and looks into the header only when it has changed.
+  unsigned* host_timeout;
   unsigned ln_nonce;    // kEpiLnFused, kEpiPartialFused: a number no earlier launch of this process had (ln_launch_tag, sk_launch_tag)
   const void* gamma;    // 16-bit [N]                                                   (kEpiLnFused)
   const void* beta;     // 16-bit [N]
@@ -165,6 +168,11 @@ __device__ __forceinline__ unsigned ln_launch_tag(const GemmParams& p) {
   return x | 1u;  // never 0: a zeroed header then never reads as "timed out"
 }
 
+__device__ __forceinline__ void ln_record_timeout(const GemmParams& p, unsigned tag) {
+  p.timeout_flag[kLnHdrTimeout] = (int)tag;
+  if (p.host_timeout) __hip_atomic_store(p.host_timeout, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Workgroup 0 records which launch the header speaks of.
 __device__ __forceinline__ void ln_sign_header(const GemmParams& p, unsigned tag) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -216,7 +224,7 @@ __device__ __forceinline__ void ln_gather(const GemmParams& p, unsigned tag, siz
           missing &= ~(1u << u);
       if (missing == 0) break;
       if (++polls > p.spin_limit) {
-        p.timeout_flag[kLnHdrTimeout] = (int)tag;
+        ln_record_timeout(p, tag);
 #pragma unroll
         for (int u = 0; u < INFLIGHT; ++u)
           if (missing & (1u << u)) {
@@ -519,8 +527,6 @@ struct GemmTile {
     const T* b_base = B_KMAJOR ? (const T*)p.B + ((size_t)kb * N + col0) : (const T*)p.B + ((size_t)col0 * K + kb);
     unsigned bytes_a = klen > 0 ? ((unsigned)(rows_a - 1) * K + klen) * 2u : 0u;
     unsigned bytes_b = klen > 0 ? ((unsigned)(rows_b - 1) * K + klen) * 2u : 0u;
-    const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(a_base, bytes_a);
-    const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(b_base, bytes_b);
     // kEpiStoreLoop: the same for the next tile of this workgroup (neither split-K nor the [K][N]
     // layout nor a short K tile exist in that mode: the host sees to it)
     auto set_tile = [&](int id) __attribute__((always_inline)) {

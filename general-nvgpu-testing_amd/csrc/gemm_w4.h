@@ -734,7 +734,7 @@ struct GemmW4 {
               missing &= ~(1u << u);
           if (missing == 0) break;
           if (++polls > p.spin_limit) {
-            p.timeout_flag[kLnHdrTimeout] = (int)tag;
+            ln_record_timeout(p, tag);
 #pragma unroll
             for (int u = 0; u < INFLIGHT; ++u)
               if (missing & (1u << u)) {
