@@ -1430,8 +1430,15 @@ struct GemmTile {
   }
 };
 
+// Wavefront tiles of up to 32 blocks fit 256 registers.  Told so (two wavefronts per SIMD must fit), the compiler keeps
+// the accumulators in ordinary registers; with 512 to use it puts them into accumulation registers, rotates them through
+// spare ones where a loop's ends join (32 moves per K tile of the 128 x 64 tile) and reads every one back in the
+// epilogue.  Same machine: 2048 x 1024 x 2048 in 128 x 64 tiles 17.6 -> 15.2 us, 4096 x 2048 x 1024 in 256 x 128 tiles of
+// 128 x 64 wavefronts 20.0 -> 17.3, in 128 x 256 tiles of 64 x 128 20.2 -> 17.2, 1024^3 5.27 -> 5.11.
+constexpr int min_waves_per_simd(int TM, int TN) { return TM * TN <= 32 * 256 ? 2 : 1; }
+
 template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false>
-__global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
+__global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, min_waves_per_simd(BM / WAVES_M, BN / WAVES_N))
     gemmrc_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   GemmTile<T, BM, BN, WAVES_M, WAVES_N, EPI, AST, BST, B_KMAJOR>::run(p, smem);
