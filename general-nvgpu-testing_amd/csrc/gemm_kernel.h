@@ -18,6 +18,9 @@
 //     and the ds_read_b128 fragment reads are both bank-conflict free;
 //   * global -> LDS goes through buffer loads that write LDS directly (no VGPR staging);
 //     rows past the matrix edge are outside the buffer descriptor and never touch memory;
+//   * KG > 1: KG groups of wavefronts, each with an LDS ring of its own, share the output tile and
+//     take every KG-th K tile; one barrier serves KG K tiles, and the groups' sums meet in LDS
+//     behind the last one, added in group order (deep_shape below);
 //   * A has AST slots and B has BST slots (3 + 2 for the 256x256 tile = all 160 KiB of LDS).
 //     While tile h feeds the MFMAs, B tile h+BST-1 and A tile h+AST-1 are in flight, their
 //     loads issued one at a time between rows of MFMAs so the vector-memory path (64 B/clk)
@@ -309,22 +312,34 @@ __device__ __forceinline__ void bare_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// A-slot count of the "deep" pipeline of a tile shape: as many slots as 160 KiB of LDS hold with one
-// slot fewer for B, at most 8.  Small tiles get a long prefetch queue this way, which is what a
-// split-K workgroup (few tiles in flight per CU, every byte fetched exactly once) needs to keep HBM busy.
-constexpr int deep_a_slots(int BM, int BN) {
+// The "deep" pipeline of a tile shape: what runs when a CU has one workgroup to itself.
+//   * Tiles of four wavefronts up to 128 x 64: two K groups (GemmTile's KG), each with a ring of its own.  A lone
+//     group's K tile is a chain -- barrier, LDS reads, MFMAs -- of 190 ns on 64 x 64 tiles however far ahead the loads
+//     are; two groups run two chains side by side, 145 ns per K tile, where the fills (16 KiB at 122 GB/s: 134 ns) are the
+//     next limit.  Same machine, one ring of 8 + 7 slots -> two of 5 + 4: 16 x 4096 x 4096 15.1 -> 12.1 us,
+//     1 x 1024 x 9480 30.9 -> 23.2, 768 x 1024 x 2048 9.5 -> 8.3, 1024 x 1024 x 4096 15.8 -> 14.0, split-K
+//     256 x 256 x 32768 12.8 -> 12.0; [K][N] 1024 x 1024 x 4096 21.9 -> 18.0.  128 x 64 and 64 x 128 tiles (one ring of
+//     7 + 6 or 6 + 5 slots -> two of 3 + 3): 16 x 4096 x 4096 21.2 -> 17.1 and 21.2 -> 18.5.  Four groups of 3 + 2 slots:
+//     no faster than two, and slower wherever memory, not L2, is what the loads wait for (16 x 11008 x 4096 18.2).
+//   * The others: one group, as many A slots as 160 KiB of LDS hold with one slot fewer for B, at most 8.
+struct DeepShape {
+  int a_slots, b_slots, k_groups;
+};
+constexpr DeepShape deep_shape(int BM, int BN, int NW) {
+  if (NW == 4 && BM * BN <= 64 * 64) return {5, 4, 2};
+  if (NW == 4 && BM * BN <= 128 * 64) return {3, 3, 2};
   int a = 8;
   while (a > 3 && (a * BM + (a - 1) * BN) * kRowBytes > 160 * 1024) --a;
-  return a;
+  return {a, a - 1, 1};
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false, int KG = 1>
 struct GemmTile {
   using Traits = ElemTraits<T>;
   using vec8 = typename Traits::vec8;
   using vec4 = typename Traits::vec4;
 
-  static constexpr int NW = WAVES_M * WAVES_N;
+  static constexpr int NW = WAVES_M * WAVES_N;  // wavefronts of a group (KG groups share a workgroup: see run)
   static constexpr int NT = NW * 64;
   // Wavefronts that issue the global->LDS loads.  With two wavefronts per SIMD the hardware favours the
   // older one of each pair (wavefronts 0 .. NW/2-1) when both have an MFMA ready, so those finish a K tile
@@ -341,7 +356,7 @@ struct GemmTile {
   static constexpr int A_BYTES = BM * kRowBytes;
   static constexpr int B_BYTES = BN * kRowBytes;
   static constexpr int B_REGION = AST * A_BYTES;  // A slots first, then B slots
-  static constexpr int LDS_BYTES = AST * A_BYTES + BST * B_BYTES;
+  static constexpr int LDS_BYTES = AST * A_BYTES + BST * B_BYTES;  // of one group
   static constexpr int LA = (BM * kChunksPerRow) / NTL;  // buffer loads per wavefront per A tile
   static constexpr int LB = (BN * kChunksPerRow) / NTL;
   static constexpr int LOADS = LA + LB;
@@ -363,7 +378,8 @@ struct GemmTile {
   static_assert((BM * kChunksPerRow) % NTL == 0 && (BN * kChunksPerRow) % NTL == 0,
                 "every wavefront must move a whole number of 1 KiB chunks per tile");
   static_assert(AST >= 2 && BST >= 2 && (AST == BST || AST == BST + 1), "slot counts");
-  static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
+  static_assert(KG * LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
+  static_assert(KG == 1 || (NW <= 4 && !SIDE && !LOOP && (KG - 1) * BM * BN * 4 <= KG * LDS_BYTES), "K groups");
   static_assert(WAIT_STEADY < 64, "vmcnt range");
   static_assert(BM * 8 * (4 * WAVES_N + 2) <= LDS_BYTES, "row statistics scratch of the LayerNorm epilogues");
 
@@ -457,8 +473,11 @@ struct GemmTile {
     }
   }
 
-  static __device__ __forceinline__ void run(const GemmParams& p, char* smem) {
-    const int tid = threadIdx.x;
+  static __device__ __forceinline__ void run(const GemmParams& p, char* smem_base) {
+    // K groups: group kg multiplies K tiles kg, kg + KG, ... of the whole output tile with a ring of LDS slots of its own.
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+    char* const smem = smem_base + kg * LDS_BYTES;
+    const int tid = (int)threadIdx.x - kg * NT;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WAVES_M;
@@ -467,6 +486,7 @@ struct GemmTile {
     if constexpr (EPI == kEpiPartialFused) {
       const int multiplying = p.tiles_m * p.tiles_n * p.splits;
       if ((int)blockIdx.x >= multiplying) {  // (uniform)
+        if (kg != 0) return;
         const int r = (int)blockIdx.x - multiplying;
         if (p.sk_out == 4) splitk_reduce_part_of<4>(p, r);
         else if (p.sk_out == 2) splitk_reduce_part_of<2>(p, r);
@@ -515,7 +535,8 @@ struct GemmTile {
       k_tail = kBK;
       --kt_full;
     }
-    const int n_tiles = kt_full + (k_tail ? 1 : 0);  // the short tile, if any, is tile 0
+    const int n_all = kt_full + (k_tail ? 1 : 0);  // the short tile, if any, is tile 0
+    const int n_tiles = KG == 1 ? n_all : (n_all - kg + KG - 1) / KG;  // of this group; its tile t is tile t * KG + kg of all
 
     // Buffer descriptors cover exactly the rows of this tile that exist and the K range of
     // this slice; anything else is out of range: reads return zero and touch no memory.
@@ -559,7 +580,10 @@ struct GemmTile {
     }
 
     // First K element (inside the slice) of tile t: the short tile comes first.
-    auto tile_koff = [&](int t) { return k_tail ? (t == 0 ? kt_full * kBK : (t - 1) * kBK) : t * kBK; };
+    auto tile_koff = [&](int t_group) {
+      const int t = t_group * KG + kg;
+      return k_tail ? (t == 0 ? kt_full * kBK : (t - 1) * kBK) : t * kBK;
+    };
 
     // ---- global -> LDS ------------------------------------------------------------------
     // One buffer load (1 KiB per wavefront) of A tile t / B tile t into its slot.  Tiles past the end
@@ -938,7 +962,7 @@ struct GemmTile {
         }
       };
       if constexpr (!LOOP) {  // (no short tile there: the host sees to it; its registers would not fit beside the accumulators)
-        if (k_tail && loader) {
+        if (k_tail && loader && kg == 0) {
           ShortTile st;
           load_short_tile(st, k_tail);
           fills(std::true_type{});
@@ -972,6 +996,7 @@ struct GemmTile {
       } else {
         for (int h = 0; h < n_tiles; ++h) tile_body(h, std::false_type{}, W16{});
       }
+      if (KG > 1 && n_tiles < (n_all + KG - 1) / KG) bare_barrier();  // the other groups' last tile
       wait_vm_and_lds<0>();  // the empty fills of the last iterations must be gone before LDS is reused
       // Drain: the second half of the last tile is in set 1.
       if constexpr (B_KMAJOR) {
@@ -1000,6 +1025,27 @@ struct GemmTile {
         else side_load(0, W4{});
       }
       if constexpr (!LOOP) k_loop_and_drain();
+    } else if (KG > 1 && n_all > 0) {
+      bare_barrier();
+    }
+    if constexpr (KG > 1) {
+      // The groups' sums meet in group 0, added in group order; the other groups are done.
+      __syncthreads();  // every group's slots are dead
+      f32x4* sums = (f32x4*)smem_base;
+      if (kg > 0) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) sums[((kg - 1) * FM * FN + i * FN + j) * NT + tid] = acc[i][j];
+      }
+      __syncthreads();
+      if (kg > 0) return;
+#pragma unroll
+      for (int g = 0; g < KG - 1; ++g)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] += sums[(g * FM * FN + i * FN + j) * NT + tid];
     }
 
     // ---- per-row statistics of the tile (LayerNorm epilogues) -------------------------------
@@ -1437,11 +1483,11 @@ struct GemmTile {
 // 128 x 64 wavefronts 20.0 -> 17.3, in 128 x 256 tiles of 64 x 128 20.2 -> 17.2, 1024^3 5.27 -> 5.11.
 constexpr int min_waves_per_simd(int TM, int TN) { return TM * TN <= 32 * 256 ? 2 : 1; }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false>
-__global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, min_waves_per_simd(BM / WAVES_M, BN / WAVES_N))
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false, int KG = 1>
+__global__ void __launch_bounds__(WAVES_M* WAVES_N * 64 * KG, (KG > 2 ? KG : min_waves_per_simd(BM / WAVES_M, BN / WAVES_N)))
     gemmrc_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  GemmTile<T, BM, BN, WAVES_M, WAVES_N, EPI, AST, BST, B_KMAJOR>::run(p, smem);
+  GemmTile<T, BM, BN, WAVES_M, WAVES_N, EPI, AST, BST, B_KMAJOR, KG>::run(p, smem);
 }
 
 }  // namespace beam

@@ -43,13 +43,13 @@ inline hipError_t allow_lds_once(std::atomic<unsigned long long>& done, const vo
   return hipSuccess;
 }
 
-template <typename T, int BM, int BN, int WVM, int WVN, int EPI, int AST, int BST, bool B_KMAJOR = false>
+template <typename T, int BM, int BN, int WVM, int WVN, int EPI, int AST, int BST, bool B_KMAJOR = false, int KG = 1>
 hipError_t launch_gemm(const GemmParams& p, dim3 grid, hipStream_t stream) {
-  using Tile = GemmTile<T, BM, BN, WVM, WVN, EPI, AST, BST, B_KMAJOR>;
-  auto kern = gemmrc_kernel<T, BM, BN, WVM, WVN, EPI, AST, BST, B_KMAJOR>;
+  using Tile = GemmTile<T, BM, BN, WVM, WVN, EPI, AST, BST, B_KMAJOR, KG>;
+  auto kern = gemmrc_kernel<T, BM, BN, WVM, WVN, EPI, AST, BST, B_KMAJOR, KG>;
   static std::atomic<unsigned long long> configured{0};
-  if (hipError_t e = allow_lds_once(configured, reinterpret_cast<const void*>(kern), Tile::LDS_BYTES); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, grid, dim3(Tile::NT), Tile::LDS_BYTES, stream, p);
+  if (hipError_t e = allow_lds_once(configured, reinterpret_cast<const void*>(kern), KG * Tile::LDS_BYTES); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, grid, dim3(KG * Tile::NT), KG * Tile::LDS_BYTES, stream, p);
   return hipGetLastError();
 }
 
@@ -63,9 +63,9 @@ GemmLauncher loop_launcher() {
     return nullptr;
 }
 
-template <typename T, int BM, int BN, int WVM, int WVN, int AST, int BST>
+template <typename T, int BM, int BN, int WVM, int WVN, int AST, int BST, int KG = 1>
 GemmLauncher partial_fused_launcher() {
-  if constexpr (BM * BN <= 128 * 128) return launch_gemm<T, BM, BN, WVM, WVN, kEpiPartialFused, AST, BST>;
+  if constexpr (BM * BN <= 128 * 128) return launch_gemm<T, BM, BN, WVM, WVN, kEpiPartialFused, AST, BST, false, KG>;
   else return nullptr;
 }
 
@@ -80,15 +80,16 @@ KernelSet make_kernel_set() {
   k.threads = WVM * WVN * 64;
   k.lds_bytes = GemmTile<_Float16, BM, BN, WVM, WVN, kEpiStore, 3, 2>::LDS_BYTES;
   k.lds_bytes_shallow = GemmTile<_Float16, BM, BN, WVM, WVN, kEpiStore, 2, 2>::LDS_BYTES;
-  constexpr int DA = deep_a_slots(BM, BN);
-  k.lds_bytes_deep = GemmTile<_Float16, BM, BN, WVM, WVN, kEpiStore, DA, DA - 1>::LDS_BYTES;
+  constexpr DeepShape deep = deep_shape(BM, BN, WVM * WVN);
+  constexpr int DA = deep.a_slots, DB = deep.b_slots, KG = deep.k_groups;
+  k.lds_bytes_deep = KG * GemmTile<_Float16, BM, BN, WVM, WVN, kEpiStore, DA, DB, false, KG>::LDS_BYTES;
 #define BEAM_FILL(D, T)                                                             \
   k.launch[D][kEpiStore][0] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, 3, 2>;     \
   k.launch[D][kEpiStore][1] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, 2, 2>;     \
-  k.launch[D][kEpiStore][2] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, DA, DA - 1>; \
+  k.launch[D][kEpiStore][2] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, DA, DB, false, KG>; \
   k.launch[D][kEpiPartial][0] = launch_gemm<T, BM, BN, WVM, WVN, kEpiPartial, 3, 2>; \
   k.launch[D][kEpiPartial][1] = launch_gemm<T, BM, BN, WVM, WVN, kEpiPartial, 2, 2>; \
-  k.launch[D][kEpiPartial][2] = launch_gemm<T, BM, BN, WVM, WVN, kEpiPartial, DA, DA - 1>; \
+  k.launch[D][kEpiPartial][2] = launch_gemm<T, BM, BN, WVM, WVN, kEpiPartial, DA, DB, false, KG>; \
   k.launch[D][kEpiLnStats][2] = nullptr;                                               \
   k.launch[D][kEpiLnFused][2] = nullptr;                                               \
   k.launch[D][kEpiLnStats][0] = launch_gemm<T, BM, BN, WVM, WVN, kEpiLnStats, 3, 2>; \
@@ -100,13 +101,13 @@ KernelSet make_kernel_set() {
   k.launch[D][kEpiStoreSide][2] = nullptr; \
   k.launch_kmajor[D][0] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, 3, 2, true>; \
   k.launch_kmajor[D][1] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, 2, 2, true>; \
-  k.launch_kmajor[D][2] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, DA, DA - 1, true>; \
+  k.launch_kmajor[D][2] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, DA, DB, true, KG>; \
   k.launch[D][kEpiStoreLoop][0] = loop_launcher<T, BM, BN, WVM, WVN>();              \
   k.launch[D][kEpiStoreLoop][1] = nullptr;                                            \
   k.launch[D][kEpiStoreLoop][2] = nullptr;                                            \
   k.launch_partial_fused[D][0] = partial_fused_launcher<T, BM, BN, WVM, WVN, 3, 2>();  \
   k.launch_partial_fused[D][1] = partial_fused_launcher<T, BM, BN, WVM, WVN, 2, 2>();  \
-  k.launch_partial_fused[D][2] = partial_fused_launcher<T, BM, BN, WVM, WVN, DA, DA - 1>();
+  k.launch_partial_fused[D][2] = partial_fused_launcher<T, BM, BN, WVM, WVN, DA, DB, KG>();
   BEAM_FILL(0, _Float16)
   BEAM_FILL(1, __bf16)
 #undef BEAM_FILL

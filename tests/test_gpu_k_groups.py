@@ -1,0 +1,34 @@
+"""Tiles whose K tiles are dealt to groups of wavefronts: fewer K tiles than groups, counts that the groups share
+unevenly, and a short last K tile.  Bound: close_enough's, the one of every other GEMM test."""
+import numpy as np
+import pytest
+
+from test_gpu_edges import close_enough
+from test_gpu_gemm import F16, BF16
+from test_gpu_unaligned import run
+
+pytestmark = pytest.mark.gpu
+
+DEEP_GROUP_TILES = [(64, 64, 32, 32), (128, 64, 64, 32), (64, 128, 32, 64)]
+
+
+@pytest.mark.parametrize("K", [8, 64, 65, 128, 136, 192, 257, 320, 585])
+@pytest.mark.parametrize("tile", DEEP_GROUP_TILES)
+def test_deep_tiles(gpu, beamc, oracle, tile, K):
+    import ctypes
+    L = beamc.lib
+    cfg = beamc.TileConfig(*tile, 2, 0).to_c()
+    for (M, N), dtype in (((130, 72), F16), ((33, 129), BF16)):
+        a, b = beamc.host_uniform((M, K), dtype, 83, 0), beamc.host_uniform((N, K), dtype, 83, 1)
+        bt = np.ascontiguousarray(b.T)
+        ref = oracle.gemmrc(a, b, dtype)
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, dtype, ctypes.byref(cfg), None), a, b, (M, N), dtype, (0, 0, 0))
+        close_enough(oracle, out, ref, K, dtype, f"gemmrc {(M, N, K)}")
+        nn = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, dtype, ctypes.byref(cfg), None), a, bt, (M, N), dtype, (0, 0, 0))
+        assert (nn == out).all(), f"[K][N] {(M, N, K)}: differs from [N][K]"
+        for slices in (2, 3):
+            ws = beamc.DeviceArray((L.beam_splitk_workspace_bytes(M, N, slices),), itemsize=1)
+            out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, dtype, ctypes.byref(cfg), slices, ws.ptr, ws.nbytes, None),
+                      a, b, (M, N), dtype, (0, 0, 0))
+            ws.free()
+            close_enough(oracle, out, ref, K, dtype, f"split-K {(M, N, K)} in {slices}")
