@@ -600,7 +600,12 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   beam_tile_cfg c;
   const KernelSet* ks;
   if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks))) return rc;
-  if (!cfg && c.pipeline == 2) c.pipeline = 0;  // the default for split-K-shaped problems
+  // Too few workgroups to keep memory busy for the side job (the deep pipeline's problems): the two kernels one after
+  // the other.
+  if (!cfg && c.pipeline == 2) {
+    if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
+    return beam_silu(X, Y, count, dtype, stream);
+  }
   if (c.pipeline == 2) return fail(BEAM_ERR_UNSUPPORTED, "the side job runs with pipeline 0 or 1");
   GemmParams p = base_params(A, B, M, N, K, c);
   p.C = C;
