@@ -447,6 +447,28 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
   return BEAM_OK;
 }
 
+// Which form of the kernel for few rows (gemm_rows.h), if any, runs c = a @ b^T.  bf16, us, tiled kernel -> this one:
+//   * Up to 16 columns for every CU, one form is ahead for every K: 4096 columns, M = 16 K = 128 3.6 -> 3.3,
+//     K = 16384 37.3 -> 25.7; M = 64 K = 128 3.9 -> 3.6, K = 1024 5.0 -> 4.1, K = 16384 41.9 -> 33.1.
+//   * Beyond that the fetches of A add up, and B's become the bound.  M <= 16, K <= 4096: 64 columns per workgroup,
+//     M = 1: 5000 x 4096 11.7 -> 7.9, 16384 x 1024 7.4 -> 3.8, 11008 x 4096 15.0 -> 14.5 (M = 16 15.6 -> 15.5),
+//     16384 x 3000 17.6 -> 15.9; the tiled kernel is ahead from there on (16384 x 4088 20.6, here 27.2) and where K is
+//     so short that the workgroups' starts count (65536 x 512 11.0, here 12.1).
+//   * Longer K: 16 columns, fewer wavefronts: M = 16 6000 x 9000 26.8 -> 23.3, 8192 x 11008 32.1 -> 27.8, but
+//     10000 x 6000 21.4, here 23.0.
+//   * M <= 32: 32 columns per workgroup, 8192 x 1024 5.1 -> 4.3, x 2048 7.6 -> 6.4; 16384 x 512 3.7, here 5.0.
+RowsPlan rows_plan(int M, int N, int K, int cus) {
+  if (M > 64 || K % 8 != 0 || K > kRowsMaxK) return kRowsNone;
+  const long cols = N, round = 16L * cus;  // columns of one workgroup of 16 per CU
+  if (cols <= round) return kRowsNarrow;
+  if (M <= 16) {
+    if (K > 4096) return cols <= 2 * round ? kRowsDeep : kRowsNone;
+    return K >= 512 && cols <= 4 * round && cols * K <= (3L << 24) ? kRowsWide : kRowsNone;
+  }
+  if (M <= 32 && cols <= 2 * round && K >= 1024 && K <= 2048) return kRowsWide;
+  return kRowsNone;
+}
+
 }  // namespace
 
 extern "C" {
@@ -467,13 +489,17 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, false, false, st));
     return BEAM_OK;
   }
+  const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
+  if (const RowsPlan plan = cfg ? kRowsNone : rows_plan(M, N, K, cus); plan != kRowsNone) {
+    BEAM_HIP(launch_gemm_rows(plan, A, B, C, M, N, K, dtype, st));
+    return BEAM_OK;
+  }
   beam_tile_cfg c;
   const KernelSet* ks;
   if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, -1, true))) return rc;
   GemmParams p = base_params(A, B, M, N, K, c);
   p.C = C;
   const long tiles = (long)p.tiles_m * p.tiles_n;
-  const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   // The 256 x 256 tile of four 128 x 128 wavefronts has a kernel of its own (gemm_w4.h), built for problems
   // of a round of workgroups or more: one workgroup per CU walks its tiles with the operand ring running
   // through the tile boundaries.  It is what the tile {256, 256, 128, 128} means wherever its preconditions
@@ -600,9 +626,9 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   beam_tile_cfg c;
   const KernelSet* ks;
   if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks))) return rc;
-  // Too few workgroups to keep memory busy for the side job (the deep pipeline's problems): the two kernels one after
-  // the other.
-  if (!cfg && c.pipeline == 2) {
+  // Too few workgroups to keep memory busy for the side job (the deep pipeline's problems, few rows): the two kernels one
+  // after the other.
+  if (!cfg && (c.pipeline == 2 || rows_plan(M, N, K, g_dev.cus > 0 ? g_dev.cus : 256) != kRowsNone)) {
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }

@@ -152,6 +152,16 @@ hipError_t launch_gemm_w4_kmajor(const GemmParams& p, int dtype, dim3 grid, hipS
 // workgroup per CU) makes them walk, which needs tiles_n <= kW4LnCompactTiles.  gamma and beta 16-byte aligned as well.
 constexpr int kW4LnCompactTiles = 32;
 hipError_t launch_gemm_w4_ln(const GemmParams& p, int dtype, dim3 grid, hipStream_t stream);
+// c = a @ b^T for few rows (gemm_rows.h); needs 8 <= K <= kRowsMaxK, K % 8 == 0, and M <= 64 (narrow), 16 (deep) or
+// 32 (wide).
+enum RowsPlan : int {
+  kRowsNone = 0,
+  kRowsNarrow = 1,  // 16 columns per workgroup, 8 or 4 wavefronts
+  kRowsDeep = 2,    // 16 columns, 4 wavefronts
+  kRowsWide = 3,    // 64 (M <= 16) or 32 columns, 4 wavefronts
+};
+constexpr int kRowsMaxK = 1 << 23;
+hipError_t launch_gemm_rows(RowsPlan plan, const void* A, const void* B, void* C, int M, int N, int K, int dtype, hipStream_t stream);
 // Measurement only: the split-K partial kernel of the 64 x 128 (wave 32 x 64) or 64 x 64 (wave 32 x 32) tile, deep
 // pipeline, fp16, with its loads and fragment reads but no MFMAs and no stores (kEpiProbeLoads); hipErrorInvalidValue
 // for any other tile.

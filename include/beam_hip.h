@@ -66,7 +66,8 @@ int beam_default_config(int M, int N, int K, beam_tile_cfg* cfg, int* split_k);
 
 /* ---- tiled GEMM ------------------------------------------------------------------------ */
 
-/* cfg == NULL: beam_default_config() picks the tile (never a split).
+/* cfg == NULL: beam_default_config() picks the tile (never a split); up to 64 rows of A may run on a kernel of their own
+ * that has no tile to name.
  * Replaces entry_cutlass_gemmrc / entry_cutlass_gemmrc_spec
  * (cuda/cutlass_kernels/main.cc:11-15, cutlass_gemmrc.cu:21-40,55-111). */
 int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int dtype,
