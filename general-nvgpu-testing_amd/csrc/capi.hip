@@ -628,7 +628,8 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks))) return rc;
   // Too few workgroups to keep memory busy for the side job (the deep pipeline's problems, few rows): the two kernels one
   // after the other.
-  if (!cfg && (c.pipeline == 2 || rows_plan(M, N, K, g_dev.cus > 0 ? g_dev.cus : 256) != kRowsNone)) {
+  const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
+  if (!cfg && (c.pipeline == 2 || rows_plan(M, N, K, cus) != kRowsNone)) {
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }
@@ -653,6 +654,15 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
     }
   }
   p.side_iters = (int)(((count >> 3) * (16 / p.side_width) + per_pass - 1) / per_pass);
+  // A job that outlasts the loop goes on at 0.4-1.4 us for every 16 bytes per thread; with a round of workgroups or less,
+  // from 8 such passes on, a launch of its own (3 us and 11 us per 16 Mi elements) is ahead.  Fused, then two launches:
+  // 256^3 with 2^20 elements (28 passes) 15.8, 6.5 us; 1024^3 with 2^24 (16) 30.3, 20.7; 4096 x 4096 x 256 with 2^24 (12)
+  // 28.9, 26.4; but 1536 x 1536 x 512 with 2^22 (7) 9.4, 10.5.  With several rounds the later workgroups hide it:
+  // 8192 x 8192 x 256 with 2^26 (12) 110.8, 117.7.
+  if (!cfg && wgs <= cus && p.side_iters - k_tiles > 8) {
+    if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
+    return beam_silu(X, Y, count, dtype, stream);
+  }
   BEAM_HIP(ks->launch[dtype][kEpiStoreSide][c.pipeline](p, dim3((unsigned)wgs, 1, 1), (hipStream_t)stream));
   return BEAM_OK;
 }
