@@ -54,11 +54,12 @@ struct Device {
 };
 Device g_dev;
 std::mutex g_dev_mu;
-// A word of pinned host memory that every fused GEMM+LayerNorm launch in which a workgroup gave up sets to its own tag
-// (made once, by beam_init; the process keeps it).  A checked call that finds it as it was before its launch knows that
-// nobody gave up, without copying the workspace header back: that blocking copy of 16 bytes cost more than a small
-// call's kernel (64 x 64 x 64: 24 us of a checked call beyond its launch with the copy, 11 without).  Tags never repeat, so any time-out between the two looks changes the word, whichever thread's or stream's
-// launch it was; the header then says whose.
+// A word of pinned host memory that a fused GEMM+LayerNorm launch sets when a workgroup in it gives up (made once, by
+// beam_init; the process keeps it, and it stays set).  While it is zero no launch of the process has ever given up, and a
+// checked call is done without copying the workspace header back: that blocking copy of 16 bytes cost more than a small
+// call's kernel (64 x 64 x 64: 24 us of a checked call beyond its launch with the copy, 11 without).  After the first
+// time-out every checked call reads its header.  (One word cannot tell more: launches of other streams and threads write
+// it too, so comparing it before and after a launch could miss this launch's own time-out between two of another's.)
 unsigned* g_ln_host_timeout = nullptr;
 // Polls before a waiting thread gives up: of statistics slots in the fused LayerNorm (3-4 us each once the pauses
 // between tries have grown: about 60 ms), of a tile's flags in the one-launch split-K (about 1 us each).  What a
@@ -310,12 +311,15 @@ int beam_init(void) {
   }
   g_dev.status = BEAM_OK;
   void* word = nullptr;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // the first call may come while a stream is being captured
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (hipHostMalloc(&word, 64, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
     *(unsigned*)word = 0;
     g_ln_host_timeout = (unsigned*)word;
   } else {
     (void)hipGetLastError();  // without it every checked call reads the header
   }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
   void* ignored;
   return scratch_on_current_device(&ignored);  // the no-allocation entry point's memory, looked up at set-up
 }
@@ -1221,7 +1225,6 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   int rc = beam_init();
   if (rc && M > 0 && N > 0) return rc;
   const volatile unsigned* word = g_ln_host_timeout;
-  const unsigned before = word ? *word : 0u;
   rc = beam_gemmrc_ln_ex(A, B, gamma, beta, eps, Y, M, N, K, dtype, cfg, BEAM_LN_AUTO, ws, ws_bytes, stream);
   if (rc || capturing != hipStreamCaptureStatusNone || M == 0 || N == 0) return rc;
   bool generic;
@@ -1232,7 +1235,7 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
     return BEAM_OK;  // nothing in the call waits for anything
   if (word) {
     BEAM_HIP(hipStreamSynchronize(st));
-    if (*word == before) return BEAM_OK;
+    if (*word == 0) return BEAM_OK;
   }
   int timed_out = 0;
   if ((rc = beam_gemmrc_ln_timed_out(ws, stream, &timed_out))) return rc;

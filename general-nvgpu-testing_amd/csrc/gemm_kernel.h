@@ -112,8 +112,8 @@ struct GemmParams {
   float* next_stats;    // kEpiLnFused: 8-byte words [tiles_m][tiles_n][BM] = (M2, ~tag)
   // kEpiLnFused: the workspace header (tile_map.h: kLnHdr*); never has to be initialised
   int* timeout_flag;
-  // kEpiLnFused: a word in host memory that a launch in which a workgroup gave up waiting sets to its tag (may be null).
-  // The host takes an unchanged word for "nobody gave up" and looks into the header only when it has changed.
+  // kEpiLnFused: a word in host memory that a launch in which a workgroup gave up waiting sets (may be null).  The host
+  // takes zero for "nobody ever gave up" and looks into the header otherwise.
   unsigned* host_timeout;
   unsigned ln_nonce;    // kEpiLnFused, kEpiPartialFused: a number no earlier launch of this process had (ln_launch_tag, sk_launch_tag)
   const void* gamma;    // 16-bit [N]                                                   (kEpiLnFused)
@@ -173,7 +173,7 @@ __device__ __forceinline__ unsigned ln_launch_tag(const GemmParams& p) {
 
 __device__ __forceinline__ void ln_record_timeout(const GemmParams& p, unsigned tag) {
   p.timeout_flag[kLnHdrTimeout] = (int)tag;
-  if (p.host_timeout) __hip_atomic_store(p.host_timeout, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (p.host_timeout) __hip_atomic_store(p.host_timeout, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Workgroup 0 records which launch the header speaks of.
