@@ -441,8 +441,12 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
     cfg->wave_m = 128;
     cfg->wave_n = 128;
   }
-  if (split_req < 0 && tiles(c.block_m, c.block_n) < cus / 2 && K >= 2048)
-    cfg->pipeline = 2;  // few workgroups per CU: a long prefetch queue keeps HBM busy
+  // One workgroup per CU under a long sum: the deep pipeline.  Less than half the CUs busy: its long prefetch queue keeps
+  // memory busy.  Tiles with two K groups: up to a full round, since a lone group's K tile is a serial chain.  64 x 128
+  // tiles, one group -> two: 8192 x 256 x 2048 17.6 -> 12.3 us, 654 x 1832 x 2104 21.5 -> 16.8, 2048 x 1024 x 2048 11.8 ->
+  // 11.4; 64 x 64 tiles 1024 x 1024 x 2048 8.1 -> 7.7.  At K = 1024 one group is ahead (5.2, 5.5; 6.7, 7.2).
+  const long picked = tiles(c.block_m, c.block_n);
+  if (split_req < 0 && K >= 2048 && (picked < cus / 2 || (picked <= cus && c.block_m * c.block_n <= 128 * 64))) cfg->pipeline = 2;
   // K slices on at most half the CUs: every workgroup has the memory system of two CUs to itself, the long
   // queue's prologue costs more than it hides (64 x 128 x 65536 in 64 slices: 8.9 against 9.9 us), and the
   // reducing workgroups of the one-launch form start on the idle CUs at once.
