@@ -580,8 +580,9 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     const KernelSet* alt_ks = nullptr;
     if ((alt.wave_n != c.wave_n) && resolve_cfg(&alt, M, N, K, &alt, &alt_ks) == BEAM_OK) c = alt, ks = alt_ks;
   }
-  // The 4-wavefront kernel, as in beam_gemmrc; the K tile's offset into B is a 32-bit scalar there.
-  const bool w4_fits = c.pipeline == 0 && K % kBK == 0 && K >= kW4MinK && ((uintptr_t)C & 15) == 0 && N <= (1 << 21) &&
+  // The 4-wavefront kernel, as in beam_gemmrc (its stores write whole chunks of 8 columns); the K tile's offset into B is a
+  // 32-bit scalar there.
+  const bool w4_fits = c.pipeline == 0 && K % kBK == 0 && K >= kW4MinK && N % 8 == 0 && ((uintptr_t)C & 15) == 0 && N <= (1 << 21) &&
                        (size_t)K * N * 2 < ((size_t)1 << 31);
   const bool w4_named = c.block_m == 256 && c.block_n == 256 && c.wave_m == 128 && c.wave_n == 128;
   if (w4_named && !w4_fits && !cfg) {

@@ -87,6 +87,21 @@ def test_every_tile(gpu, beamc, oracle):
         assert_close(oracle, out, ref_nn, K, F16, f"matmul {cfg.name}")
 
 
+# N around a chunk of 8 and around the largest tile; K a multiple of 64, which is what the 4-wavefront kernel asks of K
+@pytest.mark.parametrize("N", [257, 513, 1001, 1004])
+def test_every_tile_kmajor_whole_k_tiles(gpu, beamc, oracle, N):
+    """[K][N] with N not a multiple of 8 in every compiled tile and LDS depth, C on a 16-byte boundary: no kernel that
+    stores whole chunks may take it."""
+    M, K = 300, 192
+    L = beamc.lib
+    a, b = beamc.host_uniform((M, K), F16, 76, 0), beamc.host_uniform((K, N), F16, 76, 1)
+    ref = oracle.matmul_nn(a, b, F16)
+    for cfg in all_configs(beamc):
+        c = cfg.to_c()
+        out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, ctypes.byref(c), None), a, b, (M, N), F16, (0, 0, 0))
+        assert_close(oracle, out, ref, K, F16, f"matmul {cfg.name} N={N}")
+
+
 # the persistent kernels: more tiles than CUs, K a multiple of 64, operands off a 16-byte boundary
 @pytest.mark.parametrize("wave_n", [64, 128])
 def test_walking_kernels_at_any_address(gpu, beamc, oracle, wave_n):
