@@ -441,8 +441,8 @@ def gemmrc_ln(a, b, c, gamma, beta, eps: float = 1e-5, config: Optional[TileConf
         raise BeamError(1, "gamma and beta must be [N] of the same dtype as a, b, c")
     cfg = config.to_c() if config is not None else None
     cfgp = ctypes.byref(cfg) if cfg else None
-    # gamma or beta off an 8-byte boundary: the plain kernels, which need room for an fp32 copy of the product
-    aligned = ((pg | pbt) & 7) == 0
+    # operands off their boundaries may run on the plain kernels, which need room for an fp32 copy of the product
+    aligned = ((pa | pb | pc) & 15) == 0 and ((pg | pbt) & 7) == 0
     need = lib.beam_gemmrc_ln_workspace_bytes_for(M, N, K, cfgp, mode) if aligned else lib.beam_gemmrc_ln_workspace_bytes_ex(M, N, cfgp, mode)
     ws = _get_ln_workspace(need)
     if check and mode == LN_AUTO:

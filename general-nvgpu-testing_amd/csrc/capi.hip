@@ -991,8 +991,10 @@ static int ln_resolve_cfg(const beam_tile_cfg* cfg, int M, int N, int K, int mod
 // What a GEMM+LayerNorm call does and the workspace it needs: one function, so that the entry point and the
 // workspace queries cannot disagree.
 //   plain     the problem is outside what the tiled kernels take (K below 8 or beyond a descriptor, gamma or beta not
-//             8-byte aligned): plain GEMM into fp32 X, then a row-wise LayerNorm.  (Also for the one combination
-//             that has always been computed and never refused: BEAM_LN_FUSED where it does not apply, K % 8 != 0.)
+//             8-byte aligned): plain GEMM into fp32 X, then a row-wise LayerNorm
+//   unaligned rows of A or B off 16 bytes or Y off 8 (rows_unaligned; K % 8 != 0 implies it).  The tiled kernels take
+//             them; where they would refuse the call (BEAM_LN_FUSED where it does not apply) it runs on the plain ones,
+//             which never refused such operands
 //   capturing the stream is being captured: AUTO then means two passes (a replayed graph may share the device with
 //             other work, which the fused kernel's residency argument does not cover); an explicit FUSED is honoured
 //   wide_io   Y, gamma and beta are 16-byte aligned (the 4-wavefront kernel's vector accesses)
@@ -1003,7 +1005,8 @@ struct LnPlan {
   bool w4;  // fused, on the kernel of gemm_w4.h
   size_t need;
 };
-static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool plain, bool capturing, bool wide_io, LnPlan* out) {
+static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool plain, bool unaligned, bool capturing, bool wide_io,
+                   LnPlan* out) {
   out->ks = nullptr;
   out->w4 = false;
   if (plain) {
@@ -1015,7 +1018,7 @@ static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool
   int rc = ln_resolve_cfg(cfg, M, N, K, mode, &out->c, &out->ks);
   if (rc) return rc;
   beam_tile_cfg& c = out->c;
-  if (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N) && K % 8 != 0) {
+  if (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N) && (unaligned || K % 8 != 0)) {
     out->kind = LnPlan::kPlain;
     out->need = ln_generic_need(M, N);
     return BEAM_OK;
@@ -1047,9 +1050,9 @@ size_t beam_gemmrc_ln_workspace_bytes_for(int M, int N, int K, const beam_tile_c
   if ((K > 0 && K < 8) || K > kMaxK) return ln_generic_need(M, N);
   (void)beam_init();  // AUTO depends on the device
   LnPlan eager, captured;
-  if (ln_plan(M, N, K, cfg, mode, false, false, true, &eager)) return 0;
+  if (ln_plan(M, N, K, cfg, mode, false, false, false, true, &eager)) return 0;
   if (mode != BEAM_LN_AUTO) return eager.need;
-  if (ln_plan(M, N, K, cfg, mode, false, true, true, &captured)) return eager.need;
+  if (ln_plan(M, N, K, cfg, mode, false, false, true, true, &captured)) return eager.need;
   return eager.need > captured.need ? eager.need : captured.need;
 }
 
@@ -1082,7 +1085,8 @@ size_t beam_gemmrc_ln_workspace_bytes(int M, int N, const beam_tile_cfg* cfg) {
 
 size_t beam_dbg_ln_plan_bytes(int M, int N, int K, const beam_tile_cfg* cfg, int mode, int plain, int capturing, int wide_io) {
   LnPlan plan;
-  if (M <= 0 || N <= 0 || K < 0 || ln_plan(M, N, K, cfg, mode, plain != 0 || (K > 0 && K < 8) || K > kMaxK, capturing != 0, wide_io != 0, &plan)) return 0;
+  if (M <= 0 || N <= 0 || K < 0 || ln_plan(M, N, K, cfg, mode, plain != 0 || (K > 0 && K < 8) || K > kMaxK, false, capturing != 0,
+                                                     wide_io != 0, &plan)) return 0;
   return plan.need;
 }
 
@@ -1119,7 +1123,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (st != nullptr) (void)hipStreamIsCapturing(st, &capturing);
   LnPlan plan;
-  if ((rc = ln_plan(M, N, K, cfg, mode, ln_is_generic(generic, gamma, beta), capturing != hipStreamCaptureStatusNone,
+  if ((rc = ln_plan(M, N, K, cfg, mode, ln_is_generic(generic, gamma, beta), rows_unaligned(A, B, Y, K), capturing != hipStreamCaptureStatusNone,
                     (((uintptr_t)Y | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0, &plan)))
     return rc;
   const size_t need = plan.need;
@@ -1235,7 +1239,7 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   bool generic;
   (void)check_problem(A, B, Y, M, N, K, dtype, &generic);
   LnPlan plan;
-  if (ln_plan(M, N, K, cfg, BEAM_LN_AUTO, ln_is_generic(generic, gamma, beta), false,
+  if (ln_plan(M, N, K, cfg, BEAM_LN_AUTO, ln_is_generic(generic, gamma, beta), rows_unaligned(A, B, Y, K), false,
               (((uintptr_t)Y | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0, &plan) || plan.kind != LnPlan::kFused)
     return BEAM_OK;  // nothing in the call waits for anything
   if (word) {
@@ -1335,7 +1339,7 @@ int beam_bench(int op, const beam_problem* q, const beam_tile_cfg* cfg, int warm
         int rc = beam_init();
         if (rc) return rc;
         LnPlan plan;
-        if ((rc = ln_plan(q->M, q->N, q->K, cfg, BEAM_LN_TWOPASS, q->K % 8 != 0 || q->K > kMaxK, false, true, &plan))) return rc;
+        if ((rc = ln_plan(q->M, q->N, q->K, cfg, BEAM_LN_TWOPASS, q->K % 8 != 0 || q->K > kMaxK, false, false, true, &plan))) return rc;
         if (plan.kind != LnPlan::kTwoPass || !q->ws || q->ws_bytes < plan.need) return fail(BEAM_ERR_WORKSPACE, "needs the workspace of a two-pass call");
         const float* stats = (const float*)((const char*)q->ws + align_up((size_t)q->M * q->N * sizeof(float), 256));
         BEAM_HIP(launch_ln_apply((const float*)q->ws, stats, q->gamma, q->beta, q->C, q->M, q->N, (q->N + plan.c.block_n - 1) / plan.c.block_n,

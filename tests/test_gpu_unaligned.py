@@ -129,3 +129,38 @@ def test_layer_norm(gpu, beamc, oracle, shape, dtype):
         ws.free()
     dg.free()
     dbt.free()
+
+
+@pytest.mark.parametrize("offs", [(1, 0, 0), (0, 3, 0), (0, 0, 1), (4, 4, 2)])
+def test_layer_norm_one_kernel_form_where_it_does_not_apply(gpu, beamc, oracle, offs):
+    """More than 64 column tiles: BEAM_LN_FUSED is refused on aligned operands and computed (by the plain kernels) on
+    others, through the C entry point and the Python operator."""
+    M, N, K = 20, 64 * 64 + 8, 64
+    L = beamc.lib
+    tile = beamc.TileConfig(64, 64, 32, 32)
+    cfg = tile.to_c()
+    a, b, g, bt = make_ln_inputs(beamc, M, N, K, F16, 77)
+    ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, F16)
+    dg, dbt = beamc.DeviceArray.from_numpy(g, F16), beamc.DeviceArray.from_numpy(bt, F16)
+    ws = beamc.DeviceArray((L.beam_gemmrc_ln_workspace_bytes_ex(M, N, ctypes.byref(cfg), beamc.LN_FUSED),), itemsize=1)
+
+    def call(pa, pb, pc):
+        return L.beam_gemmrc_ln_ex(pa, pb, dg.ptr, dbt.ptr, 1e-5, pc, M, N, K, F16, ctypes.byref(cfg), beamc.LN_FUSED, ws.ptr, ws.nbytes, None)
+
+    check_ln(oracle, run(beamc, call, a, b, (M, N), F16, offs), ref, F16, f"LN_FUSED at {offs}")
+    da, db, c = Embedded(beamc, a.shape, F16, 0, a), Embedded(beamc, b.shape, F16, 0, b), Embedded(beamc, (M, N), F16, 0)
+    assert call(da.ptr, db.ptr, c.ptr) == 2
+    views = []
+    for x, off in zip((da, db, c), offs):  # the same buffers, seen `off` elements further on (inputs: other values)
+        v = beamc.DeviceArray.__new__(beamc.DeviceArray)
+        v.shape, v.dtype, v.itemsize, v.nbytes, v.ptr = x.shape, F16, 2, 2 * x.n, x.ptr + 2 * off
+        views.append(v)
+    beamc._check(L.beam_memcpy_h2d(views[0].ptr, a.ctypes.data, a.nbytes))
+    beamc._check(L.beam_memcpy_h2d(views[1].ptr, b.ctypes.data, b.nbytes))
+    beamc.gemmrc_ln(*views, dg, dbt, config=tile, mode=beamc.LN_FUSED)
+    c.off = offs[2]
+    check_ln(oracle, c.result(), ref, F16, f"gemmrc_ln, LN_FUSED at {offs}")
+    for v in views:
+        v.ptr = 0
+    for x in (da.buf, db.buf, c.buf, dg, dbt, ws):
+        x.free()
