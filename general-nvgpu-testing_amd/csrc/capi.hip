@@ -152,7 +152,8 @@ int check_problem(const void* A, const void* B, const void* C, int M, int N, int
 }
 
 // Rows of A or B that do not start on 16 bytes, or C not on 8: what the kernels take at a lower rate (gemm_kernel.h:
-// load_short_tile), and what may call split-K without a workspace.
+// load_short_tile), and what may call split-K without a workspace.  No tile that a caller names is refused on them: where
+// the library has no kernel for it, the plain one computes the problem.
 bool rows_unaligned(const void* A, const void* B, const void* C, int K) {
   return K % 8 != 0 || (((uintptr_t)A | (uintptr_t)B) & 15) != 0 || ((uintptr_t)C & 7) != 0;
 }
@@ -504,7 +505,11 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   }
   beam_tile_cfg c;
   const KernelSet* ks;
-  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, -1, true))) return rc;
+  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, -1, true))) {
+    if (!rows_unaligned(A, B, C, K)) return rc;
+    BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, false, false, st));
+    return BEAM_OK;
+  }
   GemmParams p = base_params(A, B, M, N, K, c);
   p.C = C;
   const long tiles = (long)p.tiles_m * p.tiles_n;
@@ -564,7 +569,11 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
   }
   beam_tile_cfg c;
   const KernelSet* ks;
-  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, -1, true))) return rc;
+  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, -1, true))) {
+    if (N % 8 == 0 && !rows_unaligned(A, B, C, K)) return rc;
+    BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, true, false, st));
+    return BEAM_OK;
+  }
   if (!cfg) {
     // The library's choice is priced for B as [N][K].  In this layout a B fragment is two LDS reads, and the tiles
     // whose wavefronts are 64 columns wide pay for it: eight wavefronts of 64 x 32 instead of four of 64 x 64
@@ -634,7 +643,11 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   if ((rc = beam_init())) return rc;
   beam_tile_cfg c;
   const KernelSet* ks;
-  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks))) return rc;
+  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks))) {
+    if (!rows_unaligned(A, B, C, K)) return rc;
+    if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, cfg, stream))) return rc;
+    return beam_silu(X, Y, count, dtype, stream);
+  }
   // Too few workgroups to keep memory busy for the side job (the deep pipeline's problems, few rows): the two kernels one
   // after the other.
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
@@ -743,7 +756,7 @@ int beam_splitk_effective(int M, int N, int K, const beam_tile_cfg* cfg, int spl
   const KernelSet* ks;
   if (M <= 0 || N <= 0 || K < 0) return 1;
   if ((K > 0 && K < 8) || K > kMaxK) return 1;  // the plain kernel: no slices
-  if (resolve_cfg(cfg, M, N, K, &c, &ks, split_k > 0 ? split_k : 0)) return -1;
+  if (resolve_cfg(cfg, M, N, K, &c, &ks, split_k > 0 ? split_k : 0)) return K % 8 != 0 ? 1 : -1;
   return effective_split(M, N, K, c, split_k);
 }
 
@@ -789,7 +802,11 @@ int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int 
   }
   beam_tile_cfg c;
   const KernelSet* ks;
-  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, split_k > 0 ? split_k : 0))) return rc;
+  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, split_k > 0 ? split_k : 0))) {
+    if (!rows_unaligned(A, B, C, K)) return rc;
+    BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, false, false, st));
+    return BEAM_OK;
+  }
   int s = effective_split(M, N, K, c, split_k);
   // Operands whose rows are not 16-byte aligned may be given without room for slices (they need none: one pass).
   if (rows_unaligned(A, B, C, K) && (!ws || ws_bytes < splitk_partial_bytes(M, N, s))) s = 1;
@@ -993,8 +1010,8 @@ static int ln_resolve_cfg(const beam_tile_cfg* cfg, int M, int N, int K, int mod
 //   plain     the problem is outside what the tiled kernels take (K below 8 or beyond a descriptor, gamma or beta not
 //             8-byte aligned): plain GEMM into fp32 X, then a row-wise LayerNorm
 //   unaligned rows of A or B off 16 bytes or Y off 8 (rows_unaligned; K % 8 != 0 implies it).  The tiled kernels take
-//             them; where they would refuse the call (BEAM_LN_FUSED where it does not apply) it runs on the plain ones,
-//             which never refused such operands
+//             them; where they would refuse the call (a tile that is not compiled, BEAM_LN_FUSED where it does not apply)
+//             it runs on the plain ones, which never refused such operands
 //   capturing the stream is being captured: AUTO then means two passes (a replayed graph may share the device with
 //             other work, which the fused kernel's residency argument does not cover); an explicit FUSED is honoured
 //   wide_io   Y, gamma and beta are 16-byte aligned (the 4-wavefront kernel's vector accesses)
@@ -1016,13 +1033,13 @@ static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool
   }
   if (capturing && mode == BEAM_LN_AUTO) mode = BEAM_LN_TWOPASS;
   int rc = ln_resolve_cfg(cfg, M, N, K, mode, &out->c, &out->ks);
-  if (rc) return rc;
   beam_tile_cfg& c = out->c;
-  if (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N) && (unaligned || K % 8 != 0)) {
+  if ((unaligned || K % 8 != 0) && (rc || (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N)))) {
     out->kind = LnPlan::kPlain;
     out->need = ln_generic_need(M, N);
     return BEAM_OK;
   }
+  if (rc) return rc;
   if (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N))
     return fail(BEAM_ERR_UNSUPPORTED, "fused LayerNorm: needs a device of %d CUs and at most 64 column tiles (N=%d, block_n=%d, %d CUs)",
                 kNumXcd * 32, N, c.block_n, g_dev.cus);

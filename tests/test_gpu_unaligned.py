@@ -164,3 +164,48 @@ def test_layer_norm_one_kernel_form_where_it_does_not_apply(gpu, beamc, oracle, 
         v.ptr = 0
     for x in (da.buf, db.buf, c.buf, dg, dbt, ws):
         x.free()
+
+
+@pytest.mark.parametrize("tile", [(96, 64, 32, 32, 0, 0), (128, 128, 64, 64, 7, 0)])
+@pytest.mark.parametrize("shape,offs", [((65, 72, 65), (0, 0, 0)), ((65, 72, 64), (1, 0, 0)), ((65, 72, 64), (0, 2, 0)), ((65, 72, 64), (0, 0, 3))])
+def test_tile_that_is_not_compiled(gpu, beamc, oracle, tile, shape, offs):
+    """Rows off 16 bytes are computed whatever tile is named, by every entry point that takes one; aligned ones are
+    refused with it."""
+    M, N, K = shape
+    L = beamc.lib
+    cfg = beamc._TileCfg(*tile)
+    cp = ctypes.byref(cfg)
+    a, b, g, bt = make_ln_inputs(beamc, M, N, K, F16, 78)
+    bk = np.ascontiguousarray(b.T)
+    x = beamc.host_normal((1000,), F16, 78, 9, 0.0, 2.0)
+    dg, dbt, dx = (beamc.DeviceArray.from_numpy(v, F16) for v in (g, bt, x))
+    dy, dy2 = beamc.DeviceArray((1000,), F16), beamc.DeviceArray((1000,), F16)
+    beamc.silu(dx, dy2)
+    ws = beamc.DeviceArray((1 << 20,), itemsize=1)
+    ref, ref_nn, ref_ln = oracle.gemmrc(a, b, F16), oracle.matmul_nn(a, bk, F16), oracle.gemmrc_ln(a, b, g, bt, 1e-5, F16)
+    calls = {
+        "gemmrc": (b, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, F16, cp, None)),
+        "matmul": (bk, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, cp, None)),
+        "split-K": (b, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, F16, cp, 2, ws.ptr, ws.nbytes, None)),
+        "split-K, no workspace": (b, lambda pa, pb, pc: L.beam_gemmrc_splitk_noalloc(pa, pb, pc, M, N, K, F16, cp, 2, None)),
+        "with SiLU": (b, lambda pa, pb, pc: L.beam_parallel_gemmrc_silu(pa, pb, pc, M, N, K, dx.ptr, dy.ptr, 1000, F16, cp, None)),
+        "LayerNorm": (b, lambda pa, pb, pc: L.beam_gemmrc_ln_ex(pa, pb, dg.ptr, dbt.ptr, 1e-5, pc, M, N, K, F16, cp, beamc.LN_AUTO, ws.ptr,
+                                                                ws.nbytes, None)),
+    }
+    for what, (bb, call) in calls.items():
+        out = run(beamc, call, a, bb, (M, N), F16, offs)
+        if what == "LayerNorm":
+            check_ln(oracle, out, ref_ln, F16, what)
+        else:
+            close_enough(oracle, out, ref_nn if what == "matmul" else ref, K, F16, what)
+        if K % 8 == 0:
+            da, db, c = Embedded(beamc, a.shape, F16, 0, a), Embedded(beamc, bb.shape, F16, 0, bb), Embedded(beamc, (M, N), F16, 0)
+            assert call(da.ptr, db.ptr, c.ptr) == 2, what
+            for v in (da, db, c):
+                v.buf.free()
+    assert (dy.to_numpy() == dy2.to_numpy()).all()
+    if K % 8 != 0:
+        assert L.beam_splitk_effective(M, N, K, cp, 2) == 1
+        assert L.beam_gemmrc_ln_workspace_bytes_for(M, N, K, cp, beamc.LN_AUTO) >= M * N * 4
+    for v in (dg, dbt, dx, dy, dy2, ws):
+        v.free()
