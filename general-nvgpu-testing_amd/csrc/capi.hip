@@ -643,11 +643,13 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   if ((rc = beam_init())) return rc;
   beam_tile_cfg c;
   const KernelSet* ks;
-  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks))) {
-    if (!rows_unaligned(A, B, C, K)) return rc;
+  rc = resolve_cfg(cfg, M, N, K, &c, &ks);
+  if (cfg && (rc || c.pipeline == 2)) {  // no kernel carries a side job there
+    if (!rows_unaligned(A, B, C, K)) return rc ? rc : fail(BEAM_ERR_UNSUPPORTED, "the side job runs with pipeline 0 or 1");
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, cfg, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }
+  if (rc) return rc;
   // Too few workgroups to keep memory busy for the side job (the deep pipeline's problems, few rows): the two kernels one
   // after the other.
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
@@ -655,7 +657,6 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }
-  if (c.pipeline == 2) return fail(BEAM_ERR_UNSUPPORTED, "the side job runs with pipeline 0 or 1");
   GemmParams p = base_params(A, B, M, N, K, c);
   p.C = C;
   p.side_x = X;

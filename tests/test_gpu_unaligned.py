@@ -166,6 +166,25 @@ def test_layer_norm_one_kernel_form_where_it_does_not_apply(gpu, beamc, oracle, 
         x.free()
 
 
+@pytest.mark.parametrize("shape,offs", [((65, 72, 65), (0, 0, 0)), ((130, 72, 64), (1, 0, 0)), ((65, 200, 192), (0, 2, 0)), ((65, 72, 64), (0, 0, 3))])
+@pytest.mark.parametrize("tile", [(64, 64, 32, 32), (128, 128, 64, 64)])
+def test_side_job_beside_the_deep_pipeline(gpu, beamc, oracle, tile, shape, offs):
+    """The deep pipeline carries no side job: refused on aligned rows (test_gpu_silu), computed in two launches on others."""
+    M, N, K = shape
+    L = beamc.lib
+    cfg = beamc.TileConfig(*tile, 2, 0).to_c()
+    a, b = beamc.host_uniform((M, K), BF16, 79, 0), beamc.host_uniform((N, K), BF16, 79, 1)
+    dx = beamc.DeviceArray.from_numpy(beamc.host_normal((3001,), BF16, 79, 2, 0.0, 2.0), BF16)
+    dy, dy2 = beamc.DeviceArray((3001,), BF16), beamc.DeviceArray((3001,), BF16)
+    beamc.silu(dx, dy2)
+    out = run(beamc, lambda pa, pb, pc: L.beam_parallel_gemmrc_silu(pa, pb, pc, M, N, K, dx.ptr, dy.ptr, 3001, BF16, ctypes.byref(cfg), None),
+              a, b, (M, N), BF16, offs)
+    close_enough(oracle, out, oracle.gemmrc(a, b, BF16), K, BF16, f"{shape} at {offs}")
+    assert (dy.to_numpy() == dy2.to_numpy()).all()
+    for v in (dx, dy, dy2):
+        v.free()
+
+
 @pytest.mark.parametrize("tile", [(96, 64, 32, 32, 0, 0), (128, 128, 64, 64, 7, 0)])
 @pytest.mark.parametrize("shape,offs", [((65, 72, 65), (0, 0, 0)), ((65, 72, 64), (1, 0, 0)), ((65, 72, 64), (0, 2, 0)), ((65, 72, 64), (0, 0, 3))])
 def test_tile_that_is_not_compiled(gpu, beamc, oracle, tile, shape, offs):
