@@ -1060,6 +1060,18 @@ static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool
   return BEAM_OK;
 }
 
+// The plan of a call: the above for its operands and its workspace.  Unaligned rows have always got by with room for fp32 X
+// on 16 bytes; a workspace that has that, and not what the tiled kernels ask for, still means the plain ones.
+static int ln_plan_call(const void* A, const void* B, const void* gamma, const void* beta, const void* Y, int M, int N, int K,
+                        const beam_tile_cfg* cfg, int mode, bool generic, bool capturing, const void* ws, size_t ws_bytes, LnPlan* out) {
+  const bool unaligned = rows_unaligned(A, B, Y, K);
+  const bool wide_io = (((uintptr_t)Y | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0;
+  if (int rc = ln_plan(M, N, K, cfg, mode, ln_is_generic(generic, gamma, beta), unaligned, capturing, wide_io, out)) return rc;
+  if (unaligned && out->kind != LnPlan::kPlain && (!ws || ws_bytes < out->need || ((uintptr_t)ws & 255) != 0))
+    return ln_plan(M, N, K, cfg, mode, true, unaligned, capturing, wide_io, out);
+  return BEAM_OK;
+}
+
 // Enough for beam_gemmrc_ln_ex(M, N, K, cfg, mode) on operands aligned as the tiled kernels need them.  AUTO covers
 // both forms it can resolve to (one kernel eagerly, two passes under stream capture and as the retry of
 // beam_gemmrc_ln_checked), which also covers the plain path.
@@ -1141,8 +1153,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (st != nullptr) (void)hipStreamIsCapturing(st, &capturing);
   LnPlan plan;
-  if ((rc = ln_plan(M, N, K, cfg, mode, ln_is_generic(generic, gamma, beta), rows_unaligned(A, B, Y, K), capturing != hipStreamCaptureStatusNone,
-                    (((uintptr_t)Y | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0, &plan)))
+  if ((rc = ln_plan_call(A, B, gamma, beta, Y, M, N, K, cfg, mode, generic, capturing != hipStreamCaptureStatusNone, ws, ws_bytes, &plan)))
     return rc;
   const size_t need = plan.need;
   if (!ws || ws_bytes < need)
@@ -1257,8 +1268,7 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   bool generic;
   (void)check_problem(A, B, Y, M, N, K, dtype, &generic);
   LnPlan plan;
-  if (ln_plan(M, N, K, cfg, BEAM_LN_AUTO, ln_is_generic(generic, gamma, beta), rows_unaligned(A, B, Y, K), false,
-              (((uintptr_t)Y | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0, &plan) || plan.kind != LnPlan::kFused)
+  if (ln_plan_call(A, B, gamma, beta, Y, M, N, K, cfg, BEAM_LN_AUTO, generic, false, ws, ws_bytes, &plan) || plan.kind != LnPlan::kFused)
     return BEAM_OK;  // nothing in the call waits for anything
   if (word) {
     BEAM_HIP(hipStreamSynchronize(st));

@@ -131,6 +131,30 @@ def test_layer_norm(gpu, beamc, oracle, shape, dtype):
     dbt.free()
 
 
+@pytest.mark.parametrize("shape,offs", [((130, 3, 65), (0, 0, 0)), ((130, 257, 71), (0, 0, 0)), ((130, 257, 72), (1, 0, 0)), ((65, 72, 64), (0, 0, 3))])
+def test_layer_norm_workspace_of_the_plain_kernels(gpu, beamc, oracle, shape, offs):
+    """Unaligned rows need M * N fp32 values on a 16-byte boundary and no more, whatever the mode."""
+    M, N, K = shape
+    L = beamc.lib
+    a, b, g, bt = make_ln_inputs(beamc, M, N, K, F16, 80)
+    ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, F16)
+    dg, dbt = beamc.DeviceArray.from_numpy(g, F16), beamc.DeviceArray.from_numpy(bt, F16)
+    room = (M * N * 4 + 255) // 256 * 256
+    ws = beamc.DeviceArray((room + 16 + 256,), itemsize=1)
+    for mode in (beamc.LN_AUTO, beamc.LN_TWOPASS, beamc.LN_FUSED):
+        for at in (0, 16):
+            ws.fill_bytes(0xEE)
+            out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_ln_ex(pa, pb, dg.ptr, dbt.ptr, 1e-5, pc, M, N, K, F16, None, mode, ws.ptr + at,
+                                                                    room, None), a, b, (M, N), F16, offs)
+            check_ln(oracle, out, ref, F16, f"mode {mode}, workspace at {at}")
+            assert (ws.to_numpy(np.uint8)[room + at:] == 0xEE).all(), "written beyond the workspace"
+    out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_ln_checked(pa, pb, dg.ptr, dbt.ptr, 1e-5, pc, M, N, K, F16, None, ws.ptr + 16, room, None,
+                                                                 None), a, b, (M, N), F16, offs)
+    check_ln(oracle, out, ref, F16, "checked")
+    for v in (dg, dbt, ws):
+        v.free()
+
+
 @pytest.mark.parametrize("offs", [(1, 0, 0), (0, 3, 0), (0, 0, 1), (4, 4, 2)])
 def test_layer_norm_one_kernel_form_where_it_does_not_apply(gpu, beamc, oracle, offs):
     """More than 64 column tiles: BEAM_LN_FUSED is refused on aligned operands and computed (by the plain kernels) on
