@@ -809,8 +809,9 @@ int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int 
     return BEAM_OK;
   }
   int s = effective_split(M, N, K, c, split_k);
-  // Operands whose rows are not 16-byte aligned may be given without room for slices (they need none: one pass).
-  if (rows_unaligned(A, B, C, K) && (!ws || ws_bytes < splitk_partial_bytes(M, N, s))) s = 1;
+  // Operands whose rows are not 16-byte aligned may be given without room for slices, or with it off 16 bytes (they need
+  // none: one pass).
+  if (rows_unaligned(A, B, C, K) && (!ws || ((uintptr_t)ws & 15) != 0 || ws_bytes < splitk_partial_bytes(M, N, s))) s = 1;
   if (split_k <= 0 && g_verbose.load(std::memory_order_relaxed)) log_split_choice_once(M, N, K, dtype, c, s);
   if (s == 1) {  // nothing to reduce: the plain kernel writes C directly
     GemmParams p = base_params(A, B, M, N, K, c);

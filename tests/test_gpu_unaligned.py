@@ -62,6 +62,22 @@ def test_any_k(gpu, beamc, oracle, K, dtype):
             close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"split-K {(M, N, K)} room {room}")
 
 
+@pytest.mark.parametrize("shape,offs", [((65, 72, 321), (0, 0, 0)), ((65, 72, 320), (0, 1, 0))])
+def test_split_k_workspace_off_16_bytes(gpu, beamc, oracle, shape, offs):
+    """Unaligned rows never needed a workspace: one that is off 16 bytes is left alone."""
+    M, N, K = shape
+    L = beamc.lib
+    a, b = beamc.host_uniform((M, K), F16, 81, 0), beamc.host_uniform((N, K), F16, 81, 1)
+    ws = beamc.DeviceArray((L.beam_splitk_workspace_bytes(M, N, 3) + 256,), itemsize=1)
+    ws.fill_bytes(0xEE)
+    for at in (2, 8):
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, F16, None, 3, ws.ptr + at, ws.nbytes - at, None), a, b,
+                  (M, N), F16, offs)
+        close_enough(oracle, out, oracle.gemmrc(a, b, F16), K, F16, f"workspace at {at}")
+    assert (ws.to_numpy(np.uint8) == 0xEE).all()
+    ws.free()
+
+
 # N around one chunk, around the tiles' widths, and a last K tile that is whole (64, 128) or short
 @pytest.mark.parametrize("N", [8, 9, 63, 65, 127, 129, 255, 257, 1001])
 @pytest.mark.parametrize("dtype", [F16, BF16])
