@@ -1261,17 +1261,14 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (st != nullptr) (void)hipStreamIsCapturing(st, &capturing);
   // (captured: AUTO is two passes, which wait for nothing; a stream being captured cannot be waited for anyway)
-  int rc = beam_init();
-  if (rc && M > 0 && N > 0) return rc;
-  const volatile unsigned* word = g_ln_host_timeout;
-  rc = beam_gemmrc_ln_ex(A, B, gamma, beta, eps, Y, M, N, K, dtype, cfg, BEAM_LN_AUTO, ws, ws_bytes, stream);
+  int rc = beam_gemmrc_ln_ex(A, B, gamma, beta, eps, Y, M, N, K, dtype, cfg, BEAM_LN_AUTO, ws, ws_bytes, stream);
   if (rc || capturing != hipStreamCaptureStatusNone || M == 0 || N == 0) return rc;
   bool generic;
   (void)check_problem(A, B, Y, M, N, K, dtype, &generic);
   LnPlan plan;
   if (ln_plan_call(A, B, gamma, beta, Y, M, N, K, cfg, BEAM_LN_AUTO, generic, false, ws, ws_bytes, &plan) || plan.kind != LnPlan::kFused)
     return BEAM_OK;  // nothing in the call waits for anything
-  if (word) {
+  if (const volatile unsigned* word = g_ln_host_timeout) {
     BEAM_HIP(hipStreamSynchronize(st));
     if (*word == 0) return BEAM_OK;
   }

@@ -343,6 +343,24 @@ def test_argument_validation_without_gpu(beamc):
     assert L.beam_get_config(10 ** 6, ctypes.byref(out)) == 1
 
 
+def test_argument_validation_of_the_checked_layer_norm_without_gpu(beamc):
+    """The checked GEMM+LayerNorm looks at its arguments before it looks for a device, like the unchecked one."""
+    P = 1 << 20
+
+    def both(A, B, g, bt, eps, Y, M, N, K, dtype):
+        first = beamc.lib.beam_gemmrc_ln_ex(A, B, g, bt, eps, Y, M, N, K, dtype, None, 0, P, 1 << 30, None)
+        assert beamc.lib.beam_gemmrc_ln_checked(A, B, g, bt, eps, Y, M, N, K, dtype, None, P, 1 << 30, None, None) == first
+        return first
+
+    assert both(P, P, P, P, 1e-5, P, -1, 4, 8, 0) == 1
+    assert both(P, P, P, P, 1e-5, P, 4, 4, 8, 7) == 2
+    assert both(P, None, P, P, 1e-5, P, 4, 4, 8, 0) == 1
+    assert both(P + 1, P, P, P, 1e-5, P, 4, 4, 8, 0) == 1
+    assert both(P, P, None, P, 1e-5, P, 4, 4, 8, 0) == 1
+    assert both(P, P, P, P, -1.0, P, 4, 4, 8, 0) == 1
+    assert both(P, P, P, P, 1e-5, P, 0, 4, 8, 0) == 0
+
+
 def test_config_table(beamc):
     cfgs = beamc.list_configs()
     shapes = {(c.block_m, c.block_n, c.wave_m, c.wave_n) for c in cfgs}
