@@ -177,7 +177,8 @@ int auto_slices(long tiles, int K, int cus) {
   return s < 1 ? 1 : (int)s;
 }
 
-int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* split_k);
+// *raised (may be null): the tile's own depth is pipeline 0, and only the two K groups made it the deep pipeline.
+int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* split_k, bool* raised = nullptr);
 
 // split_req: -1 the caller cannot run K slices (no workspace); 0 it can, and leaves the number to
 // the library; > 0 it asks for that many.  The default tile is chosen for that situation.
@@ -374,7 +375,7 @@ int beam_default_config(int M, int N, int K, beam_tile_cfg* cfg, int* split_k) {
 
 namespace {
 
-int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* split_k) {
+int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* split_k, bool* raised) {
   if (!cfg) return fail(BEAM_ERR_INVALID, "null cfg");
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -447,7 +448,12 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
   // tiles, one group -> two: 8192 x 256 x 2048 17.6 -> 12.3 us, 654 x 1832 x 2104 21.5 -> 16.8, 2048 x 1024 x 2048 11.8 ->
   // 11.4; 64 x 64 tiles 1024 x 1024 x 2048 8.1 -> 7.7.  At K = 1024 one group is ahead (5.2, 5.5; 6.7, 7.2).
   const long picked = tiles(c.block_m, c.block_n);
-  if (split_req < 0 && K >= 2048 && (picked < cus / 2 || (picked <= cus && c.block_m * c.block_n <= 128 * 64))) cfg->pipeline = 2;
+  const bool few = picked < cus / 2, groups = picked <= cus && c.block_m * c.block_n <= 128 * 64;
+  if (raised) *raised = false;
+  if (split_req < 0 && K >= 2048 && (few || groups)) {
+    if (raised) *raised = !few && c.pipeline == 0;
+    cfg->pipeline = 2;
+  }
   // K slices on at most half the CUs: every workgroup has the memory system of two CUs to itself, the long
   // queue's prologue costs more than it hides (64 x 128 x 65536 in 64 slices: 8.9 against 9.9 us), and the
   // reducing workgroups of the one-launch form start on the idle CUs at once.
@@ -644,6 +650,16 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   beam_tile_cfg c;
   const KernelSet* ks;
   rc = resolve_cfg(cfg, M, N, K, &c, &ks);
+  if (cfg && !rc && c.pipeline == 2) {
+    // beam_default_config names the deep pipeline for tiles that it otherwise names with pipeline 0; passed on to here, such
+    // a tile carries the job with that
+    beam_tile_cfg own;
+    int own_split;
+    bool raised = false;
+    if (choose_default(M, N, K, -1, &own, &own_split, &raised) == BEAM_OK && raised && own.block_m == c.block_m &&
+        own.block_n == c.block_n && own.wave_m == c.wave_m && own.wave_n == c.wave_n)
+      c.pipeline = 0;
+  }
   if (cfg && (rc || c.pipeline == 2)) {  // no kernel carries a side job there
     if (!rows_unaligned(A, B, C, K)) return rc ? rc : fail(BEAM_ERR_UNSUPPORTED, "the side job runs with pipeline 0 or 1");
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, cfg, stream))) return rc;

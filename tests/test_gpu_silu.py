@@ -227,3 +227,22 @@ def test_pair_error_paths(gpu, beamc):
     assert rc == 1
     for t in (a, b, c, x, y, y2, y3):
         t.free()
+
+
+@pytest.mark.parametrize("shape", [(2048, 1024, 2048), (654, 1832, 2104), (768, 2560, 2048), (3100, 4000, 256)])
+def test_pair_takes_the_default_tile(gpu, beamc, oracle, shape):
+    """The tile that beam_default_config names can be passed on to the pair, also where the GEMM alone runs it with two K
+    groups, which carry no side job."""
+    M, N, K = shape
+    cfg, _ = beamc.default_config(M, N, K)
+    assert (cfg.pipeline == 2) == (K >= 2048)
+    a, b = beamc.host_uniform((M, K), F16, 35, 0), beamc.host_uniform((N, K), F16, 35, 1)
+    x = beamc.host_normal((70001,), F16, 35, 2, 0.0, 2.5)
+    da, db, dx = (beamc.DeviceArray.from_numpy(v, F16) for v in (a, b, x))
+    c, y = beamc.DeviceArray((M, N), F16), beamc.DeviceArray((70001,), F16)
+    beamc.parallel_gemmrc_silu(da, db, c, dx, y, config=cfg)
+    r = oracle.compare(c.to_numpy(), oracle.gemmrc(a, b, F16), F16)
+    assert r["max_abs_err"] <= oracle.gemm_tolerance(K) * r["rms_ref"]
+    assert_same_bits(y.to_numpy(), run_silu(beamc, x, F16), x, "side job")
+    for t in (da, db, dx, c, y):
+        t.free()
