@@ -666,20 +666,32 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
     return beam_silu(X, Y, count, dtype, stream);
   }
   if (rc) return rc;
-  // Too few workgroups to keep memory busy for the side job (the deep pipeline's problems, few rows): the two kernels one
-  // after the other.
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
-  if (!cfg && (c.pipeline == 2 || rows_plan(M, N, K, cus) != kRowsNone)) {
-    if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
-    return beam_silu(X, Y, count, dtype, stream);
+  const long long wgs = (long long)((M + c.block_m - 1) / c.block_m) * ((N + c.block_n - 1) / c.block_n);
+  const long long per_pass = wgs * ks->threads;  // units one K tile of the whole grid covers
+  // With the library's tile, a GEMM kernel that carries no side job and is the faster one by more than the second launch
+  // costs (2.5 us), or too few workgroups to keep memory busy for a long job: the two kernels one after the other.
+  //   * The deep pipeline: less than half the CUs busy, or tiles of 64 rows (two K groups).  2^18 elements, one launch, two
+  //     launches: 155 x 2040 x 1536 10.1, 9.1 us; 2048 x 1024 x 2048 18.9, 15.9; 580 x 968 x 5672 39.4, 29.4.  Tiles of 128
+  //     rows gain less than that: 128 x 128 (one group) 496 x 5688 x 1224 13.2, 15.3; 530 x 4400 x 3528 36.0, 37.2; 128 x 64
+  //     1377 x 1416 x 832 7.7, 9.8; 5813 x 312 x 6256 46.4, 47.2.
+  //   * Few rows, whose launch alone takes 3-5 us: from K = 768 on (1 x 512, 2^12 elements: K = 512 4.8, 5.4; K = 1024 7.1,
+  //     5.5), or from 8 passes of the grid over the job on (1 x 1024 x 64 with 2^19 9.9, 5.4; 64 x 64 x 64 with 2^12 3.6, 5.4).
+  if (!cfg) {
+    const bool two_groups = c.block_m == 64;
+    const bool deep = c.pipeline == 2 && (wgs * 2 < cus || two_groups);
+    const bool rows = rows_plan(M, N, K, cus) != kRowsNone && (K >= 768 || (count >> 3) > 8 * per_pass);
+    if (deep || rows) {
+      if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
+      return beam_silu(X, Y, count, dtype, stream);
+    }
+    if (c.pipeline == 2) c.pipeline = 0;
   }
   GemmParams p = base_params(A, B, M, N, K, c);
   p.C = C;
   p.side_x = X;
   p.side_y = Y;
   p.side_count = count;
-  const long long wgs = (long long)p.tiles_m * p.tiles_n;
-  const long long per_pass = wgs * ks->threads;  // units one K tile of the whole grid covers
   // The narrowest unit with which the job still ends inside the K loop: the work is then spread
   // evenly over the tiles instead of crowding the first ones.  A job longer than the loop keeps
   // 16-byte units and finishes after the GEMM's epilogue.
@@ -694,11 +706,12 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   }
   p.side_iters = (int)(((count >> 3) * (16 / p.side_width) + per_pass - 1) / per_pass);
   // A job that outlasts the loop goes on at 0.4-1.4 us for every 16 bytes per thread; with a round of workgroups or less,
-  // from 8 such passes on, a launch of its own (3 us and 11 us per 16 Mi elements) is ahead.  Fused, then two launches:
+  // from 8 such passes on (more behind a long loop, whose own passes are the cheaper for it: 992 x 3976 x 3288 with 2^26
+  // elements, 52 K tiles and 12 passes beyond them, 84.4, 88.9), a launch of its own (3 us and 11 us per 16 Mi elements) is ahead.  Fused, then two launches:
   // 256^3 with 2^20 elements (28 passes) 15.8, 6.5 us; 1024^3 with 2^24 (16) 30.3, 20.7; 4096 x 4096 x 256 with 2^24 (12)
   // 28.9, 26.4; but 1536 x 1536 x 512 with 2^22 (7) 9.4, 10.5.  With several rounds the later workgroups hide it:
   // 8192 x 8192 x 256 with 2^26 (12) 110.8, 117.7.
-  if (!cfg && wgs <= cus && p.side_iters - k_tiles > 8) {
+  if (!cfg && wgs <= cus && p.side_iters - k_tiles > 8 + k_tiles / 8) {
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }

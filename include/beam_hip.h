@@ -219,8 +219,9 @@ int beam_set_ln_walk(int on);
 
 /* ---- GEMM with an independent elementwise job hidden in its K loop ------------------------ */
 
-/* C = A . B^T as beam_gemmrc and, in the same launch (with cfg NULL in a second one where the GEMM has too few workgroups, or
- * too short a K loop, to carry the job), Y[i] = silu(X[i]) = X[i] / (1 + exp(-X[i]))
+/* C = A . B^T as beam_gemmrc (with cfg NULL its sums may be added in another order than there) and, in the same launch (with
+ * cfg NULL in a second one where the GEMM's own kernel is the faster by more than that costs, has too few workgroups for the
+ * job, or too short a K loop), Y[i] = silu(X[i]) = X[i] / (1 + exp(-X[i]))
  * for i in [0, count): 16-bit in, fp32 arithmetic, round-to-nearest 16-bit out.  The array is cut into
  * units of 4, 8 or 16 bytes (the narrowest with which the job still ends inside the K loop), dealt out in
  * contiguous runs over the GEMM's workgroups and carried, a few units per K tile, by the wavefronts that

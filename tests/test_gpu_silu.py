@@ -246,3 +246,29 @@ def test_pair_takes_the_default_tile(gpu, beamc, oracle, shape):
     assert_same_bits(y.to_numpy(), run_silu(beamc, x, F16), x, "side job")
     for t in (da, db, dx, c, y):
         t.free()
+
+
+# (shape, elements): few rows under a short loop and with a small job (one launch), a long loop, a long job (two launches);
+# the deep pipeline with few workgroups and with 64-row tiles (two) and 128-row tiles (one); a job far beyond the loop (two)
+@pytest.mark.parametrize("shape,count", [((16, 512, 256), 5000), ((64, 300, 767), 20001), ((16, 512, 768), 5000), ((1, 64, 64), 16385), ((33, 1000, 64), 300003),
+                                         ((256, 256, 4096), 100003), ((768, 2560, 2048), 70001), ((496, 5688, 1224), 70001), ((1377, 1416, 832), 70001),
+                                         ((256, 256, 256), 1 << 20), ((1024, 1024, 200), (1 << 22) + 5)])
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_pair_routes(gpu, beamc, oracle, shape, count, dtype):
+    """Without a tile: whether the pair is one launch or two, C and Y are whole and nothing else is written."""
+    M, N, K = shape
+    a, b = beamc.host_uniform((M, K), dtype, 36, 0), beamc.host_uniform((N, K), dtype, 36, 1)
+    x = beamc.host_normal((count,), dtype, 36, 2, 0.0, 2.5)
+    da, db, dx = (beamc.DeviceArray.from_numpy(v, dtype) for v in (a, b, x))
+    c, y = beamc.DeviceArray((M * N + 8,), dtype), beamc.DeviceArray((count + 8,), dtype)
+    c.fill_bytes(0xEE)
+    y.fill_bytes(0xEE)
+    beamc._check(beamc.lib.beam_parallel_gemmrc_silu(da.ptr, db.ptr, c.ptr, M, N, K, dx.ptr, y.ptr, count, dtype, None, None))
+    cout, yout = c.to_numpy(), y.to_numpy()
+    assert (cout[M * N:] == 0xEEEE).all() and (yout[count:] == 0xEEEE).all()
+    r = oracle.compare(cout[:M * N].reshape(M, N), oracle.gemmrc(a, b, dtype), dtype)
+    err = r["max_abs_err"] if dtype == F16 else r["max_bf16_excess"]
+    assert err <= oracle.gemm_tolerance(K) * r["rms_ref"]
+    assert_same_bits(yout[:count], run_silu(beamc, x, dtype), x, "side job")
+    for t in (da, db, dx, c, y):
+        t.free()
