@@ -462,22 +462,24 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
   return BEAM_OK;
 }
 
-// Which form of the kernel for few rows (gemm_rows.h), if any, runs c = a @ b^T.  bf16, us, tiled kernel -> this one:
-//   * Up to 16 columns for every CU, one form is ahead for every K: 4096 columns, M = 16 K = 128 3.6 -> 3.3,
-//     K = 16384 37.3 -> 25.7; M = 64 K = 128 3.9 -> 3.6, K = 1024 5.0 -> 4.1, K = 16384 41.9 -> 33.1.
+// Which form of the kernel for few rows (gemm_rows.h), if any, runs c = a @ b^T.  us, the best tiled kernel -> this one:
+//   * Up to 16 columns for every CU, 16 columns per workgroup: 4096 columns, M = 16 K = 128 3.6 -> 3.3, K = 16384
+//     37.3 -> 25.7; M = 64 K = 512 3.6 -> 3.5, K = 1024 5.0 -> 4.1, K = 16384 41.9 -> 33.1.  Beyond 32 rows the K tiles have
+//     to be more than the wavefronts: M = 64 K = 128 2.8, here 3.0, K = 320 3.1, here 3.3.
 //   * Beyond that the fetches of A add up, and B's become the bound.  M <= 16, K <= 4096: 64 columns per workgroup,
-//     M = 1: 5000 x 4096 11.7 -> 7.9, 16384 x 1024 7.4 -> 3.8, 11008 x 4096 15.0 -> 14.5 (M = 16 15.6 -> 15.5),
-//     16384 x 3000 17.6 -> 15.9; the tiled kernel is ahead from there on (16384 x 4088 20.6, here 27.2) and where K is
-//     so short that the workgroups' starts count (65536 x 512 11.0, here 12.1).
-//   * Longer K: 16 columns, fewer wavefronts: M = 16 6000 x 9000 26.8 -> 23.3, 8192 x 11008 32.1 -> 27.8, but
-//     10000 x 6000 21.4, here 23.0.
-//   * M <= 32: 32 columns per workgroup, 8192 x 1024 5.1 -> 4.3, x 2048 7.6 -> 6.4; 16384 x 512 3.7, here 5.0.
+//     M = 1: 5120 x 4096 11.7 -> 8.0, 16384 x 1024 5.4 -> 3.7, 11008 x 4096 14.8 -> 14.3, M = 16 10240 x 4096 14.8 -> 14.6,
+//     14336 x 3072 15.0 -> 14.5; the tiled kernel is ahead from there on (M = 16 11008 x 4096 15.3, here 15.6; 16384 x 4088
+//     20.6, here 27.2) and where K is so short that the workgroups' starts count (65536 x 512 11.0, here 12.1).
+//   * Longer K: 16 columns, fewer wavefronts: M = 16 6144 x 10240 24.7 -> 21.8, 7168 x 12288 29.1 -> 26.1; behind in
+//     K = 8192, the more so the wider (7168 x 8192 20.5, here 24.4; 8192 x 8192 21.5, here 29.4).
+//   * M <= 32: 32 columns per workgroup, 8192 x 1024 4.9 -> 4.2, x 2048 7.7 -> 6.4; 16384 x 512 3.7, here 5.0.
 RowsPlan rows_plan(int M, int N, int K, int cus) {
   if (M > 64 || K % 8 != 0 || K > kRowsMaxK) return kRowsNone;
   const long cols = N, round = 16L * cus;  // columns of one workgroup of 16 per CU
-  if (cols <= round) return kRowsNarrow;
+  if (cols <= round) return M <= 32 || K > 320 ? kRowsNarrow : kRowsNone;
   if (M <= 16) {
-    if (K > 4096) return cols <= 2 * round ? kRowsDeep : kRowsNone;
+    if (K > 4096) return 4 * cols <= 7 * round ? kRowsDeep : kRowsNone;
+    if (M > 8 && K > 3072 && 2 * cols > 5 * round) return kRowsNone;
     return K >= 512 && cols <= 4 * round && cols * K <= (3L << 24) ? kRowsWide : kRowsNone;
   }
   if (M <= 32 && cols <= 2 * round && K >= 1024 && K <= 2048) return kRowsWide;
