@@ -462,6 +462,17 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
   return BEAM_OK;
 }
 
+// The deep pipeline of the library's own tile as one K group (KernelSet::launch_deep_one_group), or nullptr for two.  Where
+// one row of 64 x 64 tiles nearly fills the chip, B is read once and memory is the bound; one ring of 8 + 7 slots then keeps
+// more of it in flight than two of 5 + 4.  fp16, us, two groups -> one: [N][K] from 3/4 of a round on, 33 x 12288 x 2048
+// 10.5 -> 10.1, 16 x 14336 x 8192 35.4 -> 33.9, 64 x 12288 x 16384 94.5 -> 89.6; below it 17 x 11008 x 8192 27.5, 28.4.
+// [K][N] from 7/8 on: 16 x 16384 x 8192 45.9 -> 42.6, x 12288 81.5 -> 72.7.
+GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, int N, int dtype, bool b_kmajor, int cus) {
+  if (c.pipeline != 2 || M > c.block_m) return nullptr;
+  const long tiles = (N + c.block_n - 1) / c.block_n;
+  return 8 * tiles >= (b_kmajor ? 7L : 6L) * cus ? ks.launch_deep_one_group[dtype][b_kmajor ? 1 : 0] : nullptr;
+}
+
 // Which form of the kernel for few rows (gemm_rows.h), if any, runs c = a @ b^T.  us, the best tiled kernel -> this one:
 //   * Up to 16 columns for every CU, 16 columns per workgroup: 4096 columns, M = 16 K = 128 3.6 -> 3.3, K = 16384
 //     37.3 -> 25.7; M = 64 K = 512 3.6 -> 3.5, K = 1024 5.0 -> 4.1, K = 16384 41.9 -> 33.1.  Beyond 32 rows the K tiles have
@@ -554,7 +565,8 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     BEAM_HIP(loop(p, dim3((unsigned)cus, 1, 1), st));
     return BEAM_OK;
   }
-  BEAM_HIP(ks->launch[dtype][kEpiStore][c.pipeline](p, dim3((unsigned)tiles, 1, 1), st));
+  GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, dtype, false, cus);
+  BEAM_HIP((one_group ? one_group : ks->launch[dtype][kEpiStore][c.pipeline])(p, dim3((unsigned)tiles, 1, 1), st));
   return BEAM_OK;
 }
 
@@ -609,14 +621,15 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
   }
   GemmParams p = base_params(A, B, M, N, K, c);
   p.C = C;
+  const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   if (w4_fits && w4_named) {
     const long tiles = (long)p.tiles_m * p.tiles_n;
-    const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
     p.c_streaming = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024;
     BEAM_HIP(launch_gemm_w4_kmajor(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
-  BEAM_HIP(ks->launch_kmajor[dtype][c.pipeline](p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
+  GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, dtype, true, cus);
+  BEAM_HIP((one_group ? one_group : ks->launch_kmajor[dtype][c.pipeline])(p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
   return BEAM_OK;
 }
 
@@ -847,7 +860,8 @@ int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int 
   if (s == 1) {  // nothing to reduce: the plain kernel writes C directly
     GemmParams p = base_params(A, B, M, N, K, c);
     p.C = C;
-    BEAM_HIP(ks->launch[dtype][kEpiStore][c.pipeline](p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
+    GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, dtype, false, g_dev.cus > 0 ? g_dev.cus : 256);
+    BEAM_HIP((one_group ? one_group : ks->launch[dtype][kEpiStore][c.pipeline])(p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
     return BEAM_OK;
   }
   const size_t need = splitk_partial_bytes(M, N, s);

@@ -23,6 +23,8 @@ struct KernelSet {
   GemmLauncher launch[2][kNumEpilogues][3];
   // B stored [K][N] instead of [N][K], kEpiStore only: [dtype][pipeline]
   GemmLauncher launch_kmajor[2][3];
+  // The deep pipeline as one K group where `launch` has two, 64 x 64 tiles only: [dtype][B stored [K][N]]; nullptr otherwise.
+  GemmLauncher launch_deep_one_group[2][2];
   // Split-K in one launch (kEpiPartialFused), tiles up to 128 x 128 only (what split-K problems run on):
   // [dtype][pipeline]; nullptr otherwise.
   GemmLauncher launch_partial_fused[2][3];
@@ -69,6 +71,12 @@ GemmLauncher partial_fused_launcher() {
   else return nullptr;
 }
 
+template <typename T, int BM, int BN, int WVM, int WVN, bool B_KMAJOR>
+GemmLauncher deep_one_group_launcher() {
+  if constexpr (BM * BN <= 64 * 64) return launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, 8, 7, B_KMAJOR>;
+  else return nullptr;
+}
+
 template <int BM, int BN, int TM, int TN>
 KernelSet make_kernel_set() {
   constexpr int WVM = BM / TM, WVN = BN / TN;
@@ -102,6 +110,8 @@ KernelSet make_kernel_set() {
   k.launch_kmajor[D][0] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, 3, 2, true>; \
   k.launch_kmajor[D][1] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, 2, 2, true>; \
   k.launch_kmajor[D][2] = launch_gemm<T, BM, BN, WVM, WVN, kEpiStore, DA, DB, true, KG>; \
+  k.launch_deep_one_group[D][0] = deep_one_group_launcher<T, BM, BN, WVM, WVN, false>(); \
+  k.launch_deep_one_group[D][1] = deep_one_group_launcher<T, BM, BN, WVM, WVN, true>();  \
   k.launch[D][kEpiStoreLoop][0] = loop_launcher<T, BM, BN, WVM, WVN>();              \
   k.launch[D][kEpiStoreLoop][1] = nullptr;                                            \
   k.launch[D][kEpiStoreLoop][2] = nullptr;                                            \

@@ -32,3 +32,18 @@ def test_deep_tiles(gpu, beamc, oracle, tile, K):
                       a, b, (M, N), dtype, (0, 0, 0))
             ws.free()
             close_enough(oracle, out, ref, K, dtype, f"split-K {(M, N, K)} in {slices}")
+
+
+@pytest.mark.parametrize("M,N,K,dtype", [(33, 12225, 2049, F16), (64, 12289, 2056, BF16), (17, 14273, 2120, F16), (64, 16384, 2111, BF16)])
+def test_one_row_of_tiles_that_nearly_fills_the_chip(gpu, beamc, oracle, M, N, K, dtype):
+    """The library's own choice there is the deep pipeline as one group: gemmrc, split-K with one slice, and [K][N]."""
+    L = beamc.lib
+    cfg, _ = beamc.default_config(M, N, K)
+    assert (cfg.block_m, cfg.block_n, cfg.pipeline) == (64, 64, 2)
+    a, b = beamc.host_uniform((M, K), dtype, 84, 0), beamc.host_uniform((N, K), dtype, 84, 1)
+    ref = oracle.gemmrc(a, b, dtype)
+    for what, bb, call in (("gemmrc", b, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, dtype, None, None)),
+                           ("split-K", b, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, dtype, None, 1, None, 0, None)),
+                           ("[K][N]", np.ascontiguousarray(b.T), lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, dtype, None, None))):
+        out = run(beamc, call, a, bb, (M, N), dtype, (0, 0, 0))
+        close_enough(oracle, out, ref, K, dtype, f"{what} {(M, N, K)}")
