@@ -14,9 +14,15 @@ namespace {
 template <typename T>
 struct Vec4Of;
 template <>
-struct Vec4Of<_Float16> { typedef _Float16 type __attribute__((ext_vector_type(4))); };
+struct Vec4Of<_Float16> {
+  typedef _Float16 type __attribute__((ext_vector_type(4)));
+  typedef _Float16 at_element __attribute__((ext_vector_type(4), aligned(2)));  // outputs: at any element's address
+};
 template <>
-struct Vec4Of<__bf16> { typedef __bf16 type __attribute__((ext_vector_type(4))); };
+struct Vec4Of<__bf16> {
+  typedef __bf16 type __attribute__((ext_vector_type(4)));
+  typedef __bf16 at_element __attribute__((ext_vector_type(4), aligned(2)));
+};
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -58,7 +64,7 @@ __global__ void __launch_bounds__(64) splitk_reduce_kernel(const float* __restri
     vec4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = (T)s[e];
-    *(vec4*)(C + q * 4) = o;
+    *(typename Vec4Of<T>::at_element*)(C + q * 4) = o;
   }
   // tail (mn not a multiple of 4)
   const size_t t = quads * 4 + (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -102,7 +108,7 @@ __global__ void __launch_bounds__(256) ln_apply_kernel(const float* __restrict__
       vec4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = (T)((v[e] - mean) * rstd * (float)g[e] + (float)b[e]);
-      *(vec4*)(y + n) = o;
+      *(typename Vec4Of<T>::at_element*)(y + n) = o;
     }
   } else {
     for (int n = threadIdx.x; n < N; n += blockDim.x)

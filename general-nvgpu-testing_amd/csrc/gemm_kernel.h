@@ -403,6 +403,7 @@ struct GemmTile {
     static_assert(P >= 1 && P <= NT && P * NT * OUT == BM * BN && PART_ROWS * BN == NT * OUT, "parts tile the tile");
     typedef float acc_t __attribute__((ext_vector_type(OUT)));
     typedef T out_t __attribute__((ext_vector_type(OUT)));
+    typedef T out_at_element __attribute__((ext_vector_type(OUT), aligned(2)));  // C lies at any element's address
     const int tid = threadIdx.x, lane = tid & 63;
     const int t = r / P, q = r - t * P;
     const int tm = t / p.tiles_n, tn = t - tm * p.tiles_n;
@@ -469,7 +470,7 @@ struct GemmTile {
       out_t o;
 #pragma unroll
       for (int e = 0; e < OUT; ++e) o[e] = (T)s[e];
-      *(out_t*)((T*)p.C + (size_t)m * N + n) = o;
+      *(out_at_element*)((T*)p.C + (size_t)m * N + n) = o;
     }
   }
 

@@ -62,6 +62,32 @@ def test_any_k(gpu, beamc, oracle, K, dtype):
             close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"split-K {(M, N, K)} room {room}")
 
 
+# N a multiple of 4, as the one-launch form asks for: 1, 2 and 4 outputs per thread of a reducing workgroup
+@pytest.mark.parametrize("M,N", [(65, 72), (400, 460), (640, 700)])
+@pytest.mark.parametrize("offs", [(0, 0, 1), (1, 0, 2), (0, 3, 3)])
+def test_split_k_outputs_at_any_address(gpu, beamc, oracle, M, N, offs):
+    """Both forms of the reduction store vectors of C at any element's address; same bits either way."""
+    K, slices = 392, 3
+    L = beamc.lib
+    ws = beamc.DeviceArray((L.beam_splitk_workspace_bytes(M, N, slices),), itemsize=1)
+    for dtype in (F16, BF16):
+        a, b = beamc.host_uniform((M, K), dtype, 82, 0), beamc.host_uniform((N, K), dtype, 82, 1)
+        ref = oracle.gemmrc(a, b, dtype)
+        for pipeline in (0, 2):
+            cfg = beamc.TileConfig(64, 64, 32, 32, pipeline, 0).to_c()
+            outs = []
+            for two in (False, True):
+                beamc.set_splitk_two_launches(two)
+                try:
+                    outs.append(run(beamc, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, dtype, ctypes.byref(cfg), slices, ws.ptr,
+                                                                                   ws.nbytes, None), a, b, (M, N), dtype, offs))
+                finally:
+                    beamc.set_splitk_two_launches(False)
+            close_enough(oracle, outs[0], ref, K, dtype, f"pipeline {pipeline} at {offs}")
+            assert (outs[0] == outs[1]).all()
+    ws.free()
+
+
 @pytest.mark.parametrize("shape,offs", [((65, 72, 321), (0, 0, 0)), ((65, 72, 320), (0, 1, 0))])
 def test_split_k_workspace_off_16_bytes(gpu, beamc, oracle, shape, offs):
     """Unaligned rows never needed a workspace: one that is off 16 bytes is left alone."""
@@ -127,6 +153,25 @@ def test_walking_kernels_at_any_address(gpu, beamc, oracle, wave_n):
     c = beamc.TileConfig(256, 256, 128, wave_n).to_c()
     out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, F16, ctypes.byref(c), None), a, b, (M, N), F16, (1, 3, 0))
     assert_close(oracle, out, oracle.gemmrc(a, b, F16), K, F16, f"256x256, wavefronts 128x{wave_n}")
+
+
+# N a multiple of 4 and of 8: the vector path of the normalisation pass, Y at any element's address
+@pytest.mark.parametrize("shape", [(65, 72, 64), (130, 260, 72), (33, 1028, 200)])
+@pytest.mark.parametrize("offs", [(0, 0, 1), (1, 0, 2), (0, 3, 3)])
+def test_layer_norm_outputs_at_any_address(gpu, beamc, oracle, shape, offs):
+    M, N, K = shape
+    L = beamc.lib
+    for dtype in (F16, BF16):
+        a, b, g, bt = make_ln_inputs(beamc, M, N, K, dtype, 85)
+        ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, dtype)
+        dg, dbt = beamc.DeviceArray.from_numpy(g, dtype), beamc.DeviceArray.from_numpy(bt, dtype)
+        ws = beamc.DeviceArray((L.beam_gemmrc_ln_workspace_bytes_ex(M, N, None, beamc.LN_AUTO),), itemsize=1)
+        for mode in (beamc.LN_TWOPASS, beamc.LN_FUSED):
+            out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_ln_ex(pa, pb, dg.ptr, dbt.ptr, 1e-5, pc, M, N, K, dtype, None, mode, ws.ptr,
+                                                                    ws.nbytes, None), a, b, (M, N), dtype, offs)
+            check_ln(oracle, out, ref, dtype, f"LayerNorm {shape} mode {mode} at {offs}")
+        for v in (dg, dbt, ws):
+            v.free()
 
 
 @pytest.mark.parametrize("shape", [(65, 63, 9), (130, 257, 71), (33, 1001, 331), (300, 515, 129)])
