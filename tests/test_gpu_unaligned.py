@@ -174,6 +174,50 @@ def test_layer_norm_outputs_at_any_address(gpu, beamc, oracle, shape, offs):
             v.free()
 
 
+def test_walking_kernels_at_any_address_kmajor_and_layer_norm(gpu, beamc, oracle):
+    """The 4-wavefront kernel's [K][N] and LayerNorm forms with A and B off 16 bytes: one tile per workgroup and, with more
+    tiles than CUs, several."""
+    L = beamc.lib
+    c = beamc.TileConfig(256, 256, 128, 128).to_c()
+    for M, N, K in ((300, 520, 192), (4200, 4200, 192)):
+        a, b, g, bt = make_ln_inputs(beamc, M, N, K, F16, 86)
+        bk = np.ascontiguousarray(b.T)
+        out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, ctypes.byref(c), None), a, bk, (M, N), F16, (1, 3, 0))
+        assert_close(oracle, out, oracle.matmul_nn(a, bk, F16), K, F16, f"[K][N] {(M, N, K)}")
+        dg, dbt = beamc.DeviceArray.from_numpy(g, F16), beamc.DeviceArray.from_numpy(bt, F16)
+        ws = beamc.DeviceArray((L.beam_gemmrc_ln_workspace_bytes_for(M, N, K, ctypes.byref(c), beamc.LN_FUSED),), itemsize=1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_ln_ex(pa, pb, dg.ptr, dbt.ptr, 1e-5, pc, M, N, K, F16, ctypes.byref(c), beamc.LN_FUSED,
+                                                                ws.ptr, ws.nbytes, None), a, b, (M, N), F16, (1, 3, 0))
+        check_ln(oracle, out, oracle.gemmrc_ln(a, b, g, bt, 1e-5, F16), F16, f"LayerNorm {(M, N, K)}")
+        for v in (dg, dbt, ws):
+            v.free()
+
+
+# K a multiple of 8 and not, a short K tile alone and behind whole ones; the job shorter than, and longer than, the K loop
+@pytest.mark.parametrize("K,offs", [(63, (0, 0, 0)), (137, (0, 0, 0)), (200, (1, 0, 3)), (459, (3, 1, 1))])
+@pytest.mark.parametrize("pipeline", [0, 1])
+def test_side_job(gpu, beamc, oracle, K, offs, pipeline):
+    """Every tile carries the SiLU job beside rows at any element's address."""
+    M, N = 300, 200
+    L = beamc.lib
+    a, b = beamc.host_uniform((M, K), F16, 87, 0), beamc.host_uniform((N, K), F16, 87, 1)
+    ref = oracle.gemmrc(a, b, F16)
+    for count in (5, 4099, 100003):
+        x = beamc.host_normal((count,), F16, 87, 2, 0.0, 2.0)
+        dx, want = beamc.DeviceArray.from_numpy(x, F16), beamc.DeviceArray((count,), F16)
+        beamc.silu(dx, want)
+        y = Embedded(beamc, (count,), F16, 8)
+        for t in beamc.list_configs():
+            cfg = beamc.TileConfig(t.block_m, t.block_n, t.wave_m, t.wave_n, pipeline, 0).to_c()
+            beamc._check(L.beam_memset(y.ptr, 0xEE, 2 * count))
+            out = run(beamc, lambda pa, pb, pc: L.beam_parallel_gemmrc_silu(pa, pb, pc, M, N, K, dx.ptr, y.ptr, count, F16, ctypes.byref(cfg), None),
+                      a, b, (M, N), F16, offs)
+            close_enough(oracle, out, ref, K, F16, f"{t.name} beside {count}")
+            assert (y.result() == want.to_numpy()).all(), (t.name, count)
+        for v in (dx, want, y.buf):
+            v.free()
+
+
 @pytest.mark.parametrize("shape", [(65, 63, 9), (130, 257, 71), (33, 1001, 331), (300, 515, 129)])
 @pytest.mark.parametrize("dtype", [F16, BF16])
 def test_layer_norm(gpu, beamc, oracle, shape, dtype):
