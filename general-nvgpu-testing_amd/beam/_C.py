@@ -510,8 +510,8 @@ def silu(x, y) -> None:
 
 
 def parallel_gemmrc_silu(a, b, c, x, y, config: Optional[TileConfig] = None) -> None:
-    """c = a @ b.T and, in the same launch, y = silu(x): the elementwise job is streamed through the
-    GEMM's K loop.  Reference: cutlass_parallel_gemmrc_lnr(gemmA, gemmB, gemmC, lnA, lnB),
+    """c = a @ b.T and y = silu(x): the elementwise job is streamed through the GEMM's K loop in the same launch, or,
+    with no tile given and a GEMM that is the faster without it, run in a second one.  Reference: cutlass_parallel_gemmrc_lnr(gemmA, gemmB, gemmC, lnA, lnB),
     cuda/cute_kernels/main.cc:55-76 (python/beam/_C/beam_C.pyi:20)."""
     pa, pb, pc, M, N, K, d, st = _problem(a, b, c)
     px, py, n, _, _ = _flat_pair(x, y, d)

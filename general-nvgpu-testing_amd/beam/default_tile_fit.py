@@ -3,11 +3,11 @@
 The library picks a tile for a problem without measuring anything: every CU works through
 ceil(tiles / CUs) workgroups, `occ` of them at a time (what LDS allows); a workgroup costs a fixed
 start-up / epilogue time plus its flops at the per-CU rate of its tile shape, which is higher when
-several workgroups share the CU.  Three constants per candidate tile (rate alone, rate with a full CU,
-fixed cost) are fitted to `default_tile_timings.json`: microseconds per launch of every candidate on 39
-shapes from 512^3 to 8192^3 (square, skinny, short-K), fp16, N(0,1)/sqrt(K) operands, best of two rounds
-of 40 launches each, on one MI355X.  `PARAMS` below are the constants compiled into the library
-(csrc/capi.hip, kCandidates); a test keeps the two in step.
+several workgroups share the CU.  `default_tile_timings.json` holds microseconds per launch of the candidates'
+tiles, at both depths, on 39 shapes from 512^3 to 8192^3 (square, skinny, short-K), fp16, N(0,1)/sqrt(K) operands,
+best of two rounds of 40 launches each, on one MI355X, the library as shipped.  `PARAMS` below are the constants
+compiled into the library (csrc/capi.hip, kCandidates; a test keeps the two in step): three per candidate (rate
+alone, rate with a full CU, fixed cost), fitted to an earlier table, when the deep tiles up to 128 x 64 had one K group.
 
     python -m beam.default_tile_fit              model's pick per shape against the table, mean / worst regret
     python -m beam.default_tile_fit --refit      coordinate search from PARAMS (what produced them)
@@ -29,7 +29,8 @@ A GEMM+LayerNorm call without a tile (one-kernel form) has a model of its own: o
 in the epilogue's chain of latencies, so the cost is rounds x (fixed + a tile's flops / rate) with whole rounds.
 `ln_tile_timings.json` holds microseconds per call of the one-kernel form with every compiled tile (3 + 2 slots) on 34
 shapes (fp16, N(0,1)/sqrt(K), best of two rounds, one MI355X; "default": the library's pick at the time, "plain": the
-plain GEMM); `LN_PARAMS` are the least-squares constants compiled into the library (csrc/capi.hip, kLnCandidates).
+plain GEMM); `LN_PARAMS` are the least-squares constants compiled into the library (csrc/capi.hip, kLnCandidates),
+fitted to an earlier table of the same shapes.
 
 This stands where the reference has fixed default shapes (cuda/cutlass_kernels/cutlass_gemmrc.cu:22-24).
 """
@@ -173,13 +174,26 @@ def predict(params, M, N, K):
     return best
 
 
+def as_run(name, M, N, K):
+    """The kernel the library runs for the model's pick (csrc/capi.hip, choose_default): a full round of 256 x 256 tiles as
+    four wavefronts of 128 x 128, and under a long sum the deep pipeline for few workgroups or two K groups."""
+    bm, bn, _ = CANDIDATES[name]
+    tiles = math.ceil(M / bm) * math.ceil(N / bn)
+    if (bm, bn) == (256, 256) and tiles >= CUS and K % 64 == 0 and K >= W4_MIN_K and N % 8 == 0:
+        return "256x256_w128x128"
+    if not name.endswith("_deep") and K >= 2048 and (tiles < CUS // 2 or (tiles <= CUS and bm * bn <= 128 * 64)):
+        return name + "_deep"
+    return name
+
+
 def regret(params, timings, rows=None):
-    """(geometric-mean, worst) ratio of the picked candidate's measured time to the best time of any tile."""
+    """(geometric-mean, worst) ratio of the measured time of what the library runs to the best time of any tile."""
     total, worst = 0.0, 0.0
     for key, row in timings.items():
         M, N, K = map(int, key.split("x"))
         us, name = predict(params, M, N, K)
         best = row["best_of_all_tiles"][1]
+        name = as_run(name, M, N, K)
         r = row["candidates"][name] / best
         total += math.log(r)
         worst = max(worst, r)
@@ -359,7 +373,8 @@ def collect(path):
         for x in (a, b, c):
             x.free()
         name = min(res, key=res.get)
-        out[key] = {"candidates": {n: round(res[n], 2) for n in CANDIDATES},
+        columns = sorted({n.replace("_deep", "") + depth for n in CANDIDATES for depth in ("", "_deep")} | {"256x256_w128x128"})
+        out[key] = {"candidates": {n: round(res[n], 2) for n in columns},
                     "best_of_all_tiles": [name, round(res[name], 2)]}
         print(key, out[key]["best_of_all_tiles"], flush=True)
     with open(path, "w") as f:

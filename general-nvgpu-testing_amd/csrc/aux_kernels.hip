@@ -148,7 +148,8 @@ __global__ void __launch_bounds__(256) silu_kernel(const T* __restrict__ x, T* _
 }
 
 // gemmrc for problems the tiled kernels do not take: K below 8 or beyond a buffer descriptor, the [K][N] layout with N
-// below 8, and GEMM+LayerNorm with gamma or beta off an 8-byte boundary.
+// below 8, and GEMM+LayerNorm with gamma or beta off an 8-byte boundary; and, on rows off 16 bytes, for calls that the
+// tiled kernels would refuse (a tile that is not compiled, LayerNorm with room for fp32 X only).
 // A plain LDS-tiled fp32 kernel: 64 x 64 outputs per workgroup, 16 K elements per step, 4 x 4 outputs per
 // thread, every access bounds-checked element by element.  Same arithmetic contract (16-bit inputs, fp32
 // accumulation, one rounding), far from the same speed; it exists so that no well-formed problem is refused

@@ -383,9 +383,10 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
   // them at a time (what LDS allows); a workgroup costs a fixed start-up / epilogue time plus its flops
   // at the per-CU rate of its tile shape, which is higher when several workgroups share the CU.  The
   // rates (TFLOP/s per CU, alone / with a full CU) and fixed costs (us) are fits to timings of all
-  // compiled tiles on 39 shapes from 512^3 to 8192^3 (square, skinny and short-K) on an MI355X:
-  // the pick is within 0.8% of the best tile on average, 6.7% at worst (tile-count thresholds:
-  // 6% and 76%).  The 224- and 192-row tiles are there for what 256 rows divide badly: 3072^3 is
+  // compiled tiles on 39 shapes from 512^3 to 8192^3 (square, skinny and short-K) on an MI355X, taken
+  // while the deep tiles up to 128 x 64 had one K group: they rank tiles, they are not those tiles' rates now.
+  // On timings of the present kernels (beam/default_tile_timings.json), what runs for the pick is within
+  // 0.8% of the best tile on average, 6.1% at worst (tile-count thresholds: 6% and 76%).  The 224- and 192-row tiles are there for what 256 rows divide badly: 3072^3 is
   // 0.75 of a round of 192 x 256 tiles against 0.56 of a round of 256 x 256 ones (49.5 against
   // 58.6 us), 7168^3 is 3.5 rounds of 224 x 256 tiles against 3.06 (546 against 613 us).
   struct Candidate {
@@ -991,8 +992,8 @@ static size_t ln_workspace_need(int M, int N, const beam_tile_cfg& c, int mode) 
 // tile: every workgroup ends with the epilogue's chain of latencies, so a round of workgroups costs a fixed time
 // that grows with the tile, and rounds count in whole numbers -- of bands, since a band's tiles wait for each other.
 // The model is that sentence: rounds x (fixed + flops of a tile / rate), rates (TFLOP/s per CU) and fixed costs (us)
-// fitted by least squares to the timings of every tile on 34 shapes (beam/ln_tile_timings.json: the pick is within
-// 1.5% of the best tile in the geometric mean, 16% at worst).
+// fitted by least squares to timings of every tile on 34 shapes; on those of the present kernels
+// (beam/ln_tile_timings.json) the pick is within 1.6% of the best tile in the geometric mean, 18% at worst.
 struct LnCandidate {
   beam_tile_cfg cfg;
   double rate, fixed;
@@ -1118,9 +1119,9 @@ static int ln_plan_call(const void* A, const void* B, const void* gamma, const v
   return BEAM_OK;
 }
 
-// Enough for beam_gemmrc_ln_ex(M, N, K, cfg, mode) on operands aligned as the tiled kernels need them.  AUTO covers
-// both forms it can resolve to (one kernel eagerly, two passes under stream capture and as the retry of
-// beam_gemmrc_ln_checked), which also covers the plain path.
+// Enough for beam_gemmrc_ln_ex(M, N, K, cfg, mode) with A, B, Y on 16 bytes and gamma, beta on 8.  AUTO covers both forms it
+// can resolve to (one kernel eagerly, two passes under stream capture and as the retry of beam_gemmrc_ln_checked); two
+// passes need at least what the plain kernels do.
 size_t beam_gemmrc_ln_workspace_bytes_for(int M, int N, int K, const beam_tile_cfg* cfg, int mode) {
   if (M <= 0 || N <= 0 || K < 0) return 0;
   if ((K > 0 && K < 8) || K > kMaxK) return ln_generic_need(M, N);

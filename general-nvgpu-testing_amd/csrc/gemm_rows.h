@@ -9,8 +9,8 @@
 // Two slots per wavefront and several workgroups per CU beat one workgroup with long rings (4 x 4096 x 4096: 4.1 us with 8
 // wavefronts of 2 slots, 4.6 with 5), as do 16 columns against 32 (5.0) or 64 (8.3).
 //   bf16, us, tiled kernel -> this: 1 x 1024 x 9480 23.1 -> 5.3, 4 x 4096 x 4096 11.8 -> 4.1, 16 x 1024 x 16384
-//   36.8 -> 11.5, 16 x 11008 x 4096 15.5 -> 15.7 (5.8 TB/s: memory), 16 x 16384 x 16384 112.6 -> 104.1 (5.2 TB/s),
-//   32 x 4096 x 4096 12.0 -> 7.4, 64 x 512 x 8192 20.1 -> 11.3, 64 x 64 x 512 3.6 -> 3.3.
+//   36.8 -> 11.5, 32 x 4096 x 4096 12.0 -> 7.4, 64 x 512 x 8192 20.1 -> 11.3, 64 x 64 x 512 3.6 -> 3.3.  Where memory is what
+//   bounds both, nothing: 16 x 11008 x 4096 15.6 either way (5.8 TB/s), and the tiled kernel runs it (capi.hip: rows_plan).
 #pragma once
 
 #include "gemm_kernel.h"
@@ -29,7 +29,7 @@ struct RowsTile {
   static constexpr int OUTS = MB * 16 * COLS;
   static_assert(AG == 1 || AG % 2 == 0, "rows in blocks of 16");
   static_assert(S >= 2 && (S - 1) * LOADS < 64, "vmcnt range");
-  static_assert(LDS_BYTES <= 160 * 1024 && OUTS * 4 <= S * SLOT, "two workgroups per CU; the sums reuse the ring");
+  static_assert(2 * LDS_BYTES <= 160 * 1024 && OUTS * 4 <= S * SLOT, "two workgroups per CU; the sums reuse the ring");
 
   static __device__ __forceinline__ void run(const void* A, const void* B, void* C, int M, int N, int K, char* smem) {
     using Traits = ElemTraits<T>;

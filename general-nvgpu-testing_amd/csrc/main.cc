@@ -593,7 +593,6 @@ int cli_bench(const Args& a) {
   cfg.group_m = a.num("group", cfg.group_m);
   split = a.num("splitk", splitk_like ? 0 : split);
   Problem p(M, N, K, dtype, a.str("data", "normal"));
-  if (op == BEAM_OP_MATMUL_NN && cfg.pipeline == 2) cfg.pipeline = 0;
   if (opname == "silu") {
     if (cfg.pipeline == 2) cfg.pipeline = 0;
     return cli_bench_silu(a, p, cfg);
@@ -601,14 +600,16 @@ int cli_bench(const Args& a) {
   float ms = 0;
   const std::string lnm = a.str("ln-mode", "auto");  // --op ln: auto | twopass | fused
   const int ln_mode = lnm == "twopass" ? BEAM_LN_TWOPASS : lnm == "fused" ? BEAM_LN_FUSED : BEAM_LN_AUTO;
-  // GEMM+LayerNorm without a tile on the command line: the library's own choice for that operator (a cost model
-  // of its own, not the plain GEMM's tile); the line below then names what it picked for a device of 256 CUs.
-  const bool ln_auto_tile = op == BEAM_OP_GEMM_LN && !a.has("tile") && !a.has("wave") && !a.has("pipeline") && !a.has("group");
-  if (ln_auto_tile && ln_mode != BEAM_LN_TWOPASS) {
+  // Without a tile on the command line: the library's own choice for the operator, named to nobody (few rows and the [K][N]
+  // layout run on kernels that beam_default_config does not name; GEMM+LayerNorm has a cost model of its own, and the
+  // line below names what that picks for a device of 256 CUs).  Split-K: the tile that goes with the library's slice count.
+  const bool own_tile = (op == BEAM_OP_GEMM || op == BEAM_OP_MATMUL_NN || op == BEAM_OP_GEMM_LN) && !a.has("tile") && !a.has("wave") &&
+                        !a.has("pipeline") && !a.has("group");
+  if (own_tile && op == BEAM_OP_GEMM_LN && ln_mode != BEAM_LN_TWOPASS) {
     beam_tile_cfg picked;
     if (beam_dbg_ln_default_config(M, N, K, 256, &picked) == BEAM_OK) cfg = picked;
   }
-  int rc = time_op(op, p, ln_auto_tile ? nullptr : &cfg, split, a.num("warmup", 5), a.num("iters", 20), &ms, ln_mode);
+  int rc = time_op(op, p, own_tile ? nullptr : &cfg, split, a.num("warmup", 5), a.num("iters", 20), &ms, ln_mode);
   if (rc != BEAM_OK) {
     std::fprintf(stderr, "bench failed (%d): %s\n", rc, beam_last_error());
     return 1;

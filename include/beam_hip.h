@@ -38,7 +38,8 @@ typedef struct beam_tile_cfg {
   int block_m, block_n; /* workgroup tile of C ("shape_threadblock")                          */
   int wave_m, wave_n;   /* wavefront tile ("shape_warp"); block/wave = wavefront grid         */
   int pipeline;         /* LDS slots per operand: 0 = 3 for A + 2 for B, 1 = 2 + 2,             */
-                        /* 2 = as many as fit 160 KiB, up to 8 + 7 (small tiles, split-K)       */
+                        /* 2 = as many as fit 160 KiB, up to 8 + 7; tiles up to 128 x 64: two   */
+                        /* rings for two groups of wavefronts that share the K tiles           */
   int group_m;          /* rasterisation group height in tiles; 0 = library default           */
 } beam_tile_cfg;
 
@@ -67,7 +68,8 @@ int beam_default_config(int M, int N, int K, beam_tile_cfg* cfg, int* split_k);
 /* ---- tiled GEMM ------------------------------------------------------------------------ */
 
 /* cfg == NULL: beam_default_config() picks the tile (never a split); up to 64 rows of A may run on a kernel of their own
- * that has no tile to name.
+ * that has no tile to name, or on the deep pipeline as one group of wavefronts.  Any K and any element's address; a tile
+ * that is not compiled is refused, but for rows that are not 16-byte aligned, which are computed whatever is named.
  * Replaces entry_cutlass_gemmrc / entry_cutlass_gemmrc_spec
  * (cuda/cutlass_kernels/main.cc:11-15, cutlass_gemmrc.cu:21-40,55-111). */
 int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int dtype,
@@ -108,7 +110,8 @@ size_t beam_splitk_workspace_bytes(int M, int N, int split_k);
  * launches (partial kernel, reduce kernel; the same bits) for tiles above 128 x 128, N not a multiple of
  * 4, more than 64 slices, M * N above 2^28, outputs so large that the adding workgroups would need more than
  * two rounds of the CUs, or a workspace that only holds the partial sums
- * (split_k * M * N * 4 bytes; anything smaller is BEAM_ERR_WORKSPACE).
+ * (split_k * M * N * 4 bytes; anything smaller, or off 16 bytes, is refused).  Operands whose rows are not 16-byte aligned
+ * (or C not 8-byte) run in one pass where the workspace does not hold their slices.
  * Replaces entry_cutlass_gemmrc_splitk / _spec
  * (cuda/cutlass_kernels/main.cc:17-21, cutlass_gemmrc_splitk.cu:59-105,107-195). */
 int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int K, int dtype,
@@ -137,8 +140,8 @@ int beam_set_verbose(int verbose);
  * for them, plus 256 KiB for the synchronisation words of the one-launch form, per GPU, present from the
  * first call into the library until the process ends).  No counterpart in
  * the reference; it is for callers that cannot allocate: code under HIP graph capture, tight serving
- * loops, harnesses that forbid hipMalloc.  Same results as beam_gemmrc_splitk, bit for bit.
- * split_k * M * N * 4 bytes beyond the array's size -> BEAM_ERR_WORKSPACE.  All calls on one GPU share
+ * loops, harnesses that forbid hipMalloc.  Same results as beam_gemmrc_splitk with such a workspace, bit for bit.
+ * split_k * M * N * 4 bytes beyond the array's size -> BEAM_ERR_WORKSPACE (rows that are not 16-byte aligned: one pass).  All calls on one GPU share
  * the array: calls that overlap in time on one GPU (different streams) race; order them. */
 size_t beam_splitk_noalloc_max_bytes(void);
 int beam_gemmrc_splitk_noalloc(const void* A, const void* B, void* C, int M, int N, int K, int dtype,
@@ -169,12 +172,12 @@ int beam_gemmrc_ln(const void* A, const void* B, const void* gamma, const void* 
  *   BEAM_LN_AUTO    fused when it applies, else two-pass (what beam_gemmrc_ln does); two-pass under
  *                   stream capture. */
 typedef enum beam_ln_mode { BEAM_LN_AUTO = 0, BEAM_LN_TWOPASS = 1, BEAM_LN_FUSED = 2 } beam_ln_mode;
-/* Workspace bytes.  _for is enough for the call beam_gemmrc_ln_ex(M, N, K, cfg, mode) on operands aligned as the
- * tiled kernels need them (A, B, Y 16 bytes, gamma and beta 8): exact for BEAM_LN_TWOPASS and BEAM_LN_FUSED; for
+/* Workspace bytes.  _for is enough for the call beam_gemmrc_ln_ex(M, N, K, cfg, mode) with A, B, Y on 16 bytes and gamma,
+ * beta on 8: exact for BEAM_LN_TWOPASS and BEAM_LN_FUSED; for
  * BEAM_LN_AUTO the larger of the two forms it can resolve to (one kernel eagerly; two passes under stream capture
  * and as the retry of beam_gemmrc_ln_checked).  The forms without K are enough for any call with these M, N, cfg and
  * mode: every K (cfg == NULL: every tile the library could pick), operands aligned to an element only, captured or
- * not. */
+ * not.  Rows that are not 16-byte aligned get by with M * N * 4 bytes on 16, on a slower path. */
 size_t beam_gemmrc_ln_workspace_bytes_for(int M, int N, int K, const beam_tile_cfg* cfg, int mode);
 size_t beam_gemmrc_ln_workspace_bytes_ex(int M, int N, const beam_tile_cfg* cfg, int mode);
 int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const void* beta, float eps,
@@ -233,7 +236,7 @@ int beam_set_ln_walk(int on);
  * drops whatever does not fit their K loops, every element is processed exactly once for any
  * count and any GEMM shape.  X, Y: device pointers, 16-byte aligned, count <= 1 073 741 696;
  * Y may be X (in place) but must not overlap it otherwise; neither may overlap C.
- * cfg->pipeline must be 0 or 1. */
+ * cfg->pipeline must be 0 or 1 (2 where beam_default_config names it for half a round of workgroups or more). */
 int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int N, int K, const void* X,
                               void* Y, long long count, int dtype, const beam_tile_cfg* cfg, void* stream);
 

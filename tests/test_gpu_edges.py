@@ -1,7 +1,7 @@
-"""Problems outside what the tiled kernels take -- K not a multiple of 8, the [K][N] layout with N not a
-multiple of 8, operands at addresses that are not 16-byte aligned -- are computed (by a plain kernel), never
-refused: every entry point against the oracle, to the same tolerances as everywhere else.  The reference's
-NN path masks any edge (python/beam/triton_kernels/gemm.py:62-63,75)."""
+"""Rows that are not 16-byte aligned -- K not a multiple of 8, the [K][N] layout with N not a multiple of 8, operands at
+other addresses -- are computed (by the tiled kernels; K or N below 8 by a plain one), never refused: every entry point
+against the oracle, to the same tolerances as everywhere else.  The reference's NN path masks any edge
+(python/beam/triton_kernels/gemm.py:62-63,75)."""
 
 import pytest
 
