@@ -466,11 +466,13 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
 // The deep pipeline of the library's own tile as one K group (KernelSet::launch_deep_one_group), or nullptr for two.  Where
 // one row of 64 x 64 tiles nearly fills the chip, B is read once and memory is the bound; one ring of 8 + 7 slots then keeps
 // more of it in flight than two of 5 + 4.  fp16, us, two groups -> one: [N][K] from 3/4 of a round on, 33 x 12288 x 2048
-// 10.5 -> 10.1, 16 x 14336 x 8192 35.4 -> 33.9, 64 x 12288 x 16384 94.5 -> 89.6; below it 17 x 11008 x 8192 27.5, 28.4.
-// [K][N] from 7/8 on: 16 x 16384 x 8192 45.9 -> 42.6, x 12288 81.5 -> 72.7.
-GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, int N, int dtype, bool b_kmajor, int cus) {
+// 10.5 -> 10.1, 16 x 14336 x 8192 35.4 -> 33.9, 64 x 12288 x 16384 94.5 -> 89.6; below it 17 x 11008 x 8192 27.5, 28.4, and
+// with rows off 128-byte lines, which fill LDS at half the rate, 64 x 12288 x 4104 36.9, 37.7.  [K][N] from 7/8 on:
+// 16 x 16384 x 8192 45.9 -> 42.6, x 12288 81.5 -> 72.7.
+GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, int N, int K, int dtype, bool b_kmajor, int cus) {
   if (c.pipeline != 2 || M > c.block_m) return nullptr;
   const long tiles = (N + c.block_n - 1) / c.block_n;
+  if (!b_kmajor && K % kBK != 0) return nullptr;
   return 8 * tiles >= (b_kmajor ? 7L : 6L) * cus ? ks.launch_deep_one_group[dtype][b_kmajor ? 1 : 0] : nullptr;
 }
 
@@ -479,19 +481,19 @@ GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, 
 //     37.3 -> 25.7; M = 64 K = 512 3.6 -> 3.5, K = 1024 5.0 -> 4.1, K = 16384 41.9 -> 33.1.  Beyond 32 rows the K tiles have
 //     to be more than the wavefronts: M = 64 K = 128 2.8, here 3.0, K = 320 3.1, here 3.3.
 //   * Beyond that the fetches of A add up, and B's become the bound.  M <= 16, K <= 4096: 64 columns per workgroup,
-//     M = 1: 5120 x 4096 11.7 -> 8.0, 16384 x 1024 5.4 -> 3.7, 11008 x 4096 14.8 -> 14.3, M = 16 10240 x 4096 14.8 -> 14.6,
-//     14336 x 3072 15.0 -> 14.5; the tiled kernel is ahead from there on (M = 16 11008 x 4096 15.3, here 15.6; 16384 x 4088
-//     20.6, here 27.2) and where K is so short that the workgroups' starts count (65536 x 512 11.0, here 12.1).
-//   * Longer K: 16 columns, fewer wavefronts: M = 16 6144 x 10240 24.7 -> 21.8, 7168 x 12288 29.1 -> 26.1; behind in
-//     K = 8192, the more so the wider (7168 x 8192 20.5, here 24.4; 8192 x 8192 21.5, here 29.4).
+//     M = 1: 5120 x 4096 11.7 -> 8.0, 16384 x 1024 5.4 -> 3.7, 11008 x 4096 14.8 -> 14.3; M = 16, B different in every call,
+//     11008 x 4096 21.2 -> 19.7, 12288 x 4096 22.3 -> 21.2; the tiled kernel is ahead from there on (16384 x 4088 20.6, here
+//     27.2) and where K is so short that the workgroups' starts count (65536 x 512 11.0, here 12.1).
+//   * Longer K: 16 columns, fewer wavefronts.  M = 16, B different in every call: 7680 x 10240 43.8 -> 35.4, 8192 x 8192
+//     33.8 -> 32.6, 8192 x 16384 66.2 -> 62.0.  (With the same B in every call, which then lies in the last-level cache,
+//     8192 x 8192 is 21.5, here 29.4.)  Beyond 8192 columns the tiled kernel is ahead: 10000 x 6000 21.4, here 23.0.
 //   * M <= 32: 32 columns per workgroup, 8192 x 1024 4.9 -> 4.2, x 2048 7.7 -> 6.4; 16384 x 512 3.7, here 5.0.
 RowsPlan rows_plan(int M, int N, int K, int cus) {
   if (M > 64 || K % 8 != 0 || K > kRowsMaxK) return kRowsNone;
   const long cols = N, round = 16L * cus;  // columns of one workgroup of 16 per CU
   if (cols <= round) return M <= 32 || K > 320 ? kRowsNarrow : kRowsNone;
   if (M <= 16) {
-    if (K > 4096) return 4 * cols <= 7 * round ? kRowsDeep : kRowsNone;
-    if (M > 8 && K > 3072 && 2 * cols > 5 * round) return kRowsNone;
+    if (K > 4096) return cols <= 2 * round ? kRowsDeep : kRowsNone;
     return K >= 512 && cols <= 4 * round && cols * K <= (3L << 24) ? kRowsWide : kRowsNone;
   }
   if (M <= 32 && cols <= 2 * round && K >= 1024 && K <= 2048) return kRowsWide;
@@ -566,7 +568,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     BEAM_HIP(loop(p, dim3((unsigned)cus, 1, 1), st));
     return BEAM_OK;
   }
-  GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, dtype, false, cus);
+  GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, false, cus);
   BEAM_HIP((one_group ? one_group : ks->launch[dtype][kEpiStore][c.pipeline])(p, dim3((unsigned)tiles, 1, 1), st));
   return BEAM_OK;
 }
@@ -629,7 +631,7 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     BEAM_HIP(launch_gemm_w4_kmajor(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
-  GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, dtype, true, cus);
+  GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, true, cus);
   BEAM_HIP((one_group ? one_group : ks->launch_kmajor[dtype][c.pipeline])(p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
   return BEAM_OK;
 }
@@ -861,7 +863,7 @@ int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int 
   if (s == 1) {  // nothing to reduce: the plain kernel writes C directly
     GemmParams p = base_params(A, B, M, N, K, c);
     p.C = C;
-    GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, dtype, false, g_dev.cus > 0 ? g_dev.cus : 256);
+    GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, false, g_dev.cus > 0 ? g_dev.cus : 256);
     BEAM_HIP((one_group ? one_group : ks->launch[dtype][kEpiStore][c.pipeline])(p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
     return BEAM_OK;
   }

@@ -9,8 +9,8 @@
 // Two slots per wavefront and several workgroups per CU beat one workgroup with long rings (4 x 4096 x 4096: 4.1 us with 8
 // wavefronts of 2 slots, 4.6 with 5), as do 16 columns against 32 (5.0) or 64 (8.3).
 //   bf16, us, tiled kernel -> this: 1 x 1024 x 9480 23.1 -> 5.3, 4 x 4096 x 4096 11.8 -> 4.1, 16 x 1024 x 16384
-//   36.8 -> 11.5, 32 x 4096 x 4096 12.0 -> 7.4, 64 x 512 x 8192 20.1 -> 11.3, 64 x 64 x 512 3.6 -> 3.3.  Where memory is what
-//   bounds both, nothing: 16 x 11008 x 4096 15.6 either way (5.8 TB/s), and the tiled kernel runs it (capi.hip: rows_plan).
+//   36.8 -> 11.5, 32 x 4096 x 4096 12.0 -> 7.4, 64 x 512 x 8192 20.1 -> 11.3, 64 x 64 x 512 3.6 -> 3.3.  Where B comes from
+//   memory in every call: fp16 16 x 11008 x 4096 21.2 -> 19.7 (4.6 TB/s); out of the last-level cache 15.6 either way.
 #pragma once
 
 #include "gemm_kernel.h"

@@ -22,9 +22,9 @@ def test_few_rows(gpu, beamc, oracle, M, K):
 
 
 # More columns than 16 for every one of the 256 CUs.  4097: one column in the last block; 4131: part of a block of 16, of 32 and
-# of 64; 5120: whole blocks; 7168: the last number of columns that the form for a long K takes
+# of 64; 5120: whole blocks; 8192: the last number of columns that the form for a long K takes
 @pytest.mark.parametrize("M,N,K,form", [(M, N, K, "wide") for M in (1, 8, 9, 16) for N, K in ((4097, 520), (4131, 1096), (5120, 512), (8200, 2056), (4131, 4096))] +
-                                       [(M, N, K, "deep") for M in (1, 8, 9, 16) for N, K in ((4097, 4104), (4131, 4168), (7168, 4104))] +
+                                       [(M, N, K, "deep") for M in (1, 8, 9, 16) for N, K in ((4097, 4104), (4131, 4168), (8192, 4104))] +
                                        [(M, N, K, "wide") for M in (17, 32) for N, K in ((4097, 1024), (4131, 2040), (8192, 1096))])
 def test_few_rows_of_many_columns(gpu, beamc, oracle, M, N, K, form):
     assert gpu["compute_units"] == 256  # the columns above are chosen for that

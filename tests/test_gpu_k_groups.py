@@ -34,9 +34,10 @@ def test_deep_tiles(gpu, beamc, oracle, tile, K):
             close_enough(oracle, out, ref, K, dtype, f"split-K {(M, N, K)} in {slices}")
 
 
-@pytest.mark.parametrize("M,N,K,dtype", [(33, 12225, 2049, F16), (64, 12289, 2056, BF16), (17, 14273, 2120, F16), (64, 16384, 2111, BF16)])
+@pytest.mark.parametrize("M,N,K,dtype", [(33, 12225, 2048, F16), (64, 12289, 2112, BF16), (17, 14273, 2048, F16), (64, 14337, 2111, BF16), (33, 16383, 2112, F16)])
 def test_one_row_of_tiles_that_nearly_fills_the_chip(gpu, beamc, oracle, M, N, K, dtype):
-    """The library's own choice there is the deep pipeline as one group: gemmrc, split-K with one slice, and [K][N]."""
+    """The library's own choice there is the deep pipeline as one group: gemmrc and split-K with one slice where K is a
+    multiple of 64, [K][N] from 14273 columns on."""
     L = beamc.lib
     cfg, _ = beamc.default_config(M, N, K)
     assert (cfg.block_m, cfg.block_n, cfg.pipeline) == (64, 64, 2)
