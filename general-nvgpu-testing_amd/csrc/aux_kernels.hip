@@ -120,31 +120,7 @@ __global__ void __launch_bounds__(256) ln_apply_kernel(const float* __restrict__
 // then the elements after the last whole vector.
 template <typename T>
 __global__ void __launch_bounds__(256) silu_kernel(const T* __restrict__ x, T* __restrict__ y, size_t count) {
-  typedef T vec8 __attribute__((ext_vector_type(8)));
-  const size_t vecs = count / 8;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (; v + 3 * stride < vecs; v += 4 * stride) {
-    vec8 in[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) in[u] = *(const vec8*)(x + (v + u * stride) * 8);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      vec8 out;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] = silu_16<T>(in[u][e]);
-      *(vec8*)(y + (v + u * stride) * 8) = out;
-    }
-  }
-  for (; v < vecs; v += stride) {
-    const vec8 in = *(const vec8*)(x + v * 8);
-    vec8 out;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = silu_16<T>(in[e]);
-    *(vec8*)(y + v * 8) = out;
-  }
-  const size_t i = vecs * 8 + (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) y[i] = silu_16<T>(x[i]);
+  silu_stream<T, 4>(x, y, count, (size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x);
 }
 
 // gemmrc for problems the tiled kernels do not take: K below 8 or beyond a buffer descriptor, the [K][N] layout with N

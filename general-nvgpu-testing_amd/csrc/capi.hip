@@ -476,28 +476,62 @@ GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, 
   return 8 * tiles >= (b_kmajor ? 7L : 6L) * cus ? ks.launch_deep_one_group[dtype][b_kmajor ? 1 : 0] : nullptr;
 }
 
-// Which form of the kernel for few rows (gemm_rows.h), if any, runs c = a @ b^T.  us, the best tiled kernel -> this one:
-//   * Up to 16 columns for every CU, 16 columns per workgroup: 4096 columns, M = 16 K = 128 3.6 -> 3.3, K = 16384
-//     37.3 -> 25.7; M = 64 K = 512 3.6 -> 3.5, K = 1024 5.0 -> 4.1, K = 16384 41.9 -> 33.1.  Beyond 32 rows the K tiles have
-//     to be more than the wavefronts: M = 64 K = 128 2.8, here 3.0, K = 320 3.1, here 3.3.
-//   * Beyond that the fetches of A add up, and B's become the bound.  M <= 16, K <= 4096: 64 columns per workgroup,
-//     M = 1: 5120 x 4096 11.7 -> 8.0, 16384 x 1024 5.4 -> 3.7, 11008 x 4096 14.8 -> 14.3; M = 16, B different in every call,
-//     11008 x 4096 21.2 -> 19.7, 12288 x 4096 22.3 -> 21.2; the tiled kernel is ahead from there on (16384 x 4088 20.6, here
-//     27.2) and where K is so short that the workgroups' starts count (65536 x 512 11.0, here 12.1).
-//   * Longer K: 16 columns, fewer wavefronts.  M = 16, B different in every call: 7680 x 10240 43.8 -> 35.4, 8192 x 8192
-//     33.8 -> 32.6, 8192 x 16384 66.2 -> 62.0.  (With the same B in every call, which then lies in the last-level cache,
-//     8192 x 8192 is 21.5, here 29.4.)  Beyond 8192 columns the tiled kernel is ahead: 10000 x 6000 21.4, here 23.0.
-//   * M <= 32: 32 columns per workgroup, 8192 x 1024 4.9 -> 4.2, x 2048 7.7 -> 6.4; 16384 x 512 3.7, here 5.0.
-RowsPlan rows_plan(int M, int N, int K, int cus) {
-  if (M > 64 || K % 8 != 0 || K > kRowsMaxK) return kRowsNone;
-  const long cols = N, round = 16L * cus;  // columns of one workgroup of 16 per CU
-  if (cols <= round) return M <= 32 || K > 320 ? kRowsNarrow : kRowsNone;
-  if (M <= 16) {
-    if (K > 4096) return cols <= 2 * round ? kRowsDeep : kRowsNone;
-    return K >= 512 && cols <= 4 * round && cols * K <= (3L << 24) ? kRowsWide : kRowsNone;
+// The tile of gemm_kwave.h for a problem, if any.  A CU's time there is what it fills LDS with, (rows + columns) x K of its
+// tile: so the tile with the smallest sum of which the problem has at most one for every CU.  (466 x 864 x 520: 32 x 64, 210
+// tiles, 4.6 us; 32 x 32, 405 tiles, 5.0; 300 x 400 x 513: 32 x 16, 250 tiles, 3.7, 16 x 16, 475 tiles, 4.0, 32 x 32 4.3.
+// Beyond one tile of 64 x 64 for every CU the tiled kernels are ahead: 2048 x 1024 x 2040 18.8, here 20.0.)
+//   b_kmajor: the form; on_lines: every row of A (and of B as [N][K]) starts on a 128-byte line.
+KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool on_lines, int cus) {
+  static const struct { int rows, cols; } kTiles[] = {{8, 16},  {16, 16}, {16, 32}, {32, 16}, {32, 32},
+                                                      {8, 64},  {16, 64}, {32, 64}, {64, 32}, {64, 64}};
+  const KwPlan none = {0, 0, 0, false};
+  if (K < 8 || K > kMaxK || (b_kmajor && N % 8 != 0)) return none;
+  // Longer sums of more than a handful of rows are what beam_gemmrc_splitk is for (256 x 256 x 32768: 12.2 us there, 22.0
+  // here), and a tuner that compares the two is to find it there; the line is where the two are about even (256 x 256 x 8192:
+  // 8.7, here 7.1; 128 x 128 x 16384: 8.3, here 12.0).
+  if (M > 64 && K >= 8192 && !b_kmajor) return none;
+  for (const auto& t : kTiles) {
+    if (t.rows == 8 && (M > 8 || b_kmajor)) continue;
+    const long tiles_n = (N + t.cols - 1) / t.cols, tiles = (long)((M + t.rows - 1) / t.rows) * tiles_n;
+    if (tiles > cus) continue;
+    KwPlan plan = {t.rows, t.cols, 4, false};
+    // The smallest tiles have little in flight for a wavefront: eight of them from K = 2048 on (256 x 256 x 4088 6.3 -> 5.8 us;
+    // x 1032 3.4, with eight 3.7).
+    if (t.rows <= 16 && t.cols == 16 && K >= 2048) plan.waves = 8;
+    // Whole lines where the fills saved are more than the one that every wavefront adds: K tiles x (rows + columns) of 1200
+    // (1024 x 1024 x 520, 9 x 128: 6.2 us, shifted 6.8; 466 x 864 x 1032, 17 x 96: 6.6, shifted 6.1; 256 x 256 x 2056,
+    // 33 x 32: 4.4, shifted 4.5).  8 rows are bound by latency: 1 x 1024 x 9480 6.4, shifted 7.2.
+    plan.shift = !on_lines && t.rows > 8 && (long)(K / kBK) * (t.rows + t.cols) >= 1200;
+    // A full tile per CU with rows on lines: from K = 2048 on the deep pipeline's two K groups, whose sums cost less to bring
+    // together (1024 x 1024 x 2048 8.8 us, here 9.4; 128 x 8192 x 4096 15.5, 16.6; 1024^3 8.3, here 6.8); and where one row of
+    // tiles streams B from memory (64 x 16384 x 1024 8.9, here 9.6).
+    if (t.rows * t.cols == 64 * 64 && on_lines && (K >= 2048 || M <= 64)) return none;
+    return plan;
   }
-  if (M <= 32 && cols <= 2 * round && K >= 1024 && K <= 2048) return kRowsWide;
-  return kRowsNone;
+  return none;
+}
+
+bool rows_on_lines(const void* A, const void* B, int K, bool b_kmajor) {
+  return K % kBK == 0 && (((uintptr_t)A | (b_kmajor ? 0 : (uintptr_t)B)) & 127) == 0;
+}
+
+void kw_params(KwParams* p, const KwPlan& plan, const void* A, const void* B, void* C, int M, int N, int K) {
+  p->A = A;
+  p->B = B;
+  p->C = C;
+  p->M = M;
+  p->N = N;
+  p->K = K;
+  p->tiles_m = (M + plan.rows - 1) / plan.rows;
+  p->tiles_n = (N + plan.cols - 1) / plan.cols;
+  p->group_m = 8;
+  p->divs = make_tile_divs(p->tiles_m, p->tiles_n, p->group_m);
+}
+
+hipError_t run_kwave(const KwPlan& plan, const void* A, const void* B, void* C, int M, int N, int K, int dtype, bool b_kmajor, hipStream_t st) {
+  KwParams p;
+  kw_params(&p, plan, A, B, C, M, N, K);
+  return dtype == BEAM_F16 ? launch_gemm_kwave<_Float16>(plan, p, b_kmajor, st) : launch_gemm_kwave<__bf16>(plan, p, b_kmajor, st);
 }
 
 }  // namespace
@@ -521,9 +555,11 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     return BEAM_OK;
   }
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
-  if (const RowsPlan plan = cfg ? kRowsNone : rows_plan(M, N, K, cus); plan != kRowsNone) {
-    BEAM_HIP(launch_gemm_rows(plan, A, B, C, M, N, K, dtype, st));
-    return BEAM_OK;
+  if (!cfg) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
+      BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, st));
+      return BEAM_OK;
+    }
   }
   beam_tile_cfg c;
   const KernelSet* ks;
@@ -589,6 +625,12 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
   if (generic || N < 8 || N > (N % 8 != 0 ? 1 << 23 : 1 << 24)) {
     BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, true, false, st));
     return BEAM_OK;
+  }
+  if (!cfg) {
+    if (const KwPlan kw = kw_plan(M, N, K, true, rows_on_lines(A, B, K, true), g_dev.cus > 0 ? g_dev.cus : 256); kw.rows) {
+      BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, true, st));
+      return BEAM_OK;
+    }
   }
   beam_tile_cfg c;
   const KernelSet* ks;
@@ -687,19 +729,35 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   const long long wgs = (long long)((M + c.block_m - 1) / c.block_m) * ((N + c.block_n - 1) / c.block_n);
   const long long per_pass = wgs * ks->threads;  // units one K tile of the whole grid covers
-  // With the library's tile, a GEMM kernel that carries no side job and is the faster one by more than the second launch
-  // costs (2.5 us), or too few workgroups to keep memory busy for a long job: the two kernels one after the other.
-  //   * The deep pipeline: less than half the CUs busy, or tiles of 64 rows (two K groups).  2^18 elements, one launch, two
-  //     launches: 155 x 2040 x 1536 10.1, 9.1 us; 2048 x 1024 x 2048 18.9, 15.9; 580 x 968 x 5672 39.4, 29.4.  Tiles of 128
-  //     rows gain less than that: 128 x 128 (one group) 496 x 5688 x 1224 13.2, 15.3; 530 x 4400 x 3528 36.0, 37.2; 128 x 64
-  //     1377 x 1416 x 832 7.7, 9.8; 5813 x 312 x 6256 46.4, 47.2.
-  //   * Few rows, whose launch alone takes 3-5 us: from K = 768 on (1 x 512, 2^12 elements: K = 512 4.8, 5.4; K = 1024 7.1,
-  //     5.5), or from 8 passes of the grid over the job on (1 x 1024 x 64 with 2^19 9.9, 5.4; 64 x 64 x 64 with 2^12 3.6, 5.4).
+  // With the library's tile:
+  //   * Where the GEMM runs on gemm_kwave.h, the job rides in workgroups of its own behind the tiles (one launch; two launches,
+  //     us: 256 x 256 x 512 with 2^18 elements 6.5, 10.1; 1000 x 600 x 1000 with 2^22 9.1, 12.2; 299 x 824 x 3968 with 2^24
+  //     17.6, 21.1).  Such a workgroup holds a tile's LDS, so beyond 2^23 elements, but for the 32 KiB of the smallest tiles,
+  //     too few of them are on a CU to keep memory busy: 1024^3 with 2^24 21.7, two launches 18.9.
+  //   * A GEMM kernel that carries no side job and is the faster one by more than the second launch costs (2.5 us): the deep
+  //     pipeline with less than half the CUs busy, or with tiles of 64 rows (two K groups).  One launch, two launches: 2048 x
+  //     1024 x 2048 with 2^18 elements 18.9, 15.9.  Tiles of 128 rows gain less than that: 128 x 128 (one group) 496 x 5688 x
+  //     1224 13.2, 15.3; 128 x 64 5813 x 312 x 6256 46.4, 47.2.
   if (!cfg) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
+      if (kw.rows + kw.cols > 32 && count > (1 << 23)) {
+        BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, (hipStream_t)stream));
+        return beam_silu(X, Y, count, dtype, stream);
+      }
+      KwSideParams p;
+      kw_params(&p, kw, A, B, C, M, N, K);
+      p.side_x = X;
+      p.side_y = Y;
+      p.side_count = count;
+      const long long per_wg = (long long)kw.waves * 64 * 8 * 8;  // elements of one round of a workgroup's accesses
+      const long long want = (count + per_wg - 1) / per_wg;
+      const int side = (int)(want < 8 * cus ? want : 8 * cus);
+      BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_kwave_side<_Float16>(kw, p, side, (hipStream_t)stream)
+                                 : launch_gemm_kwave_side<__bf16>(kw, p, side, (hipStream_t)stream));
+      return BEAM_OK;
+    }
     const bool two_groups = c.block_m == 64;
-    const bool deep = c.pipeline == 2 && (wgs * 2 < cus || two_groups);
-    const bool rows = rows_plan(M, N, K, cus) != kRowsNone && (K >= 768 || (count >> 3) > 8 * per_pass);
-    if (deep || rows) {
+    if (c.pipeline == 2 && (wgs * 2 < cus || two_groups)) {
       if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
       return beam_silu(X, Y, count, dtype, stream);
     }
@@ -726,8 +784,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   // A job that outlasts the loop goes on at 0.4-1.4 us for every 16 bytes per thread; with a round of workgroups or less,
   // from 8 such passes on (more behind a long loop, whose own passes are the cheaper for it: 992 x 3976 x 3288 with 2^26
   // elements, 52 K tiles and 12 passes beyond them, 84.4, 88.9), a launch of its own (3 us and 11 us per 16 Mi elements) is ahead.  Fused, then two launches:
-  // 256^3 with 2^20 elements (28 passes) 15.8, 6.5 us; 1024^3 with 2^24 (16) 30.3, 20.7; 4096 x 4096 x 256 with 2^24 (12)
-  // 28.9, 26.4; but 1536 x 1536 x 512 with 2^22 (7) 9.4, 10.5.  With several rounds the later workgroups hide it:
+  // 4096 x 4096 x 256 with 2^24 (12) 28.9, 26.4; but 1536 x 1536 x 512 with 2^22 (7) 9.4, 10.5.  With several rounds the later workgroups hide it:
   // 8192 x 8192 x 256 with 2^26 (12) 110.8, 117.7.
   if (!cfg && wgs <= cus && p.side_iters - k_tiles > 8 + k_tiles / 8) {
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;

@@ -38,4 +38,33 @@ __device__ __forceinline__ T silu_16(T x) {
   return (T)silu_f32<sizeof(T) == 2 && !__is_same(T, _Float16)>((float)x);
 }
 
+// y[i] = silu(x[i]) by thread `id` of `threads` that share the array: 16 bytes per access, U accesses in flight.
+template <typename T, int U>
+__device__ __forceinline__ void silu_stream(const T* __restrict__ x, T* __restrict__ y, size_t count, size_t id, size_t threads) {
+  typedef T vec8 __attribute__((ext_vector_type(8)));
+  const size_t vecs = count / 8;
+  size_t v = id;
+  for (; v + (U - 1) * threads < vecs; v += U * threads) {
+    vec8 in[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) in[u] = *(const vec8*)(x + (v + u * threads) * 8);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      vec8 out;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) out[e] = silu_16<T>(in[u][e]);
+      *(vec8*)(y + (v + u * threads) * 8) = out;
+    }
+  }
+  for (; v < vecs; v += threads) {
+    const vec8 in = *(const vec8*)(x + v * 8);
+    vec8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e] = silu_16<T>(in[e]);
+    *(vec8*)(y + v * 8) = out;
+  }
+  const size_t i = vecs * 8 + id;
+  if (i < count) y[i] = silu_16<T>(x[i]);
+}
+
 }  // namespace beam

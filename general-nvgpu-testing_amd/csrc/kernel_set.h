@@ -8,6 +8,7 @@
 
 #include "../../include/beam_hip.h"
 #include "gemm_kernel.h"
+#include "gemm_kwave.h"
 
 namespace beam {
 
@@ -162,16 +163,22 @@ hipError_t launch_gemm_w4_kmajor(const GemmParams& p, int dtype, dim3 grid, hipS
 // workgroup per CU) makes them walk, which needs tiles_n <= kW4LnCompactTiles.  gamma and beta 16-byte aligned as well.
 constexpr int kW4LnCompactTiles = 32;
 hipError_t launch_gemm_w4_ln(const GemmParams& p, int dtype, dim3 grid, hipStream_t stream);
-// c = a @ b^T for few rows (gemm_rows.h); needs 8 <= K <= kRowsMaxK, K % 8 == 0, and M <= 64 (narrow), 16 (deep) or
-// 32 (wide).
-enum RowsPlan : int {
-  kRowsNone = 0,
-  kRowsNarrow = 1,  // 16 columns per workgroup, 8 or 4 wavefronts
-  kRowsDeep = 2,    // 16 columns, 4 wavefronts
-  kRowsWide = 3,    // 64 (M <= 16) or 32 columns, 4 wavefronts
+// The kernel of gemm_kwave.h: workgroup tiles of at most 64 x 64 whose K range is dealt out to the wavefronts.
+struct KwPlan {
+  int rows, cols;  // workgroup tile; rows == 0: not this kernel
+  int waves;       // wavefronts of a workgroup (8 only for the tiles of 16 columns and at most 16 rows)
+  bool shift;      // fills take whole lines of memory (KwRows)
 };
-constexpr int kRowsMaxK = 1 << 23;
-hipError_t launch_gemm_rows(RowsPlan plan, const void* A, const void* B, void* C, int M, int N, int K, int dtype, hipStream_t stream);
+// Needs 8 <= K, and M <= rows for tiles of 8 rows; B stored [K][N]: N % 8 == 0 and tiles of 16 rows and more.
+template <typename T>
+hipError_t launch_gemm_kwave(const KwPlan& plan, const KwParams& p, bool b_kmajor, hipStream_t stream);
+// The GEMM with a SiLU job in `side_workgroups` more workgroups of the same launch; X and Y on 16 bytes.
+template <typename T>
+hipError_t launch_gemm_kwave_side(const KwPlan& plan, const KwSideParams& p, int side_workgroups, hipStream_t stream);
+template <> hipError_t launch_gemm_kwave_side<_Float16>(const KwPlan&, const KwSideParams&, int, hipStream_t);
+template <> hipError_t launch_gemm_kwave_side<__bf16>(const KwPlan&, const KwSideParams&, int, hipStream_t);
+template <> hipError_t launch_gemm_kwave<_Float16>(const KwPlan&, const KwParams&, bool, hipStream_t);
+template <> hipError_t launch_gemm_kwave<__bf16>(const KwPlan&, const KwParams&, bool, hipStream_t);
 // Measurement only: the split-K partial kernel of the 64 x 128 (wave 32 x 64) or 64 x 64 (wave 32 x 32) tile, deep
 // pipeline, fp16, with its loads and fragment reads but no MFMAs and no stores (kEpiProbeLoads); hipErrorInvalidValue
 // for any other tile.

@@ -67,8 +67,9 @@ int beam_default_config(int M, int N, int K, beam_tile_cfg* cfg, int* split_k);
 
 /* ---- tiled GEMM ------------------------------------------------------------------------ */
 
-/* cfg == NULL: beam_default_config() picks the tile (never a split); up to 64 rows of A may run on a kernel of their own
- * that has no tile to name, or on the deep pipeline as one group of wavefronts.  Any K and any element's address; a tile
+/* cfg == NULL: beam_default_config() picks the tile (never a split); where tiles of 64 x 64 or less fill at most one round of
+ * workgroups, the call may run on a kernel that has no tile to name (small tiles, K dealt out to the wavefronts), or on the
+ * deep pipeline as one group of wavefronts.  Any K and any element's address; a tile
  * that is not compiled is refused, but for rows that are not 16-byte aligned, which are computed whatever is named.
  * Replaces entry_cutlass_gemmrc / entry_cutlass_gemmrc_spec
  * (cuda/cutlass_kernels/main.cc:11-15, cutlass_gemmrc.cu:21-40,55-111). */
@@ -223,8 +224,8 @@ int beam_set_ln_walk(int on);
 /* ---- GEMM with an independent elementwise job hidden in its K loop ------------------------ */
 
 /* C = A . B^T as beam_gemmrc (with cfg NULL its sums may be added in another order than there) and, in the same launch (with
- * cfg NULL in a second one where the GEMM's own kernel is the faster by more than that costs, has too few workgroups for the
- * job, or too short a K loop), Y[i] = silu(X[i]) = X[i] / (1 + exp(-X[i]))
+ * cfg NULL in workgroups of its own behind the GEMM's, or in a second launch where the GEMM's own kernel is the faster by
+ * more than that costs, has too few workgroups for the job, or too short a K loop), Y[i] = silu(X[i]) = X[i] / (1 + exp(-X[i]))
  * for i in [0, count): 16-bit in, fp32 arithmetic, round-to-nearest 16-bit out.  The array is cut into
  * units of 4, 8 or 16 bytes (the narrowest with which the job still ends inside the K loop), dealt out in
  * contiguous runs over the GEMM's workgroups and carried, a few units per K tile, by the wavefronts that

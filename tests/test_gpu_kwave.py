@@ -1,0 +1,77 @@
+"""Small workgroup tiles whose K range is dealt out to the wavefronts, as calls without a named tile reach them: every tile,
+fewer K tiles than wavefronts, K tiles that end inside a chunk, rows on and off 128-byte lines (both ways of filling LDS),
+operands at any element's address inside buffers of NaNs.  Bounds: close_enough's, the one of every other GEMM test."""
+import numpy as np
+import pytest
+
+from test_gpu_edges import close_enough
+from test_gpu_gemm import F16, BF16
+from test_gpu_unaligned import run
+
+pytestmark = pytest.mark.gpu
+
+# The smallest tile of which the problem has at most 256: one shape for each, ragged in both directions where it can be.
+TILES = {"8x16": (5, 300), "16x16": (41, 100), "16x32": (297, 400), "32x16": (1030, 100), "32x32": (509, 500), "8x64": (3, 8300),
+         "16x64": (130, 1750), "32x64": (466, 864), "64x32": (1030, 475), "64x64": (1000, 1003)}
+# one chunk, one K tile, fewer K tiles than wavefronts, several for each; from about 640 (64x64) to 2500 (16x16) on, rows off
+# 128-byte lines are filled line by line
+KS = [8, 9, 64, 71, 200, 513, 1096, 2057, 3208, 3265]
+
+
+@pytest.mark.parametrize("tile", sorted(TILES))
+@pytest.mark.parametrize("K", KS)
+def test_gemmrc(gpu, beamc, oracle, tile, K):
+    assert gpu["compute_units"] == 256  # the shapes are chosen for that
+    L = beamc.lib
+    M, N = TILES[tile]
+    for dtype, offsets in ((F16, (0, 0, 0)), (BF16, (1, 3, 1)), (F16, (8, 24, 0))):
+        a, b = beamc.host_uniform((M, K), dtype, 94, 0), beamc.host_uniform((N, K), dtype, 94, 1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offsets)
+        close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"{tile} {(M, N, K)} at {offsets}")
+
+
+# [K][N]: the number of columns is a multiple of 8
+@pytest.mark.parametrize("M,N", [(41, 96), (297, 400), (1030, 104), (509, 504), (130, 1752), (466, 864), (1030, 472), (1000, 1000), (1, 4096)])
+@pytest.mark.parametrize("K", KS)
+def test_matmul_nn(gpu, beamc, oracle, M, N, K):
+    L = beamc.lib
+    for dtype, offsets in ((F16, (0, 0, 0)), (BF16, (3, 1, 1))):
+        a, b = beamc.host_uniform((M, K), dtype, 95, 0), beamc.host_uniform((K, N), dtype, 95, 1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offsets)
+        close_enough(oracle, out, oracle.matmul_nn(a, b, dtype), K, dtype, f"[K][N] {(M, N, K)} at {offsets}")
+
+
+def test_infinities_and_nan_stay_in_their_row_or_column(gpu, beamc):
+    """Line by line a fill brings chunks of two K tiles; a chunk behind the end of K must still be a zero for every row."""
+    M, N, K = 70, 90, 3001
+    L = beamc.lib
+    a, b = beamc.host_uniform((M, K), F16, 96, 0), beamc.host_uniform((N, K), F16, 96, 1)
+    a[69, 3000], a[68, 0], b[88, 1500] = 0x7E00, 0xFC00, 0x7C00
+    out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
+    assert np.isnan(out[69]).all() and not np.isfinite(out[68]).any() and not np.isfinite(out[:, 88]).any()
+    assert np.isfinite(np.delete(out[:68], 88, axis=1)).all()
+
+
+# The elementwise job rides in workgroups of its own behind the tiles'.  Counts: a tail only, one access of one thread, ragged,
+# more than one round of the accesses of every such workgroup.
+@pytest.mark.parametrize("tile", ["8x16", "16x16", "32x32", "64x64"])
+def test_silu_job(gpu, beamc, tile):
+    L = beamc.lib
+    M, N = TILES[tile]
+    for K, dtype in ((200, F16), (2600, BF16)):
+        da, db = (beamc.DeviceArray.from_numpy(beamc.host_uniform(s, dtype, 97, i), dtype) for i, s in enumerate(((M, K), (N, K))))
+        want, got = beamc.DeviceArray((M, N), dtype), beamc.DeviceArray((M, N), dtype)
+        beamc._check(L.beam_gemmrc(da.ptr, db.ptr, want.ptr, M, N, K, dtype, None, None))
+        for count in (0, 5, 8, 4099, 300007, (1 << 22) + 3):
+            dx = beamc.DeviceArray.from_numpy(beamc.host_normal((max(count, 1) + 64,), dtype, 97, 2, 0.0, 2.5), dtype)
+            y, alone = (beamc.DeviceArray((max(count, 1) + 64,), dtype) for _ in range(2))
+            for d in (got, y, alone):
+                d.fill_bytes(0xEE)
+            beamc._check(L.beam_silu(dx.ptr, alone.ptr, count, dtype, None))
+            beamc._check(L.beam_parallel_gemmrc_silu(da.ptr, db.ptr, got.ptr, M, N, K, dx.ptr, y.ptr, count, dtype, None, None))
+            assert (got.to_numpy() == want.to_numpy()).all(), (tile, K, count)
+            assert (y.to_numpy() == alone.to_numpy()).all(), (tile, K, count)  # the guard behind the array included
+            for d in (dx, y, alone):
+                d.free()
+        for d in (da, db, want, got):
+            d.free()
