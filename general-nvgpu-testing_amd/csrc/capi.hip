@@ -480,8 +480,8 @@ GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, 
 // tile: so the tile with the smallest sum of which the problem has at most one for every CU.  (466 x 864 x 520: 32 x 64, 210
 // tiles, 4.6 us; 32 x 32, 405 tiles, 5.0; 300 x 400 x 513: 32 x 16, 250 tiles, 3.7, 16 x 16, 475 tiles, 4.0, 32 x 32 4.3.
 // Beyond one tile of 64 x 64 for every CU the tiled kernels are ahead: 2048 x 1024 x 2040 18.8, here 20.0.)
-//   b_kmajor: the form; on_lines: every row of A (and of B as [N][K]) starts on a 128-byte line.
-KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool on_lines, int cus) {
+//   b_kmajor, ln: the form; on_lines: every row of A (and of B as [N][K]) starts on a 128-byte line.
+KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool on_lines, int cus) {
   static const struct { int rows, cols; } kTiles[] = {{8, 16},  {16, 16}, {16, 32}, {32, 16}, {32, 32},
                                                       {8, 64},  {16, 64}, {32, 64}, {64, 32}, {64, 64}};
   const KwPlan none = {0, 0, 0, false};
@@ -489,15 +489,15 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool on_lines, int cus) {
   // Longer sums of more than a handful of rows are what beam_gemmrc_splitk is for (256 x 256 x 32768: 12.2 us there, 22.0
   // here), and a tuner that compares the two is to find it there; the line is where the two are about even (256 x 256 x 8192:
   // 8.7, here 7.1; 128 x 128 x 16384: 8.3, here 12.0).
-  if (M > 64 && K >= 8192 && !b_kmajor) return none;
+  if (M > 64 && K >= 8192 && !b_kmajor && !ln) return none;
   for (const auto& t : kTiles) {
-    if (t.rows == 8 && (M > 8 || b_kmajor)) continue;
+    if (t.rows == 8 && (M > 8 || b_kmajor || ln)) continue;
     const long tiles_n = (N + t.cols - 1) / t.cols, tiles = (long)((M + t.rows - 1) / t.rows) * tiles_n;
-    if (tiles > cus) continue;
+    if (tiles > cus || (ln && tiles_n > 64)) continue;
     KwPlan plan = {t.rows, t.cols, 4, false};
     // The smallest tiles have little in flight for a wavefront: eight of them from K = 2048 on (256 x 256 x 4088 6.3 -> 5.8 us;
     // x 1032 3.4, with eight 3.7).
-    if (t.rows <= 16 && t.cols == 16 && K >= 2048) plan.waves = 8;
+    if (t.rows <= 16 && t.cols == 16 && K >= 2048 && !ln) plan.waves = 8;
     // Whole lines where the fills saved are more than the one that every wavefront adds: K tiles x (rows + columns) of 1200
     // (1024 x 1024 x 520, 9 x 128: 6.2 us, shifted 6.8; 466 x 864 x 1032, 17 x 96: 6.6, shifted 6.1; 256 x 256 x 2056,
     // 33 x 32: 4.4, shifted 4.5).  8 rows are bound by latency: 1 x 1024 x 9480 6.4, shifted 7.2.
@@ -505,7 +505,10 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool on_lines, int cus) {
     // A full tile per CU with rows on lines: from K = 2048 on the deep pipeline's two K groups, whose sums cost less to bring
     // together (1024 x 1024 x 2048 8.8 us, here 9.4; 128 x 8192 x 4096 15.5, 16.6; 1024^3 8.3, here 6.8); and where one row of
     // tiles streams B from memory (64 x 16384 x 1024 8.9, here 9.6).
-    if (t.rows * t.cols == 64 * 64 && on_lines && (K >= 2048 || M <= 64)) return none;
+    if (t.rows * t.cols == 64 * 64 && on_lines && !ln && (K >= 2048 || M <= 64)) return none;
+    // LayerNorm on full tiles under a short sum: the sums' way through LDS is the larger part (1024 x 1024 x 520 9.1 us, here
+    // 9.9; x 1000 12.7, 12.2; x 1528 15.8, 13.7).
+    if (t.rows * t.cols == 64 * 64 && ln && K < 600) return none;
     return plan;
   }
   return none;
@@ -556,7 +559,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   }
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
       BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, st));
       return BEAM_OK;
     }
@@ -627,7 +630,7 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     return BEAM_OK;
   }
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, true, rows_on_lines(A, B, K, true), g_dev.cus > 0 ? g_dev.cus : 256); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, true, false, rows_on_lines(A, B, K, true), g_dev.cus > 0 ? g_dev.cus : 256); kw.rows) {
       BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, true, st));
       return BEAM_OK;
     }
@@ -739,7 +742,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   //     1024 x 2048 with 2^18 elements 18.9, 15.9.  Tiles of 128 rows gain less than that: 128 x 128 (one group) 496 x 5688 x
   //     1224 13.2, 15.3; 128 x 64 5813 x 312 x 6256 46.4, 47.2.
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
       if (kw.rows + kw.cols > 32 && count > (1 << 23)) {
         BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, (hipStream_t)stream));
         return beam_silu(X, Y, count, dtype, stream);
@@ -1016,6 +1019,10 @@ static size_t ln_fused_set_bytes(size_t tiles_m, size_t tiles_n, int block_m) {
   return align_up(tiles_m * tiles_n * (size_t)block_m * 2 * sizeof(float), 256);
 }
 
+static size_t ln_fused_need(int M, int N, int block_m, int block_n) {
+  return ln_fused_header_bytes() + 2 * ln_fused_set_bytes((size_t)(M + block_m - 1) / block_m, (size_t)(N + block_n - 1) / block_n, block_m);
+}
+
 static bool ln_fused_applies_on(const beam_tile_cfg& c, const KernelSet& ks, int N, int cus) {
   // The residency argument of the fused kernel (tile_map.h: band_block_tile) is made for 8 XCDs of 32 CUs.
   if (cus != kNumXcd * 32) return false;
@@ -1040,9 +1047,8 @@ static size_t ln_generic_need(int M, int N) { return align_up((size_t)M * N * si
 
 // Bytes for tile `c` in `mode` (already resolved: two-pass or fused).
 static size_t ln_workspace_need(int M, int N, const beam_tile_cfg& c, int mode) {
-  const size_t tiles_m = (size_t)(M + c.block_m - 1) / c.block_m;
   const size_t tiles_n = (size_t)(N + c.block_n - 1) / c.block_n;
-  if (mode == BEAM_LN_FUSED) return ln_fused_header_bytes() + 2 * ln_fused_set_bytes(tiles_m, tiles_n, c.block_m);
+  if (mode == BEAM_LN_FUSED) return ln_fused_need(M, N, c.block_m, c.block_n);
   return align_up((size_t)M * N * sizeof(float), 256) + align_up((size_t)M * tiles_n * 2 * sizeof(float), 256);
 }
 
@@ -1126,19 +1132,33 @@ struct LnPlan {
   enum Kind { kPlain, kTwoPass, kFused } kind;
   beam_tile_cfg c;
   const KernelSet* ks;
-  bool w4;  // fused, on the kernel of gemm_w4.h
+  bool w4;    // fused, on the kernel of gemm_w4.h
+  KwPlan kw;  // fused, on the kernel of gemm_kwave.h if kw.rows != 0 (c and ks then say nothing)
   size_t need;
 };
+// The library's own choice of gemm_kwave.h for the one-kernel form (its workgroups must be resident at once, and its order of
+// bands is made for 8 XCDs of 32 CUs).
+static KwPlan ln_kw_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode) {
+  if (cfg || mode == BEAM_LN_TWOPASS || g_dev.cus != kNumXcd * 32) return KwPlan{0, 0, 0, false};
+  return kw_plan(M, N, K, false, true, true, g_dev.cus);
+}
 static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool plain, bool unaligned, bool capturing, bool wide_io,
                    LnPlan* out) {
   out->ks = nullptr;
   out->w4 = false;
+  out->kw = KwPlan{0, 0, 0, false};
   if (plain) {
     out->kind = LnPlan::kPlain;
     out->need = ln_generic_need(M, N);
     return BEAM_OK;
   }
   if (capturing && mode == BEAM_LN_AUTO) mode = BEAM_LN_TWOPASS;
+  out->kw = ln_kw_plan(M, N, K, cfg, mode);
+  if (out->kw.rows) {
+    out->kind = LnPlan::kFused;
+    out->need = ln_fused_need(M, N, out->kw.rows, out->kw.cols);
+    return BEAM_OK;
+  }
   int rc = ln_resolve_cfg(cfg, M, N, K, mode, &out->c, &out->ks);
   beam_tile_cfg& c = out->c;
   if ((unaligned || K % 8 != 0) && (rc || (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N)))) {
@@ -1212,6 +1232,7 @@ size_t beam_gemmrc_ln_workspace_bytes_ex(int M, int N, const beam_tile_cfg* cfg,
     take(ln_workspace_need(M, N, c, ln_resolve_mode(mode, c, *ks, N)));
     if (mode == BEAM_LN_AUTO) take(ln_workspace_need(M, N, c, BEAM_LN_TWOPASS));
   }
+  if (const KwPlan kw = ln_kw_plan(M, N, kBK, cfg, mode); kw.rows) take(ln_fused_need(M, N, kw.rows, kw.cols));
   return need;
 }
 
@@ -1273,6 +1294,26 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     return BEAM_OK;
   }
   if ((uintptr_t)ws & 255) return fail(BEAM_ERR_UNSUPPORTED, "workspace must be 256-byte aligned");
+  if (plan.kw.rows) {
+    KwPlan kw = plan.kw;
+    kw.shift = kw_plan(M, N, K, false, true, rows_on_lines(A, B, K, false), g_dev.cus).shift;
+    KwLnParams p;
+    kw_params(&p, kw, A, B, Y, M, N, K);
+    p.divs = band_order_divs(p.tiles_n, 1, -1);
+    if (capturing != hipStreamCaptureStatusNone) BEAM_HIP(launch_ln_replay_bump((int*)ws, st));
+    char* sets = (char*)ws + ln_fused_header_bytes();
+    p.stats = (float*)sets;
+    p.next_stats = (float*)(sets + ln_fused_set_bytes(p.tiles_m, p.tiles_n, kw.rows));
+    p.timeout_flag = (int*)ws;
+    p.host_timeout = g_ln_host_timeout;
+    p.gamma = gamma;
+    p.beta = beta;
+    p.ln_nonce = g_ln_nonce.fetch_add(1, std::memory_order_relaxed) + 1;
+    p.eps = eps;
+    p.spin_limit = g_ln_spin_limit.load();
+    BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_kwave_ln<_Float16>(kw, p, st) : launch_gemm_kwave_ln<__bf16>(kw, p, st));
+    return BEAM_OK;
+  }
   const beam_tile_cfg& c = plan.c;
   const KernelSet* ks = plan.ks;
   GemmParams p = base_params(A, B, M, N, K, c);

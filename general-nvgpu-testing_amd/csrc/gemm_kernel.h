@@ -150,7 +150,7 @@ struct GemmParams {
   int sk_self;
 };
 
-// ---- statistics exchange of the fused GEMM+LayerNorm (both K loops: this file's and gemm_w4.h's) ----------
+// ---- statistics exchange of the fused GEMM+LayerNorm (GemmParams here and in gemm_w4.h, KwLnParams in gemm_kwave.h) ----
 // A tile publishes, per row, two 8-byte words: (mean, tag) and (M2, ~tag), each with one device-scope atomic
 // store.  Such stores go straight through the XCD-private L2 to memory and the device-scope loads of the
 // gather come straight from it, so the exchange needs no cache-wide write-back / invalidate (a
@@ -161,7 +161,8 @@ struct GemmParams {
 // earlier launch or of another shape, or somebody else's data.  So a workspace needs no preparation, no
 // clearing between launches and no state on the host.  (A stray word passes for published with probability
 // 2^-32 per word, and both words of a row have to.)
-__device__ __forceinline__ unsigned ln_launch_tag(const GemmParams& p) {
+template <typename Params>
+__device__ __forceinline__ unsigned ln_launch_tag(const Params& p) {
   unsigned x = p.ln_nonce + (unsigned)p.timeout_flag[kLnHdrReplay] * 0x9E3779B1u;  // uniform: nobody writes it during a launch
   x ^= x >> 16;
   x *= 0x7feb352du;
@@ -171,20 +172,23 @@ __device__ __forceinline__ unsigned ln_launch_tag(const GemmParams& p) {
   return x | 1u;  // never 0: a zeroed header then never reads as "timed out"
 }
 
-__device__ __forceinline__ void ln_record_timeout(const GemmParams& p, unsigned tag) {
+template <typename Params>
+__device__ __forceinline__ void ln_record_timeout(const Params& p, unsigned tag) {
   p.timeout_flag[kLnHdrTimeout] = (int)tag;
   if (p.host_timeout) __hip_atomic_store(p.host_timeout, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Workgroup 0 records which launch the header speaks of.
-__device__ __forceinline__ void ln_sign_header(const GemmParams& p, unsigned tag) {
+template <typename Params>
+__device__ __forceinline__ void ln_sign_header(const Params& p, unsigned tag) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     p.timeout_flag[kLnHdrMagic] = kLnMagic;
     p.timeout_flag[kLnHdrLaunchTag] = (int)tag;
   }
 }
 
-__device__ __forceinline__ void ln_publish(const GemmParams& p, size_t slot, float mean, float m2, unsigned tag) {
+template <typename Params>
+__device__ __forceinline__ void ln_publish(const Params& p, size_t slot, float mean, float m2, unsigned tag) {
   const unsigned long long w0 = (unsigned long long)__float_as_uint(mean) | ((unsigned long long)tag << 32);
   const unsigned long long w1 = (unsigned long long)__float_as_uint(m2) | ((unsigned long long)(~tag) << 32);
   __hip_atomic_store((unsigned long long*)p.stats + slot, w0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -196,8 +200,8 @@ __device__ __forceinline__ void ln_publish(const GemmParams& p, size_t slot, flo
 // per thread) until both words of each of its slots carry the tag.  A thread that runs out of budget raises the
 // header's flag and poisons the pairs still missing, so that the rows concerned come out as NaN instead of as
 // plausible numbers.
-template <int NT, int INFLIGHT = 8>
-__device__ __forceinline__ void ln_gather(const GemmParams& p, unsigned tag, size_t first, int n_slots, int tid,
+template <int NT, int INFLIGHT = 8, typename Params>
+__device__ __forceinline__ void ln_gather(const Params& p, unsigned tag, size_t first, int n_slots, int tid,
                                           unsigned long long* gathered) {
   const unsigned long long* w0s = (const unsigned long long*)p.stats + first;
   const unsigned long long* w1s = (const unsigned long long*)p.next_stats + first;

@@ -50,6 +50,38 @@ struct KwSideParams : KwParams {
   long long side_count;
 };
 
+// GEMM+LayerNorm: the exchange of gemm_kernel.h, workgroups in band order (id = band * tiles_n + column tile).
+struct KwLnParams : KwParams {
+  float* stats;  // 8-byte words [tiles_m][tiles_n][ROWS] = (mean, tag)
+  float* next_stats;  // ... = (M2, ~tag)
+  int* timeout_flag;
+  unsigned* host_timeout;
+  const void* gamma;
+  const void* beta;
+  unsigned ln_nonce;
+  float eps;
+  int spin_limit;
+};
+
+// Column tiles of a band that stays together on an XCD.  A launch that shares the device and gets s of an XCD's 32 CUs still
+// finishes band by band if s is at least this many: XCD 0 starts with a whole band, and each XCD's last band is what
+// the next one's first workgroups wait for.  (Longer bands, as long as a round of workgroups: any 64 CUs do.)
+constexpr int kKwLnShortBand = 8;
+
+// Sum over W (4, 8 or 16) neighbouring lanes, the same bits in each of them.
+template <int W>
+__device__ __forceinline__ float lanes_sum(float x) {
+  static_assert(W == 4 || W == 8 || W == 16, "a row of 16 lanes at most");
+  auto add = [](float v, auto ctrl) __attribute__((always_inline)) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  x = add(x, std::integral_constant<int, 0xB1>{});                           // quad_perm 1 0 3 2
+  x = add(x, std::integral_constant<int, 0x4E>{});                           // quad_perm 2 3 0 1
+  if constexpr (W >= 8) x = add(x, std::integral_constant<int, 0x141>{});   // row_half_mirror
+  if constexpr (W >= 16) x = add(x, std::integral_constant<int, 0x140>{});  // row_mirror
+  return x;
+}
+
 // K-major B slots (64 rows of k, COLS columns): the 16-byte chunk position of chunk c of row k, for conflict-free transposing
 // reads (tile_map.h: kmajor_swizzle).  64 columns: that layout.  32 columns: four rows to a bank sweep, the segment XORed
 // with bit 3 of k.  16 columns: eight rows to a sweep, and rows 4 .. 7 and 8 .. 11 of every 16 change places.
@@ -386,6 +418,104 @@ struct KwTile {
       store_quad((T*)p.C, m, n, p.N, o);
     }
   }
+
+  // The tile's share of y = LayerNorm(x) * gamma + beta.  A thread owns QT quads of the summed tile; a row's quads are
+  // neighbouring lanes.  Beyond the product's time this is a chain of latencies: the tile's statistics to memory, the band's
+  // back, 3 us.  us, the tiled kernel (one K group, tiles of 64 x 64 and more) -> this: 100 x 304 x 3896 26.9 -> 8.8,
+  // 151 x 632 x 4384 32.0 -> 10.2, 512 x 1024 x 1000 12.0 -> 8.7, 1024 x 1024 x 3000 24.9 -> 18.2, 1298 x 312 x 7512 51.8 -> 21.4.
+  static __device__ __forceinline__ void run_ln(const KwLnParams& p, char* smem) {
+    constexpr int QT = (QUADS + NT - 1) / NT;
+    constexpr int TPR = NT / ROWS < 16 ? NT / ROWS : 16;  // threads that merge a row's statistics
+    static_assert(AG >= 2 && QUADS % 64 == 0 && (QUADS < NT || QUADS % NT == 0) && TPR * ROWS <= NT, "LayerNorm threads");
+    static_assert((64 + 1) * ROWS * 8 <= LDS_BYTES, "statistics of 64 column tiles and the row results");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Short bands stay together on an XCD, which then fetches their rows once (1298 x 312 x 7512 28.7 -> 25.9 us); long ones
+    // are spread in id order.
+    const int id = p.tiles_n <= kKwLnShortBand ? xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n) : (int)blockIdx.x;
+    const int tm = (int)fast_div((unsigned)id, p.divs.tiles), tn = id - tm * p.tiles_n;
+    const int row0 = tm * ROWS, col0 = tn * COLS;
+    const int M = p.M, N = p.N;
+    char* const ring = smem + wave * (S * SLOT);
+    f32x4 acc[MB][CB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < CB; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    multiply(p, row0, col0, wave, lane, ring, acc);
+    // a thread's columns are the same for all its quads (NT is a multiple of CG)
+    const int cg = tid % CG, n = col0 + cg * 4;
+    vec4 g, b;
+    if (N % 4 == 0 && n < N) {
+      g = *(const vec4*)((const T*)p.gamma + n);
+      b = *(const vec4*)((const T*)p.beta + n);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int nn = n + e < N ? n + e : N - 1;
+        g[e] = ((const T*)p.gamma)[nn];
+        b[e] = ((const T*)p.beta)[nn];
+      }
+    }
+    const unsigned tag = ln_launch_tag(p);
+    ln_sign_header(p, tag);
+    meet(lane, ring, acc);
+    f32x4 v[QT];
+#pragma unroll
+    for (int u = 0; u < QT; ++u) v[u] = tid + u * NT < QUADS ? total(smem, tid + u * NT) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    __syncthreads();  // the sums have been read: LDS is free
+    // the tile's (mean, M2) per row: about the tile's own mean first, so nothing cancels
+    const int cols = N - col0 < COLS ? N - col0 : COLS;
+    const size_t band = (size_t)tm * p.tiles_n * ROWS;
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      float s = 0.0f, m2 = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += n + e < N ? v[u][e] : 0.0f;
+      const float mean = lanes_sum<CG>(s) / (float)cols;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float d = n + e < N ? v[u][e] - mean : 0.0f;
+        m2 += d * d;
+      }
+      m2 = lanes_sum<CG>(m2);
+      if (cg == 0 && tid + u * NT < QUADS) ln_publish(p, band + (size_t)tn * ROWS + (tid + u * NT) / CG, mean, m2, tag);
+    }
+    float* const red = (float*)smem;          // [ROWS][2]: (mean, 1 / standard deviation) of the whole row
+    float* const gathered = red + ROWS * 2;   // [tiles_n][ROWS][2]
+    ln_gather<NT>(p, tag, band, p.tiles_n * ROWS, tid, (unsigned long long*)gathered);
+    __syncthreads();
+    if (tid < ROWS * TPR) {
+      const int r = tid / TPR, part = tid % TPR;
+      float s = 0.0f, m2 = 0.0f;
+      for (int t = part; t < p.tiles_n; t += TPR) {
+        const int w = N - t * COLS < COLS ? N - t * COLS : COLS;
+        s += (float)w * gathered[(t * ROWS + r) * 2];
+      }
+      const float mean = lanes_sum<TPR>(s) / (float)N;
+      for (int t = part; t < p.tiles_n; t += TPR) {
+        const int w = N - t * COLS < COLS ? N - t * COLS : COLS;
+        const float d = gathered[(t * ROWS + r) * 2] - mean;
+        m2 += gathered[(t * ROWS + r) * 2 + 1] + (float)w * d * d;
+      }
+      m2 = lanes_sum<TPR>(m2);
+      if (part == 0) {
+        red[r * 2] = mean;
+        red[r * 2 + 1] = 1.0f / sqrtf(m2 / (float)N + p.eps);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      const int q = tid + u * NT, m = row0 + q / CG;
+      if (q >= QUADS || m >= M || n >= N) continue;
+      const float mean = red[q / CG * 2], rstd = red[q / CG * 2 + 1];
+      vec4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (T)((v[u][e] - mean) * rstd * (float)g[e] + (float)b[e]);
+      store_quad((T*)p.C, m, n, N, o);
+    }
+  }
 };
 
 template <typename T, int AG, int CB, int NW, int S, KwRows MODE, bool KMAJOR>
@@ -407,6 +537,12 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_kwave_side_kernel(const KwSid
     return;
   }
   KwTile<T, AG, CB, NW, S, MODE, false>::run(p, smem);
+}
+
+template <typename T, int AG, int CB, int NW, int S, KwRows MODE>
+__global__ void __launch_bounds__(NW * 64, 2) gemm_kwave_ln_kernel(const KwLnParams p) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  KwTile<T, AG, CB, NW, S, MODE, false>::run_ln(p, smem);
 }
 
 }  // namespace beam

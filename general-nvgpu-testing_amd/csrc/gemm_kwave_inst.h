@@ -17,6 +17,16 @@ hipError_t launch_plain(const KwParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int AG, int CB, int NW, int S, KwRows MODE>
+hipError_t launch_ln(const KwLnParams& p, hipStream_t stream) {
+  using Tile = KwTile<KW_T, AG, CB, NW, S, MODE, false>;
+  auto kern = gemm_kwave_ln_kernel<KW_T, AG, CB, NW, S, MODE>;
+  static std::atomic<unsigned long long> configured{0};
+  if (hipError_t e = allow_lds_once(configured, reinterpret_cast<const void*>(kern), Tile::LDS_BYTES); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(NW * 64), Tile::LDS_BYTES, stream, p);
+  return hipGetLastError();
+}
+
 template <int AG, int CB, int NW>
 hipError_t launch_tile(const KwPlan& plan, const KwParams& p, bool b_kmajor, hipStream_t stream) {
   if constexpr (AG >= 2) {
@@ -41,6 +51,11 @@ hipError_t launch_side(const KwSideParams& p, int side_workgroups, hipStream_t s
 template <int AG, int CB, int NW>
 hipError_t launch_tile_side(const KwPlan& plan, const KwSideParams& p, int side_workgroups, hipStream_t stream) {
   return plan.shift ? launch_side<AG, CB, NW, kKwShift>(p, side_workgroups, stream) : launch_side<AG, CB, NW, kKwStraight>(p, side_workgroups, stream);
+}
+
+template <int AG, int CB>
+hipError_t launch_tile_ln(const KwPlan& plan, const KwLnParams& p, hipStream_t stream) {
+  return plan.shift ? launch_ln<AG, CB, 4, 2, kKwShift>(p, stream) : launch_ln<AG, CB, 4, 2, kKwStraight>(p, stream);
 }
 
 }  // namespace
@@ -76,6 +91,21 @@ hipError_t launch_gemm_kwave_side<KW_T>(const KwPlan& plan, const KwSideParams& 
     case 32 * 256 + 64: return launch_tile_side<4, 4, 4>(plan, p, n, stream);
     case 64 * 256 + 32: return launch_tile_side<8, 2, 4>(plan, p, n, stream);
     case 64 * 256 + 64: return launch_tile_side<8, 4, 4>(plan, p, n, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <>
+hipError_t launch_gemm_kwave_ln<KW_T>(const KwPlan& plan, const KwLnParams& p, hipStream_t stream) {
+  switch (plan.rows * 256 + plan.cols) {
+    case 16 * 256 + 16: return launch_tile_ln<2, 1>(plan, p, stream);
+    case 16 * 256 + 32: return launch_tile_ln<2, 2>(plan, p, stream);
+    case 32 * 256 + 16: return launch_tile_ln<4, 1>(plan, p, stream);
+    case 32 * 256 + 32: return launch_tile_ln<4, 2>(plan, p, stream);
+    case 16 * 256 + 64: return launch_tile_ln<2, 4>(plan, p, stream);
+    case 32 * 256 + 64: return launch_tile_ln<4, 4>(plan, p, stream);
+    case 64 * 256 + 32: return launch_tile_ln<8, 2>(plan, p, stream);
+    case 64 * 256 + 64: return launch_tile_ln<8, 4>(plan, p, stream);
   }
   return hipErrorInvalidValue;
 }

@@ -172,6 +172,10 @@ struct KwPlan {
 // Needs 8 <= K, and M <= rows for tiles of 8 rows; B stored [K][N]: N % 8 == 0 and tiles of 16 rows and more.
 template <typename T>
 hipError_t launch_gemm_kwave(const KwPlan& plan, const KwParams& p, bool b_kmajor, hipStream_t stream);
+// GEMM+LayerNorm in one launch: tiles of 16 rows and more, tiles_n <= 64, gamma and beta on 8 bytes, and a grid whose
+// workgroups are resident at once.
+template <typename T>
+hipError_t launch_gemm_kwave_ln(const KwPlan& plan, const KwLnParams& p, hipStream_t stream);
 // The GEMM with a SiLU job in `side_workgroups` more workgroups of the same launch; X and Y on 16 bytes.
 template <typename T>
 hipError_t launch_gemm_kwave_side(const KwPlan& plan, const KwSideParams& p, int side_workgroups, hipStream_t stream);
@@ -179,6 +183,8 @@ template <> hipError_t launch_gemm_kwave_side<_Float16>(const KwPlan&, const KwS
 template <> hipError_t launch_gemm_kwave_side<__bf16>(const KwPlan&, const KwSideParams&, int, hipStream_t);
 template <> hipError_t launch_gemm_kwave<_Float16>(const KwPlan&, const KwParams&, bool, hipStream_t);
 template <> hipError_t launch_gemm_kwave<__bf16>(const KwPlan&, const KwParams&, bool, hipStream_t);
+template <> hipError_t launch_gemm_kwave_ln<_Float16>(const KwPlan&, const KwLnParams&, hipStream_t);
+template <> hipError_t launch_gemm_kwave_ln<__bf16>(const KwPlan&, const KwLnParams&, hipStream_t);
 // Measurement only: the split-K partial kernel of the 64 x 128 (wave 32 x 64) or 64 x 64 (wave 32 x 32) tile, deep
 // pipeline, fp16, with its loads and fragment reads but no MFMAs and no stores (kEpiProbeLoads); hipErrorInvalidValue
 // for any other tile.

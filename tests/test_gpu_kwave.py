@@ -1,11 +1,14 @@
 """Small workgroup tiles whose K range is dealt out to the wavefronts, as calls without a named tile reach them: every tile,
 fewer K tiles than wavefronts, K tiles that end inside a chunk, rows on and off 128-byte lines (both ways of filling LDS),
 operands at any element's address inside buffers of NaNs.  Bounds: close_enough's, the one of every other GEMM test."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from test_gpu_edges import close_enough
 from test_gpu_gemm import F16, BF16
+from test_gpu_ln import check_ln, make_ln_inputs, run_ln
 from test_gpu_unaligned import run
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +78,81 @@ def test_silu_job(gpu, beamc, tile):
                 d.free()
         for d in (da, db, want, got):
             d.free()
+
+
+LN_TILES = {"16x16": (41, 100), "16x32": (297, 400), "32x16": (1030, 100), "32x32": (509, 500), "16x64": (130, 1750), "32x64": (466, 864),
+            "64x32": (1030, 475), "64x64": (1000, 1003), "64 column tiles": (60, 4096)}
+
+
+@pytest.mark.parametrize("tile", sorted(LN_TILES))
+@pytest.mark.parametrize("K", [8, 71, 513, 1096, 3265])
+def test_layer_norm(gpu, beamc, oracle, tile, K):
+    """One kernel (the caller's choice, so it is no fallback), columns that end inside a tile, statistics of up to 64 tiles."""
+    M, N = LN_TILES[tile]
+    for dtype in (F16, BF16):
+        a, b, g, bt = make_ln_inputs(beamc, M, N, K, dtype, 98)
+        got = run_ln(beamc, a, b, g, bt, dtype, mode=beamc.LN_FUSED)
+        check_ln(oracle, got, oracle.gemmrc_ln(a, b, g, bt, 1e-5, dtype), dtype, f"{tile} {(M, N, K)} dtype {dtype}")
+
+
+@pytest.mark.parametrize("M,N", [(41, 100), (1030, 475), (60, 4096)])
+def test_layer_norm_gives_up_and_recovers(gpu, beamc, M, N):
+    """With every wait forced to give up the kernel ends normally, its rows are NaN and the default call repeats as two passes;
+    the next call is right again, with no reset in between."""
+    K = 264
+    a, b, g, bt = make_ln_inputs(beamc, M, N, K, F16, 99)
+    good, two_pass = (run_ln(beamc, a, b, g, bt, F16, mode=m) for m in (beamc.LN_FUSED, beamc.LN_TWOPASS))
+    d = [beamc.DeviceArray.from_numpy(x) for x in (a, b, g, bt)]
+    y = beamc.DeviceArray((M, N))
+    try:
+        assert beamc.lib.beam_set_ln_spin_limit(-1) == 0
+        beamc.gemmrc_ln(d[0], d[1], y, d[2], d[3], mode=beamc.LN_FUSED, check=False)
+        beamc.sync()
+        assert beamc.gemmrc_ln_timed_out() and np.isnan(y.to_numpy().view(np.float16)).all()
+        assert beamc.gemmrc_ln(d[0], d[1], y, d[2], d[3]) is True
+        assert (y.to_numpy() == two_pass).all()
+    finally:
+        beamc.lib.beam_set_ln_spin_limit(beamc.DEFAULT_SPIN_LIMIT)
+    assert beamc.gemmrc_ln(d[0], d[1], y, d[2], d[3]) is False
+    assert (y.to_numpy() == good).all()
+    for t in d + [y]:
+        t.free()
+
+
+@pytest.mark.parametrize("M,N", [(1030, 475), (500, 1024), (60, 4096)])
+def test_layer_norm_launches_share_the_device(gpu, beamc, M, N):
+    """Two streams with launches that wait for their own workgroups: short bands, which stay on an XCD, and long ones."""
+    K, L = 520, beamc.lib
+    streams = []
+    for _ in range(2):
+        s = ctypes.c_void_p()
+        beamc._check(L.beam_stream_create(ctypes.byref(s)))
+        streams.append(s)
+    sets = []
+    for i in range(2):
+        d = [beamc.DeviceArray.from_numpy(x) for x in make_ln_inputs(beamc, M, N, K, F16, 72 + i)]
+        sets.append((d, beamc.DeviceArray((M, N)), beamc.DeviceArray((L.beam_gemmrc_ln_workspace_bytes_for(M, N, K, None, beamc.LN_FUSED),), itemsize=1)))
+
+    def launch(i, stream):
+        d, y, ws = sets[i]
+        beamc._check(L.beam_gemmrc_ln_ex(d[0].ptr, d[1].ptr, d[2].ptr, d[3].ptr, ctypes.c_float(1e-5), y.ptr, M, N, K, F16, None, beamc.LN_FUSED,
+                                         ws.ptr, ws.nbytes, stream))
+
+    want = []
+    for i in range(2):
+        launch(i, None)
+        beamc.sync()
+        want.append(sets[i][1].to_numpy().copy())
+    for rep in range(20):
+        for _ in range(4):
+            for i in range(2):
+                launch(i, streams[i])
+        for i in range(2):
+            flag = ctypes.c_int(1)
+            beamc._check(L.beam_gemmrc_ln_timed_out(sets[i][2].ptr, streams[i], ctypes.byref(flag)))
+            assert flag.value == 0 and (sets[i][1].to_numpy() == want[i]).all(), (i, rep)
+    for s in streams:
+        beamc._check(L.beam_stream_destroy(s))
+    for d, y, ws in sets:
+        for t in d + [y, ws]:
+            t.free()
