@@ -147,17 +147,18 @@ _TORCH_FIRST = False
 lib = _load()
 
 # What the operators need of torch, looked up once.  torch.cuda.current_stream() builds a Stream object after a walk
-# through the device index' conversions (2.8 us on the machine measured, three times per call before: 10.6 of a call's
-# 14.6 us); the raw handle of the current device's current stream is what a launch takes, and costs 0.1 us: a call of
-# gemmrc returns after 5.9 us, 4.3 of them in the library's launch.
+# through the device index' conversions (2.8 us on the machine measured); the raw handle of the current device's current
+# stream is what a launch takes, and costs 0.1 us.  _native (csrc/torch_binding.cc) is the ordinary call without all that:
+# plain torch tensors and no named tile.  It answers with a status, or a negative number for what it leaves to the code below.
 if _TORCH_FIRST:
+    from . import _torch_binding as _native
     import torch as _torch
     _Tensor = _torch.Tensor
     _TORCH_DTYPES = {_torch.float16: F16, _torch.bfloat16: BF16}
     _raw_stream = getattr(_torch._C, "_cuda_getCurrentRawStream", None)
     _raw_device = getattr(_torch._C, "_cuda_getDevice", None)
 else:
-    _torch = _Tensor = _raw_stream = _raw_device = None
+    _native = _torch = _Tensor = _raw_stream = _raw_device = None
     _TORCH_DTYPES = {}
 
 
@@ -362,6 +363,8 @@ def _get_workspace(nbytes: int) -> DeviceArray:
 
 def gemmrc(a, b, c, config: Optional[TileConfig] = None) -> None:
     """c = a @ b.T with the library's default tile (or `config`)."""
+    if _native is not None and config is None and (status := _native.gemmrc(a, b, c)) >= 0:
+        return _check(status)
     pa, pb, pc, M, N, K, d, st = _problem(a, b, c)
     cfg = ctypes.byref(config.to_c()) if config is not None else None
     _check(lib.beam_gemmrc(pa, pb, pc, M, N, K, d, cfg, st))
@@ -410,6 +413,10 @@ def gemmrc_splitk(a, b, c, split_k_slices: int = 0, check: bool = False) -> None
     picks the slice count as well (one full round of workgroups)
     (reference: cutlass_gemmrc_splitk, python/beam/_C/beam_C.pyi:18).  check=True waits for the
     result and raises if the one-launch form's bounded wait ran out."""
+    if _native is not None and split_k_slices <= 0 and not check:
+        ws = _workspace
+        if (status := _native.gemmrc_splitk(a, b, c, ws.ptr if ws else 0, ws.nbytes if ws else 0)) >= 0:
+            return _check(status)
     _splitk(a, b, c, None, split_k_slices, check)
 
 
@@ -434,6 +441,12 @@ def gemmrc_ln(a, b, c, gamma, beta, eps: float = 1e-5, config: Optional[TileConf
     runs out, LN_AUTO repeats the call as two passes (the return value is then True, and c is right either way) and
     an explicit LN_FUSED raises BeamError.  check=False launches and returns at once, like the other operators: the
     rows concerned are NaN if that ever happens, and gemmrc_ln_timed_out() tells."""
+    if _native is not None and config is None and mode == LN_AUTO and (ws := _ln_workspace) is not None:
+        status = _native.gemmrc_ln(a, b, c, gamma, beta, eps, check, ws.ptr, ws.nbytes)
+        if status != -1:
+            if status > 0:
+                _check(status)
+            return status == -2  # repeated as two passes
     pa, pb, pc, M, N, K, d, st = _problem(a, b, c)
     pg, sg, dg = _describe(gamma)
     pbt, sbt, dbt = _describe(beta)
@@ -471,6 +484,9 @@ def gemmrc_ln_timed_out() -> bool:
 def matmul(a, b, c=None, config: Optional[TileConfig] = None):
     """c = a @ b with a [M, K] and b [K, N], both row-major; returns c (allocated like the inputs when
     not given).  Reference: matmul(a, b) of python/beam/triton_kernels/gemm.py:78-99."""
+    if _native is not None and c is not None and config is None and (status := _native.matmul(a, b, c)) >= 0:
+        _check(status)
+        return c
     pa, sa, da = _describe(a)
     pb, sb, db = _describe(b)
     if len(sa) != 2 or len(sb) != 2 or sa[1] != sb[0]:
@@ -513,6 +529,8 @@ def parallel_gemmrc_silu(a, b, c, x, y, config: Optional[TileConfig] = None) -> 
     """c = a @ b.T and y = silu(x): the elementwise job is streamed through the GEMM's K loop in the same launch, or,
     with no tile given and a GEMM that is the faster without it, run in a second one.  Reference: cutlass_parallel_gemmrc_lnr(gemmA, gemmB, gemmC, lnA, lnB),
     cuda/cute_kernels/main.cc:55-76 (python/beam/_C/beam_C.pyi:20)."""
+    if _native is not None and config is None and (status := _native.parallel_gemmrc_silu(a, b, c, x, y)) >= 0:
+        return _check(status)
     pa, pb, pc, M, N, K, d, st = _problem(a, b, c)
     px, py, n, _, _ = _flat_pair(x, y, d)
     cfg = config.to_c() if config is not None else None
