@@ -480,12 +480,13 @@ GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, 
 // tile: so the tile with the smallest sum of which the problem has at most one for every CU.  (466 x 864 x 520: 32 x 64, 210
 // tiles, 4.6 us; 32 x 32, 405 tiles, 5.0; 300 x 400 x 513: 32 x 16, 250 tiles, 3.7, 16 x 16, 475 tiles, 4.0, 32 x 32 4.3.
 // Beyond one tile of 64 x 64 for every CU the tiled kernels are ahead: 2048 x 1024 x 2040 18.8, here 20.0.)
-//   b_kmajor, ln: the form; on_lines: every row of A (and of B as [N][K]) starts on a 128-byte line.
-KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool on_lines, int cus) {
+//   b_kmajor, ln: the form; rows: where every row of A (and of B as [N][K]) starts.
+enum RowStarts { kAnywhere, kOnChunks, kOnLines };  // at an element, on 16 bytes, on 128
+KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, RowStarts rows, int cus) {
   static const struct { int rows, cols; } kTiles[] = {{8, 16},  {16, 16}, {16, 32}, {32, 16}, {32, 32},
                                                       {8, 64},  {16, 64}, {32, 64}, {64, 32}, {64, 64}};
   const KwPlan none = {0, 0, 0, false};
-  if (K < 8 || K > kMaxK || (b_kmajor && N % 8 != 0)) return none;
+  if (K < 8 || K > kMaxK) return none;
   // Longer sums of more than a handful of rows are what beam_gemmrc_splitk is for (256 x 256 x 32768: 12.2 us there, 22.0
   // here), and a tuner that compares the two is to find it there; the line is where the two are about even (256 x 256 x 8192:
   // 8.7, here 7.1; 128 x 128 x 16384: 8.3, here 12.0).
@@ -500,12 +501,13 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool on_lines, int c
     if (t.rows <= 16 && t.cols == 16 && K >= 2048 && !ln) plan.waves = 8;
     // Whole lines where the fills saved are more than the one that every wavefront adds: K tiles x (rows + columns) of 1200
     // (1024 x 1024 x 520, 9 x 128: 6.2 us, shifted 6.8; 466 x 864 x 1032, 17 x 96: 6.6, shifted 6.1; 256 x 256 x 2056,
-    // 33 x 32: 4.4, shifted 4.5).  8 rows are bound by latency: 1 x 1024 x 9480 6.4, shifted 7.2.
-    plan.shift = !on_lines && t.rows > 8 && (long)(K / kBK) * (t.rows + t.cols) >= 1200;
+    // 33 x 32: 4.4, shifted 4.5).  8 rows are bound by latency: 1 x 1024 x 9480 6.4, shifted 7.2.  Rows off 16 bytes have chunks
+    // in two lines however they are fetched: 600 x 600 x 3004 12.6 either way, x 3001 14.3, shifted 15.9.
+    plan.shift = rows == kOnChunks && t.rows > 8 && (long)(K / kBK) * (t.rows + t.cols) >= 1200;
     // A full tile per CU with rows on lines: from K = 2048 on the deep pipeline's two K groups, whose sums cost less to bring
     // together (1024 x 1024 x 2048 8.8 us, here 9.4; 128 x 8192 x 4096 15.5, 16.6; 1024^3 8.3, here 6.8); and where one row of
     // tiles streams B from memory (64 x 16384 x 1024 8.9, here 9.6).
-    if (t.rows * t.cols == 64 * 64 && on_lines && !ln && (K >= 2048 || M <= 64)) return none;
+    if (t.rows * t.cols == 64 * 64 && rows == kOnLines && !ln && (K >= 2048 || M <= 64)) return none;
     // LayerNorm on full tiles under a short sum: the sums' way through LDS is the larger part (1024 x 1024 x 520 9.1 us, here
     // 9.9; x 1000 12.7, 12.2; x 1528 15.8, 13.7).
     if (t.rows * t.cols == 64 * 64 && ln && K < 600) return none;
@@ -514,8 +516,9 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool on_lines, int c
   return none;
 }
 
-bool rows_on_lines(const void* A, const void* B, int K, bool b_kmajor) {
-  return K % kBK == 0 && (((uintptr_t)A | (b_kmajor ? 0 : (uintptr_t)B)) & 127) == 0;
+RowStarts row_starts(const void* A, const void* B, int K, bool b_kmajor) {
+  const uintptr_t at = (uintptr_t)A | (b_kmajor ? 0 : (uintptr_t)B);
+  return K % kBK == 0 && (at & 127) == 0 ? kOnLines : K % 8 == 0 && (at & 15) == 0 ? kOnChunks : kAnywhere;
 }
 
 void kw_params(KwParams* p, const KwPlan& plan, const void* A, const void* B, void* C, int M, int N, int K) {
@@ -559,7 +562,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   }
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, false, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, false, row_starts(A, B, K, false), cus); kw.rows) {
       BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, st));
       return BEAM_OK;
     }
@@ -630,7 +633,7 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     return BEAM_OK;
   }
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, true, false, rows_on_lines(A, B, K, true), g_dev.cus > 0 ? g_dev.cus : 256); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, true, false, row_starts(A, B, K, true), g_dev.cus > 0 ? g_dev.cus : 256); kw.rows) {
       BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, true, st));
       return BEAM_OK;
     }
@@ -742,7 +745,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   //     1024 x 2048 with 2^18 elements 18.9, 15.9.  Tiles of 128 rows gain less than that: 128 x 128 (one group) 496 x 5688 x
   //     1224 13.2, 15.3; 128 x 64 5813 x 312 x 6256 46.4, 47.2.
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, false, false, rows_on_lines(A, B, K, false), cus); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, false, row_starts(A, B, K, false), cus); kw.rows) {
       if (kw.rows + kw.cols > 32 && count > (1 << 23)) {
         BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, (hipStream_t)stream));
         return beam_silu(X, Y, count, dtype, stream);
@@ -1140,7 +1143,7 @@ struct LnPlan {
 // bands is made for 8 XCDs of 32 CUs).
 static KwPlan ln_kw_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode) {
   if (cfg || mode == BEAM_LN_TWOPASS || g_dev.cus != kNumXcd * 32) return KwPlan{0, 0, 0, false};
-  return kw_plan(M, N, K, false, true, true, g_dev.cus);
+  return kw_plan(M, N, K, false, true, kOnLines, g_dev.cus);
 }
 static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool plain, bool unaligned, bool capturing, bool wide_io,
                    LnPlan* out) {
@@ -1232,7 +1235,7 @@ size_t beam_gemmrc_ln_workspace_bytes_ex(int M, int N, const beam_tile_cfg* cfg,
     take(ln_workspace_need(M, N, c, ln_resolve_mode(mode, c, *ks, N)));
     if (mode == BEAM_LN_AUTO) take(ln_workspace_need(M, N, c, BEAM_LN_TWOPASS));
   }
-  if (const KwPlan kw = ln_kw_plan(M, N, kBK, cfg, mode); kw.rows) take(ln_fused_need(M, N, kw.rows, kw.cols));
+  if (const KwPlan kw = ln_kw_plan(M, N, 1024, cfg, mode); kw.rows) take(ln_fused_need(M, N, kw.rows, kw.cols));
   return need;
 }
 
@@ -1296,7 +1299,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   if ((uintptr_t)ws & 255) return fail(BEAM_ERR_UNSUPPORTED, "workspace must be 256-byte aligned");
   if (plan.kw.rows) {
     KwPlan kw = plan.kw;
-    kw.shift = kw_plan(M, N, K, false, true, rows_on_lines(A, B, K, false), g_dev.cus).shift;
+    kw.shift = kw_plan(M, N, K, false, true, row_starts(A, B, K, false), g_dev.cus).shift;
     KwLnParams p;
     kw_params(&p, kw, A, B, Y, M, N, K);
     p.divs = band_order_divs(p.tiles_n, 1, -1);

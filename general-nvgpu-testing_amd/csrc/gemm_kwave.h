@@ -124,7 +124,10 @@ struct KwTile {
     const int M = p.M, N = p.N, K = p.K;
     const int rows_a = M - row0 < ROWS ? M - row0 : ROWS;
     const int rows_b = N - col0 < COLS ? N - col0 : COLS;
-    const int k8 = K >> 3;                 // whole chunks of 8 elements; K % 8 more come last
+    // Whole chunks of 8 elements, and up to 8 that come last.  K-major rows that are not whole chunks: the very last row is
+    // always among those, so that every row that is fetched has another one behind it and may be read to a whole chunk.
+    const bool n_odd = KMAJOR && (N & 7) != 0;
+    const int k8 = (K - (n_odd ? 1 : 0)) >> 3, rem = K - 8 * k8;
     const int n_all = (k8 + 7) >> 3;       // K tiles
     // This wavefront's K tiles are t0, t0 + EVERY, ...; may be none.  Shifted, a part of K in one piece (K tile t + 1's line
     // holds chunks of K tile t); straight, every NW-th.
@@ -186,9 +189,10 @@ struct KwTile {
         // with shifted rows of A, K tile t - 1 is multiplied when fill t has arrived
         const int koff = (t0 + (SHIFT ? t - 1 : t * EVERY)) * kBK;
         const bool exists = SHIFT ? t >= 1 && t <= n : t < n;
-        const int rows = K - koff < kBK ? K - koff : kBK;
+        // (not the rows behind the whole chunks: those of A are zeros there, and zero times infinity is not)
+        const int rows = 8 * k8 - koff < kBK ? 8 * k8 - koff : kBK;
         // (columns past N in the rows in front of the last read the next row's data and feed outputs that do not exist)
-        const __amdgpu_buffer_rsrc_t rk = make_rsrc(b_base + (exists ? (size_t)koff * N : 0), exists ? ((unsigned)(rows - 1) * (unsigned)N + (unsigned)(N - col0)) * 2u : 0u);
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(b_base + (exists ? (size_t)koff * N : 0), exists ? ((unsigned)(rows - 1) * (unsigned)N + (unsigned)(N - col0) + (n_odd ? 7u : 0u)) * 2u : 0u);
 #pragma unroll
         for (int i = 0; i < LB; ++i)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)(dst + A_BYTES + i * 1024), 16, (int)voff_b[i], 0, 0, 0);
@@ -326,9 +330,9 @@ struct KwTile {
     }
     wait_vm_and_lds<0>();  // the empty fills of the last iterations must be gone before the ring is reused
 
-    // K % 8 elements behind the last whole chunk, straight from memory: lanes 0 .. 15 hold them as the first of an MFMA's
+    // The elements behind the last whole chunk, straight from memory: lanes 0 .. 15 hold them as the first of an MFMA's
     // four groups of 8, the other lanes zeros.  A row's last 16 bytes are fetched as they stand and shifted down.
-    if (const int rem = K & 7; rem != 0 && wave == NW - 1) {  // (uniform)
+    if (rem != 0 && wave == NW - 1) {  // (uniform)
       const int r = lane & 15;
       auto row_end = [&](const T* base, int rows, int block) __attribute__((always_inline)) {
         typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
@@ -337,6 +341,7 @@ struct KwTile {
         const unsigned off = lane < 16 && row < rows ? (unsigned)row * row_bytes + row_bytes - 16u : kOobOffset;
         const u64x2 w = __builtin_bit_cast(u64x2, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
         const int bits = 128 - 16 * rem;
+        if (bits == 0) return __builtin_bit_cast(vec8, w);
         u64x2 o;
         o[0] = bits >= 64 ? w[1] >> (bits - 64) : (w[0] >> bits) | (w[1] << (64 - bits));
         o[1] = bits >= 64 ? 0ull : w[1] >> bits;

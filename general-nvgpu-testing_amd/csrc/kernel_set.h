@@ -169,7 +169,7 @@ struct KwPlan {
   int waves;       // wavefronts of a workgroup (8 only for the tiles of 16 columns and at most 16 rows)
   bool shift;      // fills take whole lines of memory (KwRows)
 };
-// Needs 8 <= K, and M <= rows for tiles of 8 rows; B stored [K][N]: N % 8 == 0 and tiles of 16 rows and more.
+// Needs 8 <= K, and M <= rows for tiles of 8 rows; B stored [K][N]: N >= 8 and tiles of 16 rows and more.
 template <typename T>
 hipError_t launch_gemm_kwave(const KwPlan& plan, const KwParams& p, bool b_kmajor, hipStream_t stream);
 // GEMM+LayerNorm in one launch: tiles of 16 rows and more, tiles_n <= 64, gamma and beta on 8 bytes, and a grid whose

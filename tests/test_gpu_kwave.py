@@ -33,8 +33,8 @@ def test_gemmrc(gpu, beamc, oracle, tile, K):
         close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"{tile} {(M, N, K)} at {offsets}")
 
 
-# [K][N]: the number of columns is a multiple of 8
-@pytest.mark.parametrize("M,N", [(41, 96), (297, 400), (1030, 104), (509, 504), (130, 1752), (466, 864), (1030, 472), (1000, 1000), (1, 4096)])
+# [K][N], rows of whole chunks and not
+@pytest.mark.parametrize("M,N", [(41, 9), (60, 69), (466, 35), (87, 998), (1000, 1003), (41, 96), (297, 400), (1030, 104), (509, 504), (130, 1752), (466, 864), (1030, 472), (1000, 1000), (1, 4096)])
 @pytest.mark.parametrize("K", KS)
 def test_matmul_nn(gpu, beamc, oracle, M, N, K):
     L = beamc.lib
@@ -53,6 +53,19 @@ def test_infinities_and_nan_stay_in_their_row_or_column(gpu, beamc):
     out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
     assert np.isnan(out[69]).all() and not np.isfinite(out[68]).any() and not np.isfinite(out[:, 88]).any()
     assert np.isfinite(np.delete(out[:68], 88, axis=1)).all()
+
+
+@pytest.mark.parametrize("N", [88, 90])
+def test_infinities_of_b_behind_the_whole_chunks(gpu, beamc, N):
+    """[K][N]: a row of B behind K's last whole chunk meets only its own elements of A, never the zeros beside them."""
+    M, K = 37, 75
+    L = beamc.lib
+    a, b = beamc.host_uniform((M, K), F16, 97, 0), beamc.host_uniform((K, N), F16, 97, 1)
+    a[:, 73] = 0x3C00  # one
+    b[73, 5], b[K - 1, 7], a[:, K - 1] = 0x7C00, 0xFC00, 0x3C00
+    out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
+    assert (out[:, 5] == np.inf).all() and (out[:, 7] == -np.inf).all()
+    assert np.isfinite(np.delete(out, (5, 7), axis=1)).all()
 
 
 # The elementwise job rides in workgroups of its own behind the tiles'.  Counts: a tail only, one access of one thread, ragged,
