@@ -181,7 +181,9 @@ def as_run(name, M, N, K):
     tiles = math.ceil(M / bm) * math.ceil(N / bn)
     if (bm, bn) == (256, 256) and tiles >= CUS and K % 64 == 0 and K >= W4_MIN_K and N % 8 == 0:
         return "256x256_w128x128"
-    if not name.endswith("_deep") and K >= 2048 and (tiles < CUS // 2 or (tiles <= CUS and bm * bn <= 128 * 64)):
+    few = K >= 2048 and tiles < CUS // 2
+    groups = tiles <= CUS and (bm * bn <= 128 * 64 if K >= 2048 else K >= 768 and bm * bn == 128 * 64)
+    if not name.endswith("_deep") and (few or groups):
         return name + "_deep"
     return name
 

@@ -445,13 +445,15 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
     cfg->wave_n = 128;
   }
   // One workgroup per CU under a long sum: the deep pipeline.  Less than half the CUs busy: its long prefetch queue keeps
-  // memory busy.  Tiles with two K groups: up to a full round, since a lone group's K tile is a serial chain.  64 x 128
-  // tiles, one group -> two: 8192 x 256 x 2048 17.6 -> 12.3 us, 654 x 1832 x 2104 21.5 -> 16.8, 2048 x 1024 x 2048 11.8 ->
-  // 11.4; 64 x 64 tiles 1024 x 1024 x 2048 8.1 -> 7.7.  At K = 1024 one group is ahead (5.2, 5.5; 6.7, 7.2).
+  // memory busy.  Tiles with two K groups: up to a full round, since a lone group's K tile is a serial chain; 64 x 64 tiles
+  // from K = 2048 on (1024^3 5.2, two groups 5.5; 1024 x 1024 x 2048 8.1, 7.7), 64 x 128 and 128 x 64 from K = 768 on (one
+  // group, two: 2048 x 1024 x 520 6.2, 6.3; x 768 8.3, 7.2; x 1024 10.0, 8.2; x 1536 13.9, 11.0; 620 x 3064 x 776 9.9, 9.3;
+  // x 1600 14.6, 11.1; [K][N] 700 x 2500 x 512 7.9, 7.3; x 1024 12.5, 10.0).
   const long picked = tiles(c.block_m, c.block_n);
-  const bool few = picked < cus / 2, groups = picked <= cus && c.block_m * c.block_n <= 128 * 64;
+  const bool few = K >= 2048 && picked < cus / 2;
+  const bool groups = picked <= cus && (K >= 2048 ? c.block_m * c.block_n <= 128 * 64 : K >= 768 && c.block_m * c.block_n == 128 * 64);
   if (raised) *raised = false;
-  if (split_req < 0 && K >= 2048 && (few || groups)) {
+  if (split_req < 0 && (few || groups)) {
     if (raised) *raised = !few && c.pipeline == 0;
     cfg->pipeline = 2;
   }
@@ -762,8 +764,8 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
                                  : launch_gemm_kwave_side<__bf16>(kw, p, side, (hipStream_t)stream));
       return BEAM_OK;
     }
-    const bool two_groups = c.block_m == 64;
-    if (c.pipeline == 2 && (wgs * 2 < cus || two_groups)) {
+    const bool two_groups = c.block_m == 64 && K >= 2048;
+    if (c.pipeline == 2 && ((wgs * 2 < cus && K >= 2048) || two_groups)) {
       if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
       return beam_silu(X, Y, count, dtype, stream);
     }

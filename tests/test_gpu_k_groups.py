@@ -48,3 +48,18 @@ def test_one_row_of_tiles_that_nearly_fills_the_chip(gpu, beamc, oracle, M, N, K
                            ("[K][N]", np.ascontiguousarray(b.T), lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, dtype, None, None))):
         out = run(beamc, call, a, bb, (M, N), dtype, (0, 0, 0))
         close_enough(oracle, out, ref, K, dtype, f"{what} {(M, N, K)}")
+
+
+@pytest.mark.parametrize("M,N,K,deep", [(1030, 1000, 704, False), (1030, 1000, 768, True), (1030, 1000, 775, True), (2048, 1024, 1100, True),
+                                        (1000, 1040, 2047, True)])
+def test_one_round_of_half_tiles(gpu, beamc, oracle, M, N, K, deep):
+    """Tiles of 64x128 and 128x64 that fill at most one round of workgroups: two K groups from K = 768 on, in both layouts."""
+    L = beamc.lib
+    cfg, _ = beamc.default_config(M, N, K)
+    assert cfg.block_m * cfg.block_n == 128 * 64 and (cfg.pipeline == 2) == deep, cfg
+    for dtype in (F16, BF16):
+        a, b = beamc.host_uniform((M, K), dtype, 85, 0), beamc.host_uniform((N, K), dtype, 85, 1)
+        ref = oracle.gemmrc(a, b, dtype)
+        for what, bb, call in (("gemmrc", b, L.beam_gemmrc), ("[K][N]", np.ascontiguousarray(b.T), L.beam_matmul_nn)):
+            out = run(beamc, lambda pa, pb, pc: call(pa, pb, pc, M, N, K, dtype, None, None), a, bb, (M, N), dtype, (0, 0, 0))
+            close_enough(oracle, out, ref, K, dtype, f"{what} {(M, N, K)}")
