@@ -864,11 +864,20 @@ static int effective_split(int M, int N, int K, const beam_tile_cfg& c, int spli
   return (ktiles + per - 1) / per;  // drop slices that would be empty
 }
 
+// The library's own choice (no tile, no slice count) for a sum that one launch without slices is the faster for: K dealt out
+// to the wavefronts of small tiles (gemm_kwave.h) where a CU then fills LDS with no more than 600 KB.
+static KwPlan splitk_kw_plan(int M, int N, int K, const beam_tile_cfg* cfg, int split_k, RowStarts rows) {
+  if (cfg || split_k > 0 || K >= 8192) return KwPlan{0, 0, 0, false};
+  const KwPlan kw = kw_plan(M, N, K, false, false, rows, g_dev.cus > 0 ? g_dev.cus : 256);
+  return (long)(kw.rows + kw.cols) * K <= 300000 ? kw : KwPlan{0, 0, 0, false};
+}
+
 int beam_splitk_effective(int M, int N, int K, const beam_tile_cfg* cfg, int split_k) {
   beam_tile_cfg c;
   const KernelSet* ks;
   if (M <= 0 || N <= 0 || K < 0) return 1;
   if ((K > 0 && K < 8) || K > kMaxK) return 1;  // the plain kernel: no slices
+  if (K > 0 && splitk_kw_plan(M, N, K, cfg, split_k, kAnywhere).rows) return 1;
   if (resolve_cfg(cfg, M, N, K, &c, &ks, split_k > 0 ? split_k : 0)) return K % 8 != 0 ? 1 : -1;
   return effective_split(M, N, K, c, split_k);
 }
@@ -911,6 +920,11 @@ int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int 
   }
   if (generic) {  // one pass of the plain kernel, no slices (beam_splitk_effective says 1)
     BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, false, false, st));
+    return BEAM_OK;
+  }
+  if (const KwPlan kw = splitk_kw_plan(M, N, K, cfg, split_k, row_starts(A, B, K, false)); kw.rows) {
+    if (g_verbose.load(std::memory_order_relaxed)) log_split_choice_once(M, N, K, dtype, beam_tile_cfg{kw.rows, kw.cols, kw.rows, kw.cols, 0, 0}, 1);
+    BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, st));
     return BEAM_OK;
   }
   beam_tile_cfg c;

@@ -44,6 +44,17 @@ def test_matmul_nn(gpu, beamc, oracle, M, N, K):
         close_enough(oracle, out, oracle.matmul_nn(a, b, dtype), K, dtype, f"[K][N] {(M, N, K)} at {offsets}")
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 16, 4096), (41, 100, 8184), (300, 24, 4951), (500, 500, 4096)])
+def test_split_k_of_a_short_sum(gpu, beamc, oracle, M, N, K):
+    """Left to the library, a sum below 8192 over few outputs runs without slices, and needs no workspace."""
+    L = beamc.lib
+    assert L.beam_splitk_effective(M, N, K, None, 0) == 1 and L.beam_splitk_effective(M, N, K, None, 4) > 1
+    for dtype, offsets in ((F16, (0, 0, 0)), (BF16, (3, 1, 1))):
+        a, b = beamc.host_uniform((M, K), dtype, 93, 0), beamc.host_uniform((N, K), dtype, 93, 1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, dtype, None, 0, None, 0, None), a, b, (M, N), dtype, offsets)
+        close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"{(M, N, K)} at {offsets}")
+
+
 def test_infinities_and_nan_stay_in_their_row_or_column(gpu, beamc):
     """Line by line a fill brings chunks of two K tiles; a chunk behind the end of K must still be a zero for every row."""
     M, N, K = 70, 90, 3001
