@@ -493,6 +493,10 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, RowStarts rows, int 
   // here), and a tuner that compares the two is to find it there; the line is where the two are about even (256 x 256 x 8192:
   // 8.7, here 7.1; 128 x 128 x 16384: 8.3, here 12.0).
   if (M > 64 && K >= 8192 && !b_kmajor && !ln) return none;
+  // A handful of rows beside more columns than 32 for every CU: B's way from memory is the bound, and the tiled kernels' long
+  // rings are ahead but for K from 512 to 4096 (16 x 11008 x 4096 19.7 us, tiled 21.2; 1 x 14704 x 9064 47.7 tiled, here 50.6;
+  // 10000 x 6000 21.4, 23.0) and up to 3 * 2^24 elements of B (16384 x 4088 20.6, here 27.2; 65536 x 512 11.0, 12.1).
+  if (M <= 16 && N > 32 * cus && !b_kmajor && !ln && (K < 512 || K > 4096 || (long)N * K > (3L << 24))) return none;
   for (const auto& t : kTiles) {
     if (t.rows == 8 && (M > 8 || b_kmajor || ln)) continue;
     const long tiles_n = (N + t.cols - 1) / t.cols, tiles = (long)((M + t.rows - 1) / t.rows) * tiles_n;
@@ -503,13 +507,17 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, RowStarts rows, int 
     if (t.rows <= 16 && t.cols == 16 && K >= 2048 && !ln) plan.waves = 8;
     // Whole lines where the fills saved are more than the one that every wavefront adds: K tiles x (rows + columns) of 1200
     // (1024 x 1024 x 520, 9 x 128: 6.2 us, shifted 6.8; 466 x 864 x 1032, 17 x 96: 6.6, shifted 6.1; 256 x 256 x 2056,
-    // 33 x 32: 4.4, shifted 4.5).  8 rows are bound by latency: 1 x 1024 x 9480 6.4, shifted 7.2.  Rows off 16 bytes have chunks
+    // 33 x 32: 4.4, shifted 4.5).  8 rows are bound by latency: 1 x 1024 x 9480 6.4, shifted 7.2; a row
+    // of tiles of 64 columns by memory: 16 x 11944 x 1064 6.7, 7.0.  Rows off 16 bytes have chunks
     // in two lines however they are fetched: 600 x 600 x 3004 12.6 either way, x 3001 14.3, shifted 15.9.
-    plan.shift = rows == kOnChunks && t.rows > 8 && (long)(K / kBK) * (t.rows + t.cols) >= 1200;
+    plan.shift = rows == kOnChunks && t.rows > 8 && !(M <= 16 && t.cols == 64) && (long)(K / kBK) * (t.rows + t.cols) >= 1200;
     // A full tile per CU with rows on lines: from K = 2048 on the deep pipeline's two K groups, whose sums cost less to bring
     // together (1024 x 1024 x 2048 8.8 us, here 9.4; 128 x 8192 x 4096 15.5, 16.6; 1024^3 8.3, here 6.8); and where one row of
     // tiles streams B from memory (64 x 16384 x 1024 8.9, here 9.6).
     if (t.rows * t.cols == 64 * 64 && rows == kOnLines && !ln && (K >= 2048 || M <= 64)) return none;
+    // ... or one row of 32 x 64 tiles does so from nearly every CU (20 x 14000 x 1500 10.7, here 11.4; 32 x 11008 x 4096 18.8,
+    // 18.1; 30 x 9000 x 3000 13.6, 12.1).
+    if (t.rows == 32 && t.cols == 64 && M <= 32 && !b_kmajor && !ln && 4 * tiles > 3L * cus) return none;
     // LayerNorm on full tiles under a short sum: the sums' way through LDS is the larger part (1024 x 1024 x 520 9.1 us, here
     // 9.9; x 1000 12.7, 12.2; x 1528 15.8, 13.7).
     if (t.rows * t.cols == 64 * 64 && ln && K < 600) return none;
