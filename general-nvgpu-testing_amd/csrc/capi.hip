@@ -660,11 +660,14 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     // whose wavefronts are 64 columns wide pay for it: eight wavefronts of 64 x 32 instead of four of 64 x 64
     // (768 x 3072 x 768: 8.3 against 12.7 us; 2048 x 2048 x 512: 7.9 against 10.0), and 128 x 64 tiles of 64 x 32
     // instead of 64 x 128 tiles of 32 x 64 where that does not make more tiles (256 x 8192 x 8192: 57 against 71).
+    // (Not where two K groups are held up by A's rows, which lie off 128-byte lines and fill LDS at half the rate: 64 of them
+    // instead of 128, 2048 x 1024 x 1032 9.8 against 10.6; x 1024 9.6, 9.1.)
     auto tiles_of = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     beam_tile_cfg alt = c;
     if (c.block_m == 128 && c.block_n == 128 && c.wave_m == 64 && c.wave_n == 64) {
       alt.wave_n = 32;
-    } else if (c.block_m == 64 && c.block_n == 128 && c.wave_m == 32 && c.wave_n == 64 && tiles_of(128, 64) <= tiles_of(64, 128)) {
+    } else if (c.block_m == 64 && c.block_n == 128 && c.wave_m == 32 && c.wave_n == 64 && tiles_of(128, 64) <= tiles_of(64, 128) &&
+               (c.pipeline != 2 || K % kBK == 0)) {
       alt.block_m = 128, alt.block_n = 64, alt.wave_m = 64, alt.wave_n = 32;
     }
     const KernelSet* alt_ks = nullptr;
