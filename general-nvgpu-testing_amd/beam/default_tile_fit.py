@@ -176,7 +176,8 @@ def predict(params, M, N, K):
 
 def as_run(name, M, N, K):
     """The kernel the library runs for the model's pick (csrc/capi.hip, choose_default): a full round of 256 x 256 tiles as
-    four wavefronts of 128 x 128, and under a long sum the deep pipeline for few workgroups or two K groups."""
+    four wavefronts of 128 x 128, under a long sum the deep pipeline for few workgroups or two K groups, and the deep
+    128 x 128 tile as four wavefronts of 64 x 64."""
     bm, bn, _ = CANDIDATES[name]
     tiles = math.ceil(M / bm) * math.ceil(N / bn)
     if (bm, bn) == (256, 256) and tiles >= CUS and K % 64 == 0 and K >= W4_MIN_K and N % 8 == 0:
@@ -184,8 +185,8 @@ def as_run(name, M, N, K):
     few = K >= 2048 and tiles < CUS // 2
     groups = tiles <= CUS and (bm * bn <= 128 * 64 if K >= 2048 else K >= 768 and bm * bn == 128 * 64)
     if not name.endswith("_deep") and (few or groups):
-        return name + "_deep"
-    return name
+        name += "_deep"
+    return "128x128_w64x64_deep" if name == "128x128_w64x32_deep" else name  # (beam_gemmrc: four wavefronts)
 
 
 def regret(params, timings, rows=None):
