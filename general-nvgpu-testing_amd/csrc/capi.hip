@@ -499,7 +499,7 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, RowStarts rows, int 
   if (M <= 16 && N > 32 * cus && !b_kmajor && !ln && (K < 512 || K > 4096 || (long)N * K > (3L << 24))) return none;
   for (const auto& t : kTiles) {
     if (t.rows == 8 && (M > 8 || b_kmajor || ln)) continue;
-    const long tiles_n = (N + t.cols - 1) / t.cols, tiles = (long)((M + t.rows - 1) / t.rows) * tiles_n;
+    const long tiles_n = ((long)N + t.cols - 1) / t.cols, tiles = ((long)M + t.rows - 1) / t.rows * tiles_n;
     if (tiles > cus || (ln && tiles_n > 64)) continue;
     KwPlan plan = {t.rows, t.cols, 4, false};
     // The smallest tiles have little in flight for a wavefront: eight of them from K = 2048 on (256 x 256 x 4088 6.3 -> 5.8 us;
