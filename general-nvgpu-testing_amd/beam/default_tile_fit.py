@@ -183,7 +183,9 @@ def as_run(name, M, N, K):
     if (bm, bn) == (256, 256) and tiles >= CUS and K % 64 == 0 and K >= W4_MIN_K and N % 8 == 0:
         return "256x256_w128x128"
     few = K >= 2048 and tiles < CUS // 2
-    groups = tiles <= CUS and (bm * bn <= 128 * 64 if K >= 2048 else K >= 768 and bm * bn == 128 * 64)
+    area = bm * bn
+    groups = tiles <= CUS and (area <= 128 * 64 if K >= 2048 else K >= 768 if area == 128 * 64 else
+                               area == 64 * 64 and K >= 384 and M > 64 and 2 * tiles > CUS)
     if not name.endswith("_deep") and (few or groups):
         name += "_deep"
     return "128x128_w64x64_deep" if name == "128x128_w64x32_deep" else name  # (beam_gemmrc: four wavefronts)

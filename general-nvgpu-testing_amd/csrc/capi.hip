@@ -445,13 +445,17 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
     cfg->wave_n = 128;
   }
   // One workgroup per CU under a long sum: the deep pipeline.  Less than half the CUs busy: its long prefetch queue keeps
-  // memory busy.  Tiles with two K groups: up to a full round, since a lone group's K tile is a serial chain; 64 x 64 tiles
-  // from K = 2048 on (1024^3 5.2, two groups 5.5; 1024 x 1024 x 2048 8.1, 7.7), 64 x 128 and 128 x 64 from K = 768 on (one
-  // group, two: 2048 x 1024 x 520 6.2, 6.3; x 768 8.3, 7.2; x 1024 10.0, 8.2; x 1536 13.9, 11.0; 620 x 3064 x 776 9.9, 9.3;
-  // x 1600 14.6, 11.1; [K][N] 700 x 2500 x 512 7.9, 7.3; x 1024 12.5, 10.0).
+  // memory busy.  Tiles with two K groups: up to a full round, since a lone group's K tile is a serial chain; 64 x 128 and
+  // 128 x 64 from K = 768 on (one group, two: 2048 x 1024 x 520 6.2, 6.3; x 768 8.3, 7.2; x 1024 10.0, 8.2; x 1536 13.9, 11.0;
+  // 620 x 3064 x 776 9.9, 9.3; x 1600 14.6, 11.1; [K][N] 700 x 2500 x 512 7.9, 7.3; x 1024 12.5, 10.0), 64 x 64 from K = 384 on
+  // (12 sets of operands in turn: 1024 x 1024 x 256 3.7, 3.9; x 384 4.6, 4.5; x 512 5.3, 4.8; x 1024 8.2, 6.1; the same operands
+  // in every call x 512 3.7, 4.3; x 1024 5.0, 5.4; x 2048 8.1, 7.7; a set for each of 96 calls x 512 7.1, 5.7; x 1024 11.7,
+  // 7.7).  Only from K = 2048 on: a single row of those,
+  // whose form as one group is made for long sums, and at most half a round, where smaller tiles run (kw_plan).
   const long picked = tiles(c.block_m, c.block_n);
   const bool few = K >= 2048 && picked < cus / 2;
-  const bool groups = picked <= cus && (K >= 2048 ? c.block_m * c.block_n <= 128 * 64 : K >= 768 && c.block_m * c.block_n == 128 * 64);
+  const int area = c.block_m * c.block_n;
+  const bool groups = picked <= cus && (K >= 2048 ? area <= 128 * 64 : area == 128 * 64 ? K >= 768 : area == 64 * 64 && K >= 384 && M > 64 && 2 * picked > cus);
   if (raised) *raised = false;
   if (split_req < 0 && (few || groups)) {
     if (raised) *raised = !few && c.pipeline == 0;
@@ -482,9 +486,9 @@ GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, 
 // tile: so the tile with the smallest sum of which the problem has at most one for every CU.  (466 x 864 x 520: 32 x 64, 210
 // tiles, 4.6 us; 32 x 32, 405 tiles, 5.0; 300 x 400 x 513: 32 x 16, 250 tiles, 3.7, 16 x 16, 475 tiles, 4.0, 32 x 32 4.3.
 // Beyond one tile of 64 x 64 for every CU the tiled kernels are ahead: 2048 x 1024 x 2040 18.8, here 20.0.)
-//   b_kmajor, ln: the form; rows: where every row of A (and of B as [N][K]) starts.
+//   b_kmajor, ln: the form; gemm: for beam_gemmrc's or beam_matmul_nn's result, not for a split-K call; rows: where every row of A (and of B as [N][K]) starts.
 enum RowStarts { kAnywhere, kOnChunks, kOnLines };  // at an element, on 16 bytes, on 128
-KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, RowStarts rows, int cus) {
+KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts rows, int cus) {
   static const struct { int rows, cols; } kTiles[] = {{8, 16},  {16, 16}, {16, 32}, {32, 16}, {32, 32},
                                                       {8, 64},  {16, 64}, {32, 64}, {64, 32}, {64, 64}};
   const KwPlan none = {0, 0, 0, false};
@@ -512,10 +516,15 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, RowStarts rows, int 
     // in two lines however they are fetched: 600 x 600 x 3004 12.6 either way, x 3001 14.3, shifted 15.9.
     plan.shift = rows == kOnChunks && t.rows > 8 && !(M <= 16 && t.cols == 64) && (long)(K / kBK) * (t.rows + t.cols) >= 1200;
     // A full tile per CU with rows on lines: from K = 2048 on the deep pipeline's two K groups, whose sums cost less to bring
-    // together (1024 x 1024 x 2048 8.8 us, here 9.4; 128 x 8192 x 4096 15.5, 16.6; 1024^3 8.3, here 6.8); and where one row of
-    // tiles streams B from memory (64 x 16384 x 1024 8.9, here 9.6).
+    // together (1024 x 1024 x 2048 8.8 us, here 9.4; 128 x 8192 x 4096 15.5, 16.6); and where one row of tiles streams B from
+    // memory (64 x 16384 x 1024 8.9, here 9.6).
     if (t.rows * t.cols == 64 * 64 && rows == kOnLines && !ln && (K >= 2048 || M <= 64)) return none;
-    // ... or one row of 32 x 64 tiles does so from nearly every CU (20 x 14000 x 1500 10.7, here 11.4; 32 x 11008 x 4096 18.8,
+    // ... and under a short sum, wherever rows start, if C's rows are whole chunks: the sums' way through LDS is the larger part
+    // (1024 columns, 12 sets of operands in turn, here -> tiled: 1024 x 256 4.7 -> 3.7, x 384 5.3 -> 4.5, x 512 5.6 -> 4.8, x 1024
+    // 6.8 -> 6.1, x 1001 9.5 -> 8.5, x 1032 8.4 -> 7.9, x 1288 9.1 -> 9.0, x 1544 9.6, 9.8; rows on lines x 1536 8.2 -> 7.9, x 1792
+    // 8.6 -> 8.2; [K][N] x 256 5.0 -> 4.2, x 512 5.8 -> 5.3, x 1024 7.0 -> 6.9, x 1536 8.3, 8.7; 1000 x 1003 x 1024 6.8, 7.7).
+    if (t.rows * t.cols == 64 * 64 && gemm && N % 8 == 0 && M > 64 && K <= (rows != kOnLines ? 1280 : b_kmajor ? 1024 : 2047)) return none;
+    // ... or one row of 32 x 64 tiles streams B from nearly every CU (20 x 14000 x 1500 10.7, here 11.4; 32 x 11008 x 4096 18.8,
     // 18.1; 30 x 9000 x 3000 13.6, 12.1).
     if (t.rows == 32 && t.cols == 64 && M <= 32 && !b_kmajor && !ln && 4 * tiles > 3L * cus) return none;
     // LayerNorm on full tiles under a short sum: the sums' way through LDS is the larger part (1024 x 1024 x 520 9.1 us, here
@@ -572,7 +581,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   }
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, false, false, row_starts(A, B, K, false), cus); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, false, true, row_starts(A, B, K, false), cus); kw.rows) {
       BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, st));
       return BEAM_OK;
     }
@@ -650,7 +659,7 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     return BEAM_OK;
   }
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, true, false, row_starts(A, B, K, true), g_dev.cus > 0 ? g_dev.cus : 256); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, true, false, true, row_starts(A, B, K, true), g_dev.cus > 0 ? g_dev.cus : 256); kw.rows) {
       BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, true, st));
       return BEAM_OK;
     }
@@ -763,11 +772,13 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   //   * A GEMM kernel that carries no side job and is the faster one by more than the second launch costs (2.5 us): the deep
   //     pipeline with less than half the CUs busy, or with tiles of 64 rows (two K groups).  One launch, two launches: 2048 x
   //     1024 x 2048 with 2^18 elements 18.9, 15.9.  Tiles of 128 rows gain less than that: 128 x 128 (one group) 496 x 5688 x
-  //     1224 13.2, 15.3; 128 x 64 5813 x 312 x 6256 46.4, 47.2.
+  //     1224 13.2, 15.3; 128 x 64 5813 x 312 x 6256 46.4, 47.2.  64 x 64 tiles with K below 2048: two launches
+  //     from K = 1024 or 2^21 elements on (1024^3 with 2^18 9.1, 9.0, with 2^22 16.3, 11.2; 1024 x 1024 x 512 with 2^18 6.1, 7.8,
+  //     with 2^22 9.9, 9.6).
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, false, false, row_starts(A, B, K, false), cus); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, false, true, row_starts(A, B, K, false), cus); kw.rows) {
       if (kw.rows + kw.cols > 32 && count > (1 << 23)) {
-        BEAM_HIP(run_kwave(kw, A, B, C, M, N, K, dtype, false, (hipStream_t)stream));
+        if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
         return beam_silu(X, Y, count, dtype, stream);
       }
       KwSideParams p;
@@ -782,7 +793,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
                                  : launch_gemm_kwave_side<__bf16>(kw, p, side, (hipStream_t)stream));
       return BEAM_OK;
     }
-    const bool two_groups = c.block_m == 64 && K >= 2048;
+    const bool two_groups = c.block_m == 64 && (K >= 2048 || (c.block_n == 64 && (K >= 1024 || count > (1 << 21))));
     if (c.pipeline == 2 && ((wgs * 2 < cus && K >= 2048) || two_groups)) {
       if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
       return beam_silu(X, Y, count, dtype, stream);
@@ -886,7 +897,7 @@ static int effective_split(int M, int N, int K, const beam_tile_cfg& c, int spli
 // to the wavefronts of small tiles (gemm_kwave.h) where a CU then fills LDS with no more than 600 KB.
 static KwPlan splitk_kw_plan(int M, int N, int K, const beam_tile_cfg* cfg, int split_k, RowStarts rows) {
   if (cfg || split_k > 0 || K >= 8192) return KwPlan{0, 0, 0, false};
-  const KwPlan kw = kw_plan(M, N, K, false, false, rows, g_dev.cus > 0 ? g_dev.cus : 256);
+  const KwPlan kw = kw_plan(M, N, K, false, false, false, rows, g_dev.cus > 0 ? g_dev.cus : 256);
   return (long)(kw.rows + kw.cols) * K <= 300000 ? kw : KwPlan{0, 0, 0, false};
 }
 
@@ -1177,7 +1188,7 @@ struct LnPlan {
 // bands is made for 8 XCDs of 32 CUs).
 static KwPlan ln_kw_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode) {
   if (cfg || mode == BEAM_LN_TWOPASS || g_dev.cus != kNumXcd * 32) return KwPlan{0, 0, 0, false};
-  return kw_plan(M, N, K, false, true, kOnLines, g_dev.cus);
+  return kw_plan(M, N, K, false, true, false, kOnLines, g_dev.cus);
 }
 static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool plain, bool unaligned, bool capturing, bool wide_io,
                    LnPlan* out) {
@@ -1333,7 +1344,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   if ((uintptr_t)ws & 255) return fail(BEAM_ERR_UNSUPPORTED, "workspace must be 256-byte aligned");
   if (plan.kw.rows) {
     KwPlan kw = plan.kw;
-    kw.shift = kw_plan(M, N, K, false, true, row_starts(A, B, K, false), g_dev.cus).shift;
+    kw.shift = kw_plan(M, N, K, false, true, false, row_starts(A, B, K, false), g_dev.cus).shift;
     KwLnParams p;
     kw_params(&p, kw, A, B, Y, M, N, K);
     p.divs = band_order_divs(p.tiles_n, 1, -1);

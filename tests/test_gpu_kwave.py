@@ -44,6 +44,19 @@ def test_matmul_nn(gpu, beamc, oracle, M, N, K):
         close_enough(oracle, out, oracle.matmul_nn(a, b, dtype), K, dtype, f"[K][N] {(M, N, K)} at {offsets}")
 
 
+# Full tiles of 64 x 64 whose rows of C are whole chunks: the tiled kernels' under a short sum, on both sides of every line
+@pytest.mark.parametrize("K", [8, 256, 383, 384, 385, 1024, 1025, 1032, 1280, 1281, 1344, 1984, 2047])
+@pytest.mark.parametrize("M,N", [(1000, 1000), (130, 5000)])
+def test_full_tiles_under_a_short_sum(gpu, beamc, oracle, M, N, K):
+    L = beamc.lib
+    for dtype, offsets in ((F16, (0, 0, 0)), (BF16, (3, 1, 1))):
+        a, b, bt = (beamc.host_uniform(s, dtype, 92, i) for i, s in enumerate(((M, K), (N, K), (K, N))))
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offsets)
+        close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"{(M, N, K)} at {offsets}")
+        out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, dtype, None, None), a, bt, (M, N), dtype, offsets)
+        close_enough(oracle, out, oracle.matmul_nn(a, bt, dtype), K, dtype, f"[K][N] {(M, N, K)} at {offsets}")
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 16, 4096), (41, 100, 8184), (300, 24, 4951), (500, 500, 4096)])
 def test_split_k_of_a_short_sum(gpu, beamc, oracle, M, N, K):
     """Left to the library, a sum below 8192 over few outputs runs without slices, and needs no workspace."""
