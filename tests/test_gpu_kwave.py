@@ -92,6 +92,25 @@ def test_infinities_of_b_behind_the_whole_chunks(gpu, beamc, N):
     assert np.isfinite(np.delete(out, (5, 7), axis=1)).all()
 
 
+@pytest.mark.parametrize("N", [9, 88, 90, 1003])
+@pytest.mark.parametrize("K", [9, 64, 75, 128, 200, 1032, 2000])
+def test_infinities_in_the_last_rows_of_b(gpu, beamc, N, K):
+    """[K][N]: a row of B behind the whole chunks meets only its own elements of A, never the zeros beside them.  With
+    N % 8 != 0 the last row of B is always one of those (8 * ((K - 1) / 8) is the first), else those of K % 8."""
+    M, L = 37, beamc.lib
+    first = 8 * ((K - 1) // 8)
+    rows = sorted({first, min(first + 1, K - 1), K - 1})
+    a = beamc.host_uniform((M, K), F16, 97, 0)
+    a[:, first:] = 0x3C00  # one
+    for row in rows:
+        for cols in ([0, 5], [1, 7], [2, 3, 4, 6], [N - 1]):
+            b = beamc.host_uniform((K, N), F16, 97, 1)
+            b[row, cols] = 0x7C00
+            out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
+            assert (out[:, cols] == np.inf).all(), (row, cols)
+            assert np.isfinite(np.delete(out, cols, axis=1)).all(), (row, cols)
+
+
 # The elementwise job rides in workgroups of its own behind the tiles'.  Counts: a tail only, one access of one thread, ragged,
 # more than one round of the accesses of every such workgroup.
 @pytest.mark.parametrize("tile", ["8x16", "16x16", "32x32", "64x64"])
