@@ -535,8 +535,10 @@ __global__ void __launch_bounds__(NW * 64, 2) gemm_kwave_kernel(const KwParams p
 }
 
 // A second launch costs 2.6 us and waits for the first one's last tile; here the array is streamed by the CUs that have no
-// tile, or no tile any more.  Such a workgroup holds a tile's LDS and registers, so a CU has only 4 to 8 wavefronts of them:
-// every thread keeps 8 accesses in flight.
+// tile, or no tile any more.  Such a workgroup holds a tile's LDS, so a CU has only 4 to 20 wavefronts of them: rounds of 8
+// accesses for every thread.  (In the tiles of up to 48 rows + columns and 32 x 32, not shifted, the compiler has two of a
+// round in flight at a time and uses fewer registers; eight, held together by a scheduling barrier, are ahead at 32 x 32 with
+// 2^24 elements, 19.2 -> 17.4 us, and behind in a long job, 256 x 256 x 128 with 2^26 51.9 -> 62.2.)
 template <typename T, int AG, int CB, int NW, int S, KwRows MODE>
 __global__ void __launch_bounds__(NW * 64, 2) gemm_kwave_side_kernel(const KwSideParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
