@@ -535,6 +535,10 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
   return none;
 }
 
+// LDS of one of its workgroups: two slots of a K tile for each wavefront, rows in blocks of 16.
+constexpr int kLdsBytes = 160 * 1024;  // of a CU
+int kw_lds_bytes(const KwPlan& plan) { return plan.waves * 2 * ((plan.rows < 16 ? 16 : plan.rows) + plan.cols) * kRowBytes; }
+
 RowStarts row_starts(const void* A, const void* B, int K, bool b_kmajor) {
   const uintptr_t at = (uintptr_t)A | (b_kmajor ? 0 : (uintptr_t)B);
   return K % kBK == 0 && (at & 127) == 0 ? kOnLines : K % 8 == 0 && (at & 15) == 0 ? kOnChunks : kAnywhere;
@@ -766,9 +770,18 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   const long long per_pass = wgs * ks->threads;  // units one K tile of the whole grid covers
   // With the library's tile:
   //   * Where the GEMM runs on gemm_kwave.h, the job rides in workgroups of its own behind the tiles (one launch; two launches,
-  //     us: 256 x 256 x 512 with 2^18 elements 6.5, 10.1; 1000 x 600 x 1000 with 2^22 9.1, 12.2; 299 x 824 x 3968 with 2^24
-  //     17.6, 21.1).  Such a workgroup holds a tile's LDS, so beyond 2^23 elements, but for the 32 KiB of the smallest tiles,
-  //     too few of them are on a CU to keep memory busy: 1024^3 with 2^24 21.7, two launches 18.9.
+  //     us: 256 x 256 x 512 with 2^18 elements 3.7, 4.6; 1000 x 1003 x 1024 with 2^22 9.5, 10.3).  Such a workgroup holds a
+  //     tile's LDS, and a long job is bound by how many wavefronts of it a CU then has (operands from memory).  12 and more,
+  //     tiles of up to 48 rows + columns: any length (297 x 400 x 1024 with 2^24 17.7, 20.1, with 2^26 52.6, 58.4).  8: up to
+  //     2^24 elements with 64 columns or whole-line fills (3 x 8304 x 1024 20.5, 22.1; 1720 deep, 14.3 Mi, 17.0, 21.6), else up to
+  //     2^23, since two accesses of a thread are in flight there and not eight (304 deep, 8.1 Mi, 9.4, 11.0; 408 deep, 13.5 Mi,
+  //     19.4, 17.5).  4: up to 2^23 (512 x 1024 x 2048 17.1, 17.4; with 2^24 26.7, 25.0).
+  //   * ... but not where such a workgroup is a CU's only one, not every one finds a CU without a tile, and sum and job are
+  //     short: it then starts behind a tile, 1-2 us that the tiled kernel's K loop hides.  (Behind the tiles, in the loop;
+  //     operands from memory, then the same in every call: 512 x 1024, 256 tiles, x 256 with 2^18 5.5, 4.5; 5.3, 3.9; with 2^20,
+  //     4 passes of that kernel's grid, 6.2, 5.9; 5.7, 4.4; x 512 with 2^18 6.4, 6.2; 5.7, 4.7, with 2^20 6.7, 9.1; x 1024 with
+  //     2^18 7.3, 9.1; 1000 x 1003 x 512 with 2^12 6.4, 7.1.  982 x 504 x 112, 248 tiles and 35 workgroups, 5.8, 4.7; 1241 x
+  //     336 x 224, 234 tiles and 14 workgroups, 4.3, 4.4.)
   //   * A GEMM kernel that carries no side job and is the faster one by more than the second launch costs (2.5 us): the deep
   //     pipeline with less than half the CUs busy, or with tiles of 64 rows (two K groups).  One launch, two launches: 2048 x
   //     1024 x 2048 with 2^18 elements 18.9, 15.9.  Tiles of 128 rows gain less than that: 128 x 128 (one group) 496 x 5688 x
@@ -777,21 +790,27 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   //     with 2^22 9.9, 9.6).
   if (!cfg) {
     if (const KwPlan kw = kw_plan(M, N, K, false, false, true, row_starts(A, B, K, false), cus); kw.rows) {
-      if (kw.rows + kw.cols > 32 && count > (1 << 23)) {
-        if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
-        return beam_silu(X, Y, count, dtype, stream);
-      }
-      KwSideParams p;
-      kw_params(&p, kw, A, B, C, M, N, K);
-      p.side_x = X;
-      p.side_y = Y;
-      p.side_count = count;
-      const long long per_wg = (long long)kw.waves * 64 * 8 * 8;  // elements of one round of a workgroup's accesses
+      const long long per_wg = (long long)kw.waves * 64 * 8 * 8;  // elements of one round of a side workgroup's accesses
       const long long want = (count + per_wg - 1) / per_wg;
-      const int side = (int)(want < 8 * cus ? want : 8 * cus);
-      BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_kwave_side<_Float16>(kw, p, side, (hipStream_t)stream)
-                                 : launch_gemm_kwave_side<__bf16>(kw, p, side, (hipStream_t)stream));
-      return BEAM_OK;
+      const int per_cu = kLdsBytes / kw_lds_bytes(kw);  // workgroups of the launch on a CU
+      const long long passes = ((count >> 3) + per_pass - 1) / per_pass;  // of the tiled kernel's grid over the job
+      const bool loop = per_cu == 1 && (long long)((M + kw.rows - 1) / kw.rows) * ((N + kw.cols - 1) / kw.cols) + want > cus && passes <= 4 &&
+                        passes * K <= 1024 && (K <= 256 || (K <= 512 && count >= (1 << 16)));
+      if (!loop) {
+        if (count > (per_cu * kw.waves >= 12 ? kMaxSideElems : per_cu * kw.waves >= 8 && (kw.shift || kw.cols == 64) ? 1 << 24 : 1 << 23)) {
+          if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
+          return beam_silu(X, Y, count, dtype, stream);
+        }
+        KwSideParams p;
+        kw_params(&p, kw, A, B, C, M, N, K);
+        p.side_x = X;
+        p.side_y = Y;
+        p.side_count = count;
+        const int side = (int)(want < 8 * cus ? want : 8 * cus);
+        BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_kwave_side<_Float16>(kw, p, side, (hipStream_t)stream)
+                                   : launch_gemm_kwave_side<__bf16>(kw, p, side, (hipStream_t)stream));
+        return BEAM_OK;
+      }
     }
     const bool two_groups = c.block_m == 64 && (K >= 2048 || (c.block_n == 64 && (K >= 1024 || count > (1 << 21))));
     if (c.pipeline == 2 && ((wgs * 2 < cus && K >= 2048) || two_groups)) {

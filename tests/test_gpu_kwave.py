@@ -117,7 +117,9 @@ def test_infinities_in_the_last_rows_of_b(gpu, beamc, N, K):
 def test_silu_job(gpu, beamc, tile):
     L = beamc.lib
     M, N = TILES[tile]
-    for K, dtype in ((200, F16), (2600, BF16)):
+    # (K above 512 for the large tile: under a shorter sum the job runs in the tiled kernel's K loop, test_silu_job_in_the_loop,
+    # whose sums are added in another order than beam_gemmrc's)
+    for K, dtype in ((520 if tile == "64x64" else 200, F16), (2600, BF16)):
         da, db = (beamc.DeviceArray.from_numpy(beamc.host_uniform(s, dtype, 97, i), dtype) for i, s in enumerate(((M, K), (N, K))))
         want, got = beamc.DeviceArray((M, N), dtype), beamc.DeviceArray((M, N), dtype)
         beamc._check(L.beam_gemmrc(da.ptr, db.ptr, want.ptr, M, N, K, dtype, None, None))
@@ -134,6 +136,42 @@ def test_silu_job(gpu, beamc, tile):
                 d.free()
         for d in (da, db, want, got):
             d.free()
+
+
+# ... or, in the largest tiles under a short sum, in the tiled kernel's K loop; a long job beside large tiles gets a launch of its
+# own.  Counts on both sides of each line (512 x 1024: a pass of the grid is 2^18 elements, 1000 x 1003: 2^19).
+@pytest.mark.parametrize("M,N", [(512, 1024), (1000, 1003), (1030, 472)])
+@pytest.mark.parametrize("K", [8, 71, 256, 264, 512, 520])
+def test_silu_job_in_the_loop(gpu, beamc, oracle, M, N, K):
+    for dtype in (F16, BF16):
+        a, b = beamc.host_uniform((M, K), dtype, 90, 0), beamc.host_uniform((N, K), dtype, 90, 1)
+        ref = oracle.gemmrc(a, b, dtype)
+        for count in (0, 5, (1 << 16) - 8, 1 << 16, 1 << 19, (1 << 19) + 8, (1 << 20) + 3, (1 << 20) + 8, (1 << 21) + 8):
+            silu_pair(beamc, oracle, a, b, ref, dtype, count)
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 256, 200), (297, 400, 71), (509, 500, 200), (1000, 1003, 1096)])
+def test_silu_long_job(gpu, beamc, oracle, M, N, K):
+    a, b = beamc.host_uniform((M, K), F16, 91, 0), beamc.host_uniform((N, K), F16, 91, 1)
+    ref = oracle.gemmrc(a, b, F16)
+    for count in (1 << 23, (1 << 23) + 8, 1 << 24, (1 << 24) + 5):
+        silu_pair(beamc, oracle, a, b, ref, F16, count)
+
+
+def silu_pair(beamc, oracle, a, b, ref, dtype, count):
+    L = beamc.lib
+    (M, K), N = a.shape, b.shape[0]
+    da, db = beamc.DeviceArray.from_numpy(a, dtype), beamc.DeviceArray.from_numpy(b, dtype)
+    dx = beamc.DeviceArray.from_numpy(beamc.host_normal((count + 64,), dtype, 97, 2, 0.0, 2.5), dtype)
+    c, y, alone = (beamc.DeviceArray(s, dtype) for s in ((M, N), (count + 64,), (count + 64,)))
+    for d in (c, y, alone):
+        d.fill_bytes(0xEE)
+    beamc._check(L.beam_silu(dx.ptr, alone.ptr, count, dtype, None))
+    beamc._check(L.beam_parallel_gemmrc_silu(da.ptr, db.ptr, c.ptr, M, N, K, dx.ptr, y.ptr, count, dtype, None, None))
+    close_enough(oracle, c.to_numpy(), ref, K, dtype, f"{(M, N, K)} beside {count} elements")
+    assert (y.to_numpy() == alone.to_numpy()).all(), (M, N, K, count)  # the guard behind the array included
+    for d in (da, db, dx, c, y, alone):
+        d.free()
 
 
 LN_TILES = {"16x16": (41, 100), "16x32": (297, 400), "32x16": (1030, 100), "32x32": (509, 500), "16x64": (130, 1750), "32x64": (466, 864),
