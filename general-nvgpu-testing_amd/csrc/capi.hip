@@ -913,7 +913,9 @@ static int effective_split(int M, int N, int K, const beam_tile_cfg& c, int spli
 }
 
 // The library's own choice (no tile, no slice count) for a sum that one launch without slices is the faster for: K dealt out
-// to the wavefronts of small tiles (gemm_kwave.h) where a CU then fills LDS with no more than 600 KB.
+// to the wavefronts of small tiles (gemm_kwave.h) where a CU then fills LDS with no more than 600 KB.  Where there is a plan
+// for rows on lines there is one for rows anywhere, not the other way round; beam_splitk_effective, which does not know where
+// the rows start, goes by the latter, and the call does as it says.
 static KwPlan splitk_kw_plan(int M, int N, int K, const beam_tile_cfg* cfg, int split_k, RowStarts rows) {
   if (cfg || split_k > 0 || K >= 8192) return KwPlan{0, 0, 0, false};
   const KwPlan kw = kw_plan(M, N, K, false, false, false, rows, g_dev.cus > 0 ? g_dev.cus : 256);
@@ -982,7 +984,7 @@ int beam_gemmrc_splitk(const void* A, const void* B, void* C, int M, int N, int 
     BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, false, false, st));
     return BEAM_OK;
   }
-  int s = effective_split(M, N, K, c, split_k);
+  int s = splitk_kw_plan(M, N, K, cfg, split_k, kAnywhere).rows ? 1 : effective_split(M, N, K, c, split_k);
   // Operands whose rows are not 16-byte aligned may be given without room for slices, or with it off 16 bytes (they need
   // none: one pass).
   if (rows_unaligned(A, B, C, K) && (!ws || ((uintptr_t)ws & 15) != 0 || ws_bytes < splitk_partial_bytes(M, N, s))) s = 1;
@@ -1312,6 +1314,23 @@ size_t beam_dbg_ln_plan_bytes(int M, int N, int K, const beam_tile_cfg* cfg, int
   if (M <= 0 || N <= 0 || K < 0 || ln_plan(M, N, K, cfg, mode, plain != 0 || (K > 0 && K < 8) || K > kMaxK, false, capturing != 0,
                                                      wide_io != 0, &plan)) return 0;
   return plan.need;
+}
+
+int beam_dbg_small_tile(int op, int M, int N, int K, int row_starts, int* rows, int* cols, int* waves, int* whole_lines) {
+  if (op < 0 || op > 3 || row_starts < kAnywhere || row_starts > kOnLines || M <= 0 || N <= 0 || K < 0 || !rows || !cols || !waves || !whole_lines)
+    return fail(BEAM_ERR_INVALID, "bad argument");
+  const RowStarts at = (RowStarts)row_starts;
+  const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
+  KwPlan kw = {0, 0, 0, false};
+  if (op == 0) kw = kw_plan(M, N, K, false, false, true, at, cus);
+  if (op == 1 && N >= 8) kw = kw_plan(M, N, K, true, false, true, at, cus);
+  if (op == 2) kw = splitk_kw_plan(M, N, K, nullptr, 0, at);
+  if (op == 3 && cus == kNumXcd * 32) kw = kw_plan(M, N, K, false, true, false, at, cus);
+  *rows = kw.rows;
+  *cols = kw.cols;
+  *waves = kw.waves;
+  *whole_lines = kw.shift ? 1 : 0;
+  return BEAM_OK;
 }
 
 int beam_dbg_set_splitk_self_reduce(int on) {

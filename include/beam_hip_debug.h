@@ -64,6 +64,11 @@ int beam_dbg_kmajor_lds_offset(int k, int n, int block_n);
  * and beta 16-byte aligned).  The entry point computes its requirement with the same function; the workspace queries
  * are tested against it.  0 on error. */
 size_t beam_dbg_ln_plan_bytes(int M, int N, int K, const beam_tile_cfg* cfg, int mode, int plain, int capturing, int wide_io);
+/* The small tile, its wavefronts, and whether LDS is filled by whole lines (1) or not (0), that a call without a named tile runs
+ * on; *rows = 0: none, the tiled kernels.  op: 0 beam_gemmrc, 1 beam_matmul_nn, 2 beam_gemmrc_splitk without a slice count,
+ * 3 beam_gemmrc_ln's one-kernel form.  row_starts, of every row of A (and of B as [N][K]): 0 at an element, 1 on 16 bytes
+ * (K % 8 == 0), 2 on 128 (K % 64 == 0).  Before a device has been probed, of one with 256 CUs. */
+int beam_dbg_small_tile(int op, int M, int N, int K, int row_starts, int* rows, int* cols, int* waves, int* whole_lines);
 /* A measurement, off by default: on != 0 makes the one-launch split-K run without reducing workgroups wherever its
  * multiplying workgroups fit one round of the CUs; the workgroup of (tile, slice s) then adds parts s, s + slices, ...
  * of its tile itself.  Same bits.  Unlike the shipped form this needs every workgroup of the launch resident at once

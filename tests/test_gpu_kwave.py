@@ -10,6 +10,7 @@ from test_gpu_edges import close_enough
 from test_gpu_gemm import F16, BF16
 from test_gpu_ln import check_ln, make_ln_inputs, run_ln
 from test_gpu_unaligned import run
+from test_host_logic import small_tile
 
 pytestmark = pytest.mark.gpu
 
@@ -66,6 +67,18 @@ def test_split_k_of_a_short_sum(gpu, beamc, oracle, M, N, K):
         a, b = beamc.host_uniform((M, K), dtype, 93, 0), beamc.host_uniform((N, K), dtype, 93, 1)
         out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, dtype, None, 0, None, 0, None), a, b, (M, N), dtype, offsets)
         close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"{(M, N, K)} at {offsets}")
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 1024, 2048), (64, 16384, 1024)])
+def test_split_k_needs_no_workspace_wherever_rows_start(gpu, beamc, oracle, M, N, K):
+    """Rows on lines run on the tiled kernels there, rows off them in small tiles; the caller is told one slice for both."""
+    L = beamc.lib
+    assert L.beam_splitk_effective(M, N, K, None, 0) == 1
+    assert small_tile(beamc, 2, M, N, K, 2)[0] == 0 and small_tile(beamc, 2, M, N, K, 1)[:2] == (64, 64)
+    a, b = beamc.host_uniform((M, K), F16, 93, 0), beamc.host_uniform((N, K), F16, 93, 1)
+    for offsets in ((0, 0, 0), (8, 24, 0)):
+        out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc_splitk(pa, pb, pc, M, N, K, F16, None, 0, None, 0, None), a, b, (M, N), F16, offsets)
+        close_enough(oracle, out, oracle.gemmrc(a, b, F16), K, F16, f"{(M, N, K)} at {offsets}")
 
 
 def test_infinities_and_nan_stay_in_their_row_or_column(gpu, beamc):

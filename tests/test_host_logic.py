@@ -496,6 +496,30 @@ def test_splitk_workspace_query_covers_every_small_tile(beamc):
                     assert have >= 4 * (64 + tiles * parts * S), (M, N, S, bm, bn)
 
 
+def small_tile(beamc, op, M, N, K, row_starts):
+    out = [ctypes.c_int() for _ in range(4)]
+    beamc._check(beamc.lib.beam_dbg_small_tile(op, M, N, K, row_starts, *map(ctypes.byref, out)))
+    return tuple(v.value for v in out)
+
+
+def test_splitk_in_small_tiles_needs_no_workspace_wherever_rows_start(beamc):
+    """beam_splitk_effective does not see the operands: what it calls one slice has to be one for rows on lines too."""
+    rng = np.random.default_rng(31)
+    several = on_lines_elsewhere = 0
+    shapes = [(1024, 1024, k) for k in range(2048, 2304 + 1, 64)] + [(64, 16384, 1024), (1000, 1024, 2048), (40, 16000, 1088)]
+    for _ in range(4000):
+        shapes.append(tuple(int(2 ** rng.uniform(lo, hi)) for lo, hi in ((0, 11), (3, 14), (3, 14))))
+    for M, N, K in shapes:
+        plans = [small_tile(beamc, 2, M, N, K, at) for at in range(1 + (K % 8 == 0) + (K % 64 == 0))]
+        if plans[0][0]:
+            assert beamc.lib.beam_splitk_effective(M, N, K, None, 0) == 1, (M, N, K)
+            on_lines_elsewhere += plans[-1][0] == 0
+        else:
+            assert not any(p[0] for p in plans), (M, N, K)
+            several += beamc.lib.beam_splitk_effective(M, N, K, None, 0) > 1
+    assert several and on_lines_elsewhere
+
+
 def test_band_orders_by_multiplication_match_their_definitions(beamc):
     """The fused GEMM+LayerNorm kernels turn a workgroup id into a tile with divisions done as multiplications; over
     every id of many grids that is the band-block order, the whole-bands-per-XCD order and the plain band-after-band
