@@ -27,15 +27,26 @@ hipError_t launch_ln(const KwLnParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Whole-line fills are for tiles above 8 rows whose K tiles x (rows + columns) are 1200 and more (kw_plan): with 16 x 16 that is
+// from K = 2400 on, where a workgroup has eight wavefronts.
+template <int AG, int CB, int NW>
+constexpr bool kShifts = AG > 1 && !(AG == 2 && CB == 1 && NW == 4);
+
 template <int AG, int CB, int NW>
 hipError_t launch_tile(const KwPlan& plan, const KwParams& p, bool b_kmajor, hipStream_t stream) {
-  if constexpr (AG >= 2) {
-    if (b_kmajor)
-      return plan.shift ? launch_plain<AG, CB, NW, 2, kKwShift, true>(p, stream) : launch_plain<AG, CB, NW, 2, kKwStraight, true>(p, stream);
-  } else if (b_kmajor) {
-    return hipErrorInvalidValue;
+  if (plan.shift) {
+    if constexpr (kShifts<AG, CB, NW>)
+      return b_kmajor ? launch_plain<AG, CB, NW, 2, kKwShift, true>(p, stream) : launch_plain<AG, CB, NW, 2, kKwShift, false>(p, stream);
+    else
+      return hipErrorInvalidValue;
   }
-  return plan.shift ? launch_plain<AG, CB, NW, 2, kKwShift, false>(p, stream) : launch_plain<AG, CB, NW, 2, kKwStraight, false>(p, stream);
+  if (b_kmajor) {
+    if constexpr (AG > 1)
+      return launch_plain<AG, CB, NW, 2, kKwStraight, true>(p, stream);
+    else
+      return hipErrorInvalidValue;
+  }
+  return launch_plain<AG, CB, NW, 2, kKwStraight, false>(p, stream);
 }
 
 template <int AG, int CB, int NW, KwRows MODE>
@@ -50,7 +61,13 @@ hipError_t launch_side(const KwSideParams& p, int side_workgroups, hipStream_t s
 
 template <int AG, int CB, int NW>
 hipError_t launch_tile_side(const KwPlan& plan, const KwSideParams& p, int side_workgroups, hipStream_t stream) {
-  return plan.shift ? launch_side<AG, CB, NW, kKwShift>(p, side_workgroups, stream) : launch_side<AG, CB, NW, kKwStraight>(p, side_workgroups, stream);
+  if (plan.shift) {
+    if constexpr (kShifts<AG, CB, NW>)
+      return launch_side<AG, CB, NW, kKwShift>(p, side_workgroups, stream);
+    else
+      return hipErrorInvalidValue;
+  }
+  return launch_side<AG, CB, NW, kKwStraight>(p, side_workgroups, stream);
 }
 
 template <int AG, int CB>

@@ -167,7 +167,7 @@ hipError_t launch_gemm_w4_ln(const GemmParams& p, int dtype, dim3 grid, hipStrea
 struct KwPlan {
   int rows, cols;  // workgroup tile; rows == 0: not this kernel
   int waves;       // wavefronts of a workgroup (8 only for the tiles of 16 columns and at most 16 rows)
-  bool shift;      // fills take whole lines of memory (KwRows)
+  bool shift;      // fills take whole lines of memory (KwRows); not compiled for tiles of 8 rows and, LayerNorm apart, 16 x 16 by four
 };
 // Needs 8 <= K, and M <= rows for tiles of 8 rows; B stored [K][N]: N >= 8 and tiles of 16 rows and more.
 template <typename T>

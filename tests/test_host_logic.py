@@ -502,6 +502,27 @@ def small_tile(beamc, op, M, N, K, row_starts):
     return tuple(v.value for v in out)
 
 
+def test_small_tiles_that_are_planned_are_compiled(beamc):
+    """Whole-line fills are compiled for tiles above 8 rows and, LayerNorm apart, not for 16 x 16 with four wavefronts; eight
+    wavefronts only for 16 columns and at most 16 rows; [K][N] and LayerNorm not for 8 rows."""
+    rng = np.random.default_rng(32)
+    seen = set()
+    for _ in range(20000):
+        M, N, K = (int(2 ** rng.uniform(lo, hi)) for lo, hi in ((0, 11), (3, 14), (3, 14)))
+        K = K // 8 * 8 + 8 if rng.random() < 0.7 else K
+        for op in range(4):
+            for at in range(1 + (K % 8 == 0) + (K % 64 == 0)):
+                rows, cols, waves, lines = small_tile(beamc, op, M, N, K, at)
+                if rows == 0:
+                    continue
+                seen.add((op, rows, cols, waves, lines))
+                assert not lines or (rows > 8 and at == 1 and (op == 3 or (rows, cols, waves) != (16, 16, 4))), (op, M, N, K, at)
+                assert waves == 4 or (waves == 8 and cols == 16 and rows <= 16 and op != 3), (op, M, N, K, at)
+                assert rows > 8 or op in (0, 2), (op, M, N, K, at)
+    # beam_gemmrc: 10 tiles, eight of them by whole lines, two also with eight wavefronts (16 x 16 by whole lines only so)
+    assert len({s for s in seen if s[0] == 0}) == 20 and len({s for s in seen if s[0] == 3}) == 16, sorted(seen)
+
+
 def test_splitk_in_small_tiles_needs_no_workspace_wherever_rows_start(beamc):
     """beam_splitk_effective does not see the operands: what it calls one slice has to be one for rows on lines too."""
     rng = np.random.default_rng(31)
