@@ -15,6 +15,7 @@ import ctypes
 import math
 import os
 import sys
+import warnings
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
 
@@ -150,10 +151,16 @@ lib = _load()
 # What the operators need of torch, looked up once.  torch.cuda.current_stream() builds a Stream object after a walk
 # through the device index' conversions (2.8 us on the machine measured); the raw handle of the current device's current
 # stream is what a launch takes, and costs 0.1 us.  _native (csrc/torch_binding.cc) is the ordinary call without all that:
-# plain torch tensors and no named tile.  It answers with a status, or a negative number for what it leaves to the code below.
+# plain torch tensors and no named tile.  It answers with a status, or a negative number for what it leaves to the code below,
+# which does everything without it, at 2-5 us more a call.
 if _TORCH_FIRST:
-    from . import _torch_binding as _native
     import torch as _torch
+    try:
+        from . import _torch_binding as _native
+    except ImportError as e:  # not built, or for another torch or Python
+        _native = None
+        warnings.warn(f"beam: the compiled torch binding cannot be loaded ({e}); calls go through ctypes, 2-5 us slower each.  "
+                      f"`make -C {os.path.join(_PKG_DIR, 'csrc')}` builds it.", RuntimeWarning)
     _Tensor = _torch.Tensor
     _TORCH_DTYPES = {_torch.float16: F16, _torch.bfloat16: BF16}
     _raw_stream = getattr(_torch._C, "_cuda_getCurrentRawStream", None)
