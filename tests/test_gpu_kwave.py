@@ -1,6 +1,7 @@
 """Small workgroup tiles whose K range is dealt out to the wavefronts, as calls without a named tile reach them: every tile,
-fewer K tiles than wavefronts, K tiles that end inside a chunk, rows on and off 128-byte lines (both ways of filling LDS),
-operands at any element's address inside buffers of NaNs.  Bounds: close_enough's, the one of every other GEMM test."""
+fewer K tiles than wavefronts (8x64, which is for K from 512 on, apart), K tiles that end inside a chunk, rows on and off 128-byte
+lines (both ways of filling LDS), operands at any element's address inside buffers of NaNs.  That the calls reach those tiles is
+a test of its own.  Bounds: close_enough's, the one of every other GEMM test."""
 import ctypes
 
 import numpy as np
@@ -22,6 +23,29 @@ TILES = {"8x16": (5, 300), "16x16": (41, 100), "16x32": (297, 400), "32x16": (10
 KS = [8, 9, 64, 71, 200, 513, 1096, 2057, 3208, 3265]
 
 
+def starts(K):
+    """Where the rows of an operand that itself starts on a line start (beam_dbg_small_tile)."""
+    return 0 if K % 8 else 2 if K % 64 == 0 else 1
+
+
+def test_calls_reach_the_tiles_that_they_are_named_after(gpu, beamc):
+    for name, (M, N) in TILES.items():
+        shape = tuple(map(int, name.split("x")))
+        plans = {K: small_tile(beamc, 0, M, N, K, starts(K)) for K in KS}
+        assert all(p[:2] == shape for K, p in plans.items() if name != "8x64" or K >= 512), (name, plans)
+        assert {p[3] for p in plans.values()} == ({0, 1} if shape[0] > 8 else {0}), (name, plans)  # both ways of filling LDS
+    reached = {small_tile(beamc, 1, M, N, K, starts(K)) for M, N in NN for K in KS}
+    tiles = {t for t in (tuple(map(int, n.split("x"))) for n in TILES) if t[0] > 8}
+    for lines in (0, 1):
+        assert {p[:2] for p in reached if p[0] and p[3] == lines} == tiles, reached
+    for name, (M, N) in LN_TILES.items():
+        plans = {K: small_tile(beamc, 3, M, N, K, starts(K)) for K in (8, 71, 513, 1096, 3208, 3265)}
+        shape = (16, 64) if name == "64 column tiles" else tuple(map(int, name.split("x")))
+        # (64 x 64 under a short sum is the tiled kernel's)
+        assert all(p[:2] == shape for K, p in plans.items() if name != "64x64" or K >= 600), (name, plans)
+        assert plans[3208][3] == 1 and plans[3265][3] == 0, (name, plans)
+
+
 @pytest.mark.parametrize("tile", sorted(TILES))
 @pytest.mark.parametrize("K", KS)
 def test_gemmrc(gpu, beamc, oracle, tile, K):
@@ -35,7 +59,11 @@ def test_gemmrc(gpu, beamc, oracle, tile, K):
 
 
 # [K][N], rows of whole chunks and not
-@pytest.mark.parametrize("M,N", [(41, 9), (60, 69), (466, 35), (87, 998), (1000, 1003), (41, 96), (297, 400), (1030, 104), (509, 504), (130, 1752), (466, 864), (1030, 472), (1000, 1000), (1, 4096)])
+NN = [(41, 9), (60, 69), (466, 35), (87, 998), (1000, 1003), (41, 96), (297, 400), (1030, 104), (509, 504), (130, 1752), (466, 864),
+      (1030, 472), (1000, 1000), (1, 4096)]
+
+
+@pytest.mark.parametrize("M,N", NN)
 @pytest.mark.parametrize("K", KS)
 def test_matmul_nn(gpu, beamc, oracle, M, N, K):
     L = beamc.lib
@@ -82,7 +110,7 @@ def test_split_k_needs_no_workspace_wherever_rows_start(gpu, beamc, oracle, M, N
 
 
 def test_infinities_and_nan_stay_in_their_row_or_column(gpu, beamc):
-    """Line by line a fill brings chunks of two K tiles; a chunk behind the end of K must still be a zero for every row."""
+    """Rows that start anywhere: a chunk behind the end of K is a zero for every row."""
     M, N, K = 70, 90, 3001
     L = beamc.lib
     a, b = beamc.host_uniform((M, K), F16, 96, 0), beamc.host_uniform((N, K), F16, 96, 1)
@@ -103,6 +131,28 @@ def test_infinities_of_b_behind_the_whole_chunks(gpu, beamc, N):
     out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
     assert (out[:, 5] == np.inf).all() and (out[:, 7] == -np.inf).all()
     assert np.isfinite(np.delete(out, (5, 7), axis=1)).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 90, 3208), (70, 96, 3272), (300, 700, 2008), (466, 864, 1096), (1000, 1003, 1160)])
+def test_infinities_by_whole_lines(gpu, beamc, M, N, K):
+    """A fill of whole lines brings chunks of two K tiles, and each wavefront has a part of K in one piece: elements at both ends
+    of K, on both sides of a line and of a wavefront's part reach every output of their row or column and no other."""
+    L = beamc.lib
+    assert small_tile(beamc, 0, M, N, K, 1)[3] == 1 and small_tile(beamc, 1, M, N, K, 1)[3] == 1
+    waves, tiles = small_tile(beamc, 0, M, N, K, 1)[2], -(-K // 64)
+    parts = {64 * (w * tiles // waves) for w in range(1, waves)}
+    ks = sorted(k for k in {0, 7, 8, 63, 64, K - 65, K - 64, K - 9, K - 8, K - 1} | parts | {k - 1 for k in parts} if 0 <= k < K)
+    a, b, bt = (beamc.host_uniform(s, F16, 96, i) for i, s in enumerate(((M, K), (N, K), (K, N))))
+    rows, cols = sorted({0, M // 2, M - 1}), sorted({1, N // 2, N - 1})
+    for k in ks:
+        a1, b1, bt1 = a.copy(), b.copy(), bt.copy()
+        a1[rows, k], b1[cols, k], bt1[k, cols] = 0x7E00, 0x7E00, 0x7E00  # NaN
+        want = np.zeros((M, N), bool)
+        want[rows, :] = want[:, cols] = True
+        for offsets in ((0, 0, 0), (8, 24, 0)):
+            for f, second in ((L.beam_gemmrc, b1), (L.beam_matmul_nn, bt1)):
+                out = run(beamc, lambda pa, pb, pc: f(pa, pb, pc, M, N, K, F16, None, None), a1, second, (M, N), F16, offsets).view(np.float16)
+                assert (np.isnan(out) == want).all() and np.isfinite(out[~want]).all(), (k, offsets)
 
 
 @pytest.mark.parametrize("N", [9, 88, 90, 1003])
@@ -200,6 +250,11 @@ def test_layer_norm(gpu, beamc, oracle, tile, K):
         a, b, g, bt = make_ln_inputs(beamc, M, N, K, dtype, 98)
         got = run_ln(beamc, a, b, g, bt, dtype, mode=beamc.LN_FUSED)
         check_ln(oracle, got, oracle.gemmrc_ln(a, b, g, bt, 1e-5, dtype), dtype, f"{tile} {(M, N, K)} dtype {dtype}")
+
+
+@pytest.mark.parametrize("tile", sorted(LN_TILES))
+def test_layer_norm_by_whole_lines(gpu, beamc, oracle, tile):
+    test_layer_norm(gpu, beamc, oracle, tile, 3208)
 
 
 @pytest.mark.parametrize("M,N", [(41, 100), (1030, 475), (60, 4096)])

@@ -39,6 +39,29 @@ def both(what, f, outs, handled=True):
     assert all((x.view(torch.int16) == y.view(torch.int16)).all() for x, y in zip(*got)), what
 
 
+def ordered(what, f, a, c):
+    """f's operand is written by work in front of it that is still running when f returns; launched on another stream, f would
+    read what was there before."""
+    late = torch.full_like(a, float("nan"))
+    big = torch.zeros(1 << 28, device="cuda", dtype=torch.int32)
+    torch.cuda.synchronize()
+    _C._native = Counting()
+    calls.clear()
+    f(a)
+    want = c.clone()
+    torch.cuda.synchronize()
+    for _ in range(8):  # 8 x 2 GiB of traffic, milliseconds
+        big.add_(1)
+    late.copy_(a)
+    f(late)
+    done = torch.cuda.Event()
+    done.record()
+    assert not done.query(), "the work in front is too short to tell"
+    torch.cuda.synchronize()
+    assert len(calls) == 2 and all(s >= 0 for _, s in calls), (what, calls)
+    assert (c.view(torch.int16) == want.view(torch.int16)).all(), what
+
+
 def same_error(what, f):
     said = []
     for binding in (Counting(), None):
@@ -70,6 +93,11 @@ for dtype in (torch.float16, torch.bfloat16):
         stream = torch.cuda.Stream()
         with torch.cuda.stream(stream):
             both("another stream", lambda: _C.gemmrc(a, b, c), [c])
+            ordered("gemmrc behind its stream's work", lambda x: _C.gemmrc(x, b, c), a, c)
+            ordered("matmul behind its stream's work", lambda x: _C.matmul(x, bt, c), a, c)
+            ordered("split-K behind its stream's work", lambda x: _C.gemmrc_splitk(x, b, c), a, c)
+            ordered("LayerNorm behind its stream's work", lambda x: _C.gemmrc_ln(x, b, c, g, be, check=False), a, c)
+            ordered("SiLU behind its stream's work", lambda x: _C.parallel_gemmrc_silu(x, b, c, x, torch.empty_like(x)), a, c)
         view = torch.randn(M + 1, K, device="cuda", dtype=dtype)[1:]  # contiguous, at another offset
         both("a view", lambda: _C.gemmrc(view, b, c), [c])
         both("a named tile", lambda: _C.gemmrc(a, b, c, config=_C.TileConfig(64, 64, 32, 32)), [c], handled=False)
