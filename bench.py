@@ -151,7 +151,7 @@ def extra_splitk_small(_C):
 
 
 def extra_splitk(_C):
-    """split-K at 256x256x32768: best (tile, S) against the best non-split tile."""
+    """split-K at 256x256x32768: best (tile, S) against the best non-split tile, and against gemmrc left to the library."""
     M, N, K = 256, 256, 32768
     a = _C.DeviceArray.from_numpy(_C.host_uniform((M, K), _C.F16, 11, 0))
     b = _C.DeviceArray.from_numpy(_C.host_uniform((N, K), _C.F16, 11, 1))
@@ -180,6 +180,7 @@ def extra_splitk(_C):
     # what a call that names neither tile nor slice count gets
     auto_cfg, auto_s = _C.default_config(M, N, K, split=True)
     auto_ms = min(_C.bench(1, a, b, c, config=None, split_k=0, warmup=20, iters=100) for _ in range(2))
+    own_plain_ms = min(_C.bench(0, a, b, c, config=None, warmup=20, iters=100) for _ in range(2))
     # what the machine allows for this launch shape: empty launches, and the chosen partial kernel with
     # nothing but its global->LDS loads and fragment reads (no MFMA, no store, no reduction)
     floor = {"empty_kernel_us": round(min(_C.bench(_C.OP_PROBE_EMPTY, a, b, c, warmup=50, iters=500) for _ in range(2)) * 1e3, 2),
@@ -200,6 +201,8 @@ def extra_splitk(_C):
             "library_choice_us": round(auto_ms * 1e3, 2), "library_choice": f"{auto_cfg.name},S={auto_s}",
             "best_nonsplit_us": round(best_plain[1] * 1e3, 2), "best_nonsplit_config": best_plain[0],
             "speedup": round(best_plain[1] / best_split[1], 2),
+            "library_nonsplit_us": round(own_plain_ms * 1e3, 2), "library_nonsplit_config": _C.gemmrc_kernel_name(M, N, K),
+            "speedup_over_library_nonsplit": round(own_plain_ms / best_split[1], 2),
             "hbm_GBs": round(bytes_alg / (best_split[1] * 1e-3) / 1e9, 1),
             "hbm_frac": round(bytes_alg / (best_split[1] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
 
@@ -328,11 +331,10 @@ def extra_sweep(_C):
             a = _C.DeviceArray.from_numpy(_C.host_uniform((M, K), dtype, 5, 0), dtype)
             b = _C.DeviceArray.from_numpy(_C.host_uniform((N, K), dtype, 5, 1), dtype)
             c = _C.DeviceArray((M, N), dtype)
-            cfg, _ = _C.default_config(M, N, K, split=False)
             ms = settled_ms(lambda w, n: _C.bench(_C.OP_GEMM, a, b, c, warmup=w, iters=n))
             for t in (a, b, c):
                 t.free()
-            out.append({"shape": [M, N, K], "dtype": name, "tile": cfg.name, "us": round(ms * 1e3, 1),
+            out.append({"shape": [M, N, K], "dtype": name, "tile": _C.gemmrc_kernel_name(M, N, K), "us": round(ms * 1e3, 1),
                         "TFLOPs": round(2.0 * M * N * K / (ms * 1e-3) / 1e12, 1)})
     return out
 

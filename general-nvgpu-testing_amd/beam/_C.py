@@ -227,6 +227,21 @@ def default_config(M: int, N: int, K: int, split: bool = False):
     return TileConfig(c.block_m, c.block_n, c.wave_m, c.wave_n, c.pipeline, c.group_m), s.value
 
 
+def gemmrc_kernel_name(M: int, N: int, K: int) -> str:
+    """What gemmrc without a tile runs on for operands that start on 128-byte lines.  default_config() names the tile to pass
+    on; small tiles whose K range is dealt out to the wavefronts (here rows x columns, wavefronts) have no such name, and the
+    deep 128x128 tile runs as four wavefronts."""
+    rows, cols, waves, lines = (ctypes.c_int() for _ in range(4))
+    starts = 2 if K % 64 == 0 else 1 if K % 8 == 0 else 0
+    _check(lib.beam_dbg_small_tile(0, M, N, K, starts, ctypes.byref(rows), ctypes.byref(cols), ctypes.byref(waves), ctypes.byref(lines)))
+    if rows.value:
+        return f"{rows.value}x{cols.value}_k{waves.value}" + ("_lines" if lines.value else "")
+    cfg, _ = default_config(M, N, K)
+    if (cfg.block_m, cfg.block_n, cfg.wave_n, cfg.pipeline) == (128, 128, 32, 2):
+        cfg = TileConfig(128, 128, 64, 64, 2, cfg.group_m)
+    return cfg.name
+
+
 def device_info() -> dict:
     name = ctypes.create_string_buffer(256)
     cus, clk, mem = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()

@@ -295,8 +295,7 @@ def _main(argv: Sequence[str]) -> int:
                     again = max(again, op.get_performance(a, b, c, warmup=20, rep=max(args.rep, 50), min_ms=5.0))
             for x in (a, b, c):
                 x.free()
-            cfg, _ = _C.default_config(M, N, K, split=False)
-            print(f"| {M}x{N}x{K} | {dtype} | {op} | {again:.1f} | {cfg.name} | {base:.1f} | {again / base:.3f} |", flush=True)
+            print(f"| {M}x{N}x{K} | {dtype} | {op} | {again:.1f} | {_C.gemmrc_kernel_name(M, N, K)} | {base:.1f} | {again / base:.3f} |", flush=True)
     return 0
 
 

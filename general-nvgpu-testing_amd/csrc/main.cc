@@ -609,10 +609,22 @@ int cli_bench(const Args& a) {
     beam_tile_cfg picked;
     if (beam_dbg_ln_default_config(M, N, K, 256, &picked) == BEAM_OK) cfg = picked;
   }
+  // ... and the small tile or the wavefronts that beam_gemmrc takes instead of the tile named (operands of their own start on lines)
+  int rows = 0, cols = 0, waves = 0, lines = 0;
+  const bool ln_two_pass = op == BEAM_OP_GEMM_LN && ln_mode == BEAM_LN_TWOPASS;
+  if (own_tile && !ln_two_pass)
+    (void)beam_dbg_small_tile(op == BEAM_OP_MATMUL_NN ? 1 : op == BEAM_OP_GEMM_LN ? 3 : 0, M, N, K, K % 64 == 0 ? 2 : K % 8 == 0 ? 1 : 0, &rows,
+                              &cols, &waves, &lines);
+  if (own_tile && op == BEAM_OP_GEMM && cfg.pipeline == 2 && cfg.block_m == 128 && cfg.block_n == 128 && cfg.wave_n == 32) cfg.wave_n = 64;
   int rc = time_op(op, p, own_tile ? nullptr : &cfg, split, a.num("warmup", 5), a.num("iters", 20), &ms, ln_mode);
   if (rc != BEAM_OK) {
     std::fprintf(stderr, "bench failed (%d): %s\n", rc, beam_last_error());
     return 1;
+  }
+  if (rows != 0) {
+    std::printf("%s %dx%dx%d %s small tile %dx%d, K over %d wavefronts%s: %.4f ms  %.1f TFLOP/s\n", opname.c_str(), M, N, K,
+                dtype ? "bf16" : "fp16", rows, cols, waves, lines ? ", whole lines" : "", ms, 2.0 * M * N * K / ms / 1e9);
+    return 0;
   }
   std::printf("%s %dx%dx%d %s tile %dx%d wave %dx%d pipeline %d group %d split %d: %.4f ms  %.1f TFLOP/s\n",
               opname.c_str(), M, N, K, dtype ? "bf16" : "fp16", cfg.block_m, cfg.block_n, cfg.wave_m, cfg.wave_n,

@@ -69,8 +69,9 @@ int beam_default_config(int M, int N, int K, beam_tile_cfg* cfg, int* split_k);
 
 /* cfg == NULL: beam_default_config() picks the tile (never a split); where tiles of 64 x 64 or less fill at most one round of
  * workgroups, the call may run on a kernel that has no tile to name (small tiles, K dealt out to the wavefronts), or on the
- * deep pipeline as one group of wavefronts.  Any K and any element's address; a tile
- * that is not compiled is refused, but for rows that are not 16-byte aligned, which are computed whatever is named.
+ * deep pipeline as one group of wavefronts; the 128 x 128 tile it runs on the deep pipeline as four wavefronts of 64 x 64, where
+ * beam_default_config names eight of 64 x 32.  Any K and any element's address; a tile that is not compiled is refused, but for
+ * rows that are not 16-byte aligned, which are computed whatever is named.
  * Replaces entry_cutlass_gemmrc / entry_cutlass_gemmrc_spec
  * (cuda/cutlass_kernels/main.cc:11-15, cutlass_gemmrc.cu:21-40,55-111). */
 int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int dtype,
