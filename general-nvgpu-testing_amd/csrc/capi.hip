@@ -447,11 +447,14 @@ int choose_default(int M, int N, int K, int split_req, beam_tile_cfg* cfg, int* 
   // One workgroup per CU under a long sum: the deep pipeline.  Less than half the CUs busy: its long prefetch queue keeps
   // memory busy.  Tiles with two K groups: up to a full round, since a lone group's K tile is a serial chain; 64 x 128 and
   // 128 x 64 from K = 768 on (one group, two: 2048 x 1024 x 520 6.2, 6.3; x 768 8.3, 7.2; x 1024 10.0, 8.2; x 1536 13.9, 11.0;
-  // 620 x 3064 x 776 9.9, 9.3; x 1600 14.6, 11.1; [K][N] 700 x 2500 x 512 7.9, 7.3; x 1024 12.5, 10.0), 64 x 64 from K = 384 on
-  // (12 sets of operands in turn: 1024 x 1024 x 256 3.7, 3.9; x 384 4.6, 4.5; x 512 5.3, 4.8; x 1024 8.2, 6.1; the same operands
-  // in every call x 512 3.7, 4.3; x 1024 5.0, 5.4; x 2048 8.1, 7.7; a set for each of 96 calls x 512 7.1, 5.7; x 1024 11.7,
-  // 7.7).  Only from K = 2048 on: a single row of those,
-  // whose form as one group is made for long sums, and at most half a round, where smaller tiles run (kw_plan).
+  // 620 x 3064 x 776 9.9, 9.3; x 1600 14.6, 11.1; [K][N] 700 x 2500 x 512 7.9, 7.3; x 1024 12.5, 10.0), 64 x 64 from K = 384 on.
+  // These lines are for operands that come from the last-level cache or memory, as weights that change from call to call do.
+  // With the same ones in every call, which then lie in the L2s, two groups are up to 0.8 us behind (their start, and the sums'
+  // way through LDS).  One group, two; 96 sets of operands in turn, 12 sets, the same ones: 1024 x 1024 x 256 4.0, 4.2; 3.8, 4.0;
+  // 2.9, 3.7; x 384 5.8, 5.2; 4.6, 4.5; 3.3, 4.0; x 512 7.1, 5.7; 5.2, 4.8; 3.6, 4.2; x 1024 11.7, 7.7; 8.3, 6.2; 5.0, 5.3; x 1536
+  // 16.3, 10.2; 11.2, 7.9; 6.5, 6.6; x 2048 20.8, 11.5; 14.0, 8.7; 7.9, 7.5; 2048 x 1024 x 768 11.0, 9.0; 8.2, 7.1; 5.6, 6.4; x 1024
+  // 13.6, 10.1; 9.8, 7.8; 6.6, 7.3; [K][N] 1024 x 1024 x 384 6.5, 5.5; 5.1, 4.8; 4.0, 4.5.  Only from K = 2048 on: a single row of
+  // those, whose form as one group is made for long sums, and at most half a round, where smaller tiles run (kw_plan).
   const long picked = tiles(c.block_m, c.block_n);
   const bool few = K >= 2048 && picked < cus / 2;
   const int area = c.block_m * c.block_n;
@@ -494,8 +497,9 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
   const KwPlan none = {0, 0, 0, false};
   if (K < 8 || K > kMaxK) return none;
   // Longer sums of more than a handful of rows are what beam_gemmrc_splitk is for (256 x 256 x 32768: 12.2 us there, 22.0
-  // here), and a tuner that compares the two is to find it there; the line is where the two are about even (256 x 256 x 8192:
-  // 8.7, here 7.1; 128 x 128 x 16384: 8.3, here 12.0).
+  // here); the line is where the two are about even (256 x 256 x 8192: 8.7, here 7.1; 128 x 128 x 16384: 8.3, here 12.0).  For
+  // beam_gemmrc, which has no slices, it is not a line of speed: such a sum stays on the tiled kernel at 20.2 us (256 x 256 x
+  // 8192; x 8184 7.4 here) and 78.7 (x 32768), so that the two calls remain the two methods that a tuner compares.
   if (M > 64 && K >= 8192 && !b_kmajor && !ln) return none;
   // A handful of rows beside more columns than 32 for every CU: B's way from memory is the bound, and the tiled kernels' long
   // rings are ahead but for K from 512 to 4096 (16 x 11008 x 4096 19.7 us, tiled 21.2; 1 x 14704 x 9064 47.7 tiled, here 50.6;

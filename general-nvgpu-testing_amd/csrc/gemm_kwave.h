@@ -16,7 +16,7 @@
 // 1000 x 1000 x 8184 43.7 -> 32.7, 466 x 864 x 1032 6.6 -> 6.1; 466 x 864 x 520 5.0 -> 5.1 (each wavefront has one fill more).
 //
 // us, the tiled kernels -> this: 256 x 256 x 4096 12.8 -> 5.7, x 8184 21.8 -> 7.6, 233 x 1416 x 1832 10.7 -> 7.4, 1284 x 80 x
-// 5464 25.8 -> 8.6, 1024 x 1024 x 4088 19.6 -> 16.8; [K][N] 512 x 768 x 4096 16.6 -> 11.4, 16 x 4096 x 4096
+// 5464 25.8 -> 8.6, 1024 x 1024 x 4088 19.5 -> 16.7; [K][N] 512 x 768 x 4096 16.6 -> 11.4, 16 x 4096 x 4096
 // 16.2 -> 11.2, 1284 x 80 x 5464 22.0 -> 12.5.  A handful of rows (which had a kernel of this kind for themselves, 16 columns,
 // straight): 4 x 4096 x 4096 7.9 -> 6.9, 64 x 4096 x 4096 10.4 -> 8.3, 16 x 8192 x 8192 33.0 -> 27.5.
 // Two slots and four wavefronts are the best of 1-4 slots and 2-16 wavefronts nearly everywhere (466 x 864 x 600: 5.2 us, 5.5
