@@ -125,7 +125,7 @@ struct KwTile {
     const int rows_a = M - row0 < ROWS ? M - row0 : ROWS;
     const int rows_b = N - col0 < COLS ? N - col0 : COLS;
     // Whole chunks of 8 elements, and up to 8 that come last.  K-major rows that are not whole chunks: the very last row is
-    // always among those, so that every row that is fetched has another one behind it and may be read to a whole chunk.
+    // always among those, so that every row that is fetched has another one behind it and may be read past its end.
     const bool n_odd = KMAJOR && (N & 7) != 0;
     const int k8 = (K - (n_odd ? 1 : 0)) >> 3, rem = K - 8 * k8;
     const int n_all = (k8 + 7) >> 3;       // K tiles
@@ -170,8 +170,6 @@ struct KwTile {
     // K-major B: chunk position q of a slot is row k = q / CPR (after kw_kmajor_row, its own inverse), chunk q % CPR ^ swizzle
     constexpr int CPR = COLS / 8;
     unsigned voff_b[LB];
-    const int kmajor_row0 = kw_kmajor_row(lane / CPR, COLS);  // ... of load 0; load i's is 64 / CPR * i further on
-    static_assert(64 / CPR % (COLS == 16 ? 16 : 1) == 0, "kw_kmajor_row moves rows within 16, alike in every load");
     if constexpr (KMAJOR) {
 #pragma unroll
       for (int i = 0; i < LB; ++i) {
@@ -191,16 +189,16 @@ struct KwTile {
         // with shifted rows of A, K tile t - 1 is multiplied when fill t has arrived
         const int koff = (t0 + (SHIFT ? t - 1 : t * EVERY)) * kBK;
         const bool exists = SHIFT ? t >= 1 && t <= n : t < n;
-        // (not the rows behind the whole chunks: those of A are zeros there, and zero times infinity is not.  Rows that are not
-        // whole chunks end up to 7 elements before the descriptor does, so there the rows themselves are counted as well)
+        // (not the rows behind the whole chunks: those of A are zeros there, and zero times infinity is not)
         const int rows = 8 * k8 - koff < kBK ? 8 * k8 - koff : kBK;
-        const int wanted = n_odd ? rows : kBK;
         // (columns past N in the rows in front of the last read the next row's data and feed outputs that do not exist)
-        const __amdgpu_buffer_rsrc_t rk = make_rsrc(b_base + (exists ? (size_t)koff * N : 0), exists ? ((unsigned)(rows - 1) * (unsigned)N + (unsigned)(N - col0) + (n_odd ? 7u : 0u)) * 2u : 0u);
+        // The range check works on whole dwords from a lane's own offset: an odd last column needs the element behind it in range,
+        // and that one alone is no whole dword of the row behind, which starts there.  (Telling the lanes of that row instead, by
+        // selects or by a branch in the loop, cost 0.5-1.4%: 288 x 448 x 4432 9.54 -> 9.67 and 9.59 us.)
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(b_base + (exists ? (size_t)koff * N : 0), exists ? ((unsigned)(rows - 1) * (unsigned)N + (unsigned)(N - col0) + (unsigned)(N & 1)) * 2u : 0u);
 #pragma unroll
         for (int i = 0; i < LB; ++i)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)(dst + A_BYTES + i * 1024), 16,
-                                                   (int)(kmajor_row0 + 64 / CPR * i < wanted ? voff_b[i] : kOobOffset), 0, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)(dst + A_BYTES + i * 1024), 16, (int)voff_b[i], 0, 0, 0);
       } else {
 #pragma unroll
         for (int i = 0; i < LB; ++i)

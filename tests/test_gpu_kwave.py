@@ -155,7 +155,7 @@ def test_infinities_by_whole_lines(gpu, beamc, M, N, K):
                 assert (np.isnan(out) == want).all() and np.isfinite(out[~want]).all(), (k, offsets)
 
 
-@pytest.mark.parametrize("N", [9, 88, 90, 1003])
+@pytest.mark.parametrize("N", [9, 10, 15, 88, 90, 92, 1003])
 @pytest.mark.parametrize("K", [9, 64, 75, 128, 200, 1032, 2000])
 def test_infinities_in_the_last_rows_of_b(gpu, beamc, N, K):
     """[K][N]: a row of B behind the whole chunks meets only its own elements of A, never the zeros beside them.  With
@@ -166,12 +166,13 @@ def test_infinities_in_the_last_rows_of_b(gpu, beamc, N, K):
     a = beamc.host_uniform((M, K), F16, 97, 0)
     a[:, first:] = 0x3C00  # one
     for row in rows:
-        for cols in ([0, 5], [1, 7], [2, 3, 4, 6], [N - 1]):
+        for cols in ([0], [1], [2], [3], [4], [5], [6], [7], [N - 1], [0, 5, N - 1]):
             b = beamc.host_uniform((K, N), F16, 97, 1)
             b[row, cols] = 0x7C00
-            out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
-            assert (out[:, cols] == np.inf).all(), (row, cols)
-            assert np.isfinite(np.delete(out, cols, axis=1)).all(), (row, cols)
+            for offsets in ((0, 0, 0), (1, 3, 1)):
+                out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, offsets).view(np.float16)
+                assert (out[:, cols] == np.inf).all(), (row, cols, offsets)
+                assert np.isfinite(np.delete(out, cols, axis=1)).all(), (row, cols, offsets)
 
 
 # The elementwise job rides in workgroups of its own behind the tiles'.  Counts: a tail only, one access of one thread, ragged,
