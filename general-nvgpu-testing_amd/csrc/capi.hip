@@ -221,6 +221,29 @@ GemmParams base_params(const void* A, const void* B, int M, int N, int K, const 
   return p;
 }
 
+// How a tiled kernel's 16-bit output leaves (StoreKind).  Rows on 64-byte sectors: through the L2.  Rows off them are written
+// in parts of a sector by two wavefronts or workgroups: left in the L2, which puts the parts together, where that saves more
+// than the write-back at the kernel's end costs.  (us, through -> cached; C in the last-level cache, then from memory.)
+//   * The kernel of gemm_w4.h, 64 contiguous bytes of a row per store: always (2048 x 1992 x 4032 68 -> 67, 77 -> 74; 4096 x
+//     4040 x 256 19 -> 15.5, 27 -> 18, x 1024 34 -> 31, 41 -> 33).
+//   * Tiles of 64 columns: always (2048 x 1992 x 256 in 64 x 64 tiles, two K groups 14.2 -> 13.7, 14.3 -> 13.8, x 1985 14.6 ->
+//     13.5; 512 x 968 x 256 4.0 -> 3.9, 4.1 -> 4.0).
+//   * The others from 20 MB on (3072 x 4040 x 256 in 128 x 128 tiles 14.0 -> 12.9, 20 -> 15, in 192 x 256 13.1, 13.3, 18 -> 14;
+//     4096 x 8136 x 1024 in 256 x 256 tiles 70 -> 63, 79 -> 68; 8192 x 8136 x 256 in 128 x 128 106 -> 71).  Below: 2048 x 1992 x
+//     1024 in 128 x 128 tiles 11.6, cached 12.0.
+//   * 256 x 256 tiles of eight wavefronts over several rounds, one workgroup per tile, wherever rows start (4096 x 8192 x 256
+//     50 -> 34, x 1024 64 -> 62).
+// (Non-temporal stores are faster still by themselves, 8192 x 8192 x 1024 in 128 x 128 tiles 161 -> 126 us, but only put the
+// cost off: with a kernel that reads the output behind it, 4096 x 4096 x 1024 takes 54.3 us written through, 56.2 so.)
+int store_kind(const beam_tile_cfg& c, const KernelSet& ks, bool w4, const void* C, int M, int N) {
+  const size_t bytes = (size_t)M * N * 2;
+  const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
+  if (!w4 && ks.threads == 512 && c.block_m * c.block_n == 256 * 256 &&
+      (long)((M + 255) / 256) * ((N + 255) / 256) > cus) return kStoreCached;
+  if (N % 32 == 0 && ((uintptr_t)C & 63) == 0) return kStoreThrough;
+  return w4 || c.block_n == 64 || bytes >= ((size_t)20 << 20) ? kStoreCached : kStoreThrough;
+}
+
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // ---- host data generation -------------------------------------------------------------
@@ -626,7 +649,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   if (w4_fits && w4_named) {
     // Non-temporal stores of C pay when C is larger than the 256 MB last-level cache (and the K loops
     // are not so short that the writes are the bound).
-    p.c_streaming = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024;
+    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, *ks, true, C, M, N);
     BEAM_HIP(launch_gemm_w4(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
@@ -644,6 +667,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     BEAM_HIP(loop(p, dim3((unsigned)cus, 1, 1), st));
     return BEAM_OK;
   }
+  p.c_store = store_kind(c, *ks, false, C, M, N);
   GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, false, cus);
   BEAM_HIP((one_group ? one_group : ks->launch[dtype][kEpiStore][c.pipeline])(p, dim3((unsigned)tiles, 1, 1), st));
   return BEAM_OK;
@@ -712,10 +736,11 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   if (w4_fits && w4_named) {
     const long tiles = (long)p.tiles_m * p.tiles_n;
-    p.c_streaming = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024;
+    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, *ks, true, C, M, N);
     BEAM_HIP(launch_gemm_w4_kmajor(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
+  p.c_store = store_kind(c, *ks, false, C, M, N);
   GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, true, cus);
   BEAM_HIP((one_group ? one_group : ks->launch_kmajor[dtype][c.pipeline])(p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
   return BEAM_OK;
@@ -850,6 +875,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }
+  p.c_store = store_kind(c, *ks, false, C, M, N);
   BEAM_HIP(ks->launch[dtype][kEpiStoreSide][c.pipeline](p, dim3((unsigned)wgs, 1, 1), (hipStream_t)stream));
   return BEAM_OK;
 }
@@ -1410,6 +1436,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   // K == 0: the kernels run with an empty K range and produce x = 0, i.e. y = beta.
   if (plan.kind == LnPlan::kFused) {
     p.C = Y;
+    p.c_store = store_kind(c, *ks, plan.w4, Y, M, N);
     // Launches that share a workspace must be ordered (same stream): overlapping ones would race on the sets.
     const size_t set_bytes = ln_fused_set_bytes(p.tiles_m, p.tiles_n, c.block_m);
     float* sets = (float*)((char*)ws + ln_fused_header_bytes());

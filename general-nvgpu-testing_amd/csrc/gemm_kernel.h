@@ -141,6 +141,7 @@ struct GemmParams {
   int side_iters;        // K tiles' worth of units per workgroup
   int side_width;        // bytes per unit
   int c_streaming;       // kEpiStoreLoop: store C non-temporal
+  int c_store;           // StoreKind of the other 16-bit epilogues
   // kEpiPartialFused: word kSkTimeout, then from word kSkFlags on one flag per (tile, part of the tile, slice);
   // behind the partial sums in the caller's workspace.  Never has to be initialised (see sk_launch_tag).
   int* sk_sync;
@@ -280,16 +281,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, un
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, kRsrcFlags);
 }
 
-// 16 bytes of output, written through the L2 to memory (device scope) instead of left dirty in it.  A kernel ends
-// only when its dirty lines have been written back; for the one-tile-per-CU kernels, whose stores all come at the
-// very end, writing through moves that work under the other workgroups' last K tiles: 1024^3 5.5 -> 5.3 us,
-// 2048 x 2048 x 512 7.1 -> 6.5 us, 3072^3 48.0 -> 47.0 us, 2048^3 and outputs of tens of MB unchanged (same machine,
-// the two builds in turn; non-temporal stores, tried beside it, lose 8% at 3000 x 5000 x 2000).
-// (The wait states behind it: a store of more than 8 bytes reads its data registers over several cycles, and a
-// vector instruction that overwrites them must not follow at once.  The compiler keeps that distance for stores it
-// emits itself; it does not look into assembly text.)
-__device__ __forceinline__ void store_through_16(void* dst, i32x4 v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
+// How 16-bit output leaves (GemmParams::c_store; the host's store_kind has the rule and what it measured).
+//   Through: through the L2 to memory (device scope).  A kernel ends only when its dirty lines have been written back; for
+//     the one-tile-per-CU kernels, whose stores all come at the very end, writing through moves that work under the other
+//     workgroups' last K tiles: 1024^3 5.5 -> 5.3 us, 2048 x 2048 x 512 7.1 -> 6.5, 3072^3 48.0 -> 47.0.
+//   Cached: left dirty in the L2, which puts the parts of a 64-byte sector together that rows off such sectors leave to two
+//     wavefronts or workgroups; written through, each part goes to memory by itself (3000 x 5000 x 256 in 256 x 256 tiles
+//     28.6 -> 18.2 us, 3000 x 4992 x 256 15.1).
+//   Streaming: non-temporal, so that the output's lines do not push operand panels out of the L2 (4096 x 8192 x 1024 in
+//     128 x 128 tiles 82.8 -> 65.4 us).
+enum StoreKind : int { kStoreThrough = 0, kStoreCached = 1, kStoreStreaming = 2 };
+
+// (The wait states: a store of more than 8 bytes reads its data registers over several cycles, and a vector instruction
+// that overwrites them must not follow at once.  The compiler keeps that distance for stores it emits itself; it does not
+// look into assembly text.)
+template <int KIND>
+__device__ __forceinline__ void store_16(void* dst, i32x4 v) {
+  if constexpr (KIND == kStoreThrough) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
+  else if constexpr (KIND == kStoreCached) asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
+  else asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
 }
 
 // s_waitcnt vmcnt(N) lgkmcnt(0): at most N of this wavefront's buffer loads still in flight,
@@ -1203,24 +1213,30 @@ struct GemmTile {
           for (int j = 0; j < FN; ++j)
             *(vec4*)(stage + i * 16 * RB + w_off + (((2 * j + (wg >> 1)) ^ chunk_xor(wr)) << 4)) = value(hf * FMH + i, j, ctx);
         }
+        // one copy of the loop for each kind, not a branch per store: the reads of a pass stay batched ahead of its stores
+        auto store_pass = [&](auto kind_tag) __attribute__((always_inline)) {
 #pragma unroll
-        for (int it = 0; it < FMH * 16 / RPI; ++it) {
-          const int r = it * RPI + srow;
-          vec8 v = *(const vec8*)(stage + r * RB + schunk * 16);
-          if ((r >> 3) & 1) v = vec8{v[4], v[5], v[6], v[7], v[0], v[1], v[2], v[3]};
-          const int n_st = col0 + wn * TN + (schunk ^ chunk_xor(r)) * 8;
-          const int m = row0 + wm * TM + hf * FMH * 16 + r;
-          if (m < M) {
-            T* dst = C + (size_t)m * N + n_st;
-            if (n_st + 7 < N) {  // (at any element's address)
-              store_through_16(dst, __builtin_bit_cast(i32x4, v));
-            } else {
+          for (int it = 0; it < FMH * 16 / RPI; ++it) {
+            const int r = it * RPI + srow;
+            vec8 v = *(const vec8*)(stage + r * RB + schunk * 16);
+            if ((r >> 3) & 1) v = vec8{v[4], v[5], v[6], v[7], v[0], v[1], v[2], v[3]};
+            const int n_st = col0 + wn * TN + (schunk ^ chunk_xor(r)) * 8;
+            const int m = row0 + wm * TM + hf * FMH * 16 + r;
+            if (m < M) {
+              T* dst = C + (size_t)m * N + n_st;
+              if (n_st + 7 < N) {  // (at any element's address)
+                store_16<decltype(kind_tag)::value>(dst, __builtin_bit_cast(i32x4, v));
+              } else {
 #pragma unroll
-              for (int e = 0; e < 8; ++e)
-                if (n_st + e < N) dst[e] = v[e];
+                for (int e = 0; e < 8; ++e)
+                  if (n_st + e < N) dst[e] = v[e];
+              }
             }
           }
-        }
+        };
+        if (p.c_store == kStoreThrough) store_pass(std::integral_constant<int, kStoreThrough>{});  // (uniform)
+        else if (p.c_store == kStoreCached) store_pass(std::integral_constant<int, kStoreCached>{});
+        else store_pass(std::integral_constant<int, kStoreStreaming>{});
       }
     };
 

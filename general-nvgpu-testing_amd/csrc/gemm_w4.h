@@ -132,8 +132,9 @@ __host__ __device__ inline int w4_b_row(int b, int r) { return 32 * (b >> 1) + 4
 // loads of the A tile after next in gaps 0, SA, ... of step B.  The path from the vector-memory unit into
 // LDS moves 64 bytes per cycle and CU, i.e. one 1 KiB load per 64 cycles (4 MFMAs) and wavefront when all
 // four issue: loads issued faster than that stall the wavefront, and with it its MFMAs, at issue.
-// C_NT: C is stored non-temporal (an output larger than the last-level cache: its lines then do not push
-// operand panels out of the caches).
+// STORE (StoreKind): kStoreStreaming: C is stored non-temporal (an output larger than the last-level cache: its lines then do
+// not push operand panels out of the caches).  The other two say how the stores behind a workgroup's last K loop leave, and
+// all of them with LN.
 // LN: the fused GEMM+LayerNorm of gemm_kernel.h (kEpiLnFused) with this K loop: output tiles in the band
 // order of tile_map.h, and after each tile's K loop the same exchange of per-row (mean, M2) pairs between the
 // column tiles of a row band, normalisation in registers, Y stored once.  A workgroup walks the ids
@@ -142,7 +143,7 @@ __host__ __device__ inline int w4_b_row(int b, int r) { return 32 * (b >> 1) + 4
 // in the plain kernel -- the next tile's first operand tiles arrive while the band's statistics are
 // exchanged (walking_layer_norm below says why nobody waits for ever).
 // B_KMAJOR: B is stored [K][N].
-template <typename T, bool C_NT = false, bool LN = false, int SB = 4, int SA = 8, int G0 = 2, bool B_KMAJOR = false>
+template <typename T, int STORE = kStoreThrough, bool LN = false, int SB = 4, int SA = 8, int G0 = 2, bool B_KMAJOR = false>
 struct GemmW4 {
   static_assert(!(LN && B_KMAJOR), "the fused LayerNorm is built for B as [N][K]");
   using Traits = ElemTraits<T>;
@@ -365,10 +366,11 @@ struct GemmW4 {
     // LAST: the stores after the workgroup's last K loop.  Nothing hides them, and a kernel ends only when its
     // dirty lines have left the L2: those go through it to memory at once (device-scope stores; 4096^3, one tile
     // per workgroup: 98.9 -> 96.5 us, fused LayerNorm 105.7 -> 103.7 us).  The stores of earlier tiles lie under
-    // the next tile's MFMAs and stay plain (written through, 8192^3 loses 0.2%).
+    // the next tile's MFMAs and stay plain (written through, 8192^3 loses 0.2%).  Rows off 64-byte sectors stay in the L2 there
+    // too, which puts the parts of a sector together (kStoreCached).
     auto store_pair = [&](auto i_tag, auto q_tag, auto last_tag) __attribute__((always_inline)) {
       constexpr int i = decltype(i_tag)::value, q = decltype(q_tag)::value;
-      constexpr int AUX = C_NT ? 2 : (decltype(last_tag)::value ? kAuxDeviceScope : 0);
+      constexpr int AUX = STORE == kStoreStreaming ? 2 : (decltype(last_tag)::value && STORE == kStoreThrough ? kAuxDeviceScope : 0);
       constexpr int R0 = 4 * (8 * i + 2 * q);  // first register of block (i, 2 q); block (i, 2 q + 1) follows
       vec8 v;
       v[0] = (T)w4_acc_read<R0 + 0>();
@@ -835,7 +837,7 @@ struct GemmW4 {
     //    follows it: two instantiations of the same source need not round alike (the compiler fuses the last
     //    multiply-add with the conversion to 16 bits in one place and not in another, which differs on ties), and
     //    a workgroup that walks its tiles must give the bits of one that has a single tile.
-    constexpr int AUX = kAuxDeviceScope;
+    constexpr int AUX = STORE == kStoreThrough ? kAuxDeviceScope : 0;
     w4_static_for<0, FM>([&](auto i_tag) __attribute__((always_inline)) {
       constexpr int i = decltype(i_tag)::value;
       const int row = wm * 128 + 16 * i + r;
@@ -859,10 +861,10 @@ struct GemmW4 {
   }
 };
 
-template <typename T, bool C_NT = false, bool LN = false, int SB = 4, int SA = 8, int G0 = 2, bool B_KMAJOR = false>
+template <typename T, int STORE = kStoreThrough, bool LN = false, int SB = 4, int SA = 8, int G0 = 2, bool B_KMAJOR = false>
 __global__ void __launch_bounds__(256) gemmrc_w4_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  GemmW4<T, C_NT, LN, SB, SA, G0, B_KMAJOR>::run(p, smem);
+  GemmW4<T, STORE, LN, SB, SA, G0, B_KMAJOR>::run(p, smem);
 }
 
 }  // namespace beam
