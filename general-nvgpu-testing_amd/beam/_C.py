@@ -129,6 +129,7 @@ def _load() -> ctypes.CDLL:
     L.beam_dbg_ln_plan_bytes.restype = sz
     L.beam_dbg_assume_compute_units.argtypes = [i]
     L.beam_dbg_small_tile.argtypes = [i, i, i, i, i] + [ctypes.POINTER(i)] * 4
+    L.beam_dbg_off_lines_tile.argtypes = [i, i, i, cfgp, ctypes.POINTER(i)]
     L.beam_set_ln_walk.argtypes = [i]
     L.beam_dbg_set_splitk_self_reduce.argtypes = [i]
     L.beam_dbg_tile_of_workgroup.argtypes = [i, i, i, i, ctypes.POINTER(i), ctypes.POINTER(i)]
@@ -229,13 +230,18 @@ def default_config(M: int, N: int, K: int, split: bool = False):
 
 def gemmrc_kernel_name(M: int, N: int, K: int) -> str:
     """What gemmrc without a tile runs on for operands that start on 128-byte lines.  default_config() names the tile to pass
-    on; small tiles whose K range is dealt out to the wavefronts (here rows x columns, wavefronts) have no such name, and the
-    deep 128x128 tile runs as four wavefronts."""
+    on; small tiles whose K range is dealt out to the wavefronts (here rows x columns, wavefronts) have no such name, the deep
+    128x128 tile runs as four wavefronts, and rows off those lines have a choice of their own (_lines: whole-line fills)."""
     rows, cols, waves, lines = (ctypes.c_int() for _ in range(4))
     starts = 2 if K % 64 == 0 else 1 if K % 8 == 0 else 0
     _check(lib.beam_dbg_small_tile(0, M, N, K, starts, ctypes.byref(rows), ctypes.byref(cols), ctypes.byref(waves), ctypes.byref(lines)))
     if rows.value:
         return f"{rows.value}x{cols.value}_k{waves.value}" + ("_lines" if lines.value else "")
+    if starts == 1:
+        tile = _TileCfg()
+        _check(lib.beam_dbg_off_lines_tile(M, N, K, ctypes.byref(tile), ctypes.byref(lines)))
+        cfg = TileConfig(*(getattr(tile, f) for f, _ in _TileCfg._fields_))
+        return cfg.name + ("_lines" if lines.value else "")
     cfg, _ = default_config(M, N, K)
     if (cfg.block_m, cfg.block_n, cfg.wave_n, cfg.pipeline) == (128, 128, 32, 2):
         cfg = TileConfig(128, 128, 64, 64, 2, cfg.group_m)

@@ -235,10 +235,10 @@ GemmParams base_params(const void* A, const void* B, int M, int N, int K, const 
 //     50 -> 34, x 1024 64 -> 62).
 // (Non-temporal stores are faster still by themselves, 8192 x 8192 x 1024 in 128 x 128 tiles 161 -> 126 us, but only put the
 // cost off: with a kernel that reads the output behind it, 4096 x 4096 x 1024 takes 54.3 us written through, 56.2 so.)
-int store_kind(const beam_tile_cfg& c, const KernelSet& ks, bool w4, const void* C, int M, int N) {
+int store_kind(const beam_tile_cfg& c, int wavefronts, bool w4, const void* C, int M, int N) {
   const size_t bytes = (size_t)M * N * 2;
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
-  if (!w4 && ks.threads == 512 && c.block_m * c.block_n == 256 * 256 &&
+  if (!w4 && wavefronts == 8 && c.block_m * c.block_n == 256 * 256 &&
       (long)((M + 255) / 256) * ((N + 255) / 256) > cus) return kStoreCached;
   if (N % 32 == 0 && ((uintptr_t)C & 63) == 0) return kStoreThrough;
   return w4 || c.block_n == 64 || bytes >= ((size_t)20 << 20) ? kStoreCached : kStoreThrough;
@@ -514,7 +514,8 @@ GemmLauncher deep_one_group(const KernelSet& ks, const beam_tile_cfg& c, int M, 
 // Beyond one tile of 64 x 64 for every CU the tiled kernels are ahead: 2048 x 1024 x 2040 18.8, here 20.0.)
 //   b_kmajor, ln: the form; gemm: for beam_gemmrc's or beam_matmul_nn's result, not for a split-K call; rows: where every row of A (and of B as [N][K]) starts.
 enum RowStarts { kAnywhere, kOnChunks, kOnLines };  // at an element, on 16 bytes, on 128
-KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts rows, int cus) {
+//   side: with a SiLU job beside it.
+KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts rows, int cus, bool side = false) {
   static const struct { int rows, cols; } kTiles[] = {{8, 16},  {16, 16}, {16, 32}, {32, 16}, {32, 32},
                                                       {8, 64},  {16, 64}, {32, 64}, {64, 32}, {64, 64}};
   const KwPlan none = {0, 0, 0, false};
@@ -551,6 +552,9 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
     // 6.8 -> 6.1, x 1001 9.5 -> 8.5, x 1032 8.4 -> 7.9, x 1288 9.1 -> 9.0, x 1544 9.6, 9.8; rows on lines x 1536 8.2 -> 7.9, x 1792
     // 8.6 -> 8.2; [K][N] x 256 5.0 -> 4.2, x 512 5.8 -> 5.3, x 1024 7.0 -> 6.9, x 1536 8.3, 8.7; 1000 x 1003 x 1024 6.8, 7.7).
     if (t.rows * t.cols == 64 * 64 && gemm && N % 8 == 0 && M > 64 && K <= (rows != kOnLines ? 1280 : b_kmajor ? 1024 : 2047)) return none;
+    // ... nor where rows are off lines but on chunks and fills would take whole lines here: so they do in the tiled kernel
+    // (kFormLines; 1100 x 544 x 1352 8.9 -> 7.3, 1402 x 664 x 2216 11.9 -> 10.4, 447 x 1912 x 7504 27.8 -> 24.9; odd N stays).
+    if (t.rows * t.cols == 64 * 64 && plan.shift && gemm && !b_kmajor && !side && N % 8 == 0) return none;
     // ... or one row of 32 x 64 tiles streams B from nearly every CU (20 x 14000 x 1500 10.7, here 11.4; 32 x 11008 x 4096 18.8,
     // 18.1; 30 x 9000 x 3000 13.6, 12.1).
     if (t.rows == 32 && t.cols == 64 && M <= 32 && !b_kmajor && !ln && 4 * tiles > 3L * cus) return none;
@@ -560,6 +564,70 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
     return plan;
   }
   return none;
+}
+
+// What beam_gemmrc without a tile runs on where rows are off 128-byte lines but on 16-byte chunks and gemm_kwave.h is not it:
+// one of the tiles whose fills take whole lines (gemm_kernel.h: Form), or one of the others, which fill at half the rate
+// there (only rows of whole lines that start behind one stay as choose_default has them).  The cost model of choose_default with constants of its own, since the straight tiles' rates are lower on such rows:
+// TFLOP/s per CU alone and with `occ` workgroups on the CU, us per round of workgroups and per launch, least squares on the logarithm over 280 shapes with M, N from 64
+// to 8192 and K from 64 to 8192 off lines.  Its pick is 1.0% (worst 18%) behind the best of these on average, 1.5% on
+// shapes that it was not fitted to; what ran before was 10% behind.  us, before -> now: 928 x 1232 x 7112 49.7 -> 27.9, 633 x
+// 6536 x 2952 38.5 -> 26.3, 1228 x 1784 x 6296 59.4 -> 36.9, 7702 x 7248 x 2472 268 -> 255, 2247 x 3736 x 216 12.7 -> 10.3.
+struct OffLinesTile {
+  beam_tile_cfg cfg;
+  bool lines;
+};
+OffLinesTile off_lines_tile(int M, int N, int K, int cus) {
+  struct Candidate {
+    beam_tile_cfg cfg;
+    bool lines;
+    int occ;
+    double alone, full, round, launch;
+  };
+  static const Candidate kCandidates[] = {
+      {{256, 256, 128, 64, 0, 0}, false, 1, 7.37, 7.37, 8.55, 0.0},
+      {{224, 256, 112, 64, 0, 0}, false, 1, 6.73, 6.73, 7.33, 0.0},
+      {{192, 256, 96, 64, 0, 0}, false, 1, 6.16, 6.16, 6.09, 0.0},
+      {{256, 128, 64, 64, 0, 0}, false, 1, 5.17, 5.17, 4.62, 0.0},
+      {{128, 256, 64, 64, 0, 0}, false, 1, 4.84, 4.84, 4.31, 0.11},
+      {{128, 128, 64, 64, 0, 0}, false, 2, 3.89, 3.81, 2.88, 1.25},
+      {{128, 128, 64, 64, 2, 0}, false, 1, 3.93, 3.93, 3.29, 1.13},
+      {{128, 64, 64, 32, 0, 0}, false, 2, 2.62, 2.76, 1.82, 1.34},
+      {{128, 64, 64, 32, 2, 0}, false, 1, 2.77, 2.77, 2.47, 1.36},
+      {{64, 128, 32, 64, 0, 0}, false, 2, 2.10, 2.71, 1.90, 0.87},
+      {{64, 128, 32, 64, 2, 0}, false, 1, 2.66, 2.66, 2.57, 1.09},
+      {{64, 64, 32, 32, 0, 0}, false, 4, 1.57, 2.24, 1.60, 0.91},
+      {{64, 64, 32, 32, 2, 0}, false, 1, 2.00, 2.00, 2.12, 0.96},
+      {{64, 64, 32, 32, 2, 0}, true, 1, 2.72, 2.72, 2.45, 0.88},
+      {{96, 64, 48, 32, 2, 0}, true, 1, 3.42, 3.42, 2.67, 0.96},
+      {{64, 128, 32, 64, 2, 0}, true, 1, 3.72, 3.72, 3.08, 0.91},
+      {{128, 64, 64, 32, 2, 0}, true, 1, 3.63, 3.63, 3.10, 1.19},
+      {{96, 128, 48, 64, 2, 0}, true, 1, 4.65, 4.65, 3.90, 0.86},
+      {{128, 128, 64, 64, 2, 0}, true, 1, 5.18, 5.18, 4.75, 0.82},
+      {{160, 128, 80, 64, 2, 0}, true, 1, 6.07, 6.07, 4.35, 0.89},
+      {{192, 128, 96, 64, 2, 0}, true, 1, 6.45, 6.45, 6.58, 0.26},
+  };
+  // What choose_default names stays unless another is 4% ahead by this model (639 x 1648 x 272 in 64 x 64 tiles 4.4 us, its
+  // best, 96 x 64, 4.9).
+  beam_tile_cfg named;
+  int split;
+  if (choose_default(M, N, K, -1, &named, &split) != BEAM_OK) named = kCandidates[0].cfg;
+  const Candidate *best = nullptr, *stays = nullptr;
+  double best_us = 0, stays_us = 0;
+  for (const Candidate& k : kCandidates) {
+    const long tiles = (long)((M + k.cfg.block_m - 1) / k.cfg.block_m) * ((N + k.cfg.block_n - 1) / k.cfg.block_n);
+    const long load = (tiles + cus - 1) / cus;  // workgroups per CU
+    const long conc = load < k.occ ? load : k.occ;
+    const double rate = k.occ == 1 ? k.alone : k.alone + (k.full - k.alone) * (double)(conc - 1) / (k.occ - 1);
+    const double mflop = 2.0e-6 * k.cfg.block_m * k.cfg.block_n * (double)(((long)K + kBK - 1) / kBK * kBK);
+    const double us = (double)((load + k.occ - 1) / k.occ) * k.round + (double)load * mflop / rate + k.launch;
+    if (!best || us < best_us) best = &k, best_us = us;
+    if (!k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline) stays = &k, stays_us = us;
+  }
+  if (stays && best_us > 0.96 * stays_us) best = stays;
+  OffLinesTile t = {best->cfg, best->lines};
+  t.cfg.group_m = default_group_m(t.cfg.block_m, t.cfg.block_n);
+  return t;
 }
 
 // LDS of one of its workgroups: two slots of a K tile for each wavefront, rows in blocks of 16.
@@ -619,7 +687,20 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   }
   beam_tile_cfg c;
   const KernelSet* ks;
-  if ((rc = resolve_cfg(cfg, M, N, K, &c, &ks, -1, true))) {
+  const bool off_lines = !cfg && K % kBK != 0 && row_starts(A, B, K, false) == kOnChunks;
+  if (off_lines) {
+    const OffLinesTile t = off_lines_tile(M, N, K, cus);
+    c = t.cfg;
+    if (t.lines) {
+      GemmParams p = base_params(A, B, M, N, K, c);
+      p.C = C;
+      p.c_store = store_kind(c, 4, false, C, M, N);
+      const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, 1);
+      BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_lines<_Float16>(c.block_m, c.block_n, p, grid, st) : launch_gemm_lines<__bf16>(c.block_m, c.block_n, p, grid, st));
+      return BEAM_OK;
+    }
+  }
+  if ((rc = resolve_cfg(off_lines ? &c : cfg, M, N, K, &c, &ks, -1, true))) {
     if (!rows_unaligned(A, B, C, K)) return rc;
     BEAM_HIP(launch_generic_gemm(A, B, C, M, N, K, dtype, false, false, st));
     return BEAM_OK;
@@ -649,7 +730,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   if (w4_fits && w4_named) {
     // Non-temporal stores of C pay when C is larger than the 256 MB last-level cache (and the K loops
     // are not so short that the writes are the bound).
-    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, *ks, true, C, M, N);
+    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, ks->threads / 64, true, C, M, N);
     BEAM_HIP(launch_gemm_w4(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
@@ -667,7 +748,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     BEAM_HIP(loop(p, dim3((unsigned)cus, 1, 1), st));
     return BEAM_OK;
   }
-  p.c_store = store_kind(c, *ks, false, C, M, N);
+  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N);
   GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, false, cus);
   BEAM_HIP((one_group ? one_group : ks->launch[dtype][kEpiStore][c.pipeline])(p, dim3((unsigned)tiles, 1, 1), st));
   return BEAM_OK;
@@ -736,11 +817,11 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   if (w4_fits && w4_named) {
     const long tiles = (long)p.tiles_m * p.tiles_n;
-    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, *ks, true, C, M, N);
+    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, ks->threads / 64, true, C, M, N);
     BEAM_HIP(launch_gemm_w4_kmajor(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
-  p.c_store = store_kind(c, *ks, false, C, M, N);
+  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N);
   GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, true, cus);
   BEAM_HIP((one_group ? one_group : ks->launch_kmajor[dtype][c.pipeline])(p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
   return BEAM_OK;
@@ -818,7 +899,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   //     from K = 1024 or 2^21 elements on (1024^3 with 2^18 9.1, 9.0, with 2^22 16.3, 11.2; 1024 x 1024 x 512 with 2^18 6.1, 7.8,
   //     with 2^22 9.9, 9.6).
   if (!cfg) {
-    if (const KwPlan kw = kw_plan(M, N, K, false, false, true, row_starts(A, B, K, false), cus); kw.rows) {
+    if (const KwPlan kw = kw_plan(M, N, K, false, false, true, row_starts(A, B, K, false), cus, true); kw.rows) {
       const long long per_wg = (long long)kw.waves * 64 * 8 * 8;  // elements of one round of a side workgroup's accesses
       const long long want = (count + per_wg - 1) / per_wg;
       const int per_cu = kLdsBytes / kw_lds_bytes(kw);  // workgroups of the launch on a CU
@@ -875,7 +956,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }
-  p.c_store = store_kind(c, *ks, false, C, M, N);
+  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N);
   BEAM_HIP(ks->launch[dtype][kEpiStoreSide][c.pipeline](p, dim3((unsigned)wgs, 1, 1), (hipStream_t)stream));
   return BEAM_OK;
 }
@@ -1363,6 +1444,14 @@ int beam_dbg_small_tile(int op, int M, int N, int K, int row_starts, int* rows, 
   return BEAM_OK;
 }
 
+int beam_dbg_off_lines_tile(int M, int N, int K, beam_tile_cfg* cfg, int* whole_lines) {
+  if (M <= 0 || N <= 0 || K < 8 || !cfg || !whole_lines) return fail(BEAM_ERR_INVALID, "null pointer or empty problem");
+  const OffLinesTile t = off_lines_tile(M, N, K, g_dev.cus > 0 ? g_dev.cus : 256);
+  *cfg = t.cfg;
+  *whole_lines = t.lines ? 1 : 0;
+  return BEAM_OK;
+}
+
 int beam_dbg_set_splitk_self_reduce(int on) {
   g_splitk_self_reduce.store(on != 0);
   return BEAM_OK;
@@ -1436,7 +1525,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   // K == 0: the kernels run with an empty K range and produce x = 0, i.e. y = beta.
   if (plan.kind == LnPlan::kFused) {
     p.C = Y;
-    p.c_store = store_kind(c, *ks, plan.w4, Y, M, N);
+    p.c_store = store_kind(c, ks->threads / 64, plan.w4, Y, M, N);
     // Launches that share a workspace must be ordered (same stream): overlapping ones would race on the sets.
     const size_t set_bytes = ln_fused_set_bytes(p.tiles_m, p.tiles_n, c.block_m);
     float* sets = (float*)((char*)ws + ln_fused_header_bytes());

@@ -347,7 +347,25 @@ constexpr DeepShape deep_shape(int BM, int BN, int NW) {
   return {a, a - 1, 1};
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false, int KG = 1>
+// How fills take K elements, and how K groups share the work.
+//
+// Fills of LDS move one 128-byte line of memory per two clocks, whether they use the whole line or a part of it.  A row whose
+// K elements do not start on a line (K % 64 != 0, or such an address) has every 128-byte K tile in two lines, so a fill of
+// that K tile takes twice as long, and that bounds tiles up to 128 x 128 and 192 x 128 (1228 x 1784 x 6296 in 128 x 128 tiles 77 us, x 6272,
+// whose rows start on lines, 57).  With kFormLines a fill takes whole lines, whatever K elements those are: in fill t a row's
+// chunks c < 8 - phase (phase: 16-byte chunks between the start of its first line and the row) belong to K tile t, and the
+// others, in front of them in the same line, to K tile t - 1.  A chunk keeps its place in the slot.  So K tile t is read from
+// two slots, its own and the one behind it, each lane from the slot that holds its chunk: one select per operand and step.
+// It costs one slot of the ring and a fill.  Where a chunk is no K element of this workgroup's the fill leaves zeros; K ends
+// with a chunk (K % 8 == 0) and rows start on one.  Any phase gives the right result; the right one gives one line per row and fill.
+//   us, straight -> lines: 128 x 128 tiles 1228 x 1784 x 6296 77.2 -> 57.7, 3644 x 1024 x 4816 57.3 -> 47.5; 64 x 128 928 x 1232
+//   x 7112 63.8 -> 44.7; 64 x 64 531 x 1000 x 4944 22.7 -> 17.0; on rows of whole lines 1 to 10% behind (2048^3 18.6, 20.6).
+// kFormLineHalves: the two K groups share one ring, group g multiplies half g of every K tile.  A wavefront then has its
+// SIMD's other one to hide behind, as with two rings, and the ring is twice as deep.  (Two rings are ahead for 64 x 64 and
+// 96 x 64 tiles, 9.7 against 10.5 at 1024 x 1024 x 2040, one group for 160 x 128.)
+enum Form : int { kFormStraight = 0, kFormLines = 1, kFormLineHalves = 2 };
+
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false, int KG = 1, int FORM = 0>
 struct GemmTile {
   using Traits = ElemTraits<T>;
   using vec8 = typename Traits::vec8;
@@ -360,7 +378,11 @@ struct GemmTile {
   // early and idle at the barrier while the younger ones are the critical path: the older half therefore
   // issues every load, two wavefronts' worth each, and the younger half none (8192^3: +3.7%; on all-zero
   // data, where the power cap does not hide it, +21%).
-  static constexpr int LDW = NW >= 8 ? NW / 2 : NW;
+  static constexpr bool HALVES = FORM == kFormLineHalves;
+  static constexpr bool LINES = FORM != kFormStraight;
+  static constexpr int GROUPS = HALVES ? 1 : KG;  // rings, and groups that take whole K tiles
+  static constexpr int LDW = HALVES ? (BM % 64 == 0 && BN % 64 == 0 ? 2 * NW : NW) : NW >= 8 ? NW / 2 : NW;
+  static constexpr bool ALL_LOAD = LDW == (HALVES ? 2 * NW : NW);
   static constexpr int NTL = LDW * 64;  // threads that issue loads
   static constexpr int TM = BM / WAVES_M;  // wavefront tile
   static constexpr int TN = BN / WAVES_N;
@@ -374,7 +396,7 @@ struct GemmTile {
   static constexpr int LA = (BM * kChunksPerRow) / NTL;  // buffer loads per wavefront per A tile
   static constexpr int LB = (BN * kChunksPerRow) / NTL;
   static constexpr int LOADS = LA + LB;
-  static constexpr int ROWS = KSTEPS * FM;                 // rows of MFMAs per K tile
+  static constexpr int ROWS = (HALVES ? 1 : KSTEPS) * FM;  // rows of MFMAs per K tile and wavefront
   static constexpr int PER_ROW = (LOADS + ROWS - 1) / ROWS;  // buffer loads issued after each row
   // Loads that may still be in flight when tile h is needed: the A tiles and B tiles beyond h.
   // The side job adds SV buffer stores and SV buffer loads at the end of every K tile of a loader
@@ -383,17 +405,21 @@ struct GemmTile {
   static constexpr bool LOOP = (EPI == kEpiStoreLoop);
   // global stores of one wavefront per tile when its output leaves as whole rows, 16 bytes per lane
   static constexpr int NST = TM * (TN / 8) / 64;
-  static constexpr int SV = NW / LDW;  // side vectors per loader thread per K tile
+  static constexpr int SV = HALVES ? 1 : NW / LDW;  // side vectors per loader thread per K tile
+  static constexpr int LIVE = LINES ? 3 : 2;  // slots not in flight at a K tile's wait: its own (with lines two) and the next to be refilled
   static constexpr int WAIT_STEADY =
-      (AST - 2) * LA + (BST - 2) * LB + (SIDE ? 2 * SV * ((AST < BST ? AST : BST) - 1) : 0);
+      (AST - LIVE) * LA + (BST - LIVE) * LB + (SIDE ? 2 * SV * ((AST < BST ? AST : BST) - 1) : 0);
 
   static_assert(KSTEPS == 2, "the step pipeline below is written for two 32-wide steps per tile");
   static_assert(TM % 16 == 0 && TN % 16 == 0, "wavefront tile must be made of 16x16 blocks");
   static_assert((BM * kChunksPerRow) % NTL == 0 && (BN * kChunksPerRow) % NTL == 0,
                 "every wavefront must move a whole number of 1 KiB chunks per tile");
   static_assert(AST >= 2 && BST >= 2 && (AST == BST || AST == BST + 1), "slot counts");
-  static_assert(KG * LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
-  static_assert(KG == 1 || (NW <= 4 && !SIDE && !LOOP && (KG - 1) * BM * BN * 4 <= KG * LDS_BYTES), "K groups");
+  static_assert(GROUPS * LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
+  static_assert(KG == 1 || (NW <= 4 && !SIDE && !LOOP && (KG - 1) * BM * BN * 4 <= GROUPS * LDS_BYTES), "K groups");
+  static_assert(!HALVES || KG == 2, "two halves of a K tile");
+  static_assert(!LINES || NW == 4, "whole lines: the rows of a thread's fills lie a multiple of 16 apart");
+  static_assert(!LINES || (AST >= 3 && BST >= 3 && !SIDE && !LOOP && !B_KMAJOR), "whole lines");
   static_assert(WAIT_STEADY < 64, "vmcnt range");
   static_assert(BM * 8 * (4 * WAVES_N + 2) <= LDS_BYTES, "row statistics scratch of the LayerNorm epilogues");
 
@@ -491,10 +517,12 @@ struct GemmTile {
   static __device__ __forceinline__ void run(const GemmParams& p, char* smem_base) {
     // K groups: group kg multiplies K tiles kg, kg + KG, ... of the whole output tile with a ring of LDS slots of its own.
     const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
-    char* const smem = smem_base + kg * LDS_BYTES;
+    char* const smem = smem_base + (HALVES ? 0 : kg * LDS_BYTES);
     const int tid = (int)threadIdx.x - kg * NT;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ltid = HALVES ? (int)threadIdx.x : tid;  // among the threads that fill a ring
+    const int lwave = HALVES ? kg * NW + wave : wave;
     const int wm = wave % WAVES_M;
     const int wn = wave / WAVES_M;
 
@@ -544,14 +572,17 @@ struct GemmTile {
     // [K][N] with rows of B that are not whole 16-byte chunks: the last K tile is treated as a short one even if it
     // is whole, because the last row's last chunk must not be fetched as it stands (see load_short_tile).
     const bool n_odd = B_KMAJOR && (N & 7) != 0;
-    int kt_full = klen / kBK;
-    int k_tail = klen - kt_full * kBK;
+    int kt_full = LINES ? (klen + kBK - 1) / kBK : klen / kBK;
+    int k_tail = LINES ? 0 : klen - kt_full * kBK;
     if (n_odd && k_tail == 0 && kt_full > 0) {
       k_tail = kBK;
       --kt_full;
     }
     const int n_all = kt_full + (k_tail ? 1 : 0);  // the short tile, if any, is tile 0
-    const int n_tiles = KG == 1 ? n_all : (n_all - kg + KG - 1) / KG;  // of this group; its tile t is tile t * KG + kg of all
+    // Of this group.  Its tile t is tile t * GROUPS + kg of all; with lines a part of K in one piece, from k_first on.
+    const int k_first = LINES && GROUPS > 1 ? kg * n_all / GROUPS : 0;
+    const int n_tiles = GROUPS == 1 ? n_all : LINES ? (kg + 1) * n_all / GROUPS - k_first : (n_all - kg + GROUPS - 1) / GROUPS;
+    const int n_most = (n_all + GROUPS - 1) / GROUPS;  // of any group
 
     // Buffer descriptors cover exactly the rows of this tile that exist and the K range of
     // this slice; anything else is out of range: reads return zero and touch no memory.
@@ -578,25 +609,54 @@ struct GemmTile {
     };
 
     unsigned voff_a[LA], voff_b[LB];
+    // Whole lines (Form): 16-byte chunks between the start of row r's first line and the row, the same for rows 16 apart.
+    auto phase_of = [&](const T* base, int r) __attribute__((always_inline)) {
+      return LINES ? (int)(((unsigned)(size_t)base + (unsigned)r * (unsigned)K * 2u) & 127u) >> 4 : 0;
+    };
+    // Of the chunks that a thread fetches for an operand: the first fill with one of this group's, and how many.
+    struct Range {
+      int first;
+      unsigned count;
+    };
+    Range range_a{0, 0}, range_b{0, 0};
+    // (Offsets count from a line in front of the rows, so that none is negative; rows that do not exist are out of range by
+    // their own offset.)
+    auto lines_setup = [&](const T* base, int rows, unsigned* voff, int loads) __attribute__((always_inline)) -> Range {
+      const int r = ltid >> 3;
+      const int c = (ltid & 7) ^ swizzle_of_row(r);
+      const int late = c + phase_of(base, r) >= 8 ? 1 : 0;
 #pragma unroll
-    for (int i = 0; i < LA; ++i) voff_a[i] = chunk_voffset(i * NTL + tid, K);
+      for (int i = 0; i < loads; ++i) {
+        const int row = r + i * (NTL / 8);
+        voff[i] = row < rows ? (unsigned)kRowBytes + (unsigned)row * (unsigned)K * 2u + (unsigned)(c - 8 * late) * 16u : kOobOffset;
+      }
+      const int left = (klen >> 3) - 8 * k_first - c;  // chunks from this one on, to the end of K
+      int cnt = left > 0 ? (left + 7) >> 3 : 0;
+      return Range{late, (unsigned)(cnt < n_tiles ? cnt : n_tiles)};
+    };
+    if constexpr (LINES) {
+      range_a = lines_setup(a_base, rows_a, voff_a, LA);
+      range_b = lines_setup(b_base, rows_b, voff_b, LB);
+    }
 #pragma unroll
-    for (int i = 0; i < LB; ++i) {
+    for (int i = 0; i < (LINES ? 0 : LA); ++i) voff_a[i] = chunk_voffset(i * NTL + ltid, K);
+#pragma unroll
+    for (int i = 0; i < (LINES ? 0 : LB); ++i) {
       if (B_KMAJOR) {
         // LDS position q of the stage: row k = q / CPR, and the chunk that lives there is position ^ swizzle
         constexpr int CPR = BN / 8;
-        const int q = i * NTL + tid;
+        const int q = i * NTL + ltid;
         const int k = q / CPR;
         const int chunk = (q % CPR) ^ kmajor_swizzle(k, BN);
         voff_b[i] = ((unsigned)k * (unsigned)N + (unsigned)chunk * 8u) * 2u;
       } else {
-        voff_b[i] = chunk_voffset(i * NTL + tid, K);
+        voff_b[i] = chunk_voffset(i * NTL + ltid, K);
       }
     }
 
     // First K element (inside the slice) of tile t: the short tile comes first.
     auto tile_koff = [&](int t_group) {
-      const int t = t_group * KG + kg;
+      const int t = LINES ? k_first + t_group : GROUPS == 1 ? t_group : t_group * KG + kg;
       return k_tail ? (t == 0 ? kt_full * kBK : (t - 1) * kBK) : t * kBK;
     };
 
@@ -605,13 +665,25 @@ struct GemmTile {
     // of the K range get an empty descriptor: the load is still issued and counted (the pipeline below
     // has no special cases for its last iterations) but touches no memory.
     auto load_a = [&](int i, int t) __attribute__((always_inline)) {
-      char* dst = smem + (t % AST) * A_BYTES + wave * 1024 + i * (NTL * 16);
+      char* dst = smem + (t % AST) * A_BYTES + lwave * 1024 + i * (NTL * 16);
+      if constexpr (LINES) {
+        const __amdgpu_buffer_rsrc_t r = make_rsrc((const char*)a_base - kRowBytes, bytes_a + kRowBytes);
+        const unsigned off = (unsigned)(t - range_a.first) < range_a.count ? voff_a[i] : kOobOffset;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, (int)off, tile_koff(t) * 2, 0, 0);
+        return;
+      }
       const __amdgpu_buffer_rsrc_t r = make_rsrc(a_base, t < n_tiles ? bytes_a : 0u);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16,
                                                (int)voff_a[i], tile_koff(t) * 2, 0, 0);
     };
     auto load_b = [&](int i, int t) __attribute__((always_inline)) {
-      char* dst = smem + B_REGION + (t % BST) * B_BYTES + wave * 1024 + i * (NTL * 16);
+      char* dst = smem + B_REGION + (t % BST) * B_BYTES + lwave * 1024 + i * (NTL * 16);
+      if constexpr (LINES) {
+        const __amdgpu_buffer_rsrc_t r = make_rsrc((const char*)b_base - kRowBytes, bytes_b + kRowBytes);
+        const unsigned off = (unsigned)(t - range_b.first) < range_b.count ? voff_b[i] : kOobOffset;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, (int)off, tile_koff(t) * 2, 0, 0);
+        return;
+      }
       if (B_KMAJOR) {
         // Rows koff .. koff + kBK of the slice, as many as exist: rows past the end of K and the
         // columns past the last row's end are out of range and read as zeros.  (Columns past N in
@@ -641,7 +713,7 @@ struct GemmTile {
     // for the one trip to memory.
     // (A K-major B with whole chunks needs none of this: its rows past the end of K are out of range by themselves.
     // With N % 8 != 0 the chunk that the very last row of B ends inside is fetched the same way.)
-    const bool loader = LDW == NW || wave < LDW;
+    const bool loader = ALL_LOAD || lwave < LDW;
     struct ShortTile {
       i32x4 a[LA], b[LB];
     };
@@ -712,7 +784,14 @@ struct GemmTile {
     // 16x16x32 operand: lane l supplies row (l & 15), K elements 8*(l>>4) .. +7 of the step.
     int frag_off[KSTEPS];
 #pragma unroll
-    for (int kk = 0; kk < KSTEPS; ++kk) frag_off[kk] = lds_offset(lane & 15, 4 * kk + (lane >> 4));
+    for (int kk = 0; kk < KSTEPS; ++kk) frag_off[kk] = lds_offset(lane & 15, 4 * (HALVES ? kg : kk) + (lane >> 4));  // HALVES: the group's half
+    // whole lines: the lanes whose chunk of a K tile arrives with the fill behind that tile's own
+    bool late_a[KSTEPS], late_b[KSTEPS];
+#pragma unroll
+    for (int kk = 0; kk < KSTEPS; ++kk) {
+      late_a[kk] = LINES && 4 * (HALVES ? kg : kk) + (lane >> 4) + phase_of(a_base, lane & 15) >= 8;
+      late_b[kk] = LINES && 4 * (HALVES ? kg : kk) + (lane >> 4) + phase_of(b_base, lane & 15) >= 8;
+    }
     const int a_wave_off = wm * TM * kRowBytes;
     const int b_wave_off = B_KMAJOR ? 0 : wn * TN * kRowBytes;
     // K-major B: a fragment (16 columns x 32 rows of k) is two transposing 8-byte reads.  In the
@@ -932,7 +1011,7 @@ struct GemmTile {
     // second half of tile h-1 (set 1) while reading the first half of tile h into set 0; step 1
     // multiplies set 0 while reading the second half of tile h into set 1.
     bool stores_pending = false;  // kEpiStoreLoop: a store epilogue precedes the tile being started
-    auto tile_body = [&](int h, auto ld_tag, auto w_tag) __attribute__((always_inline)) {
+    auto tile_body = [&](int h, auto ld_tag, auto w_tag, auto par_tag) __attribute__((always_inline)) {
       // my fills of tile h have landed; my reads of tile h-1 are done
       if constexpr (!decltype(ld_tag)::value) {
         wait_lds<0>();  // a wavefront that loads nothing has no fills to wait for
@@ -946,11 +1025,23 @@ struct GemmTile {
       bare_barrier();  // ... and so have everyone else's: the slots of tile h-1 are free
       const char* sa = smem + (h % AST) * A_BYTES + a_wave_off;
       const char* sb = smem + B_REGION + (h % BST) * B_BYTES + b_wave_off;
-      // per-step offset of the B fragments: a swizzled chunk of the row, or 32 rows of k
-      const int sb0 = B_KMAJOR ? 0 : frag_off[0];
-      const int sb1 = B_KMAJOR ? 32 * BN * 2 : frag_off[1];
-      step(sa + frag_off[0], sb + sb0, fa1, fa0, fb1, fb0, h, std::integral_constant<int, 0>{}, ld_tag, w_tag);
-      step(sa + frag_off[1], sb + sb1, fa0, fa1, fb0, fb1, h, std::integral_constant<int, FM>{}, ld_tag, w_tag);
+      // where a step reads: a swizzled chunk of the row (whole lines: in the fill that holds it), or 32 rows of k
+      auto a_at = [&](int kk) __attribute__((always_inline)) -> const char* {
+        if constexpr (LINES) return smem + (late_a[kk] ? ((h + 1) % AST) * A_BYTES : (h % AST) * A_BYTES) + (a_wave_off + frag_off[kk]);
+        return sa + frag_off[kk];
+      };
+      auto b_at = [&](int kk) __attribute__((always_inline)) -> const char* {
+        if constexpr (LINES) return smem + (B_REGION + (late_b[kk] ? ((h + 1) % BST) * B_BYTES : (h % BST) * B_BYTES)) + (b_wave_off + frag_off[kk]);
+        return sb + (B_KMAJOR ? kk * (32 * BN * 2) : frag_off[kk]);
+      };
+      if constexpr (HALVES) {
+        // this group's half of tile h is read while its half of tile h - 1 is multiplied
+        if constexpr (decltype(par_tag)::value == 0) step(a_at(0), b_at(0), fa1, fa0, fb1, fb0, h, std::integral_constant<int, 0>{}, ld_tag, w_tag);
+        else step(a_at(0), b_at(0), fa0, fa1, fb0, fb1, h, std::integral_constant<int, 0>{}, ld_tag, w_tag);
+      } else {
+        step(a_at(0), b_at(0), fa1, fa0, fb1, fb0, h, std::integral_constant<int, 0>{}, ld_tag, w_tag);
+        step(a_at(1), b_at(1), fa0, fa1, fb0, fb1, h, std::integral_constant<int, FM>{}, ld_tag, w_tag);
+      }
       if constexpr (SIDE && decltype(ld_tag)::value) {
         side_store(h, w_tag);
         side_load(h + 1, w_tag);
@@ -977,7 +1068,7 @@ struct GemmTile {
         }
       };
       if constexpr (!LOOP) {  // (no short tile there: the host sees to it; its registers would not fit beside the accumulators)
-        if (k_tail && loader && kg == 0) {
+        if (!LINES && k_tail && loader && kg == 0) {
           ShortTile st;
           load_short_tile(st, k_tail);
           fills(std::true_type{});
@@ -994,24 +1085,40 @@ struct GemmTile {
       // two straight-line versions of the loop, with and without the loads: a branch around every load
       // would cut each row of MFMAs into several scheduling regions
       // (and the side job one version per unit width: the unit's elements are dealt to rows at compile time)
-      if constexpr (SIDE) {
-        if (!loader) {
-          for (int h = 0; h < n_tiles; ++h) tile_body(h, std::false_type{}, W16{});
-        } else if (p.side_width == 16) {
-          for (int h = 0; h < n_tiles; ++h) tile_body(h, std::true_type{}, W16{});
-        } else if (p.side_width == 8) {
-          for (int h = 0; h < n_tiles; ++h) tile_body(h, std::true_type{}, W8{});
+      using Even = std::integral_constant<int, 0>;
+      using Odd = std::integral_constant<int, 1>;
+      auto loop = [&](auto ld_tag, auto w_tag) __attribute__((always_inline)) {
+        if constexpr (HALVES) {
+          int h = 0;
+          for (; h + 1 < n_tiles; h += 2) {
+            tile_body(h, ld_tag, w_tag, Even{});
+            tile_body(h + 1, ld_tag, w_tag, Odd{});
+          }
+          if (h < n_tiles) {
+            tile_body(h, ld_tag, w_tag, Even{});
+            // the drain takes set 1
+#pragma unroll
+            for (int i = 0; i < FM; ++i) fa1[i] = fa0[i];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) fb1[j] = fb0[j];
+          }
         } else {
-          for (int h = 0; h < n_tiles; ++h) tile_body(h, std::true_type{}, W4{});
+          for (int h = 0; h < n_tiles; ++h) tile_body(h, ld_tag, w_tag, Even{});
         }
-      } else if constexpr (LDW == NW) {
-        for (int h = 0; h < n_tiles; ++h) tile_body(h, std::true_type{}, W16{});
+      };
+      if constexpr (SIDE) {
+        if (!loader) loop(std::false_type{}, W16{});
+        else if (p.side_width == 16) loop(std::true_type{}, W16{});
+        else if (p.side_width == 8) loop(std::true_type{}, W8{});
+        else loop(std::true_type{}, W4{});
+      } else if constexpr (ALL_LOAD) {
+        loop(std::true_type{}, W16{});
       } else if (loader) {
-        for (int h = 0; h < n_tiles; ++h) tile_body(h, std::true_type{}, W16{});
+        loop(std::true_type{}, W16{});
       } else {
-        for (int h = 0; h < n_tiles; ++h) tile_body(h, std::false_type{}, W16{});
+        loop(std::false_type{}, W16{});
       }
-      if (KG > 1 && n_tiles < (n_all + KG - 1) / KG) bare_barrier();  // the other groups' last tile
+      if (GROUPS > 1 && n_tiles < n_most) bare_barrier();  // the other groups' last tile
       wait_vm_and_lds<0>();  // the empty fills of the last iterations must be gone before LDS is reused
       // Drain: the second half of the last tile is in set 1.
       if constexpr (B_KMAJOR) {
@@ -1040,7 +1147,7 @@ struct GemmTile {
         else side_load(0, W4{});
       }
       if constexpr (!LOOP) k_loop_and_drain();
-    } else if (KG > 1 && n_all > 0) {
+    } else if (GROUPS > 1 && n_all > 0) {
       bare_barrier();
     }
     if constexpr (KG > 1) {
@@ -1504,11 +1611,11 @@ struct GemmTile {
 // 128 x 64 wavefronts 20.0 -> 17.3, in 128 x 256 tiles of 64 x 128 20.2 -> 17.2, 1024^3 5.27 -> 5.11.
 constexpr int min_waves_per_simd(int TM, int TN) { return TM * TN <= 32 * 256 ? 2 : 1; }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false, int KG = 1>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int AST, int BST, bool B_KMAJOR = false, int KG = 1, int FORM = 0>
 __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64 * KG, (KG > 2 ? KG : min_waves_per_simd(BM / WAVES_M, BN / WAVES_N)))
     gemmrc_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  GemmTile<T, BM, BN, WAVES_M, WAVES_N, EPI, AST, BST, B_KMAJOR, KG>::run(p, smem);
+  GemmTile<T, BM, BN, WAVES_M, WAVES_N, EPI, AST, BST, B_KMAJOR, KG, FORM>::run(p, smem);
 }
 
 }  // namespace beam

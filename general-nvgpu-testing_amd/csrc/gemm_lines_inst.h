@@ -1,0 +1,26 @@
+// The tiles of gemm_kernel.h whose fills take whole 128-byte lines, and their launcher, for one element type (BEAM_T).
+#include "kernel_set.h"
+
+namespace beam {
+
+template <int BM, int BN, int S, int KG, int FORM>
+static hipError_t launch_lines_t(const GemmParams& p, dim3 grid, hipStream_t stream) {
+  using Tile = GemmTile<BEAM_T, BM, BN, 2, 2, kEpiStore, S, S, false, KG, FORM>;
+  auto kern = gemmrc_kernel<BEAM_T, BM, BN, 2, 2, kEpiStore, S, S, false, KG, FORM>;
+  static std::atomic<unsigned long long> configured{0};
+  constexpr int LDS = Tile::GROUPS * Tile::LDS_BYTES;
+  if (hipError_t e = allow_lds_once(configured, reinterpret_cast<const void*>(kern), LDS); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, grid, dim3(KG * Tile::NT), LDS, stream, p);
+  return hipGetLastError();
+}
+
+template <>
+hipError_t launch_gemm_lines<BEAM_T>(int block_m, int block_n, const GemmParams& p, dim3 grid, hipStream_t stream) {
+#define BEAM_LINES(BM, BN, S, KG, FORM) \
+  if (block_m == BM && block_n == BN) return launch_lines_t<BM, BN, S, KG, FORM>(p, grid, stream);
+  BEAM_FOR_EACH_LINES_TILE(BEAM_LINES)
+#undef BEAM_LINES
+  return hipErrorInvalidValue;
+}
+
+}  // namespace beam

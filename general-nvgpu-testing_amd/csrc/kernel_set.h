@@ -185,6 +185,21 @@ template <> hipError_t launch_gemm_kwave<_Float16>(const KwPlan&, const KwParams
 template <> hipError_t launch_gemm_kwave<__bf16>(const KwPlan&, const KwParams&, bool, hipStream_t);
 template <> hipError_t launch_gemm_kwave_ln<_Float16>(const KwPlan&, const KwLnParams&, hipStream_t);
 template <> hipError_t launch_gemm_kwave_ln<__bf16>(const KwPlan&, const KwLnParams&, hipStream_t);
+// The tiles of gemm_kernel.h whose fills take whole 128-byte lines (Form), 2 x 2 wavefronts a group: (workgroup tile M, N, LDS
+// slots of each operand, K groups, Form).  Needs K % 8 == 0 and A and B ([N][K]) on 16 bytes.
+#define BEAM_FOR_EACH_LINES_TILE(X)      \
+  X(64, 64, 5, 2, kFormLines)            \
+  X(96, 64, 4, 2, kFormLines)            \
+  X(64, 128, 6, 2, kFormLineHalves)      \
+  X(128, 64, 6, 2, kFormLineHalves)      \
+  X(96, 128, 5, 2, kFormLineHalves)      \
+  X(128, 128, 5, 2, kFormLineHalves)     \
+  X(160, 128, 4, 1, kFormLines)          \
+  X(192, 128, 4, 2, kFormLineHalves)
+template <typename T>
+hipError_t launch_gemm_lines(int block_m, int block_n, const GemmParams& p, dim3 grid, hipStream_t stream);
+template <> hipError_t launch_gemm_lines<_Float16>(int, int, const GemmParams&, dim3, hipStream_t);
+template <> hipError_t launch_gemm_lines<__bf16>(int, int, const GemmParams&, dim3, hipStream_t);
 // Measurement only: the split-K partial kernel of the 64 x 128 (wave 32 x 64) or 64 x 64 (wave 32 x 32) tile, deep
 // pipeline, fp16, with its loads and fragment reads but no MFMAs and no stores (kEpiProbeLoads); hipErrorInvalidValue
 // for any other tile.

@@ -615,7 +615,9 @@ int cli_bench(const Args& a) {
   if (own_tile && !ln_two_pass)
     (void)beam_dbg_small_tile(op == BEAM_OP_MATMUL_NN ? 1 : op == BEAM_OP_GEMM_LN ? 3 : 0, M, N, K, K % 64 == 0 ? 2 : K % 8 == 0 ? 1 : 0, &rows,
                               &cols, &waves, &lines);
-  if (own_tile && op == BEAM_OP_GEMM && cfg.pipeline == 2 && cfg.block_m == 128 && cfg.block_n == 128 && cfg.wave_n == 32) cfg.wave_n = 64;
+  const bool off_lines = own_tile && op == BEAM_OP_GEMM && rows == 0 && K >= 8 && K % 8 == 0 && K % 64 != 0;
+  if (off_lines) (void)beam_dbg_off_lines_tile(M, N, K, &cfg, &lines);
+  else if (own_tile && op == BEAM_OP_GEMM && cfg.pipeline == 2 && cfg.block_m == 128 && cfg.block_n == 128 && cfg.wave_n == 32) cfg.wave_n = 64;
   int rc = time_op(op, p, own_tile ? nullptr : &cfg, split, a.num("warmup", 5), a.num("iters", 20), &ms, ln_mode);
   if (rc != BEAM_OK) {
     std::fprintf(stderr, "bench failed (%d): %s\n", rc, beam_last_error());
@@ -626,8 +628,8 @@ int cli_bench(const Args& a) {
                 dtype ? "bf16" : "fp16", rows, cols, waves, lines ? ", whole lines" : "", ms, 2.0 * M * N * K / ms / 1e9);
     return 0;
   }
-  std::printf("%s %dx%dx%d %s tile %dx%d wave %dx%d pipeline %d group %d split %d: %.4f ms  %.1f TFLOP/s\n",
-              opname.c_str(), M, N, K, dtype ? "bf16" : "fp16", cfg.block_m, cfg.block_n, cfg.wave_m, cfg.wave_n,
+  std::printf("%s %dx%dx%d %s tile %dx%d wave %dx%d%s pipeline %d group %d split %d: %.4f ms  %.1f TFLOP/s\n",
+              opname.c_str(), M, N, K, dtype ? "bf16" : "fp16", cfg.block_m, cfg.block_n, cfg.wave_m, cfg.wave_n, lines ? " whole lines" : "",
               cfg.pipeline, cfg.group_m, split, ms, 2.0 * M * N * K / ms / 1e9);
   return 0;
 }

@@ -69,6 +69,10 @@ size_t beam_dbg_ln_plan_bytes(int M, int N, int K, const beam_tile_cfg* cfg, int
  * 3 beam_gemmrc_ln's one-kernel form.  row_starts, of every row of A (and of B as [N][K]): 0 at an element, 1 on 16 bytes
  * (K % 8 == 0), 2 on 128 (K % 64 == 0).  Before a device has been probed, of one with 256 CUs. */
 int beam_dbg_small_tile(int op, int M, int N, int K, int row_starts, int* rows, int* cols, int* waves, int* whole_lines);
+/* The tile that beam_gemmrc without one runs on where beam_dbg_small_tile says none and the rows of A and B start on 16 bytes
+ * but not on 128 (K % 64 != 0), and whether its fills take whole 128-byte lines (*whole_lines = 1: such a tile need not be in
+ * beam_get_config's table). */
+int beam_dbg_off_lines_tile(int M, int N, int K, beam_tile_cfg* cfg, int* whole_lines);
 /* A measurement, off by default: on != 0 makes the one-launch split-K run without reducing workgroups wherever its
  * multiplying workgroups fit one round of the CUs; the workgroup of (tile, slice s) then adds parts s, s + slices, ...
  * of its tile itself.  Same bits.  Unlike the shipped form this needs every workgroup of the launch resident at once

@@ -1,0 +1,44 @@
+"""Tiles whose fills of LDS take whole 128-byte lines of memory (gemm_kernel.h: Form), as calls without a tile reach them: rows
+off lines but on 16-byte chunks.  Shapes end inside a tile in both directions; K is one chunk, ends with and just behind a K tile,
+has fewer K tiles than groups and slots, and many; rows take every phase (an operand may itself start behind a line).  Operands
+lie inside buffers of NaNs.  That the calls reach those tiles is a test of its own.  Bounds: close_enough's."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from test_gpu_edges import close_enough
+from test_gpu_gemm import BF16, F16
+from test_gpu_unaligned import run
+from test_host_logic import small_tile
+
+pytestmark = pytest.mark.gpu
+
+KS = [8, 56, 72, 136, 328, 1096, 2008, 3208]
+# A shape for each tile, its choice for K from 1096 on
+TILES = {(64, 64): (1000, 1000), (96, 64): (2913, 464), (64, 128): (329, 4648), (128, 64): (1271, 1592), (96, 128): (1477, 2024),
+         (128, 128): (399, 7968), (160, 128): (633, 6536), (192, 128): (760, 6536)}
+
+
+def off_lines_tile(beamc, M, N, K):
+    tile, lines = beamc._TileCfg(), ctypes.c_int()
+    beamc._check(beamc.lib.beam_dbg_off_lines_tile(M, N, K, ctypes.byref(tile), ctypes.byref(lines)))
+    return (tile.block_m, tile.block_n), lines.value
+
+
+def test_calls_reach_the_tiles_that_they_are_named_after(gpu, beamc):
+    assert gpu["compute_units"] == 256
+    for tile, (M, N) in TILES.items():
+        for K in (K for K in KS if K >= 1096):
+            assert small_tile(beamc, 0, M, N, K, 1)[0] == 0 and off_lines_tile(beamc, M, N, K) == (tile, 1), (tile, K)
+
+
+@pytest.mark.parametrize("tile", sorted(TILES))
+@pytest.mark.parametrize("K", KS)
+def test_gemmrc(gpu, beamc, oracle, tile, K):
+    L = beamc.lib
+    M, N = TILES[tile]
+    dtype, offsets = ((F16, (0, 0, 0)), (BF16, (8, 24, 1)), (F16, (24, 16, 3)), (BF16, (0, 8, 0)))[KS.index(K) % 4]
+    a, b = beamc.host_uniform((M, K), dtype, 71, 0), beamc.host_uniform((N, K), dtype, 71, 1)
+    out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offsets)
+    close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"{tile} {(M, N, K)} at {offsets}")
