@@ -232,16 +232,20 @@ GemmParams base_params(const void* A, const void* B, int M, int N, int K, const 
 //     4096 x 8136 x 1024 in 256 x 256 tiles 70 -> 63, 79 -> 68; 8192 x 8136 x 256 in 128 x 128 106 -> 71).  Below: 2048 x 1992 x
 //     1024 in 128 x 128 tiles 11.6, cached 12.0.
 //   * 256 x 256 tiles of eight wavefronts over several rounds, one workgroup per tile, wherever rows start (4096 x 8192 x 256
-//     50 -> 34, x 1024 64 -> 62).
+//     50 -> 34, x 1024 64 -> 62; not LayerNorm's, 8192 x 8192 x 1024 143, 147).
+//   * Rows on 32 bytes: of these only gemm_w4.h's (4096 x 4048 x 1024 33.7 -> 29.9) and the wide tiles of a plain product (5000 x
+//     5008 x 1000 54.5 -> 53.8); 64 columns 1024 x 2000 x 256 4.46, cached 4.53, LayerNorm 4385 x 5232 x 392 41.9, 44.3.
 // (Non-temporal stores are faster still by themselves, 8192 x 8192 x 1024 in 128 x 128 tiles 161 -> 126 us, but only put the
 // cost off: with a kernel that reads the output behind it, 4096 x 4096 x 1024 takes 54.3 us written through, 56.2 so.)
-int store_kind(const beam_tile_cfg& c, int wavefronts, bool w4, const void* C, int M, int N) {
+int store_kind(const beam_tile_cfg& c, int wavefronts, bool w4, const void* C, int M, int N, bool ln = false) {
   const size_t bytes = (size_t)M * N * 2;
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
-  if (!w4 && wavefronts == 8 && c.block_m * c.block_n == 256 * 256 &&
+  if (!w4 && !ln && wavefronts == 8 && c.block_m * c.block_n == 256 * 256 &&
       (long)((M + 255) / 256) * ((N + 255) / 256) > cus) return kStoreCached;
   if (N % 32 == 0 && ((uintptr_t)C & 63) == 0) return kStoreThrough;
-  return w4 || c.block_n == 64 || bytes >= ((size_t)20 << 20) ? kStoreCached : kStoreThrough;
+  if (w4) return kStoreCached;
+  if (N % 16 == 0 && ((uintptr_t)C & 31) == 0 && (ln || c.block_n == 64)) return kStoreThrough;
+  return c.block_n == 64 || bytes >= ((size_t)20 << 20) ? kStoreCached : kStoreThrough;
 }
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -1525,7 +1529,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   // K == 0: the kernels run with an empty K range and produce x = 0, i.e. y = beta.
   if (plan.kind == LnPlan::kFused) {
     p.C = Y;
-    p.c_store = store_kind(c, ks->threads / 64, plan.w4, Y, M, N);
+    p.c_store = store_kind(c, ks->threads / 64, plan.w4, Y, M, N, true);
     // Launches that share a workspace must be ordered (same stream): overlapping ones would race on the sets.
     const size_t set_bytes = ln_fused_set_bytes(p.tiles_m, p.tiles_n, c.block_m);
     float* sets = (float*)((char*)ws + ln_fused_header_bytes());
