@@ -577,11 +577,11 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
 // to 8192 and K from 64 to 8192 off lines.  Its pick is 1.0% (worst 18%) behind the best of these on average, 1.5% on
 // shapes that it was not fitted to; what ran before was 10% behind.  us, before -> now: 928 x 1232 x 7112 49.7 -> 27.9, 633 x
 // 6536 x 2952 38.5 -> 26.3, 1228 x 1784 x 6296 59.4 -> 36.9, 7702 x 7248 x 2472 268 -> 255, 2247 x 3736 x 216 12.7 -> 10.3.
-struct OffLinesTile {
+struct LineChoice {
   beam_tile_cfg cfg;
-  bool lines;
+  bool lines;  // cfg is a tile of launch_gemm_lines
 };
-OffLinesTile off_lines_tile(int M, int N, int K, int cus) {
+LineChoice off_lines_tile(int M, int N, int K, int cus) {
   struct Candidate {
     beam_tile_cfg cfg;
     bool lines;
@@ -629,7 +629,7 @@ OffLinesTile off_lines_tile(int M, int N, int K, int cus) {
     if (!k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline) stays = &k, stays_us = us;
   }
   if (stays && best_us > 0.96 * stays_us) best = stays;
-  OffLinesTile t = {best->cfg, best->lines};
+  LineChoice t = {best->cfg, best->lines};
   t.cfg.group_m = default_group_m(t.cfg.block_m, t.cfg.block_n);
   return t;
 }
@@ -693,7 +693,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   const KernelSet* ks;
   const bool off_lines = !cfg && K % kBK != 0 && row_starts(A, B, K, false) == kOnChunks;
   if (off_lines) {
-    const OffLinesTile t = off_lines_tile(M, N, K, cus);
+    const LineChoice t = off_lines_tile(M, N, K, cus);
     c = t.cfg;
     if (t.lines) {
       GemmParams p = base_params(A, B, M, N, K, c);
@@ -1302,6 +1302,63 @@ static int ln_resolve_cfg(const beam_tile_cfg* cfg, int M, int N, int K, int mod
   return BEAM_OK;
 }
 
+// The one-kernel form among all tiles, those whose fills take whole lines (gemm_kernel.h: Form) included, for rows on 16 bytes;
+// `named` is ln_choose_tile's.  The model above with constants for rows on 128-byte lines and off them: TFLOP/s per CU, us per
+// round of bands and per launch, least squares on the logarithm over 160 and 200 shapes with M from 64 to 8192, N and K from 256 to 8192.
+// `named` stays unless another tile is 4% ahead by it.  Its pick is 1.8% (off lines) and 3.3% (on) behind the best tile on
+// average, `named` 12 and 11%; the tiles with rings deeper than 3 + 2 slots are ahead on lines too.  us, before -> now: 1978 x 2120 x
+// 4888 86 -> 59, 2908 x 328 x 5736 51 -> 33, 1891 x 920 x 3704 40 -> 28, 6257 x 2744 x 4688 243 -> 196; on lines 1064 x 1040 x
+// 3776 42 -> 29, 126 x 6720 x 1472 21.6 -> 19.0.
+static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) {
+  struct Candidate {
+    beam_tile_cfg cfg;
+    bool lines;
+    double rate[2], round[2], launch[2];  // rows off lines, on lines
+  };
+  static const Candidate kCandidates[] = {
+      {{256, 256, 128, 128, 0, 0}, false, {0, 7.60}, {0, 14.89}, {0, 0}},  // (only where it is `named`)
+      {{256, 256, 128, 64, 0, 0}, false, {6.99, 7.79}, {16.42, 16.95}, {0, 0}},
+      {{224, 256, 112, 64, 0, 0}, false, {6.59, 7.53}, {14.53, 15.39}, {0, 0}},
+      {{192, 256, 96, 64, 0, 0}, false, {6.05, 7.19}, {13.07, 14.04}, {0, 0}},
+      {{256, 128, 64, 64, 0, 0}, false, {4.84, 6.41}, {11.32, 12.29}, {0, 0}},
+      {{128, 256, 64, 64, 0, 0}, false, {4.53, 5.74}, {9.83, 10.90}, {0, 0}},
+      {{128, 128, 64, 32, 0, 0}, false, {3.77, 4.50}, {4.72, 4.60}, {4.29, 4.99}},
+      {{64, 128, 32, 64, 0, 0}, false, {2.29, 2.59}, {2.04, 2.03}, {5.90, 6.00}},
+      {{64, 64, 32, 32, 0, 0}, false, {1.67, 2.10}, {1.00, 1.05}, {6.00, 6.00}},
+      {{96, 64, 48, 32, 2, 0}, true, {3.32, 3.30}, {9.20, 9.03}, {0, 0}},
+      {{64, 128, 32, 64, 2, 0}, true, {3.70, 3.58}, {9.48, 9.51}, {0, 0}},
+      {{128, 64, 64, 32, 2, 0}, true, {3.55, 3.61}, {10.07, 9.82}, {0, 0}},
+      {{96, 128, 48, 64, 2, 0}, true, {4.52, 4.28}, {11.08, 10.91}, {0, 0}},
+      {{128, 128, 64, 64, 2, 0}, true, {5.24, 5.08}, {12.33, 12.32}, {0, 0}},
+      {{160, 128, 80, 64, 2, 0}, true, {5.91, 5.77}, {12.13, 12.24}, {0, 0}},
+      {{192, 128, 96, 64, 2, 0}, true, {6.41, 6.03}, {15.03, 14.95}, {0, 0}},
+  };
+  const int on = K % kBK == 0 ? 1 : 0;
+  const Candidate *best = nullptr, *stays = nullptr;
+  double best_us = 0, stays_us = 0;
+  for (const Candidate& k : kCandidates) {
+    const beam_tile_cfg& t = k.cfg;
+    const bool is_named = !k.lines && t.block_m == named.block_m && t.block_n == named.block_n && t.wave_n == named.wave_n;
+    if (t.wave_m == 128 && t.wave_n == 128 && !is_named) continue;
+    const int tiles_m = (M + t.block_m - 1) / t.block_m, tiles_n = (N + t.block_n - 1) / t.block_n;
+    if (tiles_n > 64 || k.rate[on] == 0) continue;
+    if (!k.lines) {
+      beam_tile_cfg c;
+      const KernelSet* ks;
+      if (resolve_cfg(&t, M, N, K, &c, &ks) || !ln_fused_applies_on(c, *ks, N, kNumXcd * 32)) continue;
+    }
+    const int bands_per_round = kNumXcd * 32 / tiles_n;
+    const double us = k.launch[on] + (double)((tiles_m + bands_per_round - 1) / bands_per_round) *
+                                         (k.round[on] + 2.0e-6 * t.block_m * t.block_n * (double)(((long)K + kBK - 1) / kBK * kBK) / k.rate[on]);
+    if (!best || us < best_us) best = &k, best_us = us;
+    if (is_named) stays = &k, stays_us = us;
+  }
+  if (!best || (stays && best_us > 0.96 * stays_us)) return LineChoice{named, false};
+  LineChoice c = {best->cfg, best->lines};
+  c.cfg.group_m = default_group_m(c.cfg.block_m, c.cfg.block_n);
+  return c;
+}
+
 // What a GEMM+LayerNorm call does and the workspace it needs: one function, so that the entry point and the
 // workspace queries cannot disagree.
 //   plain     the problem is outside what the tiled kernels take (K below 8 or beyond a descriptor, gamma or beta not
@@ -1317,6 +1374,7 @@ struct LnPlan {
   beam_tile_cfg c;
   const KernelSet* ks;
   bool w4;    // fused, on the kernel of gemm_w4.h
+  bool lines;  // fused, in a tile whose fills take whole lines (ks then says nothing)
   KwPlan kw;  // fused, on the kernel of gemm_kwave.h if kw.rows != 0 (c and ks then say nothing)
   size_t need;
 };
@@ -1330,6 +1388,7 @@ static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool
                    LnPlan* out) {
   out->ks = nullptr;
   out->w4 = false;
+  out->lines = false;
   out->kw = KwPlan{0, 0, 0, false};
   if (plain) {
     out->kind = LnPlan::kPlain;
@@ -1351,6 +1410,19 @@ static int ln_plan(int M, int N, int K, const beam_tile_cfg* cfg, int mode, bool
     return BEAM_OK;
   }
   if (rc) return rc;
+  if (!cfg && mode != BEAM_LN_TWOPASS && !unaligned && K >= 8 && K % 8 == 0 && g_dev.cus == kNumXcd * 32) {
+    const LineChoice t = ln_line_tile(M, N, K, c);
+    if (t.lines) {
+      c = t.cfg;
+      out->ks = nullptr;
+      out->lines = true;
+      out->kind = LnPlan::kFused;
+      out->need = ln_fused_need(M, N, c.block_m, c.block_n);
+      return BEAM_OK;
+    }
+    c = t.cfg;
+    if ((rc = resolve_cfg(&c, M, N, K, &c, &out->ks))) return rc;
+  }
   if (mode == BEAM_LN_FUSED && !ln_fused_applies(c, *out->ks, N))
     return fail(BEAM_ERR_UNSUPPORTED, "fused LayerNorm: needs a device of %d CUs and at most 64 column tiles (N=%d, block_n=%d, %d CUs)",
                 kNumXcd * 32, N, c.block_n, g_dev.cus);
@@ -1391,7 +1463,12 @@ size_t beam_gemmrc_ln_workspace_bytes_for(int M, int N, int K, const beam_tile_c
   (void)beam_init();  // AUTO depends on the device
   LnPlan eager, captured;
   if (ln_plan(M, N, K, cfg, mode, false, false, false, true, &eager)) return 0;
-  if (mode != BEAM_LN_AUTO) return eager.need;
+  if (mode != BEAM_LN_AUTO) {
+    // rows off 16 bytes have a tile of their own choice, and more column tiles perhaps
+    LnPlan off;
+    if (ln_plan(M, N, K, cfg, mode, false, true, false, true, &off) == BEAM_OK && off.kind == eager.kind && off.need > eager.need) return off.need;
+    return eager.need;
+  }
   if (ln_plan(M, N, K, cfg, mode, false, false, true, true, &captured)) return eager.need;
   return eager.need > captured.need ? eager.need : captured.need;
 }
@@ -1417,6 +1494,11 @@ size_t beam_gemmrc_ln_workspace_bytes_ex(int M, int N, const beam_tile_cfg* cfg,
     if (mode == BEAM_LN_AUTO) take(ln_workspace_need(M, N, c, BEAM_LN_TWOPASS));
   }
   if (const KwPlan kw = ln_kw_plan(M, N, 1024, cfg, mode); kw.rows) take(ln_fused_need(M, N, kw.rows, kw.cols));
+  if (mode != BEAM_LN_TWOPASS) {
+#define BEAM_LINES(BM, BN, S, KG, FORM) if ((N + BN - 1) / BN <= 64) take(ln_fused_need(M, N, BM, BN));
+    BEAM_FOR_EACH_LINES_TILE(BEAM_LINES)
+#undef BEAM_LINES
+  }
   return need;
 }
 
@@ -1450,7 +1532,7 @@ int beam_dbg_small_tile(int op, int M, int N, int K, int row_starts, int* rows, 
 
 int beam_dbg_off_lines_tile(int M, int N, int K, beam_tile_cfg* cfg, int* whole_lines) {
   if (M <= 0 || N <= 0 || K < 8 || !cfg || !whole_lines) return fail(BEAM_ERR_INVALID, "null pointer or empty problem");
-  const OffLinesTile t = off_lines_tile(M, N, K, g_dev.cus > 0 ? g_dev.cus : 256);
+  const LineChoice t = off_lines_tile(M, N, K, g_dev.cus > 0 ? g_dev.cus : 256);
   *cfg = t.cfg;
   *whole_lines = t.lines ? 1 : 0;
   return BEAM_OK;
@@ -1529,7 +1611,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   // K == 0: the kernels run with an empty K range and produce x = 0, i.e. y = beta.
   if (plan.kind == LnPlan::kFused) {
     p.C = Y;
-    p.c_store = store_kind(c, ks->threads / 64, plan.w4, Y, M, N, true);
+    p.c_store = store_kind(c, plan.lines ? 4 : ks->threads / 64, plan.w4, Y, M, N, true);
     // Launches that share a workspace must be ordered (same stream): overlapping ones would race on the sets.
     const size_t set_bytes = ln_fused_set_bytes(p.tiles_m, p.tiles_n, c.block_m);
     float* sets = (float*)((char*)ws + ln_fused_header_bytes());
@@ -1591,6 +1673,11 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
       const unsigned cus = (unsigned)g_dev.cus;
       const bool walk = grid > cus && p.tiles_n <= kW4LnCompactTiles && !g_ln_no_walk.load(std::memory_order_relaxed);
       BEAM_HIP(launch_gemm_w4_ln(p, dtype, dim3(walk ? cus : grid, 1, 1), st));
+      return BEAM_OK;
+    }
+    if (plan.lines) {
+      BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_lines_ln<_Float16>(c.block_m, c.block_n, p, dim3(grid, 1, 1), st)
+                                 : launch_gemm_lines_ln<__bf16>(c.block_m, c.block_n, p, dim3(grid, 1, 1), st));
       return BEAM_OK;
     }
     BEAM_HIP(ks->launch[dtype][kEpiLnFused][c.pipeline](p, dim3(grid, 1, 1), st));
@@ -1953,6 +2040,17 @@ int beam_dbg_ln_default_config(int M, int N, int K, int compute_units, beam_tile
   if (!cfg || M <= 0 || N <= 0 || K <= 0) return fail(BEAM_ERR_INVALID, "bad argument");
   const KernelSet* ks = nullptr;
   return ln_choose_tile(M, N, K, compute_units, cfg, &ks) ? BEAM_OK : BEAM_ERR_UNSUPPORTED;
+}
+
+int beam_dbg_ln_line_tile(int M, int N, int K, beam_tile_cfg* cfg, int* whole_lines) {
+  beam_tile_cfg named;
+  const KernelSet* ks;
+  if (M <= 0 || N <= 0 || K < 8 || K % 8 != 0 || !cfg || !whole_lines) return fail(BEAM_ERR_INVALID, "null pointer or not a problem on 16-byte rows");
+  if (!ln_choose_tile(M, N, K, kNumXcd * 32, &named, &ks)) return fail(BEAM_ERR_UNSUPPORTED, "no one-kernel form for N=%d", N);
+  const LineChoice t = ln_line_tile(M, N, K, named);
+  *cfg = t.cfg;
+  *whole_lines = t.lines ? 1 : 0;
+  return BEAM_OK;
 }
 
 int beam_dbg_w4_kmajor_swizzle(int k) { return w4_kmajor_swizzle(k); }

@@ -198,7 +198,12 @@ template <> hipError_t launch_gemm_kwave_ln<__bf16>(const KwPlan&, const KwLnPar
   X(192, 128, 4, 2, kFormLineHalves)
 template <typename T>
 hipError_t launch_gemm_lines(int block_m, int block_n, const GemmParams& p, dim3 grid, hipStream_t stream);
+// GEMM+LayerNorm in one launch: parameters as for the kEpiLnFused kernels.
+template <typename T>
+hipError_t launch_gemm_lines_ln(int block_m, int block_n, const GemmParams& p, dim3 grid, hipStream_t stream);
 template <> hipError_t launch_gemm_lines<_Float16>(int, int, const GemmParams&, dim3, hipStream_t);
+template <> hipError_t launch_gemm_lines_ln<_Float16>(int, int, const GemmParams&, dim3, hipStream_t);
+template <> hipError_t launch_gemm_lines_ln<__bf16>(int, int, const GemmParams&, dim3, hipStream_t);
 template <> hipError_t launch_gemm_lines<__bf16>(int, int, const GemmParams&, dim3, hipStream_t);
 // Measurement only: the split-K partial kernel of the 64 x 128 (wave 32 x 64) or 64 x 64 (wave 32 x 32) tile, deep
 // pipeline, fp16, with its loads and fragment reads but no MFMAs and no stores (kEpiProbeLoads); hipErrorInvalidValue

@@ -605,9 +605,11 @@ int cli_bench(const Args& a) {
   // line below names what that picks for a device of 256 CUs).  Split-K: the tile that goes with the library's slice count.
   const bool own_tile = (op == BEAM_OP_GEMM || op == BEAM_OP_MATMUL_NN || op == BEAM_OP_GEMM_LN) && !a.has("tile") && !a.has("wave") &&
                         !a.has("pipeline") && !a.has("group");
+  int ln_lines = 0;
   if (own_tile && op == BEAM_OP_GEMM_LN && ln_mode != BEAM_LN_TWOPASS) {
     beam_tile_cfg picked;
     if (beam_dbg_ln_default_config(M, N, K, 256, &picked) == BEAM_OK) cfg = picked;
+    if (K >= 8 && K % 8 == 0) (void)beam_dbg_ln_line_tile(M, N, K, &cfg, &ln_lines);
   }
   // ... and the small tile or the wavefronts that beam_gemmrc takes instead of the tile named (operands of their own start on lines)
   int rows = 0, cols = 0, waves = 0, lines = 0;
@@ -629,7 +631,7 @@ int cli_bench(const Args& a) {
     return 0;
   }
   std::printf("%s %dx%dx%d %s tile %dx%d wave %dx%d%s pipeline %d group %d split %d: %.4f ms  %.1f TFLOP/s\n",
-              opname.c_str(), M, N, K, dtype ? "bf16" : "fp16", cfg.block_m, cfg.block_n, cfg.wave_m, cfg.wave_n, lines ? " whole lines" : "",
+              opname.c_str(), M, N, K, dtype ? "bf16" : "fp16", cfg.block_m, cfg.block_n, cfg.wave_m, cfg.wave_n, lines || ln_lines ? " whole lines" : "",
               cfg.pipeline, cfg.group_m, split, ms, 2.0 * M * N * K / ms / 1e9);
   return 0;
 }

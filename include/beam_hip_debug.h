@@ -81,7 +81,10 @@ int beam_dbg_set_splitk_self_reduce(int on);
 /* For tests on a host without a GPU: the CU count the library's choices assume when no device could be probed
  * (refused once a device has been). */
 int beam_dbg_assume_compute_units(int compute_units);
-/* The tile a beam_gemmrc_ln call without a tile takes for its one-kernel form on a device of `compute_units` CUs
+/* What a beam_gemmrc_ln call without a tile, on a device of 256 CUs and rows on 16 bytes, takes for its one-kernel form where
+ * beam_dbg_small_tile says none, and whether its fills take whole 128-byte lines (as in beam_dbg_off_lines_tile). */
+int beam_dbg_ln_line_tile(int M, int N, int K, beam_tile_cfg* cfg, int* whole_lines);
+/* The tile that it takes among those of beam_get_config's table, and on rows off 16 bytes, on a device of `compute_units` CUs
  * (the library's LayerNorm cost model; BEAM_ERR_UNSUPPORTED where that form applies with no tile). */
 int beam_dbg_ln_default_config(int M, int N, int K, int compute_units, beam_tile_cfg* cfg);
 /* The 4-wavefront kernel with B stored [K][N] (256 columns, 512 bytes per row of k in an LDS slot): the XOR code of

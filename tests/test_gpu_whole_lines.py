@@ -9,6 +9,7 @@ import pytest
 
 from test_gpu_edges import close_enough
 from test_gpu_gemm import BF16, F16
+from test_gpu_ln import check_ln, make_ln_inputs, run_ln
 from test_gpu_unaligned import run
 from test_host_logic import small_tile
 
@@ -20,9 +21,9 @@ TILES = {(64, 64): (1000, 1000), (96, 64): (2913, 464), (64, 128): (329, 4648), 
          (128, 128): (399, 7968), (160, 128): (633, 6536), (192, 128): (760, 6536)}
 
 
-def off_lines_tile(beamc, M, N, K):
+def off_lines_tile(beamc, M, N, K, plan="beam_dbg_off_lines_tile"):
     tile, lines = beamc._TileCfg(), ctypes.c_int()
-    beamc._check(beamc.lib.beam_dbg_off_lines_tile(M, N, K, ctypes.byref(tile), ctypes.byref(lines)))
+    beamc._check(getattr(beamc.lib, plan)(M, N, K, ctypes.byref(tile), ctypes.byref(lines)))
     return (tile.block_m, tile.block_n), lines.value
 
 
@@ -42,3 +43,24 @@ def test_gemmrc(gpu, beamc, oracle, tile, K):
     a, b = beamc.host_uniform((M, K), dtype, 71, 0), beamc.host_uniform((N, K), dtype, 71, 1)
     out = run(beamc, lambda pa, pb, pc: L.beam_gemmrc(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offsets)
     close_enough(oracle, out, oracle.gemmrc(a, b, dtype), K, dtype, f"{tile} {(M, N, K)} at {offsets}")
+
+
+# GEMM+LayerNorm: a shape for each tile, K off lines and on them; the last two have more tiles than CUs
+LN_TILES = {(96, 64): (1064, 1040, 1480), (64, 128): (163, 6232, 2056), (128, 64): (1240, 1592, 2008),
+            (96, 128): (449, 4352, 968), (128, 128): (399, 7968, 2056), (160, 128): (795, 5016, 744), (192, 128): (2912, 2008, 1680)}
+
+
+def test_layernorm_reaches_them(gpu, beamc):
+    for tile, shape in LN_TILES.items():
+        assert off_lines_tile(beamc, *shape, "beam_dbg_ln_line_tile") == (tile, 1), (tile, shape)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("tile", sorted(LN_TILES))
+def test_layernorm(gpu, beamc, oracle, tile, dtype):
+    M, N, K = LN_TILES[tile]
+    for k in (K, (K + 63) // 64 * 64):
+        a, b, g, bt = make_ln_inputs(beamc, M, N, k, dtype, 72)
+        ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, dtype)
+        for mode in (beamc.LN_AUTO, beamc.LN_FUSED):
+            check_ln(oracle, run_ln(beamc, a, b, g, bt, dtype, mode=mode), ref, dtype, f"{tile} {(M, N, k)} mode {mode}")
