@@ -129,6 +129,7 @@ def _load() -> ctypes.CDLL:
     L.beam_dbg_ln_plan_bytes.restype = sz
     L.beam_dbg_assume_compute_units.argtypes = [i]
     L.beam_dbg_small_tile.argtypes = [i, i, i, i, i] + [ctypes.POINTER(i)] * 4
+    L.beam_dbg_nn_off_lines_tile.argtypes = [i, i, i, cfgp, cfgp, ctypes.POINTER(i)]
     L.beam_dbg_off_lines_tile.argtypes = L.beam_dbg_ln_line_tile.argtypes = [i, i, i, cfgp, ctypes.POINTER(i)]
     L.beam_set_ln_walk.argtypes = [i]
     L.beam_dbg_set_splitk_self_reduce.argtypes = [i]

@@ -557,8 +557,9 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
     // 8.6 -> 8.2; [K][N] x 256 5.0 -> 4.2, x 512 5.8 -> 5.3, x 1024 7.0 -> 6.9, x 1536 8.3, 8.7; 1000 x 1003 x 1024 6.8, 7.7).
     if (t.rows * t.cols == 64 * 64 && gemm && N % 8 == 0 && M > 64 && K <= (rows != kOnLines ? 1280 : b_kmajor ? 1024 : 2047)) return none;
     // ... nor where rows are off lines but on chunks and fills would take whole lines here: so they do in the tiled kernel
-    // (kFormLines; 1100 x 544 x 1352 8.9 -> 7.3, 1402 x 664 x 2216 11.9 -> 10.4, 447 x 1912 x 7504 27.8 -> 24.9; odd N stays).
-    if (t.rows * t.cols == 64 * 64 && plan.shift && gemm && !b_kmajor && !side && N % 8 == 0) return none;
+    // (kFormLines; 1100 x 544 x 1352 8.9 -> 7.3, 1402 x 664 x 2216 11.9 -> 10.4, 447 x 1912 x 7504 27.8 -> 24.9; [K][N] 3393 x
+    // 184 x 2168 13.0 -> 12.0, 147 x 3952 x 2824 14.6 -> 13.4).  Rows of C that are not whole chunks stay.
+    if (t.rows * t.cols == 64 * 64 && plan.shift && gemm && !side && N % 8 == 0) return none;
     // ... or one row of 32 x 64 tiles streams B from nearly every CU (20 x 14000 x 1500 10.7, here 11.4; 32 x 11008 x 4096 18.8,
     // 18.1; 30 x 9000 x 3000 13.6, 12.1).
     if (t.rows == 32 && t.cols == 64 && M <= 32 && !b_kmajor && !ln && 4 * tiles > 3L * cus) return none;
@@ -629,6 +630,62 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
     if (!k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline) stays = &k, stays_us = us;
   }
   if (stays && best_us > 0.96 * stays_us) best = stays;
+  LineChoice t = {best->cfg, best->lines};
+  t.cfg.group_m = default_group_m(t.cfg.block_m, t.cfg.block_n);
+  return t;
+}
+
+// The same for beam_matmul_nn, where only rows of A can be off lines for K's sake: whole chunks in B's rows (N % 8 == 0), and not.
+// Fitted to 100 and 60 shapes with M and N from 32 and 64 to 8192 (5001); `named` is what choose_default's tile has become there,
+// and stays unless another is 8% ahead by the model: 7.3% and 5.6% faster than `named` on average.  us, before -> now: 3059 x 368
+// x 7800 45.8 -> 35.5, 841 x 6176 x 1416 23.8 -> 21.6, 1369 x 957 x 208 7.6 -> 6.1, 4397 x 3888 x 280 24.2 -> 23.0.
+LineChoice nn_off_lines_tile(int M, int N, int K, const beam_tile_cfg& named, int cus) {
+  struct Candidate {
+    beam_tile_cfg cfg;
+    bool lines;
+    int occ;
+    double alone[2], full[2], round[2], launch[2];  // N % 8 == 0, else
+  };
+  static const Candidate kCandidates[] = {
+      {{256, 256, 128, 64, 0, 0}, false, 1, {7.34, 7.85}, {7.34, 7.85}, {8.27, 7.56}, {0, 2.82}},
+      {{224, 256, 112, 64, 0, 0}, false, 1, {7.05, 7.31}, {7.05, 7.31}, {7.45, 6.95}, {0, 2.69}},
+      {{192, 256, 96, 64, 0, 0}, false, 1, {6.51, 6.92}, {6.51, 6.92}, {6.59, 6.38}, {0, 2.55}},
+      {{256, 128, 64, 64, 0, 0}, false, 1, {5.14, 5.76}, {5.14, 5.76}, {4.74, 4.65}, {0, 2.96}},
+      {{128, 256, 64, 64, 0, 0}, false, 1, {5.10, 5.29}, {5.10, 5.29}, {4.69, 4.52}, {0, 2.73}},
+      {{128, 128, 64, 32, 0, 0}, false, 2, {3.93, 4.06}, {3.88, 3.37}, {3.50, 3.10}, {0.36, 2.98}},
+      {{128, 128, 64, 32, 2, 0}, false, 1, {4.09, 4.40}, {4.09, 4.40}, {3.63, 4.90}, {0.38, 1.10}},
+      {{128, 64, 64, 32, 0, 0}, false, 2, {2.25, 2.27}, {2.69, 2.76}, {2.39, 2.94}, {0.92, 0.93}},
+      {{128, 64, 64, 32, 2, 0}, false, 1, {2.58, 2.79}, {2.58, 2.79}, {2.78, 3.12}, {1.18, 1.36}},
+      {{64, 128, 32, 64, 0, 0}, false, 2, {1.96, 1.92}, {2.84, 2.81}, {2.46, 2.86}, {0.72, 1.90}},
+      {{64, 128, 32, 64, 2, 0}, false, 1, {2.97, 2.93}, {2.97, 2.93}, {3.02, 3.44}, {1.17, 1.92}},
+      {{64, 64, 32, 32, 0, 0}, false, 4, {1.29, 1.29}, {2.28, 2.52}, {2.25, 2.95}, {0.63, 0.68}},
+      {{64, 64, 32, 32, 2, 0}, false, 1, {1.96, 1.96}, {1.96, 1.96}, {2.51, 2.52}, {0.82, 1.24}},
+      {{64, 64, 32, 32, 2, 0}, true, 1, {2.26, 2.19}, {2.26, 2.19}, {2.43, 2.84}, {0.91, 1.19}},
+      {{96, 64, 48, 32, 2, 0}, true, 1, {2.80, 2.76}, {2.80, 2.76}, {2.55, 3.18}, {0.98, 1.29}},
+      {{64, 128, 32, 32, 2, 0}, true, 1, {2.74, 2.82}, {2.74, 2.82}, {2.77, 3.70}, {0.89, 1.69}},
+      {{96, 128, 48, 64, 2, 0}, true, 1, {3.68, 3.85}, {3.68, 3.85}, {3.79, 5.68}, {1.00, 1.55}},
+      {{128, 128, 64, 32, 2, 0}, true, 1, {4.28, 4.67}, {4.28, 4.67}, {3.43, 5.32}, {0.53, 0.93}},
+      {{160, 128, 80, 64, 2, 0}, true, 1, {4.21, 4.48}, {4.21, 4.48}, {3.52, 5.15}, {1.61, 2.70}},
+      {{192, 128, 96, 64, 2, 0}, true, 1, {5.15, 5.64}, {5.15, 5.64}, {5.30, 6.83}, {1.43, 2.80}},
+  };
+  const int odd = N % 8 != 0 ? 1 : 0;
+  const Candidate *best = nullptr, *stays = nullptr;
+  double best_us = 0, stays_us = 0;
+  for (const Candidate& k : kCandidates) {
+    const bool is_named = !k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline;
+    // (Rows of B that are not whole chunks under a short sum: no other wide tile.  2985 x 1381 x 360 in 128 x 128 tiles 12.7 us, by
+    // lines in 160 x 128 14.0, in 256 x 128 14.3.)
+    if (odd && K < 600 && k.cfg.block_n > 64 && !is_named) continue;
+    const long tiles = (long)((M + k.cfg.block_m - 1) / k.cfg.block_m) * ((N + k.cfg.block_n - 1) / k.cfg.block_n);
+    const long load = (tiles + cus - 1) / cus;
+    const long conc = load < k.occ ? load : k.occ;
+    const double rate = k.occ == 1 ? k.alone[odd] : k.alone[odd] + (k.full[odd] - k.alone[odd]) * (double)(conc - 1) / (k.occ - 1);
+    const double mflop = 2.0e-6 * k.cfg.block_m * k.cfg.block_n * (double)(((long)K + kBK - 1) / kBK * kBK);
+    const double us = (double)((load + k.occ - 1) / k.occ) * k.round[odd] + (double)load * mflop / rate + k.launch[odd];
+    if (!best || us < best_us) best = &k, best_us = us;
+    if (is_named) stays = &k, stays_us = us;
+  }
+  if (stays && best_us > 0.92 * stays_us) return LineChoice{named, false};
   LineChoice t = {best->cfg, best->lines};
   t.cfg.group_m = default_group_m(t.cfg.block_m, t.cfg.block_n);
   return t;
@@ -805,6 +862,21 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
     }
     const KernelSet* alt_ks = nullptr;
     if ((alt.wave_n != c.wave_n) && resolve_cfg(&alt, M, N, K, &alt, &alt_ks) == BEAM_OK) c = alt, ks = alt_ks;
+    if (K % kBK != 0 && row_starts(A, B, K, true) == kOnChunks) {
+      const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
+      const LineChoice t = nn_off_lines_tile(M, N, K, c, cus);
+      c = t.cfg;
+      if (t.lines) {
+        GemmParams p = base_params(A, B, M, N, K, c);
+        p.C = C;
+        p.c_store = store_kind(c, 4, false, C, M, N);
+        const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, 1);
+        BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_lines_kmajor<_Float16>(c.block_m, c.block_n, p, grid, st)
+                                   : launch_gemm_lines_kmajor<__bf16>(c.block_m, c.block_n, p, grid, st));
+        return BEAM_OK;
+      }
+      if ((rc = resolve_cfg(&c, M, N, K, &c, &ks))) return rc;
+    }
   }
   // The 4-wavefront kernel, as in beam_gemmrc (its stores write whole chunks of 8 columns); the K tile's offset into B is a
   // 32-bit scalar there.
@@ -1533,6 +1605,14 @@ int beam_dbg_small_tile(int op, int M, int N, int K, int row_starts, int* rows, 
 int beam_dbg_off_lines_tile(int M, int N, int K, beam_tile_cfg* cfg, int* whole_lines) {
   if (M <= 0 || N <= 0 || K < 8 || !cfg || !whole_lines) return fail(BEAM_ERR_INVALID, "null pointer or empty problem");
   const LineChoice t = off_lines_tile(M, N, K, g_dev.cus > 0 ? g_dev.cus : 256);
+  *cfg = t.cfg;
+  *whole_lines = t.lines ? 1 : 0;
+  return BEAM_OK;
+}
+
+int beam_dbg_nn_off_lines_tile(int M, int N, int K, const beam_tile_cfg* named, beam_tile_cfg* cfg, int* whole_lines) {
+  if (M <= 0 || N < 8 || K < 8 || !named || !cfg || !whole_lines) return fail(BEAM_ERR_INVALID, "null pointer or empty problem");
+  const LineChoice t = nn_off_lines_tile(M, N, K, *named, g_dev.cus > 0 ? g_dev.cus : 256);
   *cfg = t.cfg;
   *whole_lines = t.lines ? 1 : 0;
   return BEAM_OK;

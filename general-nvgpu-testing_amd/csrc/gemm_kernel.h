@@ -408,7 +408,7 @@ struct GemmTile {
   static constexpr int SV = HALVES ? 1 : NW / LDW;  // side vectors per loader thread per K tile
   static constexpr int LIVE = LINES ? 3 : 2;  // slots not in flight at a K tile's wait: its own (with lines two) and the next to be refilled
   static constexpr int WAIT_STEADY =
-      (AST - LIVE) * LA + (BST - LIVE) * LB + (SIDE ? 2 * SV * ((AST < BST ? AST : BST) - 1) : 0);
+      (AST - LIVE) * LA + (BST - (B_KMAJOR ? 2 : LIVE)) * LB + (SIDE ? 2 * SV * ((AST < BST ? AST : BST) - 1) : 0);
 
   static_assert(KSTEPS == 2, "the step pipeline below is written for two 32-wide steps per tile");
   static_assert(TM % 16 == 0 && TN % 16 == 0, "wavefront tile must be made of 16x16 blocks");
@@ -418,8 +418,8 @@ struct GemmTile {
   static_assert(GROUPS * LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
   static_assert(KG == 1 || (NW <= 4 && !SIDE && !LOOP && (KG - 1) * BM * BN * 4 <= GROUPS * LDS_BYTES), "K groups");
   static_assert(!HALVES || KG == 2, "two halves of a K tile");
-  static_assert(!LINES || NW == 4, "whole lines: the rows of a thread's fills lie a multiple of 16 apart");
-  static_assert(!LINES || (AST >= 3 && BST >= 3 && !SIDE && !LOOP && !B_KMAJOR), "whole lines");
+  static_assert(!LINES || NTL % 128 == 0, "whole lines: the rows of a thread's fills lie a multiple of 16 apart");
+  static_assert(!LINES || (AST >= 3 && BST >= 3 && !SIDE && !LOOP && (!B_KMAJOR || AST == BST + 1)), "whole lines");
   static_assert(WAIT_STEADY < 64, "vmcnt range");
   static_assert(BM * 8 * (4 * WAVES_N + 2) <= LDS_BYTES, "row statistics scratch of the LayerNorm epilogues");
 
@@ -569,12 +569,16 @@ struct GemmTile {
     int klen = K - kb;
     if (klen > p.k_slice) klen = p.k_slice;
     if (klen < 0) klen = 0;
+    // [K][N] with whole lines of A and rows of B that are not whole chunks: the last 8 elements of K are multiplied straight
+    // from memory behind the loop (the host sees to K % 8 == 0), so that every row of B that is fetched has another behind it.
+    const bool last_chunk_apart = LINES && B_KMAJOR && (N & 7) != 0;
+    if (last_chunk_apart) klen -= 8;
     // [K][N] with rows of B that are not whole 16-byte chunks: the last K tile is treated as a short one even if it
     // is whole, because the last row's last chunk must not be fetched as it stands (see load_short_tile).
     const bool n_odd = B_KMAJOR && (N & 7) != 0;
     int kt_full = LINES ? (klen + kBK - 1) / kBK : klen / kBK;
     int k_tail = LINES ? 0 : klen - kt_full * kBK;
-    if (n_odd && k_tail == 0 && kt_full > 0) {
+    if (!LINES && n_odd && k_tail == 0 && kt_full > 0) {
       k_tail = kBK;
       --kt_full;
     }
@@ -592,7 +596,7 @@ struct GemmTile {
     // B as [N][K] (rows of K): like A.  B as [K][N] (B_KMAJOR): the tile's columns start at col0 of
     // row kb; a descriptor is made per K tile (load_b) so that it ends with the tile's last row.
     const T* b_base = B_KMAJOR ? (const T*)p.B + ((size_t)kb * N + col0) : (const T*)p.B + ((size_t)col0 * K + kb);
-    unsigned bytes_a = klen > 0 ? ((unsigned)(rows_a - 1) * K + klen) * 2u : 0u;
+    unsigned bytes_a = klen > 0 ? ((unsigned)(rows_a - 1) * K + klen) * 2u : 0u;  // (whole lines: chunks behind klen are masked)
     unsigned bytes_b = klen > 0 ? ((unsigned)(rows_b - 1) * K + klen) * 2u : 0u;
     // kEpiStoreLoop: the same for the next tile of this workgroup (neither split-K nor the [K][N]
     // layout nor a short K tile exist in that mode: the host sees to it)
@@ -636,12 +640,12 @@ struct GemmTile {
     };
     if constexpr (LINES) {
       range_a = lines_setup(a_base, rows_a, voff_a, LA);
-      range_b = lines_setup(b_base, rows_b, voff_b, LB);
+      if constexpr (!B_KMAJOR) range_b = lines_setup(b_base, rows_b, voff_b, LB);
     }
 #pragma unroll
     for (int i = 0; i < (LINES ? 0 : LA); ++i) voff_a[i] = chunk_voffset(i * NTL + ltid, K);
 #pragma unroll
-    for (int i = 0; i < (LINES ? 0 : LB); ++i) {
+    for (int i = 0; i < (LINES && !B_KMAJOR ? 0 : LB); ++i) {
       if (B_KMAJOR) {
         // LDS position q of the stage: row k = q / CPR, and the chunk that lives there is position ^ swizzle
         constexpr int CPR = BN / 8;
@@ -678,7 +682,7 @@ struct GemmTile {
     };
     auto load_b = [&](int i, int t) __attribute__((always_inline)) {
       char* dst = smem + B_REGION + (t % BST) * B_BYTES + lwave * 1024 + i * (NTL * 16);
-      if constexpr (LINES) {
+      if constexpr (LINES && !B_KMAJOR) {
         const __amdgpu_buffer_rsrc_t r = make_rsrc((const char*)b_base - kRowBytes, bytes_b + kRowBytes);
         const unsigned off = (unsigned)(t - range_b.first) < range_b.count ? voff_b[i] : kOobOffset;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, (int)off, tile_koff(t) * 2, 0, 0);
@@ -693,7 +697,10 @@ struct GemmTile {
         if (rows > kBK) rows = kBK;
         // (n_odd: another row of at least 8 elements follows every tile fetched here, so its last row may be read to a
         // whole chunk; the range check works on whole dwords and would cut an odd last column off)
-        const unsigned bytes = (t < n_tiles && rows > 0) ? ((unsigned)(rows - 1) * N + rows_b + (n_odd ? 7 : 0)) * 2u : 0u;
+        // (Whole lines: behind the last row that is multiplied here A's are zeros, and zero times infinity is not; one element
+        // is enough for an odd last column's dword, and too little for one of the row behind.)
+        const unsigned more = LINES ? (unsigned)(N & 1) : n_odd ? 7u : 0u;
+        const unsigned bytes = (t < n_tiles && rows > 0) ? ((unsigned)(rows - 1) * N + rows_b + more) * 2u : 0u;
         const __amdgpu_buffer_rsrc_t r = make_rsrc(b_base + (size_t)koff * N, bytes);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16,
                                                  (int)voff_b[i], 0, 0, 0);
@@ -790,7 +797,7 @@ struct GemmTile {
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
       late_a[kk] = LINES && 4 * (HALVES ? kg : kk) + (lane >> 4) + phase_of(a_base, lane & 15) >= 8;
-      late_b[kk] = LINES && 4 * (HALVES ? kg : kk) + (lane >> 4) + phase_of(b_base, lane & 15) >= 8;
+      late_b[kk] = LINES && !B_KMAJOR && 4 * (HALVES ? kg : kk) + (lane >> 4) + phase_of(b_base, lane & 15) >= 8;
     }
     const int a_wave_off = wm * TM * kRowBytes;
     const int b_wave_off = B_KMAJOR ? 0 : wn * TN * kRowBytes;
@@ -1031,8 +1038,8 @@ struct GemmTile {
         return sa + frag_off[kk];
       };
       auto b_at = [&](int kk) __attribute__((always_inline)) -> const char* {
-        if constexpr (LINES) return smem + (B_REGION + (late_b[kk] ? ((h + 1) % BST) * B_BYTES : (h % BST) * B_BYTES)) + (b_wave_off + frag_off[kk]);
-        return sb + (B_KMAJOR ? kk * (32 * BN * 2) : frag_off[kk]);
+        if constexpr (LINES && !B_KMAJOR) return smem + (B_REGION + (late_b[kk] ? ((h + 1) % BST) * B_BYTES : (h % BST) * B_BYTES)) + (b_wave_off + frag_off[kk]);
+        return sb + (B_KMAJOR ? (HALVES ? kg : kk) * (32 * BN * 2) : frag_off[kk]);
       };
       if constexpr (HALVES) {
         // this group's half of tile h is read while its half of tile h - 1 is multiplied
@@ -1097,10 +1104,14 @@ struct GemmTile {
           if (h < n_tiles) {
             tile_body(h, ld_tag, w_tag, Even{});
             // the drain takes set 1
+            if constexpr (B_KMAJOR) wait_lds<0>();  // (reads that the compiler does not see)
 #pragma unroll
             for (int i = 0; i < FM; ++i) fa1[i] = fa0[i];
 #pragma unroll
-            for (int j = 0; j < FN; ++j) fb1[j] = fb0[j];
+            for (int j = 0; j < FN; ++j) {
+              if constexpr (B_KMAJOR) asm volatile("" : "+v"(fb0[j]));
+              fb1[j] = fb0[j];
+            }
           }
         } else {
           for (int h = 0; h < n_tiles; ++h) tile_body(h, ld_tag, w_tag, Even{});
@@ -1149,6 +1160,27 @@ struct GemmTile {
       if constexpr (!LOOP) k_loop_and_drain();
     } else if (GROUPS > 1 && n_all > 0) {
       bare_barrier();
+    }
+    if constexpr (LINES && B_KMAJOR) {
+      if (last_chunk_apart && kg == 0) {  // (uniform) lanes 0 .. 15 hold the 8 elements, as the first of an MFMA's four groups
+        const int r = lane & 15;
+        vec8 fb[FN];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const int n = col0 + wn * TN + j * 16 + r;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) fb[j][e] = lane < 16 && n < N ? ((const T*)p.B)[(size_t)(K - 8 + e) * N + n] : (T)0.0f;
+        }
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(a_base, (unsigned)rows_a * (unsigned)K * 2u);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          const int row = wm * TM + i * 16 + r;
+          const unsigned off = lane < 16 && row < rows_a ? ((unsigned)row * (unsigned)K + (unsigned)K - 8u) * 2u : kOobOffset;
+          const vec8 fa = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] = Traits::mfma(fb[j], fa, acc[i][j]);
+        }
+      }
     }
     if constexpr (KG > 1) {
       // The groups' sums meet in group 0, added in group order; the other groups are done.

@@ -198,6 +198,20 @@ template <> hipError_t launch_gemm_kwave_ln<__bf16>(const KwPlan&, const KwLnPar
   X(192, 128, 4, 2, kFormLineHalves)
 template <typename T>
 hipError_t launch_gemm_lines(int block_m, int block_n, const GemmParams& p, dim3 grid, hipStream_t stream);
+// B stored [K][N], fills of A by whole lines: (workgroup tile M, N, wavefronts M, N of a group, LDS slots of B (A has one more), K
+// groups, Form).  Needs K % 8 == 0, A on 16 bytes and N >= 8.
+#define BEAM_FOR_EACH_KMAJOR_LINES_TILE(X)    \
+  X(64, 64, 2, 2, 4, 2, kFormLines)           \
+  X(96, 64, 2, 2, 3, 2, kFormLines)           \
+  X(64, 128, 2, 4, 6, 1, kFormLines)          \
+  X(96, 128, 2, 2, 5, 2, kFormLineHalves)     \
+  X(128, 128, 2, 4, 4, 1, kFormLines)         \
+  X(160, 128, 2, 2, 3, 1, kFormLines)         \
+  X(192, 128, 2, 2, 3, 2, kFormLineHalves)
+template <typename T>
+hipError_t launch_gemm_lines_kmajor(int block_m, int block_n, const GemmParams& p, dim3 grid, hipStream_t stream);
+template <> hipError_t launch_gemm_lines_kmajor<_Float16>(int, int, const GemmParams&, dim3, hipStream_t);
+template <> hipError_t launch_gemm_lines_kmajor<__bf16>(int, int, const GemmParams&, dim3, hipStream_t);
 // GEMM+LayerNorm in one launch: parameters as for the kEpiLnFused kernels.
 template <typename T>
 hipError_t launch_gemm_lines_ln(int block_m, int block_n, const GemmParams& p, dim3 grid, hipStream_t stream);

@@ -73,6 +73,8 @@ int beam_dbg_small_tile(int op, int M, int N, int K, int row_starts, int* rows, 
  * but not on 128 (K % 64 != 0), and whether its fills take whole 128-byte lines (*whole_lines = 1: such a tile need not be in
  * beam_get_config's table). */
 int beam_dbg_off_lines_tile(int M, int N, int K, beam_tile_cfg* cfg, int* whole_lines);
+/* The same for beam_matmul_nn and rows of A; `named`: the tile that it would run on otherwise. */
+int beam_dbg_nn_off_lines_tile(int M, int N, int K, const beam_tile_cfg* named, beam_tile_cfg* cfg, int* whole_lines);
 /* A measurement, off by default: on != 0 makes the one-launch split-K run without reducing workgroups wherever its
  * multiplying workgroups fit one round of the CUs; the workgroup of (tile, slice s) then adds parts s, s + slices, ...
  * of its tile itself.  Same bits.  Unlike the shipped form this needs every workgroup of the launch resident at once

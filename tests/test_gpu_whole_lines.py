@@ -64,3 +64,54 @@ def test_layernorm(gpu, beamc, oracle, tile, dtype):
         ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, dtype)
         for mode in (beamc.LN_AUTO, beamc.LN_FUSED):
             check_ln(oracle, run_ln(beamc, a, b, g, bt, dtype, mode=mode), ref, dtype, f"{tile} {(M, N, k)} mode {mode}")
+
+
+# [K][N]: shapes that reach each tile, B's rows of whole chunks and not
+NN_TILES = [((64, 64), (155, 4720, 360)), ((64, 64), (2086, 368, 2632)), ((64, 128), (655, 2896, 432)), ((96, 64), (714, 1432, 200)),
+            ((96, 64), (860, 1229, 2312)), ((96, 64), (215, 5103, 952)), ((96, 128), (2197, 1384, 2120)), ((96, 128), (551, 3597, 4784)),
+            ((128, 128), (723, 3752, 376)), ((128, 128), (2472, 1152, 600)), ((160, 128), (1428, 3456, 336)), ((160, 128), (3677, 1242, 1232)),
+            ((192, 128), (1296, 4320, 1136)), ((192, 128), (1713, 3017, 1688))]
+
+
+def nn_tile(beamc, M, N, K):
+    named, _ = beamc.default_config(M, N, K)
+    named, tile, lines = named.to_c(), beamc._TileCfg(), ctypes.c_int()
+    beamc._check(beamc.lib.beam_dbg_nn_off_lines_tile(M, N, K, ctypes.byref(named), ctypes.byref(tile), ctypes.byref(lines)))
+    return (tile.block_m, tile.block_n), lines.value
+
+
+def test_matmul_nn_reaches_them(gpu, beamc):
+    for tile, (M, N, K) in NN_TILES:
+        assert small_tile(beamc, 1, M, N, K, 1)[0] == 0 and nn_tile(beamc, M, N, K) == (tile, 1), (tile, (M, N, K))
+
+
+@pytest.mark.parametrize("tile,shape", NN_TILES)
+def test_matmul_nn(gpu, beamc, oracle, tile, shape):
+    L = beamc.lib
+    M, N, K = shape
+    for dtype, offsets in ((F16, (0, 0, 0)), (BF16, (8, 3, 1))):
+        a, b = beamc.host_uniform((M, K), dtype, 73, 0), beamc.host_uniform((K, N), dtype, 73, 1)
+        out = run(beamc, lambda pa, pb, pc: L.beam_matmul_nn(pa, pb, pc, M, N, K, dtype, None, None), a, b, (M, N), dtype, offsets)
+        close_enough(oracle, out, oracle.matmul_nn(a, b, dtype), K, dtype, f"[K][N] {tile} {(M, N, K)} at {offsets}")
+
+
+@pytest.mark.parametrize("M,N,K", [(5681, 57, 2008), (3817, 364, 880), (860, 1229, 2312), (714, 1432, 200)])
+def test_infinities_of_b_reach_their_columns_only(gpu, beamc, M, N, K):
+    """The rows of B behind the last K tile of the loop, and at both ends of K, meet only their own elements of A."""
+    a, b = beamc.host_uniform((M, K), F16, 74, 0), beamc.host_uniform((K, N), F16, 74, 1)
+    rows = [0, 63, 64, K // 2, K - 9, K - 8, K - 1]
+    for i, k in enumerate(rows):
+        a[:, k], b[k, 2 * i] = 0x3C00, 0x7C00  # one, infinity
+    out = run(beamc, lambda pa, pb, pc: beamc.lib.beam_matmul_nn(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
+    cols = [2 * i for i in range(len(rows))]
+    assert (out[:, cols] == np.inf).all() and np.isfinite(np.delete(out, cols, axis=1)).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1100, 1000, 1096), (929, 1232, 200), (1478, 2024, 2008)])
+def test_infinities_stay_in_their_row_or_column(gpu, beamc, M, N, K):
+    a, b = beamc.host_uniform((M, K), F16, 75, 0), beamc.host_uniform((N, K), F16, 75, 1)
+    for i, k in enumerate([0, 7, 8, 63, 64, K // 2, K - 1]):
+        a[10 * i, k], b[10 * i + 5, k] = 0xFC00, 0x7C00
+    out = run(beamc, lambda pa, pb, pc: beamc.lib.beam_gemmrc(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
+    assert not np.isfinite(out[0:70:10]).any() and not np.isfinite(out[:, 5:75:10]).any()
+    assert np.isfinite(np.delete(np.delete(out, range(0, 70, 10), axis=0), range(5, 75, 10), axis=1)).all()
