@@ -231,20 +231,21 @@ GemmParams base_params(const void* A, const void* B, int M, int N, int K, const 
 //   * The others from 20 MB on (3072 x 4040 x 256 in 128 x 128 tiles 14.0 -> 12.9, 20 -> 15, in 192 x 256 13.1, 13.3, 18 -> 14;
 //     4096 x 8136 x 1024 in 256 x 256 tiles 70 -> 63, 79 -> 68; 8192 x 8136 x 256 in 128 x 128 106 -> 71).  Below: 2048 x 1992 x
 //     1024 in 128 x 128 tiles 11.6, cached 12.0.
-//   * 256 x 256 tiles of eight wavefronts over several rounds, one workgroup per tile, wherever rows start (4096 x 8192 x 256
-//     50 -> 34, x 1024 64 -> 62; not LayerNorm's, 8192 x 8192 x 1024 143, 147).
+//   * 256 x 256 tiles of eight wavefronts over several rounds under a short sum, one workgroup per tile, wherever rows start
+//     (8192 x 8192 x 256 106 -> 65, 119 -> 62; 4096 x 8192 x 1024 58.8, 59.9; 64 -> 62; 7079 x 4544 x 1840 [K][N] 96.7, 98.5),
+//     but not beside a side job (8192 x 4096 x 256 with 2^25 elements 51.9, 53.3).
 //   * Rows on 32 bytes: of these only gemm_w4.h's (4096 x 4048 x 1024 33.7 -> 29.9) and the wide tiles of a plain product (5000 x
 //     5008 x 1000 54.5 -> 53.8); 64 columns 1024 x 2000 x 256 4.46, cached 4.53, LayerNorm 4385 x 5232 x 392 41.9, 44.3.
 // (Non-temporal stores are faster still by themselves, 8192 x 8192 x 1024 in 128 x 128 tiles 161 -> 126 us, but only put the
 // cost off: with a kernel that reads the output behind it, 4096 x 4096 x 1024 takes 54.3 us written through, 56.2 so.)
-int store_kind(const beam_tile_cfg& c, int wavefronts, bool w4, const void* C, int M, int N, bool ln = false) {
+int store_kind(const beam_tile_cfg& c, int wavefronts, bool w4, const void* C, int M, int N, int K, bool fused = false) {
   const size_t bytes = (size_t)M * N * 2;
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
-  if (!w4 && !ln && wavefronts == 8 && c.block_m * c.block_n == 256 * 256 &&
+  if (!w4 && !fused && wavefronts == 8 && K < 1024 && c.block_m * c.block_n == 256 * 256 &&
       (long)((M + 255) / 256) * ((N + 255) / 256) > cus) return kStoreCached;
   if (N % 32 == 0 && ((uintptr_t)C & 63) == 0) return kStoreThrough;
   if (w4) return kStoreCached;
-  if (N % 16 == 0 && ((uintptr_t)C & 31) == 0 && (ln || c.block_n == 64)) return kStoreThrough;
+  if (N % 16 == 0 && ((uintptr_t)C & 31) == 0 && (fused || c.block_n == 64)) return kStoreThrough;
   return c.block_n == 64 || bytes >= ((size_t)20 << 20) ? kStoreCached : kStoreThrough;
 }
 
@@ -755,7 +756,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     if (t.lines) {
       GemmParams p = base_params(A, B, M, N, K, c);
       p.C = C;
-      p.c_store = store_kind(c, 4, false, C, M, N);
+      p.c_store = store_kind(c, 4, false, C, M, N, K);
       const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, 1);
       BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_lines<_Float16>(c.block_m, c.block_n, p, grid, st) : launch_gemm_lines<__bf16>(c.block_m, c.block_n, p, grid, st));
       return BEAM_OK;
@@ -791,7 +792,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
   if (w4_fits && w4_named) {
     // Non-temporal stores of C pay when C is larger than the 256 MB last-level cache (and the K loops
     // are not so short that the writes are the bound).
-    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, ks->threads / 64, true, C, M, N);
+    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, ks->threads / 64, true, C, M, N, K);
     BEAM_HIP(launch_gemm_w4(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
@@ -809,7 +810,7 @@ int beam_gemmrc(const void* A, const void* B, void* C, int M, int N, int K, int 
     BEAM_HIP(loop(p, dim3((unsigned)cus, 1, 1), st));
     return BEAM_OK;
   }
-  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N);
+  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N, K);
   GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, false, cus);
   BEAM_HIP((one_group ? one_group : ks->launch[dtype][kEpiStore][c.pipeline])(p, dim3((unsigned)tiles, 1, 1), st));
   return BEAM_OK;
@@ -869,7 +870,7 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
       if (t.lines) {
         GemmParams p = base_params(A, B, M, N, K, c);
         p.C = C;
-        p.c_store = store_kind(c, 4, false, C, M, N);
+        p.c_store = store_kind(c, 4, false, C, M, N, K);
         const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, 1);
         BEAM_HIP(dtype == BEAM_F16 ? launch_gemm_lines_kmajor<_Float16>(c.block_m, c.block_n, p, grid, st)
                                    : launch_gemm_lines_kmajor<__bf16>(c.block_m, c.block_n, p, grid, st));
@@ -893,11 +894,11 @@ int beam_matmul_nn(const void* A, const void* B, void* C, int M, int N, int K, i
   const int cus = g_dev.cus > 0 ? g_dev.cus : 256;
   if (w4_fits && w4_named) {
     const long tiles = (long)p.tiles_m * p.tiles_n;
-    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, ks->threads / 64, true, C, M, N);
+    p.c_store = (size_t)M * N * 2 >= ((size_t)256 << 20) && K >= 1024 ? kStoreStreaming : store_kind(c, ks->threads / 64, true, C, M, N, K);
     BEAM_HIP(launch_gemm_w4_kmajor(p, dtype, dim3((unsigned)(tiles < cus ? tiles : cus), 1, 1), st));
     return BEAM_OK;
   }
-  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N);
+  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N, K);
   GemmLauncher one_group = cfg ? nullptr : deep_one_group(*ks, c, M, N, K, dtype, true, cus);
   BEAM_HIP((one_group ? one_group : ks->launch_kmajor[dtype][c.pipeline])(p, dim3((unsigned)(p.tiles_m * p.tiles_n), 1, 1), st));
   return BEAM_OK;
@@ -1032,7 +1033,7 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }
-  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N);
+  p.c_store = store_kind(c, ks->threads / 64, false, C, M, N, K, true);
   BEAM_HIP(ks->launch[dtype][kEpiStoreSide][c.pipeline](p, dim3((unsigned)wgs, 1, 1), (hipStream_t)stream));
   return BEAM_OK;
 }
@@ -1691,7 +1692,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
   // K == 0: the kernels run with an empty K range and produce x = 0, i.e. y = beta.
   if (plan.kind == LnPlan::kFused) {
     p.C = Y;
-    p.c_store = store_kind(c, plan.lines ? 4 : ks->threads / 64, plan.w4, Y, M, N, true);
+    p.c_store = store_kind(c, plan.lines ? 4 : ks->threads / 64, plan.w4, Y, M, N, K, true);
     // Launches that share a workspace must be ordered (same stream): overlapping ones would race on the sets.
     const size_t set_bytes = ln_fused_set_bytes(p.tiles_m, p.tiles_n, c.block_m);
     float* sets = (float*)((char*)ws + ln_fused_header_bytes());
