@@ -1024,12 +1024,20 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
     }
   }
   p.side_iters = (int)(((count >> 3) * (16 / p.side_width) + per_pass - 1) / per_pass);
-  // A job that outlasts the loop goes on at 0.4-1.4 us for every 16 bytes per thread; with a round of workgroups or less,
-  // from 8 such passes on (more behind a long loop, whose own passes are the cheaper for it: 992 x 3976 x 3288 with 2^26
-  // elements, 52 K tiles and 12 passes beyond them, 84.4, 88.9), a launch of its own (3 us and 11 us per 16 Mi elements) is ahead.  Fused, then two launches:
-  // 4096 x 4096 x 256 with 2^24 (12) 28.9, 26.4; but 1536 x 1536 x 512 with 2^22 (7) 9.4, 10.5.  With several rounds the later workgroups hide it:
-  // 8192 x 8192 x 256 with 2^26 (12) 110.8, 117.7.
-  if (!cfg && wgs <= cus && p.side_iters - k_tiles > 8 + k_tiles / 8) {
+  // Two launches, where the job outlasts the loop or the GEMM alone takes its rows by whole lines, which no kernel with a side
+  // job does; the second launch costs about 2.5 us and the job alone 3 us to 1 Mi elements, 8 at 9 Mi, 20 at 25 Mi.  Over 106
+  // shapes from 256 x 256 x 256 to 8192^3 with 2^18 to 2^26 elements this rule took 7% off the mean of what one launch took.
+  //   * Behind the loop a pass costs 0.4-1.4 us for 16 bytes per thread; a long loop's own passes are the cheaper for it.  One
+  //     launch, then two, us: 1602 x 2624 x 320 with 10 Mi (14 passes behind it) 24.7, 16.8; 2156 x 3680 x 448 with 31 Mi (24)
+  //     41.6, 37.2; 1226 x 7304 x 320 with 15 Mi (8) 35.6, 23.9; 5000 x 4000 x 512 with 64 Mi (18) 99.0, 82.3; but 7276 x 392 x
+  //     256 with 7 Mi (1) 12.0, 13.6.  Tiles of eight wavefronts, one on a CU, move more in a pass, and their later rounds hide
+  //     the earlier ones' passes: 5632 x 5632 x 256 in two rounds with 60 Mi (28) 90.5, 73.8; 8192 x 4096 x 256 in two with 64 Mi
+  //     (28) 91.8, 83.6, with 32 Mi (12) 51.9, 57.3; 8192 x 8192 x 512 in four with 64 Mi (8) 127.9, 135.0.
+  //   * By whole lines, with 2^20 elements or K from 2048 on: 1787 x 2648 x 744 with 38 Mi 73.8, 46.6; 1157 x 3216 x 3880 with
+  //     0.5 Mi 56.0, 33.3; 679 x 3080 x 4880 with 2.3 Mi 46.5, 34.3; but 4155 x 496 x 560 with 0.6 Mi 10.4, 11.8.
+  const bool by_lines = K % kBK != 0 && row_starts(A, B, K, false) == kOnChunks && (count >= (1 << 20) || K >= 2048) && off_lines_tile(M, N, K, cus).lines;
+  const long long behind = (ks->threads == 512 ? 8 * ((wgs + cus - 1) / cus) : 4) + k_tiles / 8;
+  if (!cfg && (by_lines || p.side_iters - k_tiles > behind)) {
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
     return beam_silu(X, Y, count, dtype, stream);
   }

@@ -9,6 +9,7 @@ import pytest
 
 from test_gpu_edges import close_enough
 from test_gpu_gemm import BF16, F16
+from test_gpu_kwave import silu_pair
 from test_gpu_ln import check_ln, make_ln_inputs, run_ln
 from test_gpu_unaligned import run
 from test_host_logic import small_tile
@@ -115,3 +116,11 @@ def test_infinities_stay_in_their_row_or_column(gpu, beamc, M, N, K):
     out = run(beamc, lambda pa, pb, pc: beamc.lib.beam_gemmrc(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, 0, 0)).view(np.float16)
     assert not np.isfinite(out[0:70:10]).any() and not np.isfinite(out[:, 5:75:10]).any()
     assert np.isfinite(np.delete(np.delete(out, range(0, 70, 10), axis=0), range(5, 75, 10), axis=1)).all()
+
+
+@pytest.mark.parametrize("M,N,K,count", [(566, 3648, 1304, (1 << 20) - 8), (566, 3648, 1304, 1 << 20), (679, 3080, 4880, 4096),
+                                         (1602, 2624, 320, 10 << 20), (2176, 2176, 256, 3 << 20), (3072, 3072, 256, 60 << 18)])
+def test_silu_job_beside(gpu, beamc, oracle, M, N, K, count):
+    """An elementwise job on either side of the lines from which it gets a launch of its own: by whole lines, behind the loop."""
+    a, b = beamc.host_uniform((M, K), BF16, 74, 0), beamc.host_uniform((N, K), BF16, 74, 1)
+    silu_pair(beamc, oracle, a, b, oracle.gemmrc(a, b, BF16), BF16, count)
