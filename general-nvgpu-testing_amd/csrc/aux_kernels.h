@@ -20,6 +20,7 @@ hipError_t launch_ln_apply(const float* X, const float* stats, const void* gamma
 
 // One thread moves on the replay counter in the header of a fused GEMM+LayerNorm workspace: recorded in front
 // of a fused launch when the stream is being captured (see ln_launch_tag in gemm_kernel.h).
+hipError_t launch_tell_host(unsigned* word, unsigned value, hipStream_t stream);
 hipError_t launch_ln_replay_bump(int* header, hipStream_t stream);
 
 // gemmrc without any condition on K, N or alignment (slow; what the tiled kernels refuse runs here):

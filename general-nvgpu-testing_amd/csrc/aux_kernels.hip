@@ -216,6 +216,11 @@ __global__ void __launch_bounds__(256) ln_rows_kernel(const float* __restrict__ 
 // workspace header.  Whatever the word held before, it holds something else afterwards.
 __global__ void ln_replay_bump_kernel(int* hdr) { hdr[kLnHdrReplay] = hdr[kLnHdrReplay] + 1; }
 
+// Runs behind a stream's work and tells the host so (capi.hip: wait_for_stream).
+__global__ void __launch_bounds__(64) tell_host_kernel(unsigned* word, unsigned value) {
+  if (threadIdx.x == 0) __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void empty_kernel(int* p) {
   if (p && threadIdx.x == 0x7fffffff) *p = 1;  // never true: keeps the argument alive
 }
@@ -244,6 +249,11 @@ hipError_t launch_silu(const void* x, void* y, size_t count, int dtype, hipStrea
   else
     hipLaunchKernelGGL(silu_kernel<_Float16>, dim3((unsigned)blocks), dim3(256), 0, stream, (const _Float16*)x,
                        (_Float16*)y, count);
+  return hipGetLastError();
+}
+
+hipError_t launch_tell_host(unsigned* word, unsigned value, hipStream_t stream) {
+  hipLaunchKernelGGL(tell_host_kernel, dim3(1), dim3(64), 0, stream, word, value);
   return hipGetLastError();
 }
 

@@ -57,10 +57,53 @@ std::mutex g_dev_mu;
 // A word of pinned host memory that a fused GEMM+LayerNorm launch sets when a workgroup in it gives up (made once, by
 // beam_init; the process keeps it, and it stays set).  While it is zero no launch of the process has ever given up, and a
 // checked call is done without copying the workspace header back: that blocking copy of 16 bytes cost more than a small
-// call's kernel (64 x 64 x 64: 24 us of a checked call beyond its launch with the copy, 11 without).  After the first
+// call's kernel (64 x 64 x 64: 24 us of a checked call beyond its launch with the copy, 11 without, 7 as wait_for_stream waits).  After the first
 // time-out every checked call reads its header.  (One word cannot tell more: launches of other streams and threads write
 // it too, so comparing it before and after a launch could miss this launch's own time-out between two of another's.)
 unsigned* g_ln_host_timeout = nullptr;
+
+// Words of pinned host memory, a 64-byte line each, through which a kernel at a stream's end tells a waiting thread that it has
+// come there (wait_for_stream).  Allocated with the word above; a call holds one while it waits, and without a free one waits as
+// hipStreamSynchronize does.
+constexpr int kWaitWords = 64;
+constexpr int kWaitStride = 16;  // unsigned per line
+unsigned* g_wait_words = nullptr;
+std::atomic<unsigned long long> g_wait_free{~0ull};
+std::atomic<unsigned> g_wait_value{0};
+
+int take_wait_word() {
+  unsigned long long free = g_wait_free.load(std::memory_order_relaxed);
+  while (free != 0)
+    if (g_wait_free.compare_exchange_weak(free, free & (free - 1), std::memory_order_acquire)) return __builtin_ctzll(free);
+  return -1;
+}
+void give_wait_word(int i) { g_wait_free.fetch_or(1ull << i, std::memory_order_release); }
+
+// Waits until everything that `st` holds has run; not for a stream that is being captured.  hipStreamSynchronize puts a packet
+// behind the last kernel that writes caches back for the host and raises a signal: 12.2 us from an empty kernel's launch to its
+// return.  A kernel of one wavefront that writes a word which this thread watches: 9.5 (the stream's kernels run one after
+// another, and each one's end has made its writes visible to the next).  Long waits are left to the runtime.
+hipError_t wait_for_stream(hipStream_t st) {
+  const int i = g_wait_words ? take_wait_word() : -1;
+  if (i < 0) return hipStreamSynchronize(st);
+  unsigned* const word = g_wait_words + i * kWaitStride;
+  const unsigned value = g_wait_value.fetch_add(1, std::memory_order_relaxed) + 1;
+  if (launch_tell_host(word, value, st) == hipSuccess) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    do {
+      for (int spin = 0; spin < 32; ++spin) {
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == value) {
+          give_wait_word(i);
+          return hipSuccess;
+        }
+        __builtin_ia32_pause();
+      }
+    } while (std::chrono::steady_clock::now() < until);
+  }
+  const hipError_t e = hipStreamSynchronize(st);
+  if (e == hipSuccess) give_wait_word(i);  // its kernel has run; after an error it may not have, and the word stays taken
+  return e;
+}
 // Polls before a waiting thread gives up: of statistics slots in the fused LayerNorm (3-4 us each once the pauses
 // between tries have grown: about 60 ms), of a tile's flags in the one-launch split-K (about 1 us each).  What a
 // workgroup legitimately waits for is resident with it and at most a tile's K loop behind, so the bound is there
@@ -343,9 +386,10 @@ int beam_init(void) {
   void* word = nullptr;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // the first call may come while a stream is being captured
   (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (hipHostMalloc(&word, 64, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
-    *(unsigned*)word = 0;
+  if (hipHostMalloc(&word, 64 * (1 + kWaitWords), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+    std::memset(word, 0, 64 * (1 + kWaitWords));
     g_ln_host_timeout = (unsigned*)word;
+    g_wait_words = (unsigned*)word + kWaitStride;
   } else {
     (void)hipGetLastError();  // without it every checked call reads the header
   }
@@ -1801,7 +1845,7 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   if (ln_plan_call(A, B, gamma, beta, Y, M, N, K, cfg, BEAM_LN_AUTO, generic, false, ws, ws_bytes, &plan) || plan.kind != LnPlan::kFused)
     return BEAM_OK;  // nothing in the call waits for anything
   if (const volatile unsigned* word = g_ln_host_timeout) {
-    BEAM_HIP(hipStreamSynchronize(st));
+    BEAM_HIP(wait_for_stream(st));
     if (*word == 0) return BEAM_OK;
   }
   int timed_out = 0;

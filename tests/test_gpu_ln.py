@@ -382,3 +382,51 @@ def test_walking_kernel_ends_when_every_wait_gives_up(gpu, beamc):
     assert (y.to_numpy() == good).all()
     for x in (da, db, dg, dbt, y):
         x.free()
+
+
+def test_checked_calls_wait_for_their_result(gpu, beamc):
+    """When a checked call returns, its result is there for a copy that nothing orders behind it: for each of several threads
+    on streams of their own, and for a call that waits longer than it watches for its end."""
+    import ctypes
+    import threading
+    L, chk, F32 = beamc.lib, beamc._check, ctypes.c_float
+    shapes = [(96, 200, 72), (512, 1024, 256), (300, 264, 1000), (64, 4096, 136)]
+    bad = []
+
+    def worker(t):
+        M, N, K = shapes[t % len(shapes)]
+        a, b, g_, bt = make_ln_inputs(beamc, M, N, K, BF16, 60 + t)
+        da, db, dg, dbt = (beamc.DeviceArray.from_numpy(x, BF16) for x in (a, b, g_, bt))
+        y, ws = beamc.DeviceArray((M, N), BF16), beamc.DeviceArray((L.beam_gemmrc_ln_workspace_bytes_for(M, N, K, None, beamc.LN_AUTO),), itemsize=1)
+        stream = ctypes.c_void_p()
+        chk(L.beam_stream_create(ctypes.byref(stream)))
+        call = lambda: chk(L.beam_gemmrc_ln_checked(da.ptr, db.ptr, dg.ptr, dbt.ptr, F32(1e-5), y.ptr, M, N, K, BF16, None, ws.ptr, ws.nbytes, stream, None))
+        call()
+        want = y.to_numpy().copy()
+        for _ in range(10):
+            y.fill_bytes(0xEE)
+            chk(L.beam_sync(None))
+            call()
+            if not (y.to_numpy() == want).all():
+                bad.append((t, M, N, K))
+        chk(L.beam_stream_destroy(stream))
+
+    threads = [threading.Thread(target=worker, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    # 4 ms of other work in front of the call
+    M, N, K = 512, 1024, 256
+    a, b, g_, bt = make_ln_inputs(beamc, M, N, K, BF16, 70)
+    da, db, dg, dbt = (beamc.DeviceArray.from_numpy(x, BF16) for x in (a, b, g_, bt))
+    y, big, out = beamc.DeviceArray((M, N), BF16), beamc.DeviceArray((8192, 8192), BF16), beamc.DeviceArray((8192, 8192), BF16)
+    big.fill_bytes(0)
+    beamc.gemmrc_ln(da, db, y, dg, dbt)
+    want = y.to_numpy().copy()
+    y.fill_bytes(0xEE)
+    for _ in range(8):
+        chk(L.beam_gemmrc(big.ptr, big.ptr, out.ptr, 8192, 8192, 8192, BF16, None, None))
+    assert beamc.gemmrc_ln(da, db, y, dg, dbt) is False
+    assert (y.to_numpy() == want).all()
