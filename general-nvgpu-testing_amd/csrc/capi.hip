@@ -1484,6 +1484,27 @@ static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) 
   return c;
 }
 
+// The order of a GEMM+LayerNorm launch without padding (band_order_tile's group_n): plain ids, or groups of G bands where what
+// the XCDs fetch, 8 / G of all rows and G times all columns, becomes less by a fifth; plain ids fetch 8 times the rows and, where
+// 8 does not divide a band's column tiles, 8 times the columns.  A group takes 64 CUs at most, as a band does.  us, plain -> so,
+// in the tiles of gemm_kwave.h: 1713 x 288 x 6992 36.9 -> 21.7 (G = 4), 39 x 3680 x 7808 30.5 -> 19.1 (1), 281 x 1696 x 1880
+// 16.2 -> 11.1 (1), 524 x 1440 x 3080 24.0 -> 17.9 (2), 130 x 712 x 2240 9.6 -> 6.8 (1), over 90 shapes, K from 500 to 8192, 10%
+// on average; in larger ones 690 x 2904 x 5696 54.3 -> 35.4, 5161 x 1128 x 2408 47.0 -> 33.6, 2702 x 2368 x 2752 46.7 -> 38.3,
+// 3959 x 419 x 424 13.9 -> 10.9, over 150 shapes 5%.  Where little is filled into LDS in all (7 Mi elements, under a short sum 12)
+// the fabric is no bound, and a few instructions in front of the first load are 0.1 us (28 x 264 x 3008 6.1, 6.2; 2464 x 416 x
+// 256 8.6, 8.8); nor is it for two bands of the larger tiles (84 x 5128 x 2264 20.5, 20.9).
+static int band_group(int M, int N, int K, int rows, int cols) {
+  const int tiles_m = (M + rows - 1) / rows, tiles_n = (N + cols - 1) / cols;
+  if (tiles_m < (rows * cols > 64 * 64 ? 3 : 2) || (double)tiles_m * tiles_n * (rows + cols) * K < (K < 1024 ? 12e6 : 7e6)) return -1;
+  double most = 0.8 * (8.0 * M + (tiles_n % 8 ? 8.0 : 1.0) * N);
+  int order = -1;
+  for (int lg = 0; lg <= 3 && (1 << lg) <= tiles_m && (lg == 0 || tiles_n << lg <= 64); ++lg) {
+    const double fetched = (8.0 * M) / (1 << lg) + (double)N * (1 << lg);
+    if (fetched <= most) order = -2 - lg, most = fetched;
+  }
+  return order;
+}
+
 // What a GEMM+LayerNorm call does and the workspace it needs: one function, so that the entry point and the
 // workspace queries cannot disagree.
 //   plain     the problem is outside what the tiled kernels take (K below 8 or beyond a descriptor, gamma or beta not
@@ -1724,6 +1745,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     KwLnParams p;
     kw_params(&p, kw, A, B, Y, M, N, K);
     p.divs = band_order_divs(p.tiles_n, 1, -1);
+    p.band_group = p.tiles_n <= kKwLnShortBand ? -1 : band_group(M, N, K, kw.rows, kw.cols);
     if (capturing != hipStreamCaptureStatusNone) BEAM_HIP(launch_ln_replay_bump((int*)ws, st));
     char* sets = (char*)ws + ln_fused_header_bytes();
     p.stats = (float*)sets;
@@ -1785,7 +1807,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     const int rounds_grouped = whole_bands ? (p.tiles_m + kNumXcd * bx - 1) / (kNumXcd * bx) : rounds_spread;
     const long per_xcd = ((long)p.tiles_m * p.tiles_n + kNumXcd - 1) / kNumXcd;
     if ((per_xcd + 31) / 32 < rounds_grouped) {
-      p.group_n = -1;
+      p.group_n = band_group(M, N, K, c.block_m, c.block_n);
       grid = (unsigned)(p.tiles_m * p.tiles_n);
     } else if (whole_bands) {
       p.group_n = 0;
@@ -2201,6 +2223,9 @@ int beam_dbg_band_block_tile(int wg, int tiles_m, int tiles_n, int gb, int gc, i
 
 int beam_dbg_band_block_grid(int tiles_m, int gb, int gc) { return band_block_grid(tiles_m, gb, gc); }
 
+int beam_dbg_ln_band_order(int M, int N, int K, int rows, int cols) {
+  return M < 1 || N < 1 || K < 1 || rows < 1 || cols < 1 ? 0 : band_group(M, N, K, rows, cols);
+}
 int beam_dbg_band_order_tile(int id, int tiles_m, int tiles_n, int group_m, int group_n, int* tm, int* tn) {
   if (tiles_m < 1 || tiles_n < 1 || group_m < 1 || id < 0 || !tm || !tn) return fail(BEAM_ERR_INVALID, "bad band-order query");
   const TileCoord t = band_order_tile(id, tiles_m, tiles_n, group_m, group_n, band_order_divs(tiles_n, group_m, group_n));

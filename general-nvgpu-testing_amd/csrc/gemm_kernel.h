@@ -126,7 +126,7 @@ struct GemmParams {
   int splits;    // number of K slices (1 = no split); the grid holds tiles_m * tiles_n * splits workgroups
   int group_m;   // rasterisation group height in tiles (fused LayerNorm: bands per band group)
   int group_n;   // fused LayerNorm: columns of a band group owned by one XCD; 0: whole bands, group_m of them, per XCD;
-                 // -1: band after band, workgroup id = band * tiles_n + column (no padding)
+                 // -1: band after band, workgroup id = band * tiles_n + column (no padding); less: band_group_tile
   int ln_ids;    // fused LayerNorm on the kernel of gemm_w4.h: ids of that order, padding included; the grid may be smaller
                  // (a workgroup then walks the ids blockIdx, blockIdx + gridDim, ...)
   TileDivs divs; // the tile maps' divisors as multipliers (tile_map.h), made by the host from tiles_m, tiles_n, group_m
@@ -550,7 +550,7 @@ struct GemmTile {
     if (EPI == kEpiLnFused) {
       tc = p.group_n > 0    ? band_block_tile(blockIdx.x, p.tiles_m, p.tiles_n, p.group_m, p.group_n)
            : p.group_n == 0 ? band_xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, p.group_m)
-                            : TileCoord{(int)blockIdx.x / p.tiles_n, (int)blockIdx.x % p.tiles_n};
+                            : band_order_tile(blockIdx.x, p.tiles_m, p.tiles_n, 1, p.group_n, p.divs);
       if (tc.tm < 0) return;
     } else if (p.splits > 1) {
       const int tiles = p.tiles_m * p.tiles_n;

@@ -50,7 +50,7 @@ struct KwSideParams : KwParams {
   long long side_count;
 };
 
-// GEMM+LayerNorm: the exchange of gemm_kernel.h, workgroups in band order (id = band * tiles_n + column tile).
+// GEMM+LayerNorm: the exchange of gemm_kernel.h, workgroups in one of the orders without padding.
 struct KwLnParams : KwParams {
   float* stats;  // 8-byte words [tiles_m][tiles_n][ROWS] = (mean, tag)
   float* next_stats;  // ... = (M2, ~tag)
@@ -61,6 +61,7 @@ struct KwLnParams : KwParams {
   unsigned ln_nonce;
   float eps;
   int spin_limit;
+  int band_group;  // band_order_tile's group_n
 };
 
 // Column tiles of a band that stays together on an XCD.  A launch that shares the device and gets s of an XCD's 32 CUs still
@@ -439,9 +440,10 @@ struct KwTile {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // Short bands stay together on an XCD, which then fetches their rows once (1298 x 312 x 7512 28.7 -> 25.9 us); long ones
-    // are spread in id order.
+    // are spread (capi.hip: band_group).
     const int id = p.tiles_n <= kKwLnShortBand ? xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n) : (int)blockIdx.x;
-    const int tm = (int)fast_div((unsigned)id, p.divs.tiles), tn = id - tm * p.tiles_n;
+    const TileCoord tc = band_order_tile(id, p.tiles_m, p.tiles_n, 1, p.band_group, p.divs);
+    const int tm = tc.tm, tn = tc.tn;
     const int row0 = tm * ROWS, col0 = tn * COLS;
     const int M = p.M, N = p.N;
     char* const ring = smem + wave * (S * SLOT);

@@ -190,6 +190,29 @@ BEAM_HD TileCoord band_block_tile(int wg, int tiles_m, int tiles_n, int gb, int 
   return t;
 }
 
+// The same contract without padding, for ids that follow one another through whole bands: groups of G = 1 << lg bands (1 to 8),
+// G * tiles_n at most the CUs that a launch can count on; in a group the XCDs congruent modulo G hold a band, and an XCD holds
+// about the same columns in every group, however tiles_n divides.  An XCD then fetches the rows of one band of a group and
+// G / 8 of the columns; of plain ids (id = band * tiles_n + column) all rows and, where 8 does not divide tiles_n, all columns.
+// The bands behind the last whole group go one by one.  band = id / tiles_n.  Bijection on [0, tiles_m * tiles_n).
+BEAM_HD TileCoord band_group_tile(int id, int band, int tiles_m, int tiles_n, int lg) {
+  int first = band >> lg << lg;
+  if (first + (1 << lg) > tiles_m) {
+    first = band;
+    lg = 0;
+  }
+  const int start = first * tiles_n, x = id & 7;
+  const int q = (tiles_n << lg) >> 3, r = (tiles_n << lg) & 7;  // of a group's workgroups an XCD gets q, r of them one more
+  const unsigned ones = (1u << r) - 1u, turn = (unsigned)start & 7u;
+  const unsigned more = (ones << turn | ones >> (8u - turn)) & 0xffu;  // ... these
+  // the XCDs of this band in front of this one
+  const unsigned below = (lg == 0 ? 0xffu : lg == 1 ? 0x55u : lg == 2 ? 0x11u : 0x01u) << (x & ((1 << lg) - 1)) & ((1u << x) - 1u);
+  TileCoord t;
+  t.tm = first + (x & ((1 << lg) - 1));
+  t.tn = (x >> lg) * q + __builtin_popcount(more & below) + ((id - start) >> 3);
+  return t;
+}
+
 // Number of workgroups of that padded grid.
 BEAM_HD int band_block_grid(int tiles_m, int gb, int gc) {
   return kNumXcd * ((tiles_m + gb - 1) / gb) * gb * gc;
@@ -245,7 +268,8 @@ BEAM_HD TileCoord tile_of_workgroup(int wg, int tiles_m, int tiles_n, int group_
 // The three workgroup orders of the fused GEMM+LayerNorm as one map with its divisions done by multiplication (what
 // the kernels call; a host test walks it against the defining functions above over every id of many grids).
 //   group_n > 0: band_block_tile with gb = group_m, gc = group_n;  group_n == 0: band_xcd_tile with bx = group_m;
-//   group_n < 0: band after band, id = band * tiles_n + column, no padding.
+//   group_n == -1: band after band, id = band * tiles_n + column, no padding;  group_n < -1: band_group_tile with
+//   lg = -2 - group_n.
 BEAM_HD TileDivs band_order_divs(int tiles_n, int group_m, int group_n) {
   TileDivs d;
   const int g = group_m < 1 ? 1 : group_m;
@@ -260,7 +284,7 @@ BEAM_HD TileCoord band_order_tile(int id, int tiles_m, int tiles_n, int group_m,
   if (group_n < 0) {
     t.tm = (int)fast_div((unsigned)id, dv.tiles);
     t.tn = id - t.tm * tiles_n;
-    return t;
+    return group_n < -1 ? band_group_tile(id, t.tm, tiles_m, tiles_n, -2 - group_n) : t;
   }
   const int xcd = id % kNumXcd;
   const int local = id / kNumXcd;

@@ -99,9 +99,11 @@ int beam_dbg_w4_kmajor_read_offset(int wn, int b, int g, int e, int q);
 int beam_dbg_band_block_tile(int wg, int tiles_m, int tiles_n, int gb, int gc, int* tm, int* tn);
 int beam_dbg_band_block_grid(int tiles_m, int gb, int gc);
 /* The three orders as the kernels compute them, divisions done by multiplication: group_n > 0 is the band-block
- * order with gb = group_m and gc = group_n, group_n == 0 the whole-bands order with bx = group_m, group_n < 0 plain
- * band after band (id = band * tiles_n + column). */
+ * order with gb = group_m and gc = group_n, group_n == 0 the whole-bands order with bx = group_m, group_n == -1 plain
+ * band after band (id = band * tiles_n + column), group_n < -1 the same in groups of 1 << (-2 - group_n) bands. */
 int beam_dbg_band_order_tile(int id, int tiles_m, int tiles_n, int group_m, int group_n, int* tm, int* tn);
+/* The group_n of the orders without padding that GEMM+LayerNorm runs in with tiles of rows x cols (0: bad argument). */
+int beam_dbg_ln_band_order(int M, int N, int K, int rows, int cols);
 /* The same for the order that keeps whole bands (bx at a time) on one XCD, used when a band is
  * short enough for it. */
 int beam_dbg_band_xcd_tile(int wg, int tiles_m, int tiles_n, int bx, int* tm, int* tn);

@@ -430,3 +430,32 @@ def test_checked_calls_wait_for_their_result(gpu, beamc):
         chk(L.beam_gemmrc(big.ptr, big.ptr, out.ptr, 8192, 8192, 8192, BF16, None, None))
     assert beamc.gemmrc_ln(da, db, y, dg, dbt) is False
     assert (y.to_numpy() == want).all()
+
+
+# (M, N, K), the tile, the order's group_n: bands in groups of 1, 2, 4 and 8, bands left over behind the last group, in the tiles
+# of the wavefront kernel and in larger ones
+BAND_GROUPS = [((39, 3680, 4008), (16, 64), -2), ((281, 1696, 1880), (32, 64), -2), ((524, 1440, 3080), (64, 64), -3), ((1713, 288, 3192), (64, 32), -4),
+               ((690, 2904, 2496), (64, 128), -2), ((2702, 2368, 1752), (256, 128), -3), ((3161, 1128, 1408), (128, 128), -4), ((6660, 328, 1728), (96, 128), -5)]
+
+
+def test_bands_in_groups_are_reached(gpu, beamc):
+    import ctypes
+    from test_host_logic import small_tile
+    for (M, N, K), tile, order in BAND_GROUPS:
+        small = small_tile(beamc, 3, M, N, K, 1)
+        if small[0]:
+            got = small[:2]
+        else:
+            cfg, lines = beamc._TileCfg(), ctypes.c_int()
+            beamc._check(beamc.lib.beam_dbg_ln_line_tile(M, N, K, ctypes.byref(cfg), ctypes.byref(lines)))
+            got = cfg.block_m, cfg.block_n
+        assert tuple(got) == tile and beamc.lib.beam_dbg_ln_band_order(M, N, K, *tile) == order, ((M, N, K), got, beamc.lib.beam_dbg_ln_band_order(M, N, K, *got))
+
+
+@pytest.mark.parametrize("shape", [s[0] for s in BAND_GROUPS] + [(3959, 419, 424)])
+def test_bands_in_groups(gpu, beamc, oracle, shape):
+    M, N, K = shape
+    a, b, g, bt = make_ln_inputs(beamc, M, N, K, BF16, 28)
+    ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, BF16)
+    for mode in (beamc.LN_AUTO, beamc.LN_FUSED):
+        check_ln(oracle, run_ln(beamc, a, b, g, bt, BF16, mode=mode), ref, BF16, f"{shape} mode {mode}")

@@ -578,6 +578,30 @@ def test_band_orders_by_multiplication_match_their_definitions(beamc):
             assert (c.value, d.value) == (wg // tiles_n, wg % tiles_n)
 
 
+@pytest.mark.parametrize("lg", [0, 1, 2, 3])
+def test_bands_in_groups(beamc, lg):
+    """The order of bands in groups of G = 1 << lg: every tile once, a group's ids together and before the next group's, in a whole
+    group a band on the XCDs of one residue modulo G, and on each XCD about the same columns in every group."""
+    import ctypes
+    L, G = beamc.lib, 1 << lg
+    c, d = ctypes.c_int(), ctypes.c_int()
+    for tiles_m, tiles_n in [(1, 1), (1, 64), (2, 9), (3, 55), (8, 8), (9, 23), (17, 10), (24, 9), (27, 9), (23, 16), (40, 7), (64, 33), (100, 1)]:
+        seen, columns = set(), {}
+        for wg in range(tiles_m * tiles_n):
+            assert L.beam_dbg_band_order_tile(wg, tiles_m, tiles_n, 1, -2 - lg, ctypes.byref(c), ctypes.byref(d)) == 0
+            tm, tn = c.value, d.value
+            assert 0 <= tm < tiles_m and 0 <= tn < tiles_n
+            seen.add((tm, tn))
+            first = wg // tiles_n // G * G
+            if first + G <= tiles_m:
+                assert first <= tm < first + G and tm % G == wg % G
+                columns.setdefault(wg % 8, set()).add(tn)
+            else:
+                assert tm == wg // tiles_n
+        assert len(seen) == tiles_m * tiles_n
+        assert all(len(v) <= -(-tiles_n * G // 8) + 1 for v in columns.values()), (tiles_m, tiles_n, columns)
+
+
 def test_division_by_multiplication(beamc):
     """The kernels divide by launch constants with a multiply-high and a shift (tile_map.h: FastDiv): exact for
     every numerator below 2^31, checked on small numbers exhaustively, around every multiple of the divisor that a
