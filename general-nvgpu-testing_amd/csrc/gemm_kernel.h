@@ -1352,30 +1352,37 @@ struct GemmTile {
           for (int j = 0; j < FN; ++j)
             *(vec4*)(stage + i * 16 * RB + w_off + (((2 * j + (wg >> 1)) ^ chunk_xor(wr)) << 4)) = value(hf * FMH + i, j, ctx);
         }
+        auto at = [&](int it, int* m, int* n_st) __attribute__((always_inline)) {
+          const int r = it * RPI + srow;
+          vec8 v = *(const vec8*)(stage + r * RB + schunk * 16);
+          if ((r >> 3) & 1) v = vec8{v[4], v[5], v[6], v[7], v[0], v[1], v[2], v[3]};
+          *n_st = col0 + wn * TN + (schunk ^ chunk_xor(r)) * 8;
+          *m = row0 + wm * TM + hf * FMH * 16 + r;
+          return v;
+        };
         // one copy of the loop for each kind, not a branch per store: the reads of a pass stay batched ahead of its stores
         auto store_pass = [&](auto kind_tag) __attribute__((always_inline)) {
 #pragma unroll
           for (int it = 0; it < FMH * 16 / RPI; ++it) {
-            const int r = it * RPI + srow;
-            vec8 v = *(const vec8*)(stage + r * RB + schunk * 16);
-            if ((r >> 3) & 1) v = vec8{v[4], v[5], v[6], v[7], v[0], v[1], v[2], v[3]};
-            const int n_st = col0 + wn * TN + (schunk ^ chunk_xor(r)) * 8;
-            const int m = row0 + wm * TM + hf * FMH * 16 + r;
-            if (m < M) {
-              T* dst = C + (size_t)m * N + n_st;
-              if (n_st + 7 < N) {  // (at any element's address)
-                store_16<decltype(kind_tag)::value>(dst, __builtin_bit_cast(i32x4, v));
-              } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                  if (n_st + e < N) dst[e] = v[e];
-              }
-            }
+            int m, n_st;
+            const vec8 v = at(it, &m, &n_st);
+            if (m < M && n_st + 7 < N) store_16<decltype(kind_tag)::value>(C + (size_t)m * N + n_st, __builtin_bit_cast(i32x4, v));  // (at any element's address)
           }
         };
         if (p.c_store == kStoreThrough) store_pass(std::integral_constant<int, kStoreThrough>{});  // (uniform)
-        else if (p.c_store == kStoreCached) store_pass(std::integral_constant<int, kStoreCached>{});
-        else store_pass(std::integral_constant<int, kStoreStreaming>{});
+        else store_pass(std::integral_constant<int, kStoreCached>{});
+        if ((N & 7) != 0 && col0 + wn * TN + TN > N) {  // the row's last chunk
+#pragma unroll 1
+          for (int it = 0; it < FMH * 16 / RPI; ++it) {
+            int m, n_st;
+            const vec8 v = at(it, &m, &n_st);
+            if (m < M && n_st < N && n_st + 7 >= N) {
+#pragma unroll
+              for (int e = 0; e < 7; ++e)
+                if (n_st + e < N) C[(size_t)m * N + n_st + e] = v[e];
+            }
+          }
+        }
       }
     };
 

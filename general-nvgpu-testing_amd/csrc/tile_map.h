@@ -130,12 +130,20 @@ BEAM_HD FastDiv make_fast_div(unsigned d) {
 BEAM_HD unsigned fast_div(unsigned n, FastDiv f) {
   return f.mul == 0u ? n : (unsigned)(((unsigned long long)n * f.mul) >> 32) >> f.shift;
 }
+// Constants of band_group_tile (band_order_divs).
+struct BandGroup {
+  int lg;            // a group has 1 << lg bands
+  int share;         // workgroups of a group that every XCD gets
+  unsigned more;     // those that get one more, of a group that starts with an id of XCD 0: a bit each, twice
+  unsigned residue;  // the XCDs 0, 1 << lg, ..: a bit each
+};
 // The divisors of a launch's tile maps (made once on the host, passed with the kernel's arguments).
 struct TileDivs {
   FastDiv group;      // group_m * tiles_n: tiles per group of tile rows
   FastDiv rows;       // group_m: tile rows of a full group
   FastDiv rows_last;  // tile rows of the last, short group (= rows when tiles_m is a multiple of group_m)
   FastDiv tiles;      // tiles_m * tiles_n (split-K: workgroup -> slice)
+  BandGroup bands;    // of band_group_tile
 };
 BEAM_HD TileDivs make_tile_divs(int tiles_m, int tiles_n, int group_m) {
   TileDivs d;
@@ -145,6 +153,7 @@ BEAM_HD TileDivs make_tile_divs(int tiles_m, int tiles_n, int group_m) {
   const int last = tiles_m % g;
   d.rows_last = make_fast_div((unsigned)(last ? last : g));
   d.tiles = make_fast_div((unsigned)(tiles_m * tiles_n));
+  d.bands = BandGroup{0, 0, 0, 0};
   return d;
 }
 
@@ -187,29 +196,6 @@ BEAM_HD TileCoord band_block_tile(int wg, int tiles_m, int tiles_n, int gb, int 
   t.tm = bg * gb + within / gc;
   t.tn = xcd * gc + within % gc;
   if (t.tm >= tiles_m || t.tn >= tiles_n) t.tm = -1;
-  return t;
-}
-
-// The same contract without padding, for ids that follow one another through whole bands: groups of G = 1 << lg bands (1 to 8),
-// G * tiles_n at most the CUs that a launch can count on; in a group the XCDs congruent modulo G hold a band, and an XCD holds
-// about the same columns in every group, however tiles_n divides.  An XCD then fetches the rows of one band of a group and
-// G / 8 of the columns; of plain ids (id = band * tiles_n + column) all rows and, where 8 does not divide tiles_n, all columns.
-// The bands behind the last whole group go one by one.  band = id / tiles_n.  Bijection on [0, tiles_m * tiles_n).
-BEAM_HD TileCoord band_group_tile(int id, int band, int tiles_m, int tiles_n, int lg) {
-  int first = band >> lg << lg;
-  if (first + (1 << lg) > tiles_m) {
-    first = band;
-    lg = 0;
-  }
-  const int start = first * tiles_n, x = id & 7;
-  const int q = (tiles_n << lg) >> 3, r = (tiles_n << lg) & 7;  // of a group's workgroups an XCD gets q, r of them one more
-  const unsigned ones = (1u << r) - 1u, turn = (unsigned)start & 7u;
-  const unsigned more = (ones << turn | ones >> (8u - turn)) & 0xffu;  // ... these
-  // the XCDs of this band in front of this one
-  const unsigned below = (lg == 0 ? 0xffu : lg == 1 ? 0x55u : lg == 2 ? 0x11u : 0x01u) << (x & ((1 << lg) - 1)) & ((1u << x) - 1u);
-  TileCoord t;
-  t.tm = first + (x & ((1 << lg) - 1));
-  t.tn = (x >> lg) * q + __builtin_popcount(more & below) + ((id - start) >> 3);
   return t;
 }
 
@@ -265,6 +251,20 @@ BEAM_HD TileCoord tile_of_workgroup(int wg, int tiles_m, int tiles_n, int group_
   return grouped_tile(xcd_remap(wg, tiles_m * tiles_n), tiles_m, tiles_n, group_m, dv);
 }
 
+// The band orders' contract without padding, for ids that follow one another through whole bands: groups of G = 1 << lg bands
+// (1 to 8), G * tiles_n at most the CUs that a launch can count on; in a group the XCDs congruent modulo G hold a band, and an
+// XCD holds about the same columns in every group, however tiles_n divides.  An XCD then fetches the rows of one band of a group
+// and G / 8 of the columns; of plain ids (id = band * tiles_n + column) all rows and, where 8 does not divide tiles_n, all
+// columns.  The bands behind the last whole group keep plain ids.  band = id / tiles_n.  Bijection on [0, tiles_m * tiles_n).
+// (Every instruction here is in front of a launch's first load: 100 of them, as a first form had, were 0.3 us of 7.)
+BEAM_HD TileCoord band_group_tile(int id, int band, int tiles_m, int tiles_n, const BandGroup& g) {
+  const int bands = 1 << g.lg, first = band & -bands;
+  if (first + bands > tiles_m) return TileCoord{band, id - band * tiles_n};
+  const int start = first * tiles_n, x = id & 7, b = x & (bands - 1);
+  const unsigned below = (g.residue << b) & ((1u << x) - 1u);  // the XCDs of this band in front of this one
+  return TileCoord{first + b, (x >> g.lg) * g.share + __builtin_popcount((g.more >> (8 - (start & 7))) & below) + ((id - start) >> 3)};
+}
+
 // The three workgroup orders of the fused GEMM+LayerNorm as one map with its divisions done by multiplication (what
 // the kernels call; a host test walks it against the defining functions above over every id of many grids).
 //   group_n > 0: band_block_tile with gb = group_m, gc = group_n;  group_n == 0: band_xcd_tile with bx = group_m;
@@ -277,14 +277,18 @@ BEAM_HD TileDivs band_order_divs(int tiles_n, int group_m, int group_n) {
   d.rows = make_fast_div((unsigned)(group_n > 0 ? group_n : (tiles_n < 1 ? 1 : tiles_n)));  // columns of an XCD's block
   d.rows_last = d.rows;
   d.tiles = make_fast_div((unsigned)(tiles_n < 1 ? 1 : tiles_n));
+  const int lg = group_n < -1 ? -2 - group_n : 0;
+  const unsigned residue[4] = {0xff, 0x55, 0x11, 0x01};
+  d.bands = BandGroup{lg, (tiles_n << lg) >> 3, ((1u << ((tiles_n << lg) & 7)) - 1u) * 0x101u, residue[lg & 3]};
   return d;
 }
 BEAM_HD TileCoord band_order_tile(int id, int tiles_m, int tiles_n, int group_m, int group_n, const TileDivs& dv) {
   TileCoord t;
   if (group_n < 0) {
     t.tm = (int)fast_div((unsigned)id, dv.tiles);
+    if (group_n < -1) return band_group_tile(id, t.tm, tiles_m, tiles_n, dv.bands);
     t.tn = id - t.tm * tiles_n;
-    return group_n < -1 ? band_group_tile(id, t.tm, tiles_m, tiles_n, -2 - group_n) : t;
+    return t;
   }
   const int xcd = id % kNumXcd;
   const int local = id / kNumXcd;
