@@ -1744,8 +1744,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     kw.shift = kw_plan(M, N, K, false, true, false, row_starts(A, B, K, false), g_dev.cus).shift;
     KwLnParams p;
     kw_params(&p, kw, A, B, Y, M, N, K);
-    p.divs = band_order_divs(p.tiles_n, 1, -1);
-    p.band_group = p.tiles_n <= kKwLnShortBand ? -1 : band_group(M, N, K, kw.rows, kw.cols);
+    p.divs = band_order_divs(p.tiles_n, 1, p.tiles_n <= kKwLnShortBand ? -1 : band_group(M, N, K, kw.rows, kw.cols));
     if (capturing != hipStreamCaptureStatusNone) BEAM_HIP(launch_ln_replay_bump((int*)ws, st));
     char* sets = (char*)ws + ln_fused_header_bytes();
     p.stats = (float*)sets;

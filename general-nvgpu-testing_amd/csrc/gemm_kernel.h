@@ -550,7 +550,7 @@ struct GemmTile {
     if (EPI == kEpiLnFused) {
       tc = p.group_n > 0    ? band_block_tile(blockIdx.x, p.tiles_m, p.tiles_n, p.group_m, p.group_n)
            : p.group_n == 0 ? band_xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, p.group_m)
-                            : band_order_tile(blockIdx.x, p.tiles_m, p.tiles_n, 1, p.group_n, p.divs);
+                            : unpadded_band_tile(blockIdx.x, p.tiles_m, p.tiles_n, p.divs);
       if (tc.tm < 0) return;
     } else if (p.splits > 1) {
       const int tiles = p.tiles_m * p.tiles_n;

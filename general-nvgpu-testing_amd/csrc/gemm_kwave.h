@@ -61,7 +61,6 @@ struct KwLnParams : KwParams {
   unsigned ln_nonce;
   float eps;
   int spin_limit;
-  int band_group;  // band_order_tile's group_n
 };
 
 // Column tiles of a band that stays together on an XCD.  A launch that shares the device and gets s of an XCD's 32 CUs still
@@ -442,7 +441,7 @@ struct KwTile {
     // Short bands stay together on an XCD, which then fetches their rows once (1298 x 312 x 7512 28.7 -> 25.9 us); long ones
     // are spread (capi.hip: band_group).
     const int id = p.tiles_n <= kKwLnShortBand ? xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n) : (int)blockIdx.x;
-    const TileCoord tc = band_order_tile(id, p.tiles_m, p.tiles_n, 1, p.band_group, p.divs);
+    const TileCoord tc = unpadded_band_tile(id, p.tiles_m, p.tiles_n, p.divs);
     const int tm = tc.tm, tn = tc.tn;
     const int row0 = tm * ROWS, col0 = tn * COLS;
     const int M = p.M, N = p.N;

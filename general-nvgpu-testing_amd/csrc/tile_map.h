@@ -132,7 +132,7 @@ BEAM_HD unsigned fast_div(unsigned n, FastDiv f) {
 }
 // Constants of band_group_tile (band_order_divs).
 struct BandGroup {
-  int lg;            // a group has 1 << lg bands
+  int lg;            // a group has 1 << lg bands; -1: plain ids
   int share;         // workgroups of a group that every XCD gets
   unsigned more;     // those that get one more, of a group that starts with an id of XCD 0: a bit each, twice
   unsigned residue;  // the XCDs 0, 1 << lg, ..: a bit each
@@ -153,7 +153,7 @@ BEAM_HD TileDivs make_tile_divs(int tiles_m, int tiles_n, int group_m) {
   const int last = tiles_m % g;
   d.rows_last = make_fast_div((unsigned)(last ? last : g));
   d.tiles = make_fast_div((unsigned)(tiles_m * tiles_n));
-  d.bands = BandGroup{0, 0, 0, 0};
+  d.bands = BandGroup{-1, 0, 0, 0};
   return d;
 }
 
@@ -265,6 +265,15 @@ BEAM_HD TileCoord band_group_tile(int id, int band, int tiles_m, int tiles_n, co
   return TileCoord{first + b, (x >> g.lg) * g.share + __builtin_popcount((g.more >> (8 - (start & 7))) & below) + ((id - start) >> 3)};
 }
 
+// Either order without padding (band_order_divs with group_n < 0).  (Which of them stands among the divisors: an argument that lies
+// behind the launch's first ones is another trip to memory in front of the first load, 0.25 us.)
+BEAM_HD TileCoord unpadded_band_tile(int id, int tiles_m, int tiles_n, const TileDivs& dv) {
+  const int band = (int)fast_div((unsigned)id, dv.tiles);
+  TileCoord t = {band, id - band * tiles_n};
+  if (dv.bands.lg >= 0) t = band_group_tile(id, band, tiles_m, tiles_n, dv.bands);
+  return t;
+}
+
 // The three workgroup orders of the fused GEMM+LayerNorm as one map with its divisions done by multiplication (what
 // the kernels call; a host test walks it against the defining functions above over every id of many grids).
 //   group_n > 0: band_block_tile with gb = group_m, gc = group_n;  group_n == 0: band_xcd_tile with bx = group_m;
@@ -277,18 +286,15 @@ BEAM_HD TileDivs band_order_divs(int tiles_n, int group_m, int group_n) {
   d.rows = make_fast_div((unsigned)(group_n > 0 ? group_n : (tiles_n < 1 ? 1 : tiles_n)));  // columns of an XCD's block
   d.rows_last = d.rows;
   d.tiles = make_fast_div((unsigned)(tiles_n < 1 ? 1 : tiles_n));
-  const int lg = group_n < -1 ? -2 - group_n : 0;
+  const int lg = group_n < -1 ? -2 - group_n : -1;
   const unsigned residue[4] = {0xff, 0x55, 0x11, 0x01};
-  d.bands = BandGroup{lg, (tiles_n << lg) >> 3, ((1u << ((tiles_n << lg) & 7)) - 1u) * 0x101u, residue[lg & 3]};
+  d.bands = lg < 0 ? BandGroup{-1, 0, 0, 0} : BandGroup{lg, (tiles_n << lg) >> 3, ((1u << ((tiles_n << lg) & 7)) - 1u) * 0x101u, residue[lg & 3]};
   return d;
 }
 BEAM_HD TileCoord band_order_tile(int id, int tiles_m, int tiles_n, int group_m, int group_n, const TileDivs& dv) {
   TileCoord t;
   if (group_n < 0) {
-    t.tm = (int)fast_div((unsigned)id, dv.tiles);
-    if (group_n < -1) return band_group_tile(id, t.tm, tiles_m, tiles_n, dv.bands);
-    t.tn = id - t.tm * tiles_n;
-    return t;
+    return unpadded_band_tile(id, tiles_m, tiles_n, dv);
   }
   const int xcd = id % kNumXcd;
   const int local = id / kNumXcd;
