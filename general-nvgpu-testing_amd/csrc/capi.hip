@@ -1432,7 +1432,7 @@ static int ln_resolve_cfg(const beam_tile_cfg* cfg, int M, int N, int K, int mod
 // round of bands and per launch, least squares on the logarithm over 160 and 200 shapes with M from 64 to 8192, N and K from 256 to 8192.
 // `named` stays unless another tile is 4% ahead by it.  Its pick is 1.8% (off lines) and 3.3% (on) behind the best tile on
 // average, `named` 12 and 11%; the tiles with rings deeper than 3 + 2 slots are ahead on lines too.  us, before -> now: 1978 x 2120 x
-// 4888 86 -> 59, 2908 x 328 x 5736 51 -> 33, 1891 x 920 x 3704 40 -> 28, 6257 x 2744 x 4688 243 -> 196; on lines 1064 x 1040 x
+// 4888 86 -> 59 (48 with bands in groups), 2908 x 328 x 5736 51 -> 33, 1891 x 920 x 3704 40 -> 28, 6257 x 2744 x 4688 243 -> 196; on lines 1064 x 1040 x
 // 3776 42 -> 29, 126 x 6720 x 1472 21.6 -> 19.0.
 static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) {
   struct Candidate {
