@@ -51,3 +51,39 @@ def test_compiler_never_touches_the_accumulators(tmp_path, source, count):
             if l.startswith(("s_add_u32 m0", ".LBB", "s_branch", "s_endpgm")) or writes.match(l):
                 break
             assert not reads.match(l), f"line {i}: `{l}` tests the condition bit an M0 add in inline assembly has overwritten"
+
+
+def test_restored_scalars_reach_memory_instructions_late_enough(tmp_path):
+    """A memory instruction may read a scalar register that a vector instruction wrote (v_readlane, which restores a
+    parked one) only 5 wait states later.  The compiler sees to that for its own instructions and does not look into
+    inline assembly: an order of the kernels' arguments that made it park more scalars put one right in front of a load
+    there, and the fused LayerNorm came out wrong (256 x 512 x 256)."""
+    out = tmp_path / "w4.s"
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Wno-unused-command-line-argument",
+                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-S", "--cuda-device-only",
+                    "-o", str(out), os.path.join(CSRC, "gemm_inst_w4.hip")], check=True, capture_output=True, timeout=600)
+
+    def scalars(text):
+        regs = {int(r) for r in re.findall(r"\bs(\d+)\b", text)}
+        for first, last in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+            regs |= set(range(int(first), int(last) + 1))
+        return regs
+
+    at, written, restores = 0, {}, 0
+    for line in out.read_text().splitlines():
+        line = line.split(";")[0].strip()
+        if not line or line.startswith(".") or line.endswith(":"):
+            continue
+        op, _, args = line.partition(" ") if " " in line else line.partition("\t")
+        first = args.split(",")[0]
+        at += int(args, 0) + 1 if op == "s_nop" else 1
+        if op.startswith(("buffer_", "global_")):
+            late = [r for r in scalars(args) if r in written and at - written[r] - 1 < 5]
+            assert not late, f"`{line}` reads s{late} {at - written[late[0]] - 1} wait states after a vector instruction wrote it"
+        elif op in ("v_readlane_b32", "v_readfirstlane_b32"):
+            restores += 1
+            written.update((r, at) for r in scalars(first))
+        elif op.startswith("s_"):
+            for r in scalars(first):
+                written.pop(r, None)
+    assert restores > 50
