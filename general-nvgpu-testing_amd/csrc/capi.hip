@@ -1865,7 +1865,7 @@ int beam_gemmrc_ln_checked(const void* A, const void* B, const void* gamma, cons
   LnPlan plan;
   if (ln_plan_call(A, B, gamma, beta, Y, M, N, K, cfg, BEAM_LN_AUTO, generic, false, ws, ws_bytes, &plan) || plan.kind != LnPlan::kFused)
     return BEAM_OK;  // nothing in the call waits for anything
-  if (const volatile unsigned* word = g_ln_host_timeout) {
+  if (const volatile unsigned* word = g_ln_host_timeout; word && *word == 0) {  // (set once: the header's reader waits by itself)
     BEAM_HIP(wait_for_stream(st));
     if (*word == 0) return BEAM_OK;
   }

@@ -384,6 +384,40 @@ def test_walking_kernel_ends_when_every_wait_gives_up(gpu, beamc):
         x.free()
 
 
+def test_checked_call_behind_a_timeout_costs_what_it_consists_of(gpu, beamc):
+    """Once a wait of the process has run out, a checked call is its launch and beam_gemmrc_ln_timed_out, and no more: medians of
+    200 calls each, in turn, within 10% (a kernel whose word nobody needs made it 15%)."""
+    import ctypes
+    import time
+    M, N, K = 512, 1024, 1024
+    L, chk, flag = beamc.lib, beamc._check, ctypes.c_int()
+    da, db, dg, dbt = (beamc.DeviceArray.from_numpy(x, BF16) for x in make_ln_inputs(beamc, M, N, K, BF16, 29))
+    y, ws = beamc.DeviceArray((M, N), BF16), beamc.DeviceArray((L.beam_gemmrc_ln_workspace_bytes_for(M, N, K, None, beamc.LN_AUTO),), itemsize=1)
+    args = (da.ptr, db.ptr, dg.ptr, dbt.ptr, ctypes.c_float(1e-5), y.ptr, M, N, K, BF16, None)
+    try:
+        chk(L.beam_set_ln_spin_limit(-1))
+        chk(L.beam_gemmrc_ln_checked(*args, ws.ptr, ws.nbytes, None, ctypes.byref(flag)))
+        assert flag.value == 1
+    finally:
+        L.beam_set_ln_spin_limit(beamc.DEFAULT_SPIN_LIMIT)
+    took = ([], [])
+    for _ in range(220):
+        t0 = time.perf_counter()
+        chk(L.beam_gemmrc_ln_checked(*args, ws.ptr, ws.nbytes, None, ctypes.byref(flag)))
+        t1 = time.perf_counter()
+        chk(L.beam_gemmrc_ln_ex(*args, beamc.LN_AUTO, ws.ptr, ws.nbytes, None))
+        chk(L.beam_gemmrc_ln_timed_out(ws.ptr, None, ctypes.byref(flag)))
+        t2 = time.perf_counter()
+        assert flag.value == 0
+        took[0].append(t1 - t0)
+        took[1].append(t2 - t1)
+    checked, parts = (sorted(t[20:])[100] * 1e6 for t in took)
+    print(f"checked {checked:.1f} us, launch and query {parts:.1f} us")
+    assert checked <= 1.1 * parts, (checked, parts)
+    for x in (da, db, dg, dbt, y, ws):
+        x.free()
+
+
 # small tiles; larger ones (a workgroup takes a CU), two of them by whole lines, with bands in groups, beside each other and small ones
 @pytest.mark.parametrize("shapes", [[(96, 200, 72), (512, 1024, 256), (300, 264, 1000), (64, 4096, 136)],
                                     [(690, 2904, 2496), (2702, 2368, 1752)], [(1064, 1040, 1000), (3161, 1128, 1408), (512, 1024, 256)]])
