@@ -18,9 +18,12 @@ hipError_t launch_ln_apply(const float* X, const float* stats, const void* gamma
                            void* Y, int M, int N, int tiles_n, int block_n, float eps, int dtype,
                            hipStream_t stream);
 
+// A wavefront on each XCD x writes `value` to words[x * kTellStride], x < 16, in host memory (capi.hip: wait_for_stream).
+constexpr int kTellStride = 16, kTellWords = 16 * kTellStride;
+hipError_t launch_tell_host(unsigned* words, unsigned value, hipStream_t stream);
+
 // One thread moves on the replay counter in the header of a fused GEMM+LayerNorm workspace: recorded in front
 // of a fused launch when the stream is being captured (see ln_launch_tag in gemm_kernel.h).
-hipError_t launch_tell_host(unsigned* word, unsigned value, hipStream_t stream);
 hipError_t launch_ln_replay_bump(int* header, hipStream_t stream);
 
 // gemmrc without any condition on K, N or alignment (slow; what the tiled kernels refuse runs here):

@@ -216,9 +216,13 @@ __global__ void __launch_bounds__(256) ln_rows_kernel(const float* __restrict__ 
 // workspace header.  Whatever the word held before, it holds something else afterwards.
 __global__ void ln_replay_bump_kernel(int* hdr) { hdr[kLnHdrReplay] = hdr[kLnHdrReplay] + 1; }
 
-// Runs behind a stream's work and tells the host so (capi.hip: wait_for_stream).
-__global__ void __launch_bounds__(64) tell_host_kernel(unsigned* word, unsigned value) {
-  if (threadIdx.x == 0) __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+// Runs behind a stream's work, a workgroup on each XCD, and tells the host so (capi.hip: wait_for_stream).  The release writes
+// back the L2 of the XCD that it runs on, for the host to see.
+__global__ void __launch_bounds__(64) tell_host_kernel(unsigned* words, unsigned value) {
+  constexpr int kXccId = 20, kBits = 4;  // hardware register XCC_ID, its low bits
+  static_assert(kTellWords == (1 << kBits) * kTellStride, "a word for every value");
+  const int xcd = __builtin_amdgcn_s_getreg(kXccId | (kBits - 1) << 11);
+  if (threadIdx.x == 0) __hip_atomic_store(words + xcd * kTellStride, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void empty_kernel(int* p) {
@@ -252,8 +256,8 @@ hipError_t launch_silu(const void* x, void* y, size_t count, int dtype, hipStrea
   return hipGetLastError();
 }
 
-hipError_t launch_tell_host(unsigned* word, unsigned value, hipStream_t stream) {
-  hipLaunchKernelGGL(tell_host_kernel, dim3(1), dim3(64), 0, stream, word, value);
+hipError_t launch_tell_host(unsigned* words, unsigned value, hipStream_t stream) {
+  hipLaunchKernelGGL(tell_host_kernel, dim3(kNumXcd), dim3(64), 0, stream, words, value);
   return hipGetLastError();
 }
 

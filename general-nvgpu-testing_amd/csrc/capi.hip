@@ -62,38 +62,42 @@ std::mutex g_dev_mu;
 // it too, so comparing it before and after a launch could miss this launch's own time-out between two of another's.)
 unsigned* g_ln_host_timeout = nullptr;
 
-// Words of pinned host memory, a 64-byte line each, through which a kernel at a stream's end tells a waiting thread that it has
-// come there (wait_for_stream).  Allocated with the word above; a call holds one while it waits, and without a free one waits as
-// hipStreamSynchronize does.
-constexpr int kWaitWords = 64;
-constexpr int kWaitStride = 16;  // unsigned per line
+// Sets of words of pinned host memory, a word for each XCD in a 64-byte line of its own, through which a kernel at a stream's end
+// tells a waiting thread that it has come there (wait_for_stream).  Allocated with the word above; a call holds a set while it
+// waits, and without a free one waits as hipStreamSynchronize does.
+constexpr int kWaitSets = 64;
 unsigned* g_wait_words = nullptr;
 std::atomic<unsigned long long> g_wait_free{~0ull};
 std::atomic<unsigned> g_wait_value{0};
 
-int take_wait_word() {
+int take_wait_set() {
   unsigned long long free = g_wait_free.load(std::memory_order_relaxed);
   while (free != 0)
     if (g_wait_free.compare_exchange_weak(free, free & (free - 1), std::memory_order_acquire)) return __builtin_ctzll(free);
   return -1;
 }
-void give_wait_word(int i) { g_wait_free.fetch_or(1ull << i, std::memory_order_release); }
+void give_wait_set(int i) { g_wait_free.fetch_or(1ull << i, std::memory_order_release); }
 
-// Waits until everything that `st` holds has run; not for a stream that is being captured.  hipStreamSynchronize puts a packet
-// behind the last kernel that writes caches back for the host and raises a signal: 12.2 us from an empty kernel's launch to its
-// return.  A kernel of one wavefront that writes a word which this thread watches: 9.5 (the stream's kernels run one after
-// another, and each one's end has made its writes visible to the next).  Long waits are left to the runtime.
+// Waits until everything that `st` holds has run and the host sees what it wrote; not for a stream that is being captured, and
+// only on a device of kNumXcd XCDs.  hipStreamSynchronize puts a packet behind the last kernel that writes caches back for the
+// host and raises a signal; a kernel of a wavefront on each XCD whose words this thread watches is 3 us shorter (a checked
+// GEMM+LayerNorm of 512 x 1024 x 1024 18.4 -> 15.4 us).  The stream's kernels run one after another, and a wavefront's store is
+// a release that writes back its XCD's L2: with all XCDs heard, nothing that the kernels in front wrote is left in an L2, be it
+// for memory of the device or of the host.  (One wavefront on one XCD, 15.2 us, says so of that XCD's L2 only.  Eight words in
+// one line, written and watched at once, 16.4 to 17.9.)  Long waits, and an XCD without a workgroup, are left to the runtime.
 hipError_t wait_for_stream(hipStream_t st) {
-  const int i = g_wait_words ? take_wait_word() : -1;
+  const int i = g_wait_words ? take_wait_set() : -1;
   if (i < 0) return hipStreamSynchronize(st);
-  unsigned* const word = g_wait_words + i * kWaitStride;
+  unsigned* const words = g_wait_words + i * kTellWords;
   const unsigned value = g_wait_value.fetch_add(1, std::memory_order_relaxed) + 1;
-  if (launch_tell_host(word, value, st) == hipSuccess) {
+  int told = 0;  // XCDs
+  if (launch_tell_host(words, value, st) == hipSuccess) {
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
     do {
       for (int spin = 0; spin < 32; ++spin) {
-        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == value) {
-          give_wait_word(i);
+        while (told < kNumXcd && __atomic_load_n(words + told * kTellStride, __ATOMIC_ACQUIRE) == value) ++told;
+        if (told == kNumXcd) {
+          give_wait_set(i);
           return hipSuccess;
         }
         __builtin_ia32_pause();
@@ -101,7 +105,7 @@ hipError_t wait_for_stream(hipStream_t st) {
     } while (std::chrono::steady_clock::now() < until);
   }
   const hipError_t e = hipStreamSynchronize(st);
-  if (e == hipSuccess) give_wait_word(i);  // its kernel has run; after an error it may not have, and the word stays taken
+  if (e == hipSuccess) give_wait_set(i);  // its kernel has run; after an error it may not have, and the set stays taken
   return e;
 }
 // Polls before a waiting thread gives up: of statistics slots in the fused LayerNorm (3-4 us each once the pauses
@@ -383,13 +387,14 @@ int beam_init(void) {
     return fail(BEAM_ERR_DEVICE, "device 0 is %s; this library holds gfx950 code only", prop.gcnArchName);
   }
   g_dev.status = BEAM_OK;
+  constexpr size_t kHostWordBytes = sizeof(unsigned) * (kTellStride + kWaitSets * kTellWords);
   void* word = nullptr;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // the first call may come while a stream is being captured
   (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (hipHostMalloc(&word, 64 * (1 + kWaitWords), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
-    std::memset(word, 0, 64 * (1 + kWaitWords));
+  if (hipHostMalloc(&word, kHostWordBytes, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+    std::memset(word, 0, kHostWordBytes);
     g_ln_host_timeout = (unsigned*)word;
-    g_wait_words = (unsigned*)word + kWaitStride;
+    g_wait_words = (unsigned*)word + kTellStride;
   } else {
     (void)hipGetLastError();  // without it every checked call reads the header
   }
