@@ -1491,7 +1491,7 @@ static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) 
 
 // The order of a GEMM+LayerNorm launch without padding (band_order_tile's group_n): plain ids, or groups of G bands where what
 // the XCDs fetch, 8 / G of all rows and G times all columns, becomes less by a fifth; plain ids fetch 8 times the rows and, where
-// 8 does not divide a band's column tiles, 8 times the columns.  A group takes 64 CUs at most, as a band does.  us, plain -> so,
+// 8 does not divide a band's column tiles, 8 times the columns.  A group is 64 workgroups at most, as a band is, 8 on each XCD.  us, plain -> so,
 // in the tiles of gemm_kwave.h: 1713 x 288 x 6992 36.9 -> 21.7 (G = 4), 39 x 3680 x 7808 30.5 -> 19.1 (1), 281 x 1696 x 1880
 // 16.2 -> 11.1 (1), 524 x 1440 x 3080 24.0 -> 17.9 (2), 130 x 712 x 2240 9.6 -> 6.8 (1), over 90 shapes, K from 500 to 8192, 10%
 // on average; in larger ones 690 x 2904 x 5696 54.3 -> 35.4, 5161 x 1128 x 2408 47.0 -> 33.6, 2702 x 2368 x 2752 46.7 -> 38.3,

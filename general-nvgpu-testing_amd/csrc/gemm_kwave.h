@@ -65,7 +65,10 @@ struct KwLnParams : KwParams {
 
 // Column tiles of a band that stays together on an XCD.  A launch that shares the device and gets s of an XCD's 32 CUs still
 // finishes band by band if s is at least this many: XCD 0 starts with a whole band, and each XCD's last band is what
-// the next one's first workgroups wait for.  (Longer bands, as long as a round of workgroups: any 64 CUs do.)
+// the next one's first workgroups wait for.  (Longer bands, and groups of bands, are up to 64 workgroups in id order: room for 8
+// of them on every XCD does, and 64 CUs of some XCDs do not.)  Two launches that wait may each hold the XCDs that the other one
+// needs, since the XCDs start launches independently: 512 x 1024 x 256 and 64 x 4096 x 136 have 256 workgroups each, of 96 and
+// 80 KiB of LDS.  The waits' bound then ends it.
 constexpr int kKwLnShortBand = 8;
 
 // Sum over W (4, 8 or 16) neighbouring lanes, the same bits in each of them.

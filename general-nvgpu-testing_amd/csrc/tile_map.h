@@ -252,7 +252,7 @@ BEAM_HD TileCoord tile_of_workgroup(int wg, int tiles_m, int tiles_n, int group_
 }
 
 // The band orders' contract without padding, for ids that follow one another through whole bands: groups of G = 1 << lg bands
-// (1 to 8), G * tiles_n at most the CUs that a launch can count on; in a group the XCDs congruent modulo G hold a band, and an
+// (1 to 8), G * tiles_n at most 64, so that room for 8 workgroups on every XCD finishes group after group; in a group the XCDs congruent modulo G hold a band, and an
 // XCD holds about the same columns in every group, however tiles_n divides.  An XCD then fetches the rows of one band of a group
 // and G / 8 of the columns; of plain ids (id = band * tiles_n + column) all rows and, where 8 does not divide tiles_n, all
 // columns.  The bands behind the last whole group keep plain ids.  band = id / tiles_n.  Bijection on [0, tiles_m * tiles_n).
