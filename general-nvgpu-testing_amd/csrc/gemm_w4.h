@@ -276,8 +276,14 @@ struct GemmW4 {
       // result alive across this statement and selects on the add's carry instead)
       asm volatile("s_add_u32 m0, %0, %1" ::"s"(st.lds), "n"(decltype(i_tag)::value * 4096) : "memory", "scc");
     };
-    auto load_tile_part = [&](const Stream& st, unsigned voff) __attribute__((always_inline)) {
-      asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(st.rows), "s"(st.koff) : "memory");
+    // A memory instruction may read a scalar that a vector instruction wrote (one restored from a lane, where the compiler parked
+    // it) only 5 wait states later, which the compiler keeps for its own instructions and not in front of assembly.  So a stream's
+    // first load behind a boundary of output tiles brings them along (three in the
+    // prologue, two in a tile's first K tile; 8192 x 8192 x 192, 4 tiles of 3 K tiles each, 54.8 us with and without).
+    auto load_tile_part = [&](const Stream& st, unsigned voff, auto fresh_tag) __attribute__((always_inline)) {
+      if constexpr (decltype(fresh_tag)::value)
+        asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(st.rows), "s"(st.koff) : "memory");
+      else asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(st.rows), "s"(st.koff) : "memory");
     };
     // (in `part`s of two or three scalar instructions, one part per gap; part < 0: all of them)
     bool wrap_a = false, wrap_b = false;
@@ -444,8 +450,9 @@ struct GemmW4 {
           else set_load_target(ld_a, std::integral_constant<int, ld_next>{});
         }
         if constexpr (ld >= 0) {
-          if constexpr (half == 0) load_tile_part(ld_b, voff_b[ld]);
-          else load_tile_part(ld_a, voff_a[ld]);
+          using Fresh = std::bool_constant<FIRST && ld == 0>;
+          if constexpr (half == 0) load_tile_part(ld_b, voff_b[ld], Fresh{});
+          else load_tile_part(ld_a, voff_a[ld], Fresh{});
         } else if constexpr (rd >= 0 && rd < B_READS) {
           if constexpr (B_KMAJOR) {
             const i32x2 v = read_b_transposed(sb, half, rd);  // K elements 0..3 (even read) or 4..7 of the lane's 8
@@ -482,7 +489,7 @@ struct GemmW4 {
       w4_static_for<0, LPT>([&](auto i_tag) __attribute__((always_inline)) {
         set_load_target(st, i_tag);
         asm volatile("s_nop 0");  // the wait state between the write of M0 and its use
-        load_tile_part(st, voff[decltype(i_tag)::value]);
+        load_tile_part(st, voff[decltype(i_tag)::value], std::bool_constant<decltype(i_tag)::value == 0>{});
       });
     };
     // Prologue: A and B of K tile 0, A of K tile 1 (oldest first: the first wait is about tile 0).
