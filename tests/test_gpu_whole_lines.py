@@ -108,6 +108,21 @@ def test_infinities_of_b_reach_their_columns_only(gpu, beamc, M, N, K):
     assert (out[:, cols] == np.inf).all() and np.isfinite(np.delete(out, cols, axis=1)).all()
 
 
+@pytest.mark.parametrize("offset", [0, 1, 3])
+@pytest.mark.parametrize("M,N,K", [(16500, 57, 616), (16500, 63, 336), (16500, 9, 2008), (16500, 58, 616), (33000, 65, 616), (33000, 127, 1112),
+                                   (48000, 121, 2008), (5681, 57, 2008)])
+def test_the_row_behind_the_last_that_is_fetched_stays_out(gpu, beamc, M, N, K, offset):
+    """All columns in one tile, rows of B not whole chunks: the descriptor of the last K tile ends with row K - 9 (an odd one an element
+    further on), inside a K tile, and A's elements behind it are zeros there.  Row K - 8 is infinite where a fetch beyond would begin;
+    times those zeros it would be NaN.  B starts on chunks and one and three elements off.  (The last shape has small tiles.)"""
+    assert small_tile(beamc, 1, M, N, K, 1)[0] or (N <= nn_tile(beamc, M, N, K)[0][1] and nn_tile(beamc, M, N, K)[1] == 1)
+    assert (K - 8) % 64 != 0
+    a, b = beamc.host_uniform((M, K), F16, 76, 0), beamc.host_uniform((K, N), F16, 76, 1)
+    a[:, K - 8], b[K - 8, :2] = 0x3C00, 0x7C00  # one, infinity
+    out = run(beamc, lambda pa, pb, pc: beamc.lib.beam_matmul_nn(pa, pb, pc, M, N, K, F16, None, None), a, b, (M, N), F16, (0, offset, 0)).view(np.float16)
+    assert (out[:, :2] == np.inf).all() and np.isfinite(out[:, 2:]).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(1100, 1000, 1096), (929, 1232, 200), (1478, 2024, 2008)])
 def test_infinities_stay_in_their_row_or_column(gpu, beamc, M, N, K):
     a, b = beamc.host_uniform((M, K), F16, 75, 0), beamc.host_uniform((N, K), F16, 75, 1)
