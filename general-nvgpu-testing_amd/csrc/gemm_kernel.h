@@ -288,8 +288,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, un
 //   Cached: left dirty in the L2, which puts the parts of a 64-byte sector together that rows off such sectors leave to two
 //     wavefronts or workgroups; written through, each part goes to memory by itself (3000 x 5000 x 256 in 256 x 256 tiles
 //     28.6 -> 18.2 us, 3000 x 4992 x 256 15.1).
-//   Streaming: non-temporal, so that the output's lines do not push operand panels out of the L2 (4096 x 8192 x 1024 in
-//     128 x 128 tiles 82.8 -> 65.4 us).
+//   Streaming: non-temporal, for outputs beyond the last-level cache (gemm_w4.h only).
 enum StoreKind : int { kStoreThrough = 0, kStoreCached = 1, kStoreStreaming = 2 };
 
 // (The wait states: a store of more than 8 bytes reads its data registers over several cycles, and a vector instruction
@@ -297,9 +296,9 @@ enum StoreKind : int { kStoreThrough = 0, kStoreCached = 1, kStoreStreaming = 2 
 // look into assembly text.)
 template <int KIND>
 __device__ __forceinline__ void store_16(void* dst, i32x4 v) {
+  static_assert(KIND == kStoreThrough || KIND == kStoreCached, "the others store through descriptors");
   if constexpr (KIND == kStoreThrough) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
-  else if constexpr (KIND == kStoreCached) asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
-  else asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
+  else asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 2" ::"v"(dst), "v"(v) : "memory");
 }
 
 // s_waitcnt vmcnt(N) lgkmcnt(0): at most N of this wavefront's buffer loads still in flight,

@@ -278,8 +278,8 @@ struct GemmW4 {
     };
     // A memory instruction may read a scalar that a vector instruction wrote (one restored from a lane, where the compiler parked
     // it) only 5 wait states later, which the compiler keeps for its own instructions and not in front of assembly.  So a stream's
-    // first load behind a boundary of output tiles brings them along (three in the
-    // prologue, two in a tile's first K tile; 8192 x 8192 x 192, 4 tiles of 3 K tiles each, 54.8 us with and without).
+    // first load behind a boundary of output tiles brings them along (FRESH: three in the prologue, two in a tile's first K tile; 8192 x
+    // 8192 x 192, 4 tiles of 3 K tiles each, 54.8 us with and without).
     auto load_tile_part = [&](const Stream& st, unsigned voff, auto fresh_tag) __attribute__((always_inline)) {
       if constexpr (decltype(fresh_tag)::value)
         asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(st.rows), "s"(st.koff) : "memory");
