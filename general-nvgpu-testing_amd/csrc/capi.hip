@@ -625,8 +625,8 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
 // one of the tiles whose fills take whole lines (gemm_kernel.h: Form), or one of the others, which fill at half the rate
 // there (only rows of whole lines that start behind one stay as choose_default has them).  The cost model of choose_default with constants of its own, since the straight tiles' rates are lower on such rows:
 // TFLOP/s per CU alone and with `occ` workgroups on the CU, us per round of workgroups and per launch, least squares on the logarithm over 280 shapes with M, N from 64
-// to 8192 and K from 64 to 8192 off lines.  Its pick is 1.0% (worst 18%) behind the best of these on average, 1.5% on
-// shapes that it was not fitted to; what ran before was 10% behind.  us, before -> now: 928 x 1232 x 7112 49.7 -> 27.9, 633 x
+// to 8192 and K from 64 to 8192 off lines (beam/line_tile_fit.py, with the timings).  On the 241 of them that come here its pick is
+// 1.1% behind the best of these on average, 18% at worst; what ran before took 14% more than the pick.  us, before -> now: 928 x 1232 x 7112 49.7 -> 27.9, 633 x
 // 6536 x 2952 38.5 -> 26.3, 1228 x 1784 x 6296 59.4 -> 36.9, 7702 x 7248 x 2472 268 -> 255, 2247 x 3736 x 216 12.7 -> 10.3.
 struct LineChoice {
   beam_tile_cfg cfg;
@@ -686,8 +686,9 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
 }
 
 // The same for beam_matmul_nn, where only rows of A can be off lines for K's sake: whole chunks in B's rows (N % 8 == 0), and not.
-// Fitted to 100 and 60 shapes with M and N from 32 and 64 to 8192 (5001); `named` is what choose_default's tile has become there,
-// and stays unless another is 8% ahead by the model: 7.3% and 5.6% faster than `named` on average.  us, before -> now: 3059 x 368
+// Fitted to 120 and 90 shapes with M and N from 32 and 64 to 8192 (5001); `named` is what choose_default's tile has become there,
+// and stays unless another is 8% ahead by the model.  On the 100 and 56 of them that come here the pick is 2.0% and 4.9% behind
+// the best on average, 20% and 37% at worst; what ran before took 7.1% and 4.6% more than the pick.  us, before -> now: 3059 x 368
 // x 7800 45.8 -> 35.5, 841 x 6176 x 1416 23.8 -> 21.6, 1369 x 957 x 208 7.6 -> 6.1, 4397 x 3888 x 280 24.2 -> 23.0.
 LineChoice nn_off_lines_tile(int M, int N, int K, const beam_tile_cfg& named, int cus) {
   struct Candidate {
@@ -1434,9 +1435,10 @@ static int ln_resolve_cfg(const beam_tile_cfg* cfg, int M, int N, int K, int mod
 
 // The one-kernel form among all tiles, those whose fills take whole lines (gemm_kernel.h: Form) included, for rows on 16 bytes;
 // `named` is ln_choose_tile's.  The model above with constants for rows on 128-byte lines and off them: TFLOP/s per CU, us per
-// round of bands and per launch, least squares on the logarithm over 160 and 200 shapes with M from 64 to 8192, N and K from 256 to 8192.
-// `named` stays unless another tile is 4% ahead by it.  Its pick is 1.8% (off lines) and 3.3% (on) behind the best tile on
-// average, `named` 12 and 11%; the tiles with rings deeper than 3 + 2 slots are ahead on lines too.  us, before -> now: 1978 x 2120 x
+// round of bands and per launch, least squares on the logarithm over 200 shapes off lines and 160 on them with M from 64 to 8192, N and K
+// from 256 to 8192 (beam/line_tile_fit.py, with the timings).  `named` stays unless another tile is 4% ahead by it.  On the 145 and 115 of them
+// that come here the pick is 1.9% (off lines) and 3.4% (on) behind the best tile on average, 46% and 28% at worst; what ran before
+// took 11% and 9% more than the pick.  The tiles with rings deeper than 3 + 2 slots are ahead on lines too.  us, before -> now: 1978 x 2120 x
 // 4888 86 -> 59 (48 with bands in groups), 2908 x 328 x 5736 51 -> 33, 1891 x 920 x 3704 40 -> 28, 6257 x 2744 x 4688 243 -> 196; on lines 1064 x 1040 x
 // 3776 42 -> 29, 126 x 6720 x 1472 21.6 -> 19.0.
 static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) {

@@ -2,6 +2,7 @@
 the split heuristic, workspace sizes, the synthetic-data generator and argument validation."""
 import ctypes
 import os
+import re
 
 import numpy as np
 import pytest
@@ -637,3 +638,40 @@ def test_tile_map_with_multipliers_is_the_map_with_divisions(beamc):
                 assert L.beam_dbg_tile_of_workgroup(wg, tiles_m, tiles_n, g, ctypes.byref(tm), ctypes.byref(tn)) == 0
                 assert L.beam_dbg_tile_of_workgroup_by_division(wg, tiles_m, tiles_n, g, ctypes.byref(um), ctypes.byref(un)) == 0
                 assert (tm.value, tn.value) == (um.value, un.value), (tiles_m, tiles_n, g, wg)
+
+
+def test_line_tile_models_come_from_their_timings(beamc):
+    """The three models that choose among all tiles, whole-line fills included (beam/line_tile_fit.py): the constants compiled in are
+    what the fit gives on the committed timings (by the times that they predict: 1%), and the library's picks are as far behind the
+    best tile there as its comments say."""
+    from beam import line_tile_fit as fit
+    L = beamc.lib
+    source = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "general-nvgpu-testing_amd", "csrc", "capi.hip")).read()
+
+    def compiled(function, values):
+        out, body = {}, source[source.index(f"LineChoice {function}("):]
+        for line in body[:body.index("  };\n  ", body.index("kCandidates[] = {"))].splitlines():
+            if tile := re.match(r"\s*\{\{(\d+), (\d+), (\d+), (\d+), (\d), 0\}, (true|false), (.*)\},", line):
+                bm, bn, wm, wn, pipe, lines, rest = tile.groups()
+                name = f"{bm}x{bn}_lines" if lines == "true" else f"{bm}x{bn}_w{wm}x{wn}" + ("_deep" if pipe == "2" else "")
+                out[name] = values([float(x) for x in re.findall(r"[\d.]+", rest)])
+        return out
+
+    constants = {"gemmrc": compiled("off_lines_tile", lambda v: v[1:]), "nn_whole": compiled("nn_off_lines_tile", lambda v: v[1::2]),
+                 "nn_odd": compiled("nn_off_lines_tile", lambda v: v[2::2]), "ln_off": compiled("ln_line_tile", lambda v: v[0::2]),
+                 "ln_on": compiled("ln_line_tile", lambda v: v[1::2])}
+    # (pick to best: geometric mean, worst; before to pick)
+    said = {"gemmrc": (1.011, 1.179, 1.140), "nn_whole": (1.020, 1.196, 1.071), "nn_odd": (1.049, 1.374, 1.046), "ln_off": (1.019, 1.464, 1.112),
+            "ln_on": (1.034, 1.277, 1.094)}
+    try:
+        L.beam_dbg_assume_compute_units(256)
+        for table, (columns, rows) in fit.load().items():
+            for c in (c for c in columns if "_not_built" not in c):
+                refit, own = fit.fit(table, c, rows), constants[table][c]
+                for M, N, K, _, t in rows:
+                    us = fit.model(table, c, M, N, K)
+                    assert c not in t or abs(us(own) / us(refit) - 1) < 0.01, (table, c, own, refit)
+            mean, worst, ahead, n = fit.regret(table, rows)
+            assert all(abs(x - y) < 0.003 for x, y in zip((mean, worst, ahead), said[table])), (table, mean, worst, ahead, n)
+    finally:
+        L.beam_dbg_assume_compute_units(0)
