@@ -63,10 +63,14 @@ std::mutex g_dev_mu;
 unsigned* g_ln_host_timeout = nullptr;
 
 // Sets of words of pinned host memory, a word for each XCD in a 64-byte line of its own, through which a kernel at a stream's end
-// tells a waiting thread that it has come there (wait_for_stream).  Allocated with the word above; a call holds a set while it
-// waits, and without a free one waits as hipStreamSynchronize does.
+// tells a waiting thread that it has come there, and an event for each (wait_for_stream).  The words are allocated with the word
+// above; a call holds a set while it waits, and without a free one waits as hipStreamSynchronize does.
 constexpr int kWaitSets = 64;
 unsigned* g_wait_words = nullptr;
+struct WaitEvent {
+  hipEvent_t event = nullptr;
+  int device = -1;
+} g_wait_events[kWaitSets];
 std::atomic<unsigned long long> g_wait_free{~0ull};
 std::atomic<unsigned> g_wait_value{0};
 
@@ -81,10 +85,30 @@ void give_wait_set(int i) { g_wait_free.fetch_or(1ull << i, std::memory_order_re
 // Waits until everything that `st` holds has run and the host sees what it wrote; not for a stream that is being captured, and
 // only on a device of kNumXcd XCDs.  hipStreamSynchronize puts a packet behind the last kernel that writes caches back for the
 // host and raises a signal; a kernel of a wavefront on each XCD whose words this thread watches is 3 us shorter (a checked
-// GEMM+LayerNorm of 512 x 1024 x 1024 18.4 -> 15.4 us).  The stream's kernels run one after another, and a wavefront's store is
+// GEMM+LayerNorm of 512 x 1024 x 1024 18.4 -> 15.4 us, without the event).  The stream's kernels run one after another, and a wavefront's store is
 // a release that writes back its XCD's L2: with all XCDs heard, nothing that the kernels in front wrote is left in an L2, be it
 // for memory of the device or of the host.  (One wavefront on one XCD, 15.2 us, says so of that XCD's L2 only.  Eight words in
 // one line, written and watched at once, 16.4 to 17.9.)  Long waits, and an XCD without a workgroup, are left to the runtime.
+// The event behind that kernel, recorded while the stream works, is for the runtime: it would otherwise find kernels whose end it
+// has not heard of, and put a packet of its own behind them when the caller synchronises or copies next.  us of the call and
+// what follows, by hipStreamSynchronize, watched without the event, with it: the next such call 19.1, 15.7, 16.8; another
+// product 22.6, 19.0, 21.1; hipDeviceSynchronize 22.3, 27.2, 21.2; a copy to the host and hipDeviceSynchronize 49.1, 52.9, 49.3.
+void record_wait_event(WaitEvent* e, hipStream_t st) {
+  int device = -1;
+  if (hipGetDevice(&device) != hipSuccess) return;
+  if (e->device != device) {  // (an event belongs to a device)
+    if (e->event) (void)hipEventDestroy(e->event);
+    *e = WaitEvent();
+    if (hipEventCreateWithFlags(&e->event, hipEventDisableTiming) != hipSuccess) {
+      e->event = nullptr;
+      (void)hipGetLastError();
+      return;
+    }
+    e->device = device;
+  }
+  if (hipEventRecord(e->event, st) != hipSuccess) (void)hipGetLastError();
+}
+
 hipError_t wait_for_stream(hipStream_t st) {
   const int i = g_wait_words ? take_wait_set() : -1;
   if (i < 0) return hipStreamSynchronize(st);
@@ -92,6 +116,7 @@ hipError_t wait_for_stream(hipStream_t st) {
   const unsigned value = g_wait_value.fetch_add(1, std::memory_order_relaxed) + 1;
   int told = 0;  // XCDs
   if (launch_tell_host(words, value, st) == hipSuccess) {
+    record_wait_event(&g_wait_events[i], st);
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
     do {
       for (int spin = 0; spin < 32; ++spin) {

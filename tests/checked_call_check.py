@@ -1,10 +1,12 @@
 """Run by test_gpu_ln.py in a process of its own: when a checked GEMM+LayerNorm returns, its result is there for a copy on another
 stream that does not wait for this one's, and in host memory for the calling thread, however long the stream's earlier work keeps
-the call waiting.  The same steps without the check find the old contents, so nothing else orders the copy."""
+the call waiting.  The same steps without the check find the old contents, so nothing else orders the copy.  And what the call
+saves is not left to whoever synchronises behind it."""
 import ctypes
 import os
 import sys
 import threading
+import time
 
 import torch
 
@@ -84,6 +86,29 @@ for c in callers:
     for fronts in (0, 1):
         y = torch.full(c.y.shape, float("nan"), dtype=BF16, pin_memory=True)
         assert not c.launch(y, fronts, True) and same(y, c.want), (c.shape, fronts)
+
+# A caller that synchronises behind the call pays what one does whose call has synchronised by itself (1.06 times it; without the
+# event that the wait records 1.24)
+M, N, K = 512, 1024, 1024
+c = Caller(M, N, K, 9)
+args = [t.data_ptr() for t in (c.a, c.b, c.gamma, c.beta)] + [ctypes.c_float(1e-5), c.y.data_ptr(), M, N, K, _C.BF16, None]
+ws, fell_back = (c.ws.data_ptr(), c.ws.numel()), ctypes.c_int()
+took = ([], [])
+for _ in range(220):
+    t0 = time.perf_counter()
+    _C._check(L.beam_gemmrc_ln_checked(*args, *ws, None, ctypes.byref(fell_back)))
+    _C._check(L.beam_sync(None))
+    t1 = time.perf_counter()
+    _C._check(L.beam_gemmrc_ln_ex(*args, _C.LN_AUTO, *ws, None))
+    _C._check(L.beam_sync(None))
+    _C._check(L.beam_sync(None))
+    took[0].append(t1 - t0)
+    took[1].append(time.perf_counter() - t1)
+    assert not fell_back.value
+checked, parts = (sorted(t[20:])[100] * 1e6 for t in took)
+print(f"{c.shape}: checked and synchronised {checked:.1f} us, synchronised twice {parts:.1f} us", flush=True)
+assert checked <= 1.15 * parts, (checked, parts)
+torch.cuda.synchronize()
 
 bad = []
 
