@@ -129,6 +129,7 @@ struct GemmParams {
                  // -1: band after band, workgroup id = band * tiles_n + column (no padding); less: band_group_tile
   int ln_ids;    // fused LayerNorm on the kernel of gemm_w4.h: ids of that order, padding included; the grid may be smaller
                  // (a workgroup then walks the ids blockIdx, blockIdx + gridDim, ...)
+  int c_store;   // StoreKind of the 16-bit epilogues other than kEpiStoreLoop's (here, in a line of the arguments that every launch reads)
   TileDivs divs; // the tile maps' divisors as multipliers (tile_map.h), made by the host from tiles_m, tiles_n, group_m
   // Side job (kEpiStoreSide): y[i] = silu(x[i]) over a flat 16-bit array.  The whole 8-element
   // groups of the array are cut into units of side_width bytes (16, 8 or 4), dealt out in
@@ -141,7 +142,6 @@ struct GemmParams {
   int side_iters;        // K tiles' worth of units per workgroup
   int side_width;        // bytes per unit
   int c_streaming;       // kEpiStoreLoop: store C non-temporal
-  int c_store;           // StoreKind of the other 16-bit epilogues
   // kEpiPartialFused: word kSkTimeout, then from word kSkFlags on one flag per (tile, part of the tile, slice);
   // behind the partial sums in the caller's workspace.  Never has to be initialised (see sk_launch_tag).
   int* sk_sync;
