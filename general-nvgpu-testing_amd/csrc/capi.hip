@@ -651,7 +651,7 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
 // there (only rows of whole lines that start behind one stay as choose_default has them).  The cost model of choose_default with constants of its own, since the straight tiles' rates are lower on such rows:
 // TFLOP/s per CU alone and with `occ` workgroups on the CU, us per round of workgroups and per launch, least squares on the logarithm over 280 shapes with M, N from 64
 // to 8192 and K from 64 to 8192 off lines (beam/line_tile_fit.py, with the timings).  On the 241 of them that come here its pick is
-// 1.1% behind the best of these on average, 18% at worst; what ran before took 14% more than the pick.  us, before -> now: 928 x 1232 x 7112 49.7 -> 27.9, 633 x
+// 0.9% behind the best of these on average, 16% at worst; what ran before took 14% more than the pick.  us, before -> now: 928 x 1232 x 7112 49.7 -> 27.9, 633 x
 // 6536 x 2952 38.5 -> 26.3, 1228 x 1784 x 6296 59.4 -> 36.9, 7702 x 7248 x 2472 268 -> 255, 2247 x 3736 x 216 12.7 -> 10.3.
 struct LineChoice {
   beam_tile_cfg cfg;
@@ -687,8 +687,9 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
       {{160, 128, 80, 64, 2, 0}, true, 1, 6.07, 6.07, 4.35, 0.89},
       {{192, 128, 96, 64, 2, 0}, true, 1, 6.45, 6.45, 6.58, 0.26},
   };
-  // What choose_default names stays unless another is 4% ahead by this model (639 x 1648 x 272 in 64 x 64 tiles 4.4 us, its
-  // best, 96 x 64, 4.9).
+  // What choose_default names stays unless another is 4% ahead by this model; 64 x 64 tiles of at most two to a CU under a sum of up
+  // to five K tiles, where the model is off by as much as its picks are ahead, unless 15% (639 x 1648 x 272 in 64 x 64 tiles 4.5 us, its
+  // best, 96 x 64 by lines, 4.8; 961 x 1400 x 216 4.5, 4.7; 321 x 3536 x 240 4.3, 4.5; but 559 x 2752 x 264 5.0, in 128 x 64 4.5).
   beam_tile_cfg named;
   int split;
   if (choose_default(M, N, K, -1, &named, &split) != BEAM_OK) named = kCandidates[0].cfg;
@@ -704,7 +705,8 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
     if (!best || us < best_us) best = &k, best_us = us;
     if (!k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline) stays = &k, stays_us = us;
   }
-  if (stays && best_us > 0.96 * stays_us) best = stays;
+  const bool short_sum = K < 320 && named.block_m * named.block_n == 64 * 64 && (long)((M + 63) / 64) * ((N + 63) / 64) <= 2L * cus;
+  if (stays && best_us > (short_sum ? 0.85 : 0.96) * stays_us) best = stays;
   LineChoice t = {best->cfg, best->lines};
   t.cfg.group_m = default_group_m(t.cfg.block_m, t.cfg.block_n);
   return t;
