@@ -701,7 +701,12 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
     const long conc = load < k.occ ? load : k.occ;
     const double rate = k.occ == 1 ? k.alone : k.alone + (k.full - k.alone) * (double)(conc - 1) / (k.occ - 1);
     const double mflop = 2.0e-6 * k.cfg.block_m * k.cfg.block_n * (double)(((long)K + kBK - 1) / kBK * kBK);
-    const double us = (double)((load + k.occ - 1) / k.occ) * k.round + (double)load * mflop / rate + k.launch;
+    double us = (double)((load + k.occ - 1) / k.occ) * k.round + (double)load * mflop / rate + k.launch;
+    // (From 192 x 128 on, a round that nearly fills the chip moves its operands at the fabric's rate: on 159 shapes 192 x 128 tiles by
+    // lines take 0.93 of the model's time with 180 tiles, 1.0 with 204, 1.1 with 240, 1.15 to 1.4 with 252, and 256 x 128 ones
+    // alike.  1422 x 4040 x 528 by lines 17.0 us, in 256 x 128 tiles 11.9; 3629 x 1624 x 504 16.0, 11.9; on those shapes the picks
+    // are 1.0% behind the best with this term and 1.7% without it.)
+    if (load == 1 && k.cfg.block_m * k.cfg.block_n >= 192 * 128 && tiles > 0.75 * cus) us *= 1 + 0.6 * ((double)tiles / cus - 0.75);
     if (!best || us < best_us) best = &k, best_us = us;
     if (!k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline) stays = &k, stays_us = us;
   }
