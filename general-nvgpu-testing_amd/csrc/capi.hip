@@ -705,10 +705,12 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
     // (From 192 x 128 on, a round that nearly fills the chip moves its operands at the fabric's rate: on 159 shapes 192 x 128 tiles by
     // lines take 0.93 of the model's time with 180 tiles, 1.0 with 204, 1.1 with 240, 1.15 to 1.4 with 252, and 256 x 128 ones
     // alike.  1422 x 4040 x 528 by lines 17.0 us, in 256 x 128 tiles 11.9; 3629 x 1624 x 504 16.0, 11.9; on those shapes the picks
-    // are 1.0% behind the best with this term and 1.7% without it.)
-    if (load == 1 && k.cfg.block_m * k.cfg.block_n >= 192 * 128 && tiles > 0.75 * cus) us *= 1 + 0.6 * ((double)tiles / cus - 0.75);
+    // are 0.9% behind the best with this term and 1.7% without it.  Not on the tile that is named, since what would take its place in
+    // two rounds is slowed by as much: 6645 x 1584 x 4192 in 245 tiles of 192 x 256 97, in 455 by lines 103.)
+    const bool is_named = !k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline;
+    if (!is_named && load == 1 && k.cfg.block_m * k.cfg.block_n >= 192 * 128 && tiles > 0.75 * cus) us *= 1 + 0.6 * ((double)tiles / cus - 0.75);
     if (!best || us < best_us) best = &k, best_us = us;
-    if (!k.lines && k.cfg.block_m == named.block_m && k.cfg.block_n == named.block_n && k.cfg.pipeline == named.pipeline) stays = &k, stays_us = us;
+    if (is_named) stays = &k, stays_us = us;
   }
   const bool short_sum = K < 320 && named.block_m * named.block_n == 64 * 64 && (long)((M + 63) / 64) * ((N + 63) / 64) <= 2L * cus;
   if (stays && best_us > (short_sum ? 0.85 : 0.96) * stays_us) best = stays;

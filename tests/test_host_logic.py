@@ -680,7 +680,7 @@ def test_line_tile_models_come_from_their_timings(beamc):
 @pytest.mark.parametrize("shape,tile", [((639, 1648, 272), (64, 64)), ((961, 1400, 216), (64, 64)), ((300, 4080, 312), (64, 64)),
                                         ((2131, 2112, 168), (160, 128)), ((1024, 4424, 304), (160, 128)), ((3559, 376, 328), (96, 64)),
                                         ((1422, 4040, 528), (256, 128)), ((3629, 1624, 504), (256, 128)), ((4400, 1352, 520), (256, 128)),
-                                        ((760, 6536, 1096), (192, 128)), ((1400, 4000, 2008), (192, 128))])
+                                        ((760, 6536, 1096), (192, 128)), ((1400, 4000, 2008), (192, 128)), ((6645, 1584, 4192 - 8), (192, 256))])
 def test_lines_of_the_choice_off_lines(beamc, shape, tile):
     """Rows off lines.  Up to five K tiles and at most two 64 x 64 tiles for every CU: those tiles run, as measured; whole-line tiles
     behind that line and in place of larger ones.  A round of 192 x 128 tiles that nearly fills the chip runs in 256 x 128 tiles
@@ -691,4 +691,4 @@ def test_lines_of_the_choice_off_lines(beamc, shape, tile):
         beamc._check(beamc.lib.beam_dbg_off_lines_tile(*shape, ctypes.byref(cfg), ctypes.byref(lines)))
     finally:
         beamc.lib.beam_dbg_assume_compute_units(0)
-    assert (cfg.block_m, cfg.block_n) == tile and lines.value == (tile not in ((64, 64), (256, 128)))
+    assert (cfg.block_m, cfg.block_n) == tile and lines.value == (tile not in ((64, 64), (256, 128), (192, 256)))
