@@ -655,7 +655,8 @@ KwPlan kw_plan(int M, int N, int K, bool b_kmajor, bool ln, bool gemm, RowStarts
 // 6536 x 2952 38.5 -> 26.3, 1228 x 1784 x 6296 59.4 -> 36.9, 7702 x 7248 x 2472 268 -> 255, 2247 x 3736 x 216 12.7 -> 10.3.
 struct LineChoice {
   beam_tile_cfg cfg;
-  bool lines;  // cfg is a tile of launch_gemm_lines
+  bool lines;        // cfg is a tile of launch_gemm_lines
+  double ahead = 0;  // us of what choose_default names beyond cfg's, by the model; off_lines_tile
 };
 LineChoice off_lines_tile(int M, int N, int K, int cus) {
   struct Candidate {
@@ -714,7 +715,7 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
   }
   const bool short_sum = K < 320 && named.block_m * named.block_n == 64 * 64 && (long)((M + 63) / 64) * ((N + 63) / 64) <= 2L * cus;
   if (stays && best_us > (short_sum ? 0.85 : 0.96) * stays_us) best = stays;
-  LineChoice t = {best->cfg, best->lines};
+  LineChoice t = {best->cfg, best->lines, best == stays ? 0 : stays ? stays_us - best_us : 1e9};
   t.cfg.group_m = default_group_m(t.cfg.block_m, t.cfg.block_n);
   return t;
 }
@@ -1118,8 +1119,18 @@ int beam_parallel_gemmrc_silu(const void* A, const void* B, void* C, int M, int 
   //     the earlier ones' passes: 5632 x 5632 x 256 in two rounds with 60 Mi (28) 90.5, 73.8; 8192 x 4096 x 256 in two with 64 Mi
   //     (28) 91.8, 83.6, with 32 Mi (12) 51.9, 57.3; 8192 x 8192 x 512 in four with 64 Mi (8) 127.9, 135.0.
   //   * By whole lines, with 2^20 elements or K from 2048 on: 1787 x 2648 x 744 with 38 Mi 73.8, 46.6; 1157 x 3216 x 3880 with
-  //     0.5 Mi 56.0, 33.3; 679 x 3080 x 4880 with 2.3 Mi 46.5, 34.3; but 4155 x 496 x 560 with 0.6 Mi 10.4, 11.8.
-  const bool by_lines = K % kBK != 0 && row_starts(A, B, K, false) == kOnChunks && (count >= (1 << 20) || K >= 2048) && off_lines_tile(M, N, K, cus).lines;
+  //     0.5 Mi 56.0, 33.3; 679 x 3080 x 4880 with 2.3 Mi 46.5, 34.3; but 4155 x 496 x 560 with 0.6 Mi 10.4, 11.8.  Where the job
+  //     ends inside the loop it is nearly free beside tiles of eight wavefronts, and the lines have to be ahead by 0.4 of what
+  //     it takes alone (1908 x 4584 x 3552 with 24 Mi, 5 us ahead, 75.0, 92.4; 1539 x 3648 x 3112 with 20 Mi, 2.6, 62.3, 67.7; but
+  //     1653 x 5272 x 4128 with 10 Mi, 6.7, 99.4, 92.6); by 1.1 us under a sum of up to seven K tiles (931 x 608 x 392 with 1.1 Mi,
+  //     0.2 us ahead, 7.0, 8.0; 557 x 2472 x 376 with 2.1 Mi, 0.8, 9.4, 10.0; but 2115 x 456 x 392 with 3.7 Mi behind the loop 14.8, 10.1).
+  bool by_lines = false;
+  if (K % kBK != 0 && row_starts(A, B, K, false) == kOnChunks && (count >= (1 << 20) || K >= 2048)) {
+    const LineChoice t = off_lines_tile(M, N, K, cus);
+    const double alone = 2.5 + 0.7 * (double)count / (1 << 20);  // us
+    const double least = p.side_iters > k_tiles ? 0 : ks->threads == 512 ? 0.4 * alone : k_tiles <= 7 ? 1.1 : 0;
+    by_lines = t.lines && t.ahead > least;
+  }
   const long long behind = (ks->threads == 512 ? 8 * ((wgs + cus - 1) / cus) : 4) + k_tiles / 8;
   if (!cfg && (by_lines || p.side_iters - k_tiles > behind)) {
     if ((rc = beam_gemmrc(A, B, C, M, N, K, dtype, nullptr, stream))) return rc;
