@@ -722,7 +722,7 @@ LineChoice off_lines_tile(int M, int N, int K, int cus) {
 
 // The same for beam_matmul_nn, where only rows of A can be off lines for K's sake: whole chunks in B's rows (N % 8 == 0), and not.
 // Fitted to 120 and 90 shapes with M and N from 32 and 64 to 8192 (5001); `named` is what choose_default's tile has become there,
-// and stays unless another is 8% ahead by the model.  On the 100 and 56 of them that come here the pick is 2.0% and 4.9% behind
+// and stays unless another is 8% ahead by the model.  On the 100 and 56 of them that come here the pick is 2.1% and 4.9% behind
 // the best on average, 20% and 37% at worst; what ran before took 7.1% and 4.6% more than the pick.  us, before -> now: 3059 x 368
 // x 7800 45.8 -> 35.5, 841 x 6176 x 1416 23.8 -> 21.6, 1369 x 957 x 208 7.6 -> 6.1, 4397 x 3888 x 280 24.2 -> 23.0.
 LineChoice nn_off_lines_tile(int M, int N, int K, const beam_tile_cfg& named, int cus) {
@@ -771,7 +771,10 @@ LineChoice nn_off_lines_tile(int M, int N, int K, const beam_tile_cfg& named, in
     if (!best || us < best_us) best = &k, best_us = us;
     if (is_named) stays = &k, stays_us = us;
   }
-  if (stays && best_us > 0.92 * stays_us) return LineChoice{named, false};
+  // (13% under a short sum, as in off_lines_tile, of 64 x 128 by lines a little longer: 1327 x 1320 x 264 in 64 x 64 tiles 5.9 us, by lines 6.1; 235
+  // x 2872 x 272 4.4, 4.7; 401 x 3912 x 336 6.2, 6.5.)
+  const bool short_sum = !odd && (K < 312 || (K < 350 && best->lines && best->cfg.block_m == 64 && best->cfg.block_n == 128));
+  if (stays && best_us > (short_sum ? 0.87 : 0.92) * stays_us) return LineChoice{named, false};
   LineChoice t = {best->cfg, best->lines};
   t.cfg.group_m = default_group_m(t.cfg.block_m, t.cfg.block_n);
   return t;
