@@ -1548,14 +1548,28 @@ static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) 
 // 3959 x 419 x 424 13.9 -> 10.9, over 150 shapes 5%.  Where little is filled into LDS in all (7 Mi elements, under a short sum 12)
 // the fabric is no bound, and a few instructions in front of the first load are 0.1 us (28 x 264 x 3008 6.1, 6.2; 2464 x 416 x
 // 256 8.6, 8.8); nor is it for two bands of the larger tiles (84 x 5128 x 2264 20.5, 20.9).
-static int band_group(int M, int N, int K, int rows, int cols) {
+//
+// More tiles than the device holds at once: the workgroups of the group that a round cuts wait for the next one, each on its CU,
+// and a longer group has more of them.  506 tiles of 224 x 256 over 256 CUs (4767 x 5736) are two rounds band after band (22 of 23: 3 wait,
+// 253 start) and three in groups of two (26 wait).  So groups no longer than take the rounds of plain ids.  us in three sets of
+// operands, plain ids, G = 1, 2 (4): 4755 x 5384 x 1368 84.2, 82.0, 112.9; 3283 x 6480 x 680 53.6, 51.1, 70.7; 6539 x 4352 x 1440 92.0, 83.8, 109.5;
+// 7779 x 3496 x 256 44.6, 42.3, 43.7 (60.0); with the same rounds 6201 x 4672 x 2024 124.7, 117.5, 114.7.  Over 479 shapes of more than
+// 256 tiles the choice was 5.6% behind the best G on average and 42% at worst, and is 0.2% and 3%.
+static int order_rounds(int tiles, int group, int slots) {
+  int rounds = 0, waiting = 0;
+  for (int done = 0; done < tiles; ++rounds, waiting = done % group) done += std::max(1, slots - waiting);
+  return rounds;
+}
+// slots: workgroups that the device holds at once.
+static int band_group(int M, int N, int K, int rows, int cols, int slots) {
   const int tiles_m = (M + rows - 1) / rows, tiles_n = (N + cols - 1) / cols;
   if (tiles_m < (rows * cols > 64 * 64 ? 3 : 2) || (double)tiles_m * tiles_n * (rows + cols) * K < (K < 1024 ? 12e6 : 7e6)) return -1;
+  const int rounds = order_rounds(tiles_m * tiles_n, tiles_n, slots);
   double most = 0.8 * (8.0 * M + (tiles_n % 8 ? 8.0 : 1.0) * N);
   int order = -1;
   for (int lg = 0; lg <= 3 && (1 << lg) <= tiles_m && (lg == 0 || tiles_n << lg <= 64); ++lg) {
     const double fetched = (8.0 * M) / (1 << lg) + (double)N * (1 << lg);
-    if (fetched <= most) order = -2 - lg, most = fetched;
+    if (fetched <= most && order_rounds(tiles_m * tiles_n, tiles_n << lg, slots) <= rounds) order = -2 - lg, most = fetched;
   }
   return order;
 }
@@ -1799,7 +1813,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     kw.shift = kw_plan(M, N, K, false, true, false, row_starts(A, B, K, false), g_dev.cus).shift;
     KwLnParams p;
     kw_params(&p, kw, A, B, Y, M, N, K);
-    p.divs = band_order_divs(p.tiles_n, 1, p.tiles_n <= kKwLnShortBand ? -1 : band_group(M, N, K, kw.rows, kw.cols));
+    p.divs = band_order_divs(p.tiles_n, 1, p.tiles_n <= kKwLnShortBand ? -1 : band_group(M, N, K, kw.rows, kw.cols, p.tiles_m * p.tiles_n));
     if (capturing != hipStreamCaptureStatusNone) BEAM_HIP(launch_ln_replay_bump((int*)ws, st));
     char* sets = (char*)ws + ln_fused_header_bytes();
     p.stats = (float*)sets;
@@ -1861,7 +1875,9 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     const int rounds_grouped = whole_bands ? (p.tiles_m + kNumXcd * bx - 1) / (kNumXcd * bx) : rounds_spread;
     const long per_xcd = ((long)p.tiles_m * p.tiles_n + kNumXcd - 1) / kNumXcd;
     if ((per_xcd + 31) / 32 < rounds_grouped) {
-      p.group_n = band_group(M, N, K, c.block_m, c.block_n);
+      // (the tiles by whole lines and those of gemm_w4.h are alone on their CU)
+      const int per_cu = plan.lines || plan.w4 ? 1 : kLdsBytes / (c.pipeline ? ks->lds_bytes_shallow : ks->lds_bytes);
+      p.group_n = band_group(M, N, K, c.block_m, c.block_n, kNumXcd * 32 * per_cu);
       grid = (unsigned)(p.tiles_m * p.tiles_n);
     } else if (whole_bands) {
       p.group_n = 0;
@@ -2278,7 +2294,7 @@ int beam_dbg_band_block_tile(int wg, int tiles_m, int tiles_n, int gb, int gc, i
 int beam_dbg_band_block_grid(int tiles_m, int gb, int gc) { return band_block_grid(tiles_m, gb, gc); }
 
 int beam_dbg_ln_band_order(int M, int N, int K, int rows, int cols) {
-  return M < 1 || N < 1 || K < 1 || rows < 1 || cols < 1 ? 0 : band_group(M, N, K, rows, cols);
+  return M < 1 || N < 1 || K < 1 || rows < 1 || cols < 1 ? 0 : band_group(M, N, K, rows, cols, kNumXcd * 32 * std::max(1, kLdsBytes / ((3 * rows + 2 * cols) * kRowBytes)));
 }
 int beam_dbg_band_order_tile(int id, int tiles_m, int tiles_n, int group_m, int group_n, int* tm, int* tn) {
   if (tiles_m < 1 || tiles_n < 1 || group_m < 1 || id < 0 || !tm || !tn) return fail(BEAM_ERR_INVALID, "bad band-order query");

@@ -2,6 +2,7 @@
 the split heuristic, workspace sizes, the synthetic-data generator and argument validation."""
 import ctypes
 import os
+import random
 import re
 
 import numpy as np
@@ -638,6 +639,38 @@ def test_tile_map_with_multipliers_is_the_map_with_divisions(beamc):
                 assert L.beam_dbg_tile_of_workgroup(wg, tiles_m, tiles_n, g, ctypes.byref(tm), ctypes.byref(tn)) == 0
                 assert L.beam_dbg_tile_of_workgroup_by_division(wg, tiles_m, tiles_n, g, ctypes.byref(um), ctypes.byref(un)) == 0
                 assert (tm.value, tn.value) == (um.value, un.value), (tiles_m, tiles_n, g, wg)
+
+
+def band_rounds(L, tiles_m, tiles_n, order, slots):
+    """Rounds of a fused GEMM+LayerNorm whose workgroups start in id order, slots at once, and stay until their band is computed."""
+    todo, left, resident, rounds = 0, {b: tiles_n for b in range(tiles_m)}, [], 0
+    tm, tn = ctypes.c_int(), ctypes.c_int()
+    while todo < tiles_m * tiles_n:
+        new = range(todo, min(todo + slots - len(resident), tiles_m * tiles_n))
+        todo = new.stop
+        for wg in new:
+            assert L.beam_dbg_band_order_tile(wg, tiles_m, tiles_n, 1, order, ctypes.byref(tm), ctypes.byref(tn)) == 0
+            left[tm.value] -= 1
+            resident.append(tm.value)
+        resident = [b for b in resident if left[b]]
+        rounds += 1
+    return rounds
+
+
+def test_bands_in_groups_take_no_more_rounds_than_plain_ids(beamc):
+    L = beamc.lib
+    # three rounds in groups of two or four bands, two in shorter ones
+    for shape, tile, order in [((4767, 5736, 784), (224, 256), -2), ((6539, 4352, 1440), (224, 256), -2),
+                               ((7779, 3496, 256), (224, 256), -3), ((4010, 4712, 528), (192, 256), -3)]:
+        assert L.beam_dbg_ln_band_order(*shape, *tile) == order, (shape, L.beam_dbg_ln_band_order(*shape, *tile))
+    rng, longer = random.Random(5), 0
+    for _ in range(300):
+        rows, cols = rng.choice([(192, 256), (224, 256), (256, 256), (256, 128)])
+        M, N, K = rng.randint(1200, 8192), rng.randint(512, 8192), rng.randint(256, 4096)
+        tiles_m, tiles_n, order = -(-M // rows), -(-N // cols), L.beam_dbg_ln_band_order(M, N, K, rows, cols)
+        longer += order < -2
+        assert order == -1 or band_rounds(L, tiles_m, tiles_n, order, 256) <= band_rounds(L, tiles_m, tiles_n, -1, 256), (M, N, K, rows, cols, order)
+    assert longer > 100, longer
 
 
 def test_line_tile_models_come_from_their_timings(beamc):
