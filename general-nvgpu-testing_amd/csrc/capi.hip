@@ -1574,6 +1574,50 @@ static int band_group(int M, int N, int K, int rows, int cols, int slots) {
   return order;
 }
 
+// The workgroup order of a GEMM+LayerNorm launch of the tiled kernels: group_m and group_n of band_order_tile, and the grid (returned).
+// per_cu: workgroups that a CU holds at once (one of the tiles by whole lines and of gemm_w4.h's).
+// Band groups: XCD x owns group_n columns of group_m bands; 8 * group_n covers a whole band and
+// group_m * group_n workgroups fit the 32 CUs of an XCD even at one workgroup per CU
+// ... or, when a band is short enough, whole bands per XCD (tile_map.h: band_xcd_tile)
+//     if that fills every XCD, takes no more rounds of workgroups than the spread order and
+//     streams no more operand panels through an XCD's L2 per round (bands + columns it touches;
+//     measured: 16384 x 2048 x 2048, 4 + 8 against 32 + 1 panels, 112 against 120 us;
+//     8192 x 8192 x 4096, 1 + 32 against 8 + 4, 419 against 400 us; 4096^3, 18 either way, 104.1
+//     against 104.8 us)
+// ... or, where those two orders' padding costs rounds of workgroups (20 column tiles are 3 per XCD on
+//     seven XCDs and none on the eighth: 3000 x 5000 x 2000 in 256 x 256 tiles puts 36 workgroups on six
+//     XCDs of 32 CUs), band after band with no padding: id = band * tiles_n + column, which the hardware's
+//     round-robin deals out evenly.
+//     So too with one column per XCD, of which every one fetches all rows and 8 - tiles_n do nothing, where groups of bands
+//     (band_group) fetch less: 3061 x 384 x 1384 in 96 x 64 tiles by whole lines 17.9 -> 10.9 us, 2382 x 432 x 2600 22.5 -> 16.3,
+//     3559 x 920 x 816 in 128 x 128 tiles 17.3 -> 14.8, 5240 x 1688 x 5656 in 192 x 256 117 -> 104; 48 shapes 0.53 to 1.01 of the
+//     time.  (With two columns and more 0.9 to 1.07.)
+// All three keep a band's workgroups together in id order, so a launch that gets only part of the device
+// still finishes band by band.  (The plain kernels' raster order streams fewer operand bytes into the L2s
+// when the whole grid is one round -- 4096^3: 204 against 303 MB, in the same time -- but loses exactly that.)
+static unsigned ln_order(GemmParams* p, int M, int N, int K, const beam_tile_cfg& c, bool w4, int per_cu) {
+  p->group_n = (p->tiles_n + kNumXcd - 1) / kNumXcd;
+  p->group_m = 32 / p->group_n;
+  if (p->group_m > p->tiles_m) p->group_m = p->tiles_m;
+  const int bx = p->tiles_n <= 32 ? 32 / p->tiles_n : 0;
+  const int rounds_spread = (p->tiles_m + p->group_m - 1) / p->group_m;
+  const bool whole_bands = bx > 0 && p->tiles_m >= kNumXcd * bx && (p->tiles_m + kNumXcd * bx - 1) / (kNumXcd * bx) <= rounds_spread &&
+                           bx + p->tiles_n <= p->group_m + p->group_n;
+  const int rounds_grouped = whole_bands ? (p->tiles_m + kNumXcd * bx - 1) / (kNumXcd * bx) : rounds_spread;
+  const long per_xcd = ((long)p->tiles_m * p->tiles_n + kNumXcd - 1) / kNumXcd;
+  const int bands_grouped = band_group(M, N, K, c.block_m, c.block_n, kNumXcd * 32 * per_cu);
+  if ((per_xcd + 31) / 32 < rounds_grouped || (p->group_n == 1 && !whole_bands && !w4 && bands_grouped < -1)) {
+    p->group_n = bands_grouped;
+    return (unsigned)(p->tiles_m * p->tiles_n);
+  }
+  if (whole_bands) {
+    p->group_n = 0;
+    p->group_m = bx;
+    return (unsigned)band_xcd_grid(p->tiles_m, p->tiles_n, bx);
+  }
+  return (unsigned)band_block_grid(p->tiles_m, p->group_m, p->group_n);
+}
+
 // What a GEMM+LayerNorm call does and the workspace it needs: one function, so that the entry point and the
 // workspace queries cannot disagree.
 //   plain     the problem is outside what the tiled kernels take (K below 8 or beyond a descriptor, gamma or beta not
@@ -1849,43 +1893,7 @@ int beam_gemmrc_ln_ex(const void* A, const void* B, const void* gamma, const voi
     p.beta = beta;
     p.eps = eps;
     p.spin_limit = g_ln_spin_limit.load();
-    // band groups: XCD x owns group_n columns of group_m bands; 8 * group_n covers a whole band and
-    // group_m * group_n workgroups fit the 32 CUs of an XCD even at one workgroup per CU
-    // ... or, when a band is short enough, whole bands per XCD (tile_map.h: band_xcd_tile)
-    //     if that fills every XCD, takes no more rounds of workgroups than the spread order and
-    //     streams no more operand panels through an XCD's L2 per round (bands + columns it touches;
-    //     measured: 16384 x 2048 x 2048, 4 + 8 against 32 + 1 panels, 112 against 120 us;
-    //     8192 x 8192 x 4096, 1 + 32 against 8 + 4, 419 against 400 us; 4096^3, 18 either way, 104.1
-    //     against 104.8 us)
-    // ... or, where those two orders' padding costs rounds of workgroups (20 column tiles are 3 per XCD on
-    //     seven XCDs and none on the eighth: 3000 x 5000 x 2000 in 256 x 256 tiles puts 36 workgroups on six
-    //     XCDs of 32 CUs), band after band with no padding: id = band * tiles_n + column, which the hardware's
-    //     round-robin deals out evenly.
-    // All three keep a band's workgroups together in id order, so a launch that gets only part of the device
-    // still finishes band by band.  (The plain kernels' raster order streams fewer operand bytes into the L2s
-    // when the whole grid is one round -- 4096^3: 204 against 303 MB, in the same time -- but loses exactly that.)
-    unsigned grid;
-    p.group_n = (p.tiles_n + kNumXcd - 1) / kNumXcd;
-    p.group_m = 32 / p.group_n;
-    if (p.group_m > p.tiles_m) p.group_m = p.tiles_m;
-    const int bx = p.tiles_n <= 32 ? 32 / p.tiles_n : 0;
-    const int rounds_spread = (p.tiles_m + p.group_m - 1) / p.group_m;
-    const bool whole_bands = bx > 0 && p.tiles_m >= kNumXcd * bx && (p.tiles_m + kNumXcd * bx - 1) / (kNumXcd * bx) <= rounds_spread &&
-                             bx + p.tiles_n <= p.group_m + p.group_n;
-    const int rounds_grouped = whole_bands ? (p.tiles_m + kNumXcd * bx - 1) / (kNumXcd * bx) : rounds_spread;
-    const long per_xcd = ((long)p.tiles_m * p.tiles_n + kNumXcd - 1) / kNumXcd;
-    if ((per_xcd + 31) / 32 < rounds_grouped) {
-      // (the tiles by whole lines and those of gemm_w4.h are alone on their CU)
-      const int per_cu = plan.lines || plan.w4 ? 1 : kLdsBytes / (c.pipeline ? ks->lds_bytes_shallow : ks->lds_bytes);
-      p.group_n = band_group(M, N, K, c.block_m, c.block_n, kNumXcd * 32 * per_cu);
-      grid = (unsigned)(p.tiles_m * p.tiles_n);
-    } else if (whole_bands) {
-      p.group_n = 0;
-      p.group_m = bx;
-      grid = (unsigned)band_xcd_grid(p.tiles_m, p.tiles_n, bx);
-    } else {
-      grid = (unsigned)band_block_grid(p.tiles_m, p.group_m, p.group_n);
-    }
+    const unsigned grid = ln_order(&p, M, N, K, c, plan.w4, plan.lines || plan.w4 ? 1 : kLdsBytes / (c.pipeline ? ks->lds_bytes_shallow : ks->lds_bytes));
     // the band orders' divisors as multipliers (tile_map.h: band_order_divs)
     p.divs = band_order_divs(p.tiles_n, p.group_m, p.group_n);
     if (plan.w4) {
@@ -2295,6 +2303,16 @@ int beam_dbg_band_block_grid(int tiles_m, int gb, int gc) { return band_block_gr
 
 int beam_dbg_ln_band_order(int M, int N, int K, int rows, int cols) {
   return M < 1 || N < 1 || K < 1 || rows < 1 || cols < 1 ? 0 : band_group(M, N, K, rows, cols, kNumXcd * 32 * std::max(1, kLdsBytes / ((3 * rows + 2 * cols) * kRowBytes)));
+}
+int beam_dbg_ln_launch_order(int M, int N, int K, int rows, int cols, int whole_lines, int* group_m, int* group_n) {
+  if (M < 1 || N < 1 || K < 1 || rows < 1 || cols < 1 || !group_m || !group_n) return 0;
+  GemmParams p;
+  p.tiles_m = (M + rows - 1) / rows, p.tiles_n = (N + cols - 1) / cols;
+  if (p.tiles_n > 64) return 0;
+  const beam_tile_cfg c = {rows, cols, 0, 0, 0, 0};
+  const unsigned grid = ln_order(&p, M, N, K, c, false, whole_lines ? 1 : std::max(1, kLdsBytes / ((3 * rows + 2 * cols) * kRowBytes)));
+  *group_m = p.group_m, *group_n = p.group_n;
+  return (int)grid;
 }
 int beam_dbg_band_order_tile(int id, int tiles_m, int tiles_n, int group_m, int group_n, int* tm, int* tn) {
   if (tiles_m < 1 || tiles_n < 1 || group_m < 1 || id < 0 || !tm || !tn) return fail(BEAM_ERR_INVALID, "bad band-order query");

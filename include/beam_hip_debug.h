@@ -104,6 +104,9 @@ int beam_dbg_band_block_grid(int tiles_m, int gb, int gc);
 int beam_dbg_band_order_tile(int id, int tiles_m, int tiles_n, int group_m, int group_n, int* tm, int* tn);
 /* The group_n of the orders without padding that GEMM+LayerNorm runs in with tiles of rows x cols (0: bad argument). */
 int beam_dbg_ln_band_order(int M, int N, int K, int rows, int cols);
+/* The order of a whole GEMM+LayerNorm launch in tiles of rows x cols (not gemm_w4.h's): group_m and group_n as above, returns the
+ * grid, 0 for a bad argument. */
+int beam_dbg_ln_launch_order(int M, int N, int K, int rows, int cols, int whole_lines, int* group_m, int* group_n);
 /* The same for the order that keeps whole bands (bx at a time) on one XCD, used when a band is
  * short enough for it. */
 int beam_dbg_band_xcd_tile(int wg, int tiles_m, int tiles_n, int bx, int* tm, int* tn);

@@ -504,3 +504,24 @@ def test_bands_in_groups(gpu, beamc, oracle, shape):
     ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, BF16)
     for mode in (beamc.LN_AUTO, beamc.LN_FUSED):
         check_ln(oracle, run_ln(beamc, a, b, g, bt, BF16, mode=mode), ref, BF16, f"{shape} mode {mode}")
+
+
+# (M, N, K), the tile and whether by whole lines, the order: 5 to 8 columns, bands left over behind the last group and none
+FEW_COLUMNS = [((2799, 408, 1352), (96, 64), 1, -5), ((2900, 488, 840), (96, 64), 1, -5), ((3722, 624, 808), (128, 128), 0, -5),
+               ((3838, 680, 584), (128, 128), 0, -5), ((3155, 816, 728), (128, 128), 0, -4), ((2728, 927, 856), (96, 128), 1, -4)]
+
+
+@pytest.mark.parametrize("shape,tile,whole_lines,order", FEW_COLUMNS)
+def test_few_columns_go_in_groups_of_bands(gpu, beamc, oracle, shape, tile, whole_lines, order):
+    import ctypes
+    M, N, K = shape
+    cfg, lines, gm, gn = beamc._TileCfg(), ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    beamc._check(beamc.lib.beam_dbg_ln_line_tile(M, N, K, ctypes.byref(cfg), ctypes.byref(lines)))
+    assert (cfg.block_m, cfg.block_n, lines.value) == (*tile, whole_lines)
+    # (a column on each XCD, and XCDs without one, before: group_n = 1 and a padded grid)
+    grid = beamc.lib.beam_dbg_ln_launch_order(M, N, K, *tile, whole_lines, ctypes.byref(gm), ctypes.byref(gn))
+    assert (grid, gn.value) == (-(-M // tile[0]) * -(-N // tile[1]), order)
+    a, b, g, bt = make_ln_inputs(beamc, M, N, K, BF16, 29)
+    ref = oracle.gemmrc_ln(a, b, g, bt, 1e-5, BF16)
+    for mode in (beamc.LN_AUTO, beamc.LN_FUSED):
+        check_ln(oracle, run_ln(beamc, a, b, g, bt, BF16, mode=mode), ref, BF16, f"{shape} mode {mode}")
