@@ -45,7 +45,9 @@ def model(table, column, M, N, K):
     mflop = 2e-6 * bm * bn * (-(-K // 64) * 64)
     if table.startswith("ln"):
         rounds = -(-tiles_m // max(1, CUS // tiles_n))
-        return lambda p: p[2] + rounds * (p[1] + mflop / p[0])
+        # the statistics of a wide band, which every workgroup reads (for the other tiles too the picks are no better)
+        wide = 0.00125 * bm * max(0, tiles_n - 20) if column.endswith("x64_lines") else 0
+        return lambda p: p[2] + rounds * (p[1] + wide + mflop / p[0])
     occ, load = workgroups_on_a_cu(column), -(-tiles_m * tiles_n // CUS)
     share = 0 if occ == 1 else (min(load, occ) - 1) / (occ - 1)
     return lambda p: -(-load // occ) * p[2] + load * mflop / (p[0] + (p[1] - p[0]) * share) + p[3]

@@ -1489,6 +1489,8 @@ static int ln_resolve_cfg(const beam_tile_cfg* cfg, int M, int N, int K, int mod
 // took 11% and 9% more than the pick.  The tiles with rings deeper than 3 + 2 slots are ahead on lines too.  us, before -> now: 1978 x 2120 x
 // 4888 86 -> 59 (48 with bands in groups), 2908 x 328 x 5736 51 -> 33, 1891 x 920 x 3704 40 -> 28, 6257 x 2744 x 4688 243 -> 196; on lines 1064 x 1040 x
 // 3776 42 -> 29, 126 x 6720 x 1472 21.6 -> 19.0.
+// 64 columns make the most column tiles, and a workgroup reads its rows' statistics of all of them: `wide`.  Without it 96 x 64 tiles
+// ran 666 x 2302 x 704 in 14.0 us, 439 x 2984 x 792 in 15.5 and 301 x 3936 x 960 in 24.6; what runs now takes 11.7, 13.4 and 21.4.
 static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) {
   struct Candidate {
     beam_tile_cfg cfg;
@@ -1505,9 +1507,9 @@ static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) 
       {{128, 128, 64, 32, 0, 0}, false, {3.77, 4.50}, {4.72, 4.60}, {4.29, 4.99}},
       {{64, 128, 32, 64, 0, 0}, false, {2.29, 2.59}, {2.04, 2.03}, {5.90, 6.00}},
       {{64, 64, 32, 32, 0, 0}, false, {1.67, 2.10}, {1.00, 1.05}, {6.00, 6.00}},
-      {{96, 64, 48, 32, 2, 0}, true, {3.32, 3.30}, {9.20, 9.03}, {0, 0}},
+      {{96, 64, 48, 32, 2, 0}, true, {3.435, 3.396}, {8.78, 8.436}, {0, 0.369}},
       {{64, 128, 32, 64, 2, 0}, true, {3.70, 3.58}, {9.48, 9.51}, {0, 0}},
-      {{128, 64, 64, 32, 2, 0}, true, {3.55, 3.61}, {10.07, 9.82}, {0, 0}},
+      {{128, 64, 64, 32, 2, 0}, true, {3.673, 3.692}, {9.27, 9.236}, {0.253, 0.1}},
       {{96, 128, 48, 64, 2, 0}, true, {4.52, 4.28}, {11.08, 10.91}, {0, 0}},
       {{128, 128, 64, 64, 2, 0}, true, {5.24, 5.08}, {12.33, 12.32}, {0, 0}},
       {{160, 128, 80, 64, 2, 0}, true, {5.91, 5.77}, {12.13, 12.24}, {0, 0}},
@@ -1528,8 +1530,9 @@ static LineChoice ln_line_tile(int M, int N, int K, const beam_tile_cfg& named) 
       if (resolve_cfg(&t, M, N, K, &c, &ks) || !ln_fused_applies_on(c, *ks, N, kNumXcd * 32)) continue;
     }
     const int bands_per_round = kNumXcd * 32 / tiles_n;
+    const double wide = k.lines && t.block_n == 64 && tiles_n > 20 ? 0.00125 * t.block_m * (tiles_n - 20) : 0;
     const double us = k.launch[on] + (double)((tiles_m + bands_per_round - 1) / bands_per_round) *
-                                         (k.round[on] + 2.0e-6 * t.block_m * t.block_n * (double)(((long)K + kBK - 1) / kBK * kBK) / k.rate[on]);
+                                         (k.round[on] + wide + 2.0e-6 * t.block_m * t.block_n * (double)(((long)K + kBK - 1) / kBK * kBK) / k.rate[on]);
     if (!best || us < best_us) best = &k, best_us = us;
     if (is_named) stays = &k, stays_us = us;
   }

@@ -710,6 +710,19 @@ def test_line_tile_models_come_from_their_timings(beamc):
         L.beam_dbg_assume_compute_units(0)
 
 
+@pytest.mark.parametrize("shape,tile,whole_lines", [((374, 4091, 496), (64, 128), 0), ((666, 2302, 704), (64, 128), 0), ((303, 3945, 720), (64, 128), 1),
+                                                    ((271, 3683, 704), (64, 128), 0), ((1662, 832, 1112), (96, 64), 1), ((408, 3048, 3984), (96, 64), 1)])
+def test_layer_norm_tiles_of_wide_bands(beamc, shape, tile, whole_lines):
+    """96 x 64 tiles by whole lines pay for the statistics of more than 20 column tiles; narrower bands and long sums still run in them."""
+    cfg, lines = beamc._TileCfg(), ctypes.c_int()
+    try:
+        beamc.lib.beam_dbg_assume_compute_units(256)
+        beamc._check(beamc.lib.beam_dbg_ln_line_tile(*shape, ctypes.byref(cfg), ctypes.byref(lines)))
+        assert ((cfg.block_m, cfg.block_n), lines.value) == (tile, whole_lines)
+    finally:
+        beamc.lib.beam_dbg_assume_compute_units(0)
+
+
 @pytest.mark.parametrize("shape,tile", [((639, 1648, 272), (64, 64)), ((961, 1400, 216), (64, 64)), ((300, 4080, 312), (64, 64)),
                                         ((2131, 2112, 168), (160, 128)), ((1024, 4424, 304), (160, 128)), ((3559, 376, 328), (96, 64)),
                                         ((1422, 4040, 528), (256, 128)), ((3629, 1624, 504), (256, 128)), ((4400, 1352, 520), (256, 128)),
